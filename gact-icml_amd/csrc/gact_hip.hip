@@ -69,6 +69,16 @@ __device__ __forceinline__ void row_all_minmax(float& lo, float& hi) {
 __device__ __forceinline__ void row_all_minmax(f16& lo, f16& hi) {
   asm(GACT_DPP_ALL("v_min_f16_dpp", "v_max_f16_dpp") : "+v"(lo), "+v"(hi));
 }
+// The same over each half of the row (8 lanes): the half mirrored, then the lanes of a quad exchanged twice.
+#define GACT_DPP_HALF_STEP(MIN, MAX, CTRL)                                 \
+  MIN " %0, %0, %0 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                \
+  MAX " %1, %1, %1 " CTRL " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void half_row_all_minmax(f16& lo, f16& hi) {
+  asm("s_nop 4\n\t" GACT_DPP_HALF_STEP("v_min_f16_dpp", "v_max_f16_dpp", "row_half_mirror") "s_nop 0\n\t"
+      GACT_DPP_HALF_STEP("v_min_f16_dpp", "v_max_f16_dpp", "quad_perm:[1,0,3,2]") "s_nop 0\n\t"
+      GACT_DPP_HALF_STEP("v_min_f16_dpp", "v_max_f16_dpp", "quad_perm:[2,3,0,1]") "s_nop 1"
+      : "+v"(lo), "+v"(hi));
+}
 // ------------------------------------------------------------------------------------------------
 // Philox4x32.  The key schedule only depends on the seed, so it stays on the scalar unit; each
 // round is two 32x32->64 multiplies and two three-input XORs (v_bitop3_b32, truth table 0x96).
@@ -261,19 +271,24 @@ template <> struct Elem<float> {
   __device__ static __forceinline__ float init_lo() { return 1e30f; }
   __device__ static __forceinline__ float init_hi() { return -1e30f; }
   __device__ static __forceinline__ float from_float(float v) { return v; }
-  // min and max of the whole group, in every lane of the row
-  __device__ static __forceinline__ void group_minmax(const Store& st, float& lo_out, float& hi_out) {
+  // min and max of the lane's chunks K0 .. K1 - 1
+  template <int K0, int K1>
+  __device__ static __forceinline__ void lane_minmax(const Store& st, float& lo_out, float& hi_out) {
     float lo = init_lo(), hi = init_hi();
 #pragma unroll
-    for (int k = 0; k < kQChunks; k++)
+    for (int k = K0; k < K1; k++)
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         lo = __builtin_fminf(lo, st.v[k][e]);
         hi = __builtin_fmaxf(hi, st.v[k][e]);
       }
-    row_all_minmax(lo, hi);
     lo_out = lo;
     hi_out = hi;
+  }
+  // min and max of the whole group, in every lane of the row
+  __device__ static __forceinline__ void group_minmax(const Store& st, float& lo_out, float& hi_out) {
+    lane_minmax<0, kQChunks>(st, lo_out, hi_out);
+    row_all_minmax(lo_out, hi_out);
   }
   __device__ static __forceinline__ void store_codes(uint8_t* p, const uint32_t (&b)[4]) {
     // the reference accumulates in a uint8_t: keep the low 8 bits of every byte
@@ -387,14 +402,14 @@ template <> struct Elem<f16> {
     asm("v_pk_max_f16 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
     return d;
   }
-  // min and max of the whole group, in every lane of the row: packed per-lane min / max from +-inf (the
-  // start values only survive in a lane whose 16 elements are all NaN), the two halves against each other,
-  // then the row reduction
-  __device__ static __forceinline__ void group_minmax(const Store& st, f16& lo_out, f16& hi_out) {
+  // min and max of the lane's chunks K0 .. K1 - 1: packed min / max from +-inf (the start values only survive in a lane
+  // whose elements are all NaN), then the two halves against each other
+  template <int K0, int K1>
+  __device__ static __forceinline__ void lane_minmax(const Store& st, f16& lo_out, f16& hi_out) {
     const f16 inf = (f16)__builtin_inff();
     f16x2 l = {inf, inf}, h = {(f16)-inf, (f16)-inf};
 #pragma unroll
-    for (int k = 0; k < kQChunks; k++)
+    for (int k = K0; k < K1; k++)
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         l = pk_min(l, st.v[k][j]);
@@ -405,9 +420,13 @@ template <> struct Elem<f16> {
         : "=v"(lo) : "v"(l));
     asm("v_max_f16_sdwa %0, %1, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1"
         : "=v"(hi) : "v"(h));
-    row_all_minmax(lo, hi);
     lo_out = lo;
     hi_out = hi;
+  }
+  // min and max of the whole group, in every lane of the row
+  __device__ static __forceinline__ void group_minmax(const Store& st, f16& lo_out, f16& hi_out) {
+    lane_minmax<0, kQChunks>(st, lo_out, hi_out);
+    row_all_minmax(lo_out, hi_out);
   }
   // range is a half operation; the quotient is a double narrowed to float and then to half
   __device__ static __forceinline__ f16 make_scale(f16 lo, f16 hi, int qmax) {
@@ -1596,6 +1615,308 @@ dequantize_kernel(const uint8_t* __restrict__ packed, const typename Elem<T>::St
                                                                                               unit, threadIdx.x % LPU, out);
 }
 
+// ------------------------------------------------------------------------------------------------
+// Groups of 64, 128 and 512 elements (config.group_size), float and half, in one pass each way.
+//
+// Quantize.  Whatever the group size, a row of 16 lanes takes spans of 512 consecutive elements in the layout of
+// quantize_kernel's pairs of groups (two halves of 256, the lane's chunks 16 chunk widths apart), because that is what a
+// block of the fast stream serves: one Philox block per lane and span.  A group is then one, two, four or eight of the
+// lane's chunks - at 64 half elements half a row's chunk, and neighbouring groups sit in the two halves of the row.  Where
+// the 8/BITS groups that share their bytes fill more than a span, two or four rows of the wave share them (ROWS) and OR
+// their bytes together at the end; a row then takes SPR spans.
+//
+// HBM-bound, as the kernels for groups of 256.  Against minimax + scale + pack (three launches, the data read twice and
+// ragged tensors copied to whole groups first): half [16384,1024], 4 bit, groups of 128: 26.7 -> 9.8 us quantize
+// (4.3 TB/s), 11.6 -> 8.7 dequantize; 67 M float elements, 8 bit: quantize 57 us (0.74 of 8 TB/s; groups of 256: 52).
+// ------------------------------------------------------------------------------------------------
+#define GROUPS_SPAN 512
+template <int LANE>
+__device__ __forceinline__ uint32_t quad_bcast_u32(uint32_t v) {   // value of lane LANE of the quad
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, LANE * 0x55, 0xf, 0xf, false);
+}
+// scale of the lane's group G from the lane that divided for it (QUAD: lane G of every quad, else lane G of the row)
+template <int G, bool QUAD>
+__device__ __forceinline__ float groups_bcast(float v) {
+  return QUAD ? __builtin_bit_cast(float, quad_bcast_u32<G & 3>(__builtin_bit_cast(uint32_t, v))) : row_bcast<G>(v);
+}
+template <int G, bool QUAD>
+__device__ __forceinline__ f16 groups_bcast(f16 v) {
+  return QUAD ? __builtin_bit_cast(f16, (uint16_t)quad_bcast_u32<G & 3>((uint32_t)__builtin_bit_cast(uint16_t, v))) : row_bcast<G>(v);
+}
+
+template <typename T, int D, int BITS>
+struct GroupsShape {
+  static constexpr int WPT = 8 / BITS;
+  static constexpr int CH = Elem<T>::kQChunks, W = Elem<T>::kQWidth;
+  static constexpr int CPS = 2 * CH;                                        // chunks of a span per lane
+  static constexpr int GPS = GROUPS_SPAN / D;                               // groups of a span
+  static constexpr bool HALF = D < 16 * W;                                  // a chunk of the row holds two groups
+  static constexpr int GL = HALF ? GPS / 2 : GPS;                           // groups of a span a lane has elements of
+  static constexpr int CPG = CPS / GL;                                      // chunks of a group per lane
+  static constexpr int SPANS = D * WPT > GROUPS_SPAN ? D * WPT / GROUPS_SPAN : 1;   // spans of a unit: whole super-groups
+  static constexpr int ROWS = SPANS < 4 ? SPANS : 4, SPR = SPANS / ROWS;
+  static constexpr int UNIT_GROUPS = SPANS * GPS;
+  static_assert(D == 64 || D == 128 || D == 512, "group sizes of the one-pass kernels");
+};
+
+template <typename T, int D, int BITS, int G>
+__device__ __forceinline__ void groups_lane_minmax(const typename Elem<T>::Store (&v)[2], T& lo, T& hi) {
+  typedef GroupsShape<T, D, BITS> S;
+  constexpr int C0 = G * S::CPG, CH = S::CH;
+  if constexpr (S::CPG <= CH) {
+    Elem<T>::template lane_minmax<C0 % CH, C0 % CH + S::CPG>(v[C0 / CH], lo, hi);
+  } else {   // a group of 512: both halves
+    T lo2, hi2;
+    Elem<T>::template lane_minmax<0, CH>(v[0], lo, hi);
+    Elem<T>::template lane_minmax<0, CH>(v[1], lo2, hi2);
+    lo = lo2 < lo ? lo2 : lo;   // never NaN: the start values are not
+    hi = hi2 > hi ? hi2 : hi;
+  }
+}
+template <typename T, int D, int BITS, int G = 0>
+__device__ __forceinline__ void groups_stats(const typename Elem<T>::Store (&v)[2], T (&lo)[GroupsShape<T, D, BITS>::GL],
+                                             T (&hi)[GroupsShape<T, D, BITS>::GL]) {
+  typedef GroupsShape<T, D, BITS> S;
+  if constexpr (G < S::GL) {
+    groups_lane_minmax<T, D, BITS, G>(v, lo[G], hi[G]);
+    if constexpr (S::HALF) half_row_all_minmax(lo[G], hi[G]);
+    else row_all_minmax(lo[G], hi[G]);
+    groups_stats<T, D, BITS, G + 1>(v, lo, hi);
+  }
+}
+template <typename T, int D, int BITS, int G = 0>
+__device__ __forceinline__ void groups_share_scale(T mine, T (&sc)[GroupsShape<T, D, BITS>::GL]) {
+  typedef GroupsShape<T, D, BITS> S;
+  if constexpr (G < S::GL) {
+    sc[G] = S::GL == 1 ? mine : groups_bcast<G, S::HALF>(mine);
+    groups_share_scale<T, D, BITS, G + 1>(mine, sc);
+  }
+}
+
+template <typename T, int D, int BITS, int NOISE>
+__global__ void __launch_bounds__(64)
+quantize_groups_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_t N, uint8_t* __restrict__ packed,
+                       T* __restrict__ scale_out, T* __restrict__ mn_out, T* __restrict__ mx_out,
+                       const float* __restrict__ noise) {
+  static_assert(NOISE != GACT_NOISE_REF, "the reference stream draws per output byte");
+  typedef GroupsShape<T, D, BITS> S;
+  constexpr int WPT = S::WPT, CH = S::CH, W = S::W, QMAX = (1 << BITS) - 1;
+  const uint32_t tile = gridDim.x - 1u - xcd_tile<GACT_XCD_RUN_Q>(blockIdx.x, gridDim.x);   // last tile first, see quantize_kernel
+  const int row = (int)(threadIdx.x >> 4), i = threadIdx.x & 15;
+  const int64_t unit = (int64_t)tile * (4 / S::ROWS) + row / S::ROWS;
+  const int part = row % S::ROWS;   // the row's share of its unit
+  if (unit * S::UNIT_GROUPS >= N) return;   // all rows of the unit
+  const uint64_t seed = seed_arg.value();
+  const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+  const int half = S::HALF ? i >> 3 : 0;
+
+  typename Elem<T>::Store v[2];
+  uint32_t acc[S::CPG][W];
+#pragma unroll
+  for (int s = 0; s < S::SPR; s++) {
+    const int64_t span = unit * S::SPANS + part * S::SPR + s;
+    load_group<T>(x, numel, span * 2, i, v[0]);
+    load_group<T>(x, numel, span * 2 + 1, i, v[1]);
+    T lo[S::GL], hi[S::GL], sc[S::GL];
+    groups_stats<T, D, BITS>(v, lo, hi);
+    {
+      // one division per lane: lane j of the row (half rows: of every quad) takes the lane group j
+      const int mine = i & (S::GL - 1);
+      T lo_m = lo[0], hi_m = hi[0];
+#pragma unroll
+      for (int g = 1; g < S::GL; g++) {
+        lo_m = mine == g ? lo[g] : lo_m;
+        hi_m = mine == g ? hi[g] : hi_m;
+      }
+      const T s_m = Elem<T>::make_scale(lo_m, hi_m, QMAX);
+      const int64_t n = span * S::GPS + (S::HALF ? 2 * mine + half : mine);
+      if ((S::HALF ? i & 7 : i) < S::GL && n < N) {
+        scale_out[n] = s_m;
+        mn_out[n] = lo_m;
+        if (mx_out) mx_out[n] = hi_m;
+      }
+      groups_share_scale<T, D, BITS>(s_m, sc);
+    }
+    uint32_t words[2][2];
+    if (NOISE == GACT_NOISE_FAST) fast_pair_words<T>(span, i, k0, k1, words);
+
+    u32x2 held = {0u, 0u};   // half rows: the finished bytes of an even super-group, until the odd one joins them
+#pragma unroll
+    for (int g = 0; g < S::GL; g++) {
+      const int first = S::HALF ? 2 * g : s * S::GPS + g;   // the (first) group within the row's unit
+      const int64_t n = span * S::GPS + (S::HALF ? 2 * g + half : g);
+      const uint32_t shift = (uint32_t)((first % WPT + (S::HALF && WPT > 1 ? half : 0) + part * S::SPR * S::GPS) * BITS);
+      if (S::ROWS > 1 ? s == 0 && g == 0 : first % WPT == 0) {
+#pragma unroll
+        for (int c = 0; c < S::CPG; c++)
+#pragma unroll
+          for (int e = 0; e < W; e++) acc[c][e] = 0;
+      }
+      const bool overflowed = Elem<T>::kRepairsInfiniteScale && Elem<T>::scale_is_inf(sc[g]);
+#pragma unroll
+      for (int c = 0; c < S::CPG; c++) {
+        const int h = (g * S::CPG + c) / CH, k = (g * S::CPG + c) % CH;
+        uint32_t code[W];
+        if (NOISE == GACT_NOISE_FAST) {
+          float cd[CH / 2][W];
+          fast_centred_draws<T>(words[h], cd);
+          if (k < CH / 2) Elem<T>::template codes<false, false, true, false>(v[h], k, lo[g], sc[g], cd[k % (CH / 2)], code);
+          else Elem<T>::template codes<false, false, true, true>(v[h], k, lo[g], sc[g], cd[k % (CH / 2)], code);
+        } else {
+          float u[W];
+#pragma unroll
+          for (int e = 0; e < W; e++) u[e] = 0.5f;
+          if (NOISE == GACT_NOISE_INJECT && n < N)
+            Elem<T>::load_noise(noise + span * GROUPS_SPAN + h * GROUP + chunk_col<T>(k, i), u);
+          Elem<T>::template codes<NOISE == GACT_NOISE_CONST, false>(v[h], k, lo[g], sc[g], u, code);
+        }
+        // a group past the last one holds zeros, whose codes are zero
+#pragma unroll
+        for (int e = 0; e < W; e++) acc[c][e] |= code[e] << shift;
+        if (__builtin_amdgcn_ballot_w64(overflowed) != 0 && overflowed) {   // rare, see Elem<T>::kRepairsInfiniteScale
+#pragma unroll
+          for (int e = 0; e < W; e++)
+            if (Elem<T>::above(v[h], k, e, lo[g])) acc[c][e] |= 0xffffffffu << shift;
+        }
+      }
+      if constexpr (S::ROWS > 1) {
+        // the bytes go out below, when the row has gone through its share
+      } else if constexpr (!S::HALF) {
+        if (first % WPT == WPT - 1) {
+          const int64_t sg = (unit * S::UNIT_GROUPS + first) / WPT;
+          if (sg * WPT < N) {
+#pragma unroll
+            for (int c = 0; c < S::CPG; c++) Elem<T>::store_codes(packed + sg * D + chunk_col<T>(c, i), acc[c]);
+          }
+        }
+      } else if (WPT == 1) {
+        if (n < N) Elem<T>::store_codes(packed + n * D + W * (i & 7), acc[0]);
+      } else if ((first + 1) % WPT == WPT - 1) {
+        // the two halves of the row hold different fields of the same bytes; super-groups go out in pairs, one per half
+        // row, so that a row writes 128 contiguous bytes
+        u32x2 w;
+        w.x = pack4(acc[0]);
+        w.y = pack4(acc[0] + 4);
+        w.x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w.x, 0x128, 0xf, 0xf, false);   // row_ror:8
+        w.y |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w.y, 0x128, 0xf, 0xf, false);
+        const int q = first / WPT;   // super-group of the span
+        if (WPT == 8 || (q & 1)) {
+          const int64_t sg = (span * S::GPS) / WPT + (WPT == 8 ? 0 : q - 1 + half);
+          const u32x2 out = {WPT == 8 || half ? w.x : held.x, WPT == 8 || half ? w.y : held.y};
+          if ((WPT < 8 || half == 0) && sg * WPT < N) stream_store(out, reinterpret_cast<u32x2*>(packed + sg * D + W * (i & 7)));
+        } else {
+          held = w;
+        }
+      }
+    }
+  }
+  if constexpr (S::ROWS > 1) {
+    // the unit is one super-group.  The lane's dwords in the order of their columns, OR-ed over the rows (every row of the
+    // unit is here); each row stores its share of them.
+    constexpr int DW = S::CPG * W / 4, OWN = DW / S::ROWS;
+    static_assert(DW % S::ROWS == 0, "rows store equal shares");
+    uint32_t pk[DW];
+#pragma unroll
+    for (int j = 0; j < DW; j++) {
+      pk[j] = pack4(&acc[j * 4 / W][(j * 4) % W]);
+#pragma unroll
+      for (int off = 16; off < 16 * S::ROWS; off <<= 1) pk[j] |= (uint32_t)__shfl_xor((int)pk[j], off, 64);
+    }
+#pragma unroll
+    for (int j = 0; j < OWN; j++) {
+      uint32_t mine = pk[j];
+#pragma unroll
+      for (int r = 1; r < S::ROWS; r++) mine = part == r ? pk[r * OWN + j] : mine;
+      const int at = part * OWN + j;   // W = 4: chunk; W = 8: half a chunk
+      const int col = W == 4 ? chunk_col<T>(at, i) : chunk_col<T>(at >> 1, i) + 4 * (at & 1);
+      stream_store(mine, reinterpret_cast<uint32_t*>(packed + unit * D + col));
+    }
+  }
+}
+
+// Dequantize.  A lane takes P 16-byte pieces of the columns of super-groups - it loads the code bytes of these columns once and
+// writes that piece of each of the super-group's 8/BITS groups - and the wave's 64 lanes cover neighbouring pieces, so a store
+// instruction writes whole groups.  Codes, scales and minima of all the pieces are asked for first.
+// WPT consecutive values from a + n0 on, in loads of up to 16 bytes where the array is aligned
+template <typename T, int WPT>
+__device__ __forceinline__ void load_stats(const T* __restrict__ a, int64_t n0, int64_t N, bool aligned, T (&v)[WPT]) {
+  if (WPT > 1 && aligned && n0 + WPT <= N) {
+    constexpr int VL = WPT * (int)sizeof(T) > 16 ? 16 / (int)sizeof(T) : (WPT > 1 ? WPT : 2);
+    typedef T vec __attribute__((ext_vector_type(VL)));
+#pragma unroll
+    for (int c = 0; c < WPT / VL; c++) {
+      const vec q = reinterpret_cast<const vec*>(a + n0)[c];
+#pragma unroll
+      for (int e = 0; e < VL; e++) v[c * VL + e] = q[e];
+    }
+  } else {
+#pragma unroll
+    for (int ni = 0; ni < WPT; ni++) v[ni] = n0 + ni < N ? a[n0 + ni] : (T)1.0f;
+  }
+}
+template <typename T, int D, int BITS, int P>
+__global__ void __launch_bounds__(256)
+dequantize_groups_kernel(const uint8_t* __restrict__ packed, const T* __restrict__ scale, const T* __restrict__ mn,
+                         int64_t numel, int64_t N, T* __restrict__ out) {
+  constexpr int WPT = 8 / BITS, W = Elem<T>::kDqWidth;
+  const uint32_t tile = xcd_tile<GACT_XCD_RUN_DQ>(blockIdx.x, gridDim.x);
+  const int64_t wave = (int64_t)tile * (blockDim.x >> 6) + wave_first(threadIdx.x >> 6);
+  const int64_t byte0 = wave * (P * 64 * W);   // the wave's first code byte
+  const int64_t n_first = byte0 / D * WPT;
+  if (n_first >= N) return;   // the whole wave
+  const OutWindow window(out + n_first * D, (numel - n_first * D) * (int64_t)sizeof(T));
+  const int lane = threadIdx.x & 63;
+  const bool aligned = ((reinterpret_cast<uintptr_t>(scale) | reinterpret_cast<uintptr_t>(mn)) & 15u) == 0;
+  uint32_t w[P][W / 4];
+  T s[P][WPT], m[P][WPT];
+#pragma unroll
+  for (int p = 0; p < P; p++) {
+    const int64_t at = byte0 + (p * 64 + lane) * W;   // the piece's code bytes
+    const int64_t n0 = at / D * WPT;
+#pragma unroll
+    for (int k = 0; k < W / 4; k++) w[p][k] = 0u;
+    if (n0 < N) {
+      if constexpr (W == 4) {
+        w[p][0] = stream_load(reinterpret_cast<const uint32_t*>(packed + at));
+      } else {
+        const u32x2 q = stream_load(reinterpret_cast<const u32x2*>(packed + at));
+        w[p][0] = q.x;
+        w[p][W / 4 - 1] = q.y;
+      }
+    }
+    load_stats<T, WPT>(scale, n0, N, aligned, s[p]);
+    load_stats<T, WPT>(mn, n0, N, aligned, m[p]);
+  }
+#pragma unroll
+  for (int p = 0; p < P; p++) {
+    const int64_t at = byte0 + (p * 64 + lane) * W;
+    const int64_t n0 = at / D * WPT;
+    const int col = (int)(at % D);
+#pragma unroll
+    for (int ni = 0; ni < WPT; ni++) {
+      const typename Elem<T>::Dq dq = Elem<T>::dq_prepare(s[p][ni], m[p][ni]);
+      T v[W];
+      if (__builtin_amdgcn_ballot_w64(!dq.fast) == 0) {
+#pragma unroll
+        for (int e = 0; e < W; e++)
+          v[e] = Elem<T>::finish(div_by_reciprocal((float)__builtin_amdgcn_ubfe(w[p][e >> 2], 8 * (e & 3) + ni * BITS, BITS), dq.s, dq.r), dq.mn);
+      } else {
+#pragma unroll
+        for (int e = 0; e < W; e++)
+          v[e] = Elem<T>::finish((float)__builtin_amdgcn_ubfe(w[p][e >> 2], 8 * (e & 3) + ni * BITS, BITS) / dq.s, dq.mn);
+      }
+      const int64_t first = (n0 + ni) * D + col;   // the piece's first element of this group
+      if (first + W <= numel) {
+        Elem<T>::template store_dq<GACT_STORE_NT_SYSTEM>(window, (uint32_t)((first - n_first * D) * (int64_t)sizeof(T)), v);
+      } else {
+#pragma unroll
+        for (int e = 0; e < W; e++)
+          if (first + e < numel) out[first + e] = v[e];
+      }
+    }
+  }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256)
 minimax256_kernel(const T* __restrict__ x, int64_t N, T* __restrict__ mn, T* __restrict__ mx) {
@@ -2531,6 +2852,90 @@ int dispatch_dequantize(int bits, const uint8_t* packed, const typename Elem<T>:
   return hipLaunchKernel(p.kernel, p.grid, p.block, args, p.lds, stream) == hipSuccess ? GACT_OK : GACT_ELAUNCH;
 }
 
+// ---- group sizes of the one-pass kernels other than 256 ----
+inline bool one_pass_group(int64_t group) { return group == 64 || group == 128 || group == 512; }
+
+template <typename T, int D, int BITS>
+LaunchPlan plan_quantize_groups(int64_t N, int noise_mode) {
+  typedef GroupsShape<T, D, BITS> S;
+  LaunchPlan p;
+  row_grid((N + S::UNIT_GROUPS - 1) / S::UNIT_GROUPS * S::ROWS, &p.grid, &p.block, 64);
+  switch (noise_mode) {
+    case GACT_NOISE_CONST: p.kernel = (const void*)quantize_groups_kernel<T, D, BITS, GACT_NOISE_CONST>; break;
+    case GACT_NOISE_INJECT: p.kernel = (const void*)quantize_groups_kernel<T, D, BITS, GACT_NOISE_INJECT>; break;
+    case GACT_NOISE_FAST: p.kernel = (const void*)quantize_groups_kernel<T, D, BITS, GACT_NOISE_FAST>; break;
+  }
+  return p;
+}
+template <typename T, int D>
+LaunchPlan plan_quantize_groups_bits(int bits, int64_t N, int noise_mode) {
+  switch (bits) {
+    case 1: return plan_quantize_groups<T, D, 1>(N, noise_mode);
+    case 2: return plan_quantize_groups<T, D, 2>(N, noise_mode);
+    case 4: return plan_quantize_groups<T, D, 4>(N, noise_mode);
+    case 8: return plan_quantize_groups<T, D, 8>(N, noise_mode);
+  }
+  return LaunchPlan();
+}
+template <typename T>
+int dispatch_quantize_groups(int64_t group, int bits, const T* x, int64_t numel, int64_t N, uint8_t* packed, T* scale, T* mn,
+                             T* mx, int noise_mode, SeedArg seed, const float* noise, hipStream_t stream) {
+  const LaunchPlan p = group == 64    ? plan_quantize_groups_bits<T, 64>(bits, N, noise_mode)
+                       : group == 128 ? plan_quantize_groups_bits<T, 128>(bits, N, noise_mode)
+                                      : plan_quantize_groups_bits<T, 512>(bits, N, noise_mode);
+  if (!p.kernel) return GACT_EINVAL;
+  void* args[] = {(void*)&seed, (void*)&x, (void*)&numel, (void*)&N, (void*)&packed, (void*)&scale, (void*)&mn, (void*)&mx, (void*)&noise};
+  return hipLaunchKernel(p.kernel, p.grid, p.block, args, p.lds, stream) == hipSuccess ? GACT_OK : GACT_ELAUNCH;
+}
+
+// One piece per lane keeps the most waves and the shortest chain in each, two keep more in flight per wave and are better once
+// the tensor fills the chip several times over.  Dequantize of groups of 128, us, buffers cold in every cache, one piece / two
+// (four and eight lose 5-100 % everywhere but float 8 bit, where they gain nothing):
+//   float 1 M elements  2 bit 2.6 / 3.3  4 bit 2.6 / 2.9  8 bit 2.6 / 2.6    4 M  2 bit 4.46 / 4.42  4 bit 4.5 / 4.9  8 bit 5.7 / 4.4
+//         17 M  2 bit 14.3 / 12.8  4 bit 15.6 / 15.4  8 bit 19.3 / 15.7    100 M  2 bit 76 / 73  4 bit 87 / 79  8 bit 101 / 78
+//   half  4 M  2 bit 3.8 / 4.9  4 bit 3.5 / 4.4  8 bit 3.7 / 4.0    17 M  2 bit 7.6 / 8.1  4 bit 9.9 / 8.5  8 bit 12.4 / 10.6
+//         50 M  1 bit 21.1 / 21.0  2 bit 23.1 / 22.1  4 bit 26.3 / 24.1  8 bit 33.1 / 28.9    100 M  1 bit 43.1 / 40.3
+// Float at 1 bit has eight stores per piece already (two pieces: 50 M 37.2 / 38.4) and gains from the occupancy cap instead
+// (40 000 bytes: 50 M 37.2 -> 35.8, 100 M 71.3 -> 66.6, 17 M 13.8 -> 13.2); the others lose by it (float 4 bit 17 %, half 20-30 %).
+template <typename T>
+constexpr int64_t groups_two_pieces_from(int bits) {   // elements
+  return sizeof(T) == 4 ? (bits == 1 ? INT64_MAX : bits == 2 ? 1LL << 22 : bits == 4 ? 1LL << 23 : 1LL << 21)
+                        : (bits == 1 ? 1LL << 26 : bits == 2 ? 1LL << 25 : bits == 4 ? 1LL << 23 : 1LL << 23);
+}
+#define GROUPS_DQ_CAP_FROM (1LL << 24)
+template <typename T, int D, int BITS>
+LaunchPlan plan_dequantize_groups_bits(int64_t N) {
+  LaunchPlan p;
+  const bool two = N * D >= groups_two_pieces_from<T>(BITS);
+  const int64_t per_wave = (two ? 2 : 1) * 64 * Elem<T>::kDqWidth;   // code bytes
+  const int64_t waves = (supergroups(N, BITS) * D + per_wave - 1) / per_wave;
+  p.kernel = two ? (const void*)dequantize_groups_kernel<T, D, BITS, 2> : (const void*)dequantize_groups_kernel<T, D, BITS, 1>;
+  p.grid = dim3((unsigned)((waves + 3) / 4));
+  p.block = dim3(256);
+  p.lds = sizeof(T) == 4 && BITS == 1 && N * D >= GROUPS_DQ_CAP_FROM ? 40000u : 0u;
+  return p;
+}
+template <typename T, int D>
+LaunchPlan plan_dequantize_groups(int bits, int64_t N) {
+  switch (bits) {
+    case 1: return plan_dequantize_groups_bits<T, D, 1>(N);
+    case 2: return plan_dequantize_groups_bits<T, D, 2>(N);
+    case 4: return plan_dequantize_groups_bits<T, D, 4>(N);
+    case 8: return plan_dequantize_groups_bits<T, D, 8>(N);
+  }
+  return LaunchPlan();
+}
+template <typename T>
+int dispatch_dequantize_groups(int64_t group, int bits, const uint8_t* packed, const T* scale, const T* mn, int64_t numel,
+                               int64_t N, T* out, hipStream_t stream) {
+  const LaunchPlan p = group == 64    ? plan_dequantize_groups<T, 64>(bits, N)
+                       : group == 128 ? plan_dequantize_groups<T, 128>(bits, N)
+                                      : plan_dequantize_groups<T, 512>(bits, N);
+  if (!p.kernel) return GACT_EINVAL;
+  void* args[] = {(void*)&packed, (void*)&scale, (void*)&mn, (void*)&numel, (void*)&N, (void*)&out};
+  return hipLaunchKernel(p.kernel, p.grid, p.block, args, p.lds, stream) == hipSuccess ? GACT_OK : GACT_ELAUNCH;
+}
+
 template <typename T>
 void launch_minimax_any(const T* x, int64_t N, int64_t D, T* mn, T* mx, hipStream_t stream) {
   const bool vec = aligned16(x);  // D % 32 == 0 keeps every row 16-byte aligned once the base is
@@ -2696,6 +3101,11 @@ int gact_unpack(const void* packed, int bits, const void* scale, const void* mn,
       return dispatch_dequantize<float>(bits, (const uint8_t*)packed, (const float*)scale, (const float*)mn, N * GROUP, N, (float*)out, s);
     return dispatch_dequantize<f16>(bits, (const uint8_t*)packed, (const f16*)scale, (const f16*)mn, N * GROUP, N, (f16*)out, s);
   }
+  if (G == 1 && one_pass_group(D) && aligned16(out) && aligned16(packed)) {
+    if (dtype == GACT_F32)
+      return dispatch_dequantize_groups<float>(D, bits, (const uint8_t*)packed, (const float*)scale, (const float*)mn, N * D, N, (float*)out, s);
+    return dispatch_dequantize_groups<f16>(D, bits, (const uint8_t*)packed, (const f16*)scale, (const f16*)mn, N * D, N, (f16*)out, s);
+  }
   if (dtype == GACT_F32)
     return unpack_any<float>((const uint8_t*)packed, bits, (const float*)scale, (const float*)mn, N, G, D, (float*)out, s);
   return unpack_any<f16>((const uint8_t*)packed, bits, (const f16*)scale, (const f16*)mn, N, G, D, (f16*)out, s);
@@ -2743,6 +3153,46 @@ int gact_dequantize(const void* packed, int bits, const void* scale, const void*
   if (dtype == GACT_BF16)
     return dispatch_dequantize<bf16>(bits, (const uint8_t*)packed, (const float*)scale, (const bf16*)mn, numel, N, (bf16*)out, s);
   return dispatch_dequantize<f16>(bits, (const uint8_t*)packed, (const f16*)scale, (const f16*)mn, numel, N, (f16*)out, s);
+}
+
+int gact_quantize_groups(const void* x, int dtype, int64_t numel, int group, int bits, int noise_mode, uint64_t seed,
+                         const uint64_t* seed_add, const float* noise, void* packed, void* scale, void* mn, void* mx,
+                         void* stream) {
+  if (group == GROUP)
+    return gact_quantize_seeded(x, dtype, numel, bits, noise_mode, seed, seed_add, noise, packed, scale, mn, mx, stream);
+  if (dtype != GACT_F32 && dtype != GACT_F16) return GACT_EINVAL;
+  if (!valid_bits(bits) || numel < 0) return GACT_EINVAL;
+  if (noise_mode < GACT_NOISE_CONST || noise_mode > GACT_NOISE_FAST) return GACT_EINVAL;
+  if (!one_pass_group(group) || noise_mode == GACT_NOISE_REF) return GACT_ESHAPE;
+  if (numel == 0) return GACT_OK;
+  if (!x || !packed || !scale || !mn) return GACT_EINVAL;
+  if (noise_mode == GACT_NOISE_INJECT && !noise) return GACT_EINVAL;
+  if (!aligned16(x) || !aligned16(packed) || (noise_mode == GACT_NOISE_INJECT && !aligned16(noise))) return GACT_EALIGN;
+  if (reinterpret_cast<uintptr_t>(seed_add) & 7u) return GACT_EALIGN;
+  const int64_t N = (numel + group - 1) / group;
+  hipStream_t s = (hipStream_t)stream;
+  fresh_launch();
+  const SeedArg sa{seed, seed_add};
+  if (dtype == GACT_F32)
+    return dispatch_quantize_groups<float>(group, bits, (const float*)x, numel, N, (uint8_t*)packed, (float*)scale, (float*)mn, (float*)mx, noise_mode, sa, noise, s);
+  return dispatch_quantize_groups<f16>(group, bits, (const f16*)x, numel, N, (uint8_t*)packed, (f16*)scale, (f16*)mn, (f16*)mx, noise_mode, sa, noise, s);
+}
+
+int gact_dequantize_groups(const void* packed, int bits, const void* scale, const void* mn, int dtype, int64_t numel, int group,
+                           void* out, void* stream) {
+  if (group == GROUP) return gact_dequantize(packed, bits, scale, mn, dtype, numel, out, stream);
+  if (dtype != GACT_F32 && dtype != GACT_F16) return GACT_EINVAL;
+  if (!valid_bits(bits) || numel < 0) return GACT_EINVAL;
+  if (!one_pass_group(group)) return GACT_ESHAPE;
+  if (numel == 0) return GACT_OK;
+  if (!packed || !scale || !mn || !out) return GACT_EINVAL;
+  if (!aligned16(out) || !aligned16(packed)) return GACT_EALIGN;
+  const int64_t N = (numel + group - 1) / group;
+  hipStream_t s = (hipStream_t)stream;
+  fresh_launch();
+  if (dtype == GACT_F32)
+    return dispatch_dequantize_groups<float>(group, bits, (const uint8_t*)packed, (const float*)scale, (const float*)mn, numel, N, (float*)out, s);
+  return dispatch_dequantize_groups<f16>(group, bits, (const uint8_t*)packed, (const f16*)scale, (const f16*)mn, numel, N, (f16*)out, s);
 }
 
 int gact_launch_geometry(int kind, int dtype, int bits, int64_t N, int* threads, int* lds_bytes, int* workgroups_per_cu) {

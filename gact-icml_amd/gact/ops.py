@@ -24,10 +24,12 @@ def _num_groups(numel):
     return (numel + config.group_size - 1) // config.group_size
 
 
-def _fused():
-    """The single-pass kernels are built for groups of 256; any other config.group_size takes the
-    extension-style sequence minimax -> pack / unpack on the zero-padded tensor, as the reference does."""
-    return config.group_size == _abi.GROUP
+def _fused(dtype):
+    """The single-pass kernels are built for groups of 256, and 64, 128 and 512 for float and half; any other
+    config.group_size takes the extension-style sequence minimax -> pack / unpack on the zero-padded tensor, as the
+    reference does."""
+    group = config.group_size
+    return group == _abi.GROUP or (group in _abi.ONE_PASS_GROUPS and dtype is not torch.bfloat16)
 
 
 def _padded_groups(input):
@@ -50,9 +52,10 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
         q_scale = input_groups.max(dim=-1, keepdim=True).values - q_min
         return input_groups, q_scale, q_min
 
-    if not _fused():
+    if not _fused(input.dtype) or (config.group_size != _abi.GROUP and noise is None
+                                   and (rng_stream or config.rng_stream) == "reference"):
         if seed_offset is not None:
-            raise RuntimeError("seed_offset needs the single-pass kernels (config.group_size 256)")
+            raise RuntimeError("seed_offset needs the single-pass kernels (config.group_size 64, 128, 256 or 512)")
         from .cpp_extension import minimax as ext_minimax
         input_groups = _padded_groups(input.contiguous()).contiguous()
         q_min, mx = ext_minimax.minimax(input_groups)
@@ -83,20 +86,17 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
                     or not noise.is_contiguous():
                 raise RuntimeError("noise must be a contiguous float32 CUDA tensor with one value per padded element")
     device = x.device
-    q_input = torch.empty(ext_quantization.packed_numel(q_bit, N, 1, _abi.GROUP), dtype=torch.int8, device=device)
+    group = config.group_size
+    q_input = torch.empty(ext_quantization.packed_numel(q_bit, N, 1, group), dtype=torch.int8, device=device)
     # bfloat16 (not in the reference) is quantized as the float values it holds: float scale, bfloat16 min
     q_scale = torch.empty((N, 1, 1), dtype=torch.float32 if dtype is torch.bfloat16 else dtype, device=device)
     q_min = torch.empty((N, 1, 1), dtype=dtype, device=device)
-    if seed_offset is None:
-        _abi.call_on(device, _abi.lib().gact_quantize, x.data_ptr(), _abi.dtype_code(dtype),
-                     x.numel(), q_bit, mode, seed, None if noise is None else noise.data_ptr(), q_input.data_ptr(),
-                     q_scale.data_ptr(), q_min.data_ptr(), None, _current_stream(device.index))
-    else:
+    if seed_offset is not None:
         if seed_offset.dtype is not torch.int64 or seed_offset.numel() != 1 or seed_offset.device != device:
             raise RuntimeError("seed_offset must be one int64 on the device of the data")
-        _abi.call_on(device, _abi.lib().gact_quantize_seeded, x.data_ptr(), _abi.dtype_code(dtype),
-                     x.numel(), q_bit, mode, seed, seed_offset.data_ptr(), None if noise is None else noise.data_ptr(),
-                     q_input.data_ptr(), q_scale.data_ptr(), q_min.data_ptr(), None, _current_stream(device.index))
+    _abi.call_on(device, _abi.lib().gact_quantize_groups, x.data_ptr(), _abi.dtype_code(dtype), x.numel(), group, q_bit, mode,
+                 seed, _abi.ptr(seed_offset), _abi.ptr(noise), q_input.data_ptr(), q_scale.data_ptr(), q_min.data_ptr(), None,
+                 _current_stream(device.index))
     return q_input, q_scale, q_min
 
 
@@ -148,7 +148,7 @@ def op_dequantize(input, input_shape):
     if q_bit == 32:
         return q_input.ravel()[:num_features].reshape(*input_shape).contiguous()
 
-    if not _fused():
+    if not _fused(q_min.dtype):
         groups = dequantize_and_unpack(q_input, input_shape, q_bit, q_scale, q_min)
         return groups.ravel()[:num_features].reshape(*input_shape).contiguous()
 
@@ -157,8 +157,9 @@ def op_dequantize(input, input_shape):
         raise RuntimeError("data must be a CUDA tensor!")
     if q_input.dtype is not torch.int8 or q_input.dim() != 1:
         raise RuntimeError("The type of data is not correct!")
+    group = config.group_size
     N = _num_groups(num_features)
-    if q_input.numel() < ext_quantization.packed_numel(q_bit, N, 1, _abi.GROUP) - 1 \
+    if q_input.numel() < ext_quantization.packed_numel(q_bit, N, 1, group) - 1 \
             or q_scale.numel() < N or q_min.numel() < N:
         raise RuntimeError("packed data / scale / min are too short for shape %s" % (tuple(input_shape),))
     dtype = q_min.dtype      # the scale's type as well, except for bfloat16 tensors, whose scale is float
@@ -166,6 +167,6 @@ def op_dequantize(input, input_shape):
         raise RuntimeError("expected scalar type of min to match scale")
     device = q_input.device
     out = torch.empty(tuple(input_shape), dtype=dtype, device=device)
-    _abi.call_on(device, _abi.lib().gact_dequantize, q_input.data_ptr(), q_bit, q_scale.data_ptr(), q_min.data_ptr(),
-                 _abi.dtype_code(dtype), num_features, out.data_ptr(), _current_stream(device.index))
+    _abi.call_on(device, _abi.lib().gact_dequantize_groups, q_input.data_ptr(), q_bit, q_scale.data_ptr(), q_min.data_ptr(),
+                 _abi.dtype_code(dtype), num_features, group, out.data_ptr(), _current_stream(device.index))
     return out

@@ -90,6 +90,16 @@ int gact_quantize_seeded(const void* x, int dtype, int64_t numel, int bits, int 
 int gact_dequantize(const void* packed, int bits, const void* scale, const void* mn, int dtype,
                     int64_t numel, void* out, void* stream);
 
+/* The same two with the group size as an argument: 256 (the entry points above), or 64, 128 and 512 for float and half
+ * (config.group_size, gact/gact/conf.py:50) and every noise stream but GACT_NOISE_REF.  Same results as zero-padding to
+ * whole groups, gact_minimax and gact_pack / gact_unpack, in one pass over the data; GACT_ESHAPE for any other group size and for
+ * GACT_NOISE_REF at a group size other than 256, which take that sequence. */
+int gact_quantize_groups(const void* x, int dtype, int64_t numel, int group, int bits, int noise_mode, uint64_t seed,
+                         const uint64_t* seed_add, const float* noise, void* packed, void* scale, void* mn, void* mx,
+                         void* stream);
+int gact_dequantize_groups(const void* packed, int bits, const void* scale, const void* mn, int dtype, int64_t numel, int group,
+                           void* out, void* stream);
+
 /* What a gact_quantize (kind 0; fast, deterministic or injected noise) or gact_dequantize (kind 1) launch of a tensor of
  * N groups is made of, without launching anything: the threads of a workgroup, the dynamic LDS the launch asks for -
  * on large tensors some kernels ask for LDS they never touch, which is how the library caps their occupancy - and
