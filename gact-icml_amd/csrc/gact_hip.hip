@@ -655,6 +655,50 @@ __device__ __forceinline__ void load_group(const T* __restrict__ x, int64_t nume
   }
 }
 
+// Where a quantize row takes its groups from: load() fills the lane's 16 elements of group n (elements past the end are
+// zero), and a contiguous source also has its elements side by side (x).
+template <typename T>
+struct ContiguousSource {
+  static constexpr bool kContiguous = true;
+  const T* x;
+  int64_t numel;
+  __device__ __forceinline__ void load(int64_t n, int i, typename Elem<T>::Store& st) const { load_group<T>(x, numel, n, i, st); }
+};
+// q = x / d for x < 2^31, as a multiplication (multiplier 0: d is 1)
+struct Divisor {
+  uint32_t d, m, s;
+  __device__ __forceinline__ uint32_t quotient(uint32_t x) const { return m ? __umulhi(x, m) >> s : x; }
+};
+// A tensor of up to four dimensions whose innermost runs are contiguous and whole 16-byte pieces (attention heads: [batch,
+// seq, heads, width] seen as [batch, heads, seq, width]): every 16-byte piece has an address of its own.  Counts and
+// strides are in pieces.
+struct GatherShape {
+  Divisor run, n2, n1;
+  int64_t s0, s1, s2;
+};
+template <typename T>
+struct GatherSource {
+  static constexpr bool kContiguous = false;
+  const T* x;
+  int64_t numel;
+  GatherShape g;
+  __device__ __forceinline__ void load(int64_t n, int i, typename Elem<T>::Store& st) const {
+    constexpr int CH = Elem<T>::kQChunks, W = Elem<T>::kQWidth;
+#pragma unroll
+    for (int k = 0; k < CH; k++) {
+      const uint32_t piece = (uint32_t)(n * (GROUP / W)) + (uint32_t)(16 * k + i);
+      if ((int64_t)piece * W < numel) {
+        const uint32_t i2 = g.run.quotient(piece), i1 = g.n2.quotient(i2), i0 = g.n1.quotient(i1);
+        const int64_t at = (int64_t)i0 * g.s0 + (int64_t)(i1 - i0 * g.n1.d) * g.s1 + (int64_t)(i2 - i1 * g.n2.d) * g.s2 + (piece - i2 * g.run.d);
+        Elem<T>::load_chunk(x + at * W, st, k);
+      } else {
+#pragma unroll
+        for (int e = 0; e < W; e++) Elem<T>::set(st, k, e, (T)0.0f);
+      }
+    }
+  }
+};
+
 // value of lane LANE of the row, in every lane of the row (DPP row_newbcast)
 template <int LANE>
 __device__ __forceinline__ uint32_t row_bcast_u32(uint32_t v) {
@@ -759,8 +803,8 @@ struct FastRow {
 //   GIVEN = true : min/max are read from mn_io / mx_io (the pack entry point's contract).
 // Codes follow quantization_cuda_kernel.cu:38-71; see Elem<T>::code1 for the arithmetic.
 // ------------------------------------------------------------------------------------------------
-template <typename T, int BITS, int NOISE, bool GIVEN, int SGR = 1, int STAGE = 0, bool LAZY = false>
-__device__ __forceinline__ void quantize_supergroup(const T* __restrict__ x, int64_t numel, int64_t N, int64_t sg0,
+template <typename T, int BITS, int NOISE, bool GIVEN, int SGR = 1, int STAGE = 0, bool LAZY = false, typename SRC>
+__device__ __forceinline__ void quantize_supergroup(const SRC& src, int64_t N, int64_t sg0,
                                                     int i, uint8_t* __restrict__ packed,
                                                     typename Elem<T>::Stat* __restrict__ scale_out,
                                                     T* mn_io, T* mx_io, uint32_t k0, uint32_t k1,
@@ -778,8 +822,10 @@ __device__ __forceinline__ void quantize_supergroup(const T* __restrict__ x, int
   // The staged path is for rows of whole groups.  The choice is made for the wave, not for the row: a wave in which
   // one row is ragged (the tensor's last) would otherwise run both paths one after the other, each with its own
   // round trip to memory - and being the tensor's last wave it would hold up the end of the kernel.
-  const bool whole_row = (n0 + GPR) * GROUP <= numel;
-  if (STAGE > 0 && STAGE < GPR && !GIVEN && NOISE != GACT_NOISE_REF && __builtin_amdgcn_ballot_w64(!whole_row) == 0) {
+  if constexpr (STAGE > 0 && STAGE < GPR && !GIVEN && NOISE != GACT_NOISE_REF && SRC::kContiguous) {
+  const T* __restrict__ x = src.x;
+  const bool whole_row = (n0 + GPR) * GROUP <= src.numel;
+  if (__builtin_amdgcn_ballot_w64(!whole_row) == 0) {
     // All groups whole: the loads in one straight line, then STAGE groups at a time as they arrive: reduce, divide
     // (lane j for group j % STAGE of the stage), encode; a super-group goes out when its last group is done.  The
     // work on the first groups overlaps the loads of the later ones within the wave, which pays where few waves
@@ -899,9 +945,10 @@ __device__ __forceinline__ void quantize_supergroup(const T* __restrict__ x, int
     }
     return;
   }
+  }
 #pragma unroll
   for (int g = 0; g < GPR; g++) {
-    if (n0 + g < N) load_group<T>(x, numel, n0 + g, i, v[g]);
+    if (n0 + g < N) src.load(n0 + g, i, v[g]);
   }
 #pragma unroll
   for (int g = 0; g < GPR; g++) {
@@ -1282,10 +1329,10 @@ __device__ __forceinline__ void quantize_block128(const T* __restrict__ x, int64
 #pragma unroll 1
     for (int q = 0; q < BITS; q++)
       if ((sg0 + q) * WPT < N)
-        quantize_supergroup<T, BITS, NOISE, false, 1>(x, numel, N, sg0 + q, i, packed, scale_out, mn_out, (T*)nullptr,
+        quantize_supergroup<T, BITS, NOISE, false, 1>(ContiguousSource<T>{x, numel}, N, sg0 + q, i, packed, scale_out, mn_out, (T*)nullptr,
                                                       (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
   } else if (sg0 * WPT < N) {
-    quantize_supergroup<T, BITS, NOISE, false, BITS, GACT_QB_STAGE>(x, numel, N, sg0, i, packed, scale_out, mn_out, (T*)nullptr,
+    quantize_supergroup<T, BITS, NOISE, false, BITS, GACT_QB_STAGE>(ContiguousSource<T>{x, numel}, N, sg0, i, packed, scale_out, mn_out, (T*)nullptr,
                                                                     (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
   }
 }
@@ -1368,6 +1415,9 @@ __device__ __forceinline__ void minimax_row(const T* __restrict__ x, int64_t N, 
 #endif
 #ifndef GACT_XCD_RUN_Q
 #define GACT_XCD_RUN_Q 128 /* quantize, 2, 4 and 8 bit: 2-6 % (half 2 bit 52.7 -> 50.2 us, float 2 bit 70.1 -> 68.8 us at 134 / 103 M elements) */
+#endif
+#ifndef GACT_XCD_RUN_TR
+#define GACT_XCD_RUN_TR 16 /* quantize of transposed tensors */
 #endif
 template <uint32_t RUN>
 __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nb) {
@@ -1473,7 +1523,7 @@ quantize_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_
   const int64_t sg0 = ((int64_t)tile * (blockDim.x >> 4) + (threadIdx.x >> 4)) * SGR;
   if (sg0 * (8 / BITS) >= N) return;
   const uint64_t seed = seed_arg.value();
-  quantize_supergroup<T, BITS, NOISE, GIVEN, SGR, STAGE, LAZY>(x, numel, N, sg0, threadIdx.x & 15, packed, scale_out, mn_io, mx_io,
+  quantize_supergroup<T, BITS, NOISE, GIVEN, SGR, STAGE, LAZY>(ContiguousSource<T>{x, numel}, N, sg0, threadIdx.x & 15, packed, scale_out, mn_io, mx_io,
                                                   (uint32_t)seed, (uint32_t)(seed >> 32), noise);
 }
 
@@ -1496,18 +1546,15 @@ __device__ __forceinline__ uint32_t pack4(const uint32_t* b) {
   // the reference accumulates in a uint8_t: keep the low 8 bits of every byte
   return (b[0] & 0xffu) | ((b[1] & 0xffu) << 8) | ((b[2] & 0xffu) << 16) | (b[3] << 24);
 }
-template <typename T, int BITS, int NOISE>
-__global__ void __launch_bounds__(256)
-quantize_wave8_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_t N, uint8_t* __restrict__ packed,
-                      typename Elem<T>::Stat* __restrict__ scale_out, T* __restrict__ mn_out, T* __restrict__ mx_out,
-                      const float* __restrict__ noise) {
+template <typename T, int BITS, int NOISE, typename SRC>
+__device__ __forceinline__ void quantize_wave8(const SeedArg& seed_arg, const SRC& src, int64_t sg, int64_t N, uint8_t* __restrict__ packed,
+                                               typename Elem<T>::Stat* __restrict__ scale_out, T* __restrict__ mn_out,
+                                               T* __restrict__ mx_out, const float* __restrict__ noise) {
   static_assert(NOISE != GACT_NOISE_REF, "the reference stream draws per output byte");
   static_assert(BITS == 1 || BITS == 2, "four rows share a super-group: two groups a row at 1 bit, one at 2 bit");
   typedef typename Elem<T>::Stat Stat;
   constexpr int WPT = 8 / BITS, GR = WPT / 4, QMAX = (1 << BITS) - 1;   // GR: groups of a row
   constexpr int CH = Elem<T>::kQChunks, W = Elem<T>::kQWidth;
-  const uint32_t tile = gridDim.x - 1u - xcd_tile<GACT_W8_RUN>(blockIdx.x, gridDim.x);   // last tile first, see quantize_kernel
-  const int64_t sg = (int64_t)tile * (blockDim.x >> 6) + (threadIdx.x >> 6);               // the wave's super-group
   const int64_t n0 = sg * WPT;
   if (n0 >= N) return;   // the whole wave
   const int lane = threadIdx.x & 63, r = lane >> 4, i = lane & 15;
@@ -1518,7 +1565,7 @@ quantize_wave8_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, 
   typename Elem<T>::Store v[GR];
 #pragma unroll
   for (int g = 0; g < GR; g++)
-    if (na + g < N) load_group<T>(x, numel, na + g, i, v[g]);
+    if (na + g < N) src.load(na + g, i, v[g]);
   Stat lo[GR], hi[GR], sc[GR];
 #pragma unroll
   for (int g = 0; g < GR; g++) {
@@ -1600,6 +1647,387 @@ quantize_wave8_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, 
   const uint32_t mine = r == 0 ? pk[0] : r == 1 ? pk[1] : r == 2 ? pk[2] : pk[3];
   const int col = W == 4 ? chunk_col<T>(r, i) : chunk_col<T>(r >> 1, i) + 4 * (r & 1);
   stream_store(mine, reinterpret_cast<uint32_t*>(packed + sg * GROUP + col));
+}
+template <typename T, int BITS, int NOISE>
+__global__ void __launch_bounds__(256)
+quantize_wave8_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_t N, uint8_t* __restrict__ packed,
+                      typename Elem<T>::Stat* __restrict__ scale_out, T* __restrict__ mn_out, T* __restrict__ mx_out,
+                      const float* __restrict__ noise) {
+  const uint32_t tile = gridDim.x - 1u - xcd_tile<GACT_W8_RUN>(blockIdx.x, gridDim.x);   // last tile first, see quantize_kernel
+  const int64_t sg = (int64_t)tile * (blockDim.x >> 6) + (threadIdx.x >> 6);               // the wave's super-group
+  quantize_wave8<T, BITS, NOISE>(seed_arg, ContiguousSource<T>{x, numel}, sg, N, packed, scale_out, mn_out, mx_out, noise);
+}
+
+// ------------------------------------------------------------------------------------------------
+// Quantize a tensor that is not contiguous, without a contiguous copy of it: groups are consecutive elements in the order of
+// the tensor's indices, wherever they lie.  The copy these kernels replace is torch's element-wise one, 0.5-2 TB/s: half
+// channels-last [64,256,56,56], 4 bit, 223 us of copy and 20 of quantize -> 43; [64,512,28,28] 107 + 12 -> 23; half heads
+// [64,12,197,64] 14 + 7 -> 8; small tensors lose a launch ([2,12,197,64] 3.6 + 3.5 -> 4.6).
+// ------------------------------------------------------------------------------------------------
+// Innermost runs contiguous (GatherSource): quantize_kernel - at 1 and 2 bit quantize_wave8_kernel, whatever the size: a row
+// of 8 or 4 groups would hold 8 to 32 addresses in flight (heads [2,12,197,64] float 2 bit 11.2 -> 4.9 us) - with an
+// address per 16-byte piece.
+template <typename T, int BITS, int NOISE>
+__global__ void __launch_bounds__(256)
+quantize_gather_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_t N, uint8_t* __restrict__ packed,
+                       typename Elem<T>::Stat* __restrict__ scale_out, T* mn_out, T* mx_out, GatherShape shape) {
+  const uint32_t tile = gridDim.x - 1u - xcd_tile<GACT_XCD_RUN_Q>(blockIdx.x, gridDim.x);
+  if constexpr (BITS <= 2) {
+    quantize_wave8<T, BITS, NOISE>(seed_arg, GatherSource<T>{x, numel, shape}, (int64_t)tile * (blockDim.x >> 6) + (threadIdx.x >> 6), N,
+                                   packed, scale_out, mn_out, mx_out, nullptr);
+    return;
+  }
+  const int64_t sg = (int64_t)tile * (blockDim.x >> 4) + (threadIdx.x >> 4);
+  if (sg * (8 / BITS) >= N) return;
+  const uint64_t seed = seed_arg.value();
+  quantize_supergroup<T, BITS, NOISE, false>(GatherSource<T>{x, numel, shape}, N, sg, threadIdx.x & 15, packed, scale_out, mn_out, mx_out,
+                                             (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
+}
+
+// Innermost dimension strided, the one before it contiguous (channels-last activations seen as [batch, channels, pixels], a
+// transposed matrix): a workgroup owns `tile` consecutive elements of the tensor in index order - whole channels and parts
+// of channels - and brings them into LDS in that order: it walks the memory rows (one pixel, all channels side by side) that hold
+// them in 16-byte pieces and scatters each piece's elements, one channel each, to where they belong.  Rows of 16 lanes then
+// quantize super-groups out of LDS.  Neighbouring tiles read other channels of the same memory rows; they run on one XCD at about
+// the same time (xcd_tile), so a line that several of them share comes from HBM once and from that XCD's L2 afterwards.
+// Bound by its two phases standing one behind the other: half [64,256,56,56] at 4 bit 54 us, of which reading and scattering
+// alone take 33 and quantizing out of LDS alone 27 (with more, smaller workgroups 41 and 21, together 51).
+struct TransposedShape {
+  int64_t sb, sk;          // strides of batch and pixel, in elements
+  uint32_t M, K;           // channels of a batch entry, pixels
+  int64_t channels;        // of all batch entries
+  int tile;                // elements of a workgroup, a multiple of 2048
+};
+// The tile in LDS: 16 bytes of padding after every group keep the elements of channels a power of two of pixels apart out of
+// each other's banks.  `at` in elements; groups start on 16-byte boundaries.
+template <typename T>
+__host__ __device__ __forceinline__ constexpr uint32_t tile_byte(uint32_t at) { return at * (uint32_t)sizeof(T) + (at / GROUP) * 16u; }
+template <typename T>
+constexpr unsigned tile_bytes(int tile) { return tile_byte<T>((uint32_t)tile) + 16u; }   // and a spare place
+template <typename T>
+struct TileSource {
+  static constexpr bool kContiguous = false;
+  const uint8_t* tile;
+  int64_t n_first;
+  __device__ __forceinline__ void load(int64_t n, int i, typename Elem<T>::Store& st) const {
+    const uint8_t* p = tile + (uint32_t)(n - n_first) * (GROUP * (uint32_t)sizeof(T) + 16u);
+#pragma unroll
+    for (int k = 0; k < Elem<T>::kQChunks; k++) Elem<T>::load_chunk(reinterpret_cast<const T*>(p) + chunk_col<T>(k, i), st, k);
+  }
+};
+#define TRANSPOSED_THREADS 512
+// ROWS neighbouring pixels of a piece per lane and step (the host picks as many as divide the number of pixels, up to 16
+// bytes of them): turned around in registers, they are one LDS write per channel.
+template <int ROWS> struct TransposedUnroll { static constexpr int value = ROWS >= 8 ? 1 : ROWS >= 4 ? 2 : 4; };   // steps in flight
+template <typename T, int BITS, int NOISE, int ROWS>
+__global__ void __launch_bounds__(TRANSPOSED_THREADS)
+quantize_transposed_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_t N, uint8_t* __restrict__ packed,
+                           typename Elem<T>::Stat* __restrict__ scale_out, T* mn_out, T* mx_out, TransposedShape g) {
+  extern __shared__ u32x4 tile_lds[];
+  uint8_t* const tile = reinterpret_cast<uint8_t*>(tile_lds);
+  constexpr int W = Elem<T>::kQWidth, WPT = 8 / BITS, U = TransposedUnroll<ROWS>::value, WAVES = TRANSPOSED_THREADS / 64;
+  constexpr uint32_t ES = sizeof(T);
+  static_assert(ROWS * ES <= 16, "one LDS write per channel");
+  const int64_t E0 = (int64_t)xcd_tile<GACT_XCD_RUN_TR>(blockIdx.x, gridDim.x) * g.tile;
+  const int L = numel - E0 < g.tile ? (int)(numel - E0) : g.tile;   // the grid has no tile past the end: at least 1
+  const int64_t ch0 = E0 / g.K, ch1 = (E0 + L - 1) / g.K;           // channels, counted over all batch entries
+  // the pixels of the tile: all of them, or (a tile smaller than a channel) L of them from its first one on, around the end
+  const uint32_t k_first = (uint32_t)L < g.K ? (uint32_t)(E0 - ch0 * g.K) : 0u;
+  const uint32_t steps = ((uint32_t)L < g.K ? (uint32_t)L : g.K) / ROWS;
+  const int64_t piece0 = ch0 / W;
+  const uint32_t pieces = (uint32_t)(ch1 / W - piece0) + 1;         // 16-byte pieces of a memory row
+  // a wave takes up to 8 pieces (128 bytes) side by side and as many rows as its lanes reach; the waves share the blocks
+  const uint32_t side = pieces < 8 ? pieces : 8, lane = threadIdx.x & 63;
+  const uint32_t rl = (uint32_t)(((float)lane + 0.5f) / (float)side), cl = lane - rl * side;
+  const uint32_t steps_at_once = 64u / side;
+  const uint32_t down = (steps + steps_at_once * U - 1) / (steps_at_once * U), across = (pieces + side - 1) / side;
+  // memory offsets are 32-bit, from the batch entry of the tile's first channel on (the host makes sure that they suffice)
+  const uint32_t b0 = (uint32_t)(ch0 / g.M);
+  const uint8_t* const base = reinterpret_cast<const uint8_t*>(x) + (int64_t)b0 * g.sb * ES;
+  const uint32_t row_bytes = (uint32_t)g.sk * ES, outside = (uint32_t)g.tile;
+  for (uint32_t block = threadIdx.x >> 6; block < down * across; block += WAVES) {
+    const uint32_t c0 = block / down, r0 = (block - c0 * down) * (steps_at_once * U) + rl;
+    const int64_t ch = (piece0 + c0 * side + cl) * W;   // the piece's first channel; M is a multiple of W: one batch entry holds it
+    const bool live = rl < steps_at_once && c0 * side + cl < pieces && ch < g.channels;
+    const uint32_t b = live ? (uint32_t)ch / g.M : b0;
+    const uint32_t column = ((b - b0) * (uint32_t)g.sb + (live ? (uint32_t)ch - b * g.M : 0u)) * ES;
+    const int at0 = (int)(ch * (int64_t)g.K - E0);      // where the first channel's pixel 0 belongs (may lie outside)
+    u32x4 v[U][ROWS];
+    uint32_t k[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const uint32_t r = r0 + u * steps_at_once;
+      k[u] = k_first + ROWS * r;
+      k[u] = k[u] >= g.K ? k[u] - g.K : k[u];
+      if (live && r < steps) {
+        const uint32_t from = column + k[u] * row_bytes;
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) v[u][j] = *reinterpret_cast<const u32x4*>(base + (from + j * row_bytes));
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (live && r0 + u * steps_at_once < steps) {
+#pragma unroll
+        for (int e = 0; e < W; e++) {
+          // channels of other tiles (before this one: a huge unsigned number) go to a spare place behind the tile
+          const uint32_t at = (uint32_t)(at0 + (int)(e * g.K)) + k[u];
+          uint8_t* const to = tile + tile_byte<T>(at < outside ? at : outside);
+          if constexpr (ES == 4 && ROWS == 4) {
+            *reinterpret_cast<u32x4*>(to) = u32x4{v[u][0][e], v[u][1][e], v[u][2][e], v[u][3][e]};
+          } else if constexpr (ES == 4) {
+            *reinterpret_cast<uint32_t*>(to) = v[u][0][e];
+          } else if constexpr (ROWS == 1) {
+            *reinterpret_cast<uint16_t*>(to) = (uint16_t)(v[u][0][e / 2] >> (16 * (e & 1)));
+          } else {
+            uint32_t pair[ROWS / 2];
+#pragma unroll
+            for (int j = 0; j < ROWS / 2; j++)
+              pair[j] = __builtin_amdgcn_perm(v[u][2 * j + 1][e / 2], v[u][2 * j][e / 2], e & 1 ? 0x07060302u : 0x05040100u);
+            if constexpr (ROWS == 8) *reinterpret_cast<u32x4*>(to) = u32x4{pair[0], pair[1], pair[2], pair[3]};
+            else *reinterpret_cast<u32x2*>(to) = u32x2{pair[0], pair[1]};
+          }
+        }
+      }
+    }
+  }
+  for (uint32_t at = (uint32_t)L + threadIdx.x; at < (uint32_t)g.tile; at += TRANSPOSED_THREADS)   // the padding of the last group
+    *reinterpret_cast<T*>(tile + tile_byte<T>(at)) = (T)0.0f;
+  __syncthreads();
+  const uint64_t seed = seed_arg.value();
+  const TileSource<T> src{tile, E0 / GROUP};
+  for (int sg = (int)(threadIdx.x >> 4); sg * WPT * GROUP < L; sg += TRANSPOSED_THREADS / 16)
+    quantize_supergroup<T, BITS, NOISE, false>(src, N, E0 / (WPT * GROUP) + sg, threadIdx.x & 15, packed, scale_out, mn_out, mx_out,
+                                               (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
+}
+
+// The same layout where channels are long (K pixels hold a super-group and more): a workgroup owns a strip of channels, 128 bytes
+// of every memory row, and walks along the pixels in chunks of 256, the next chunk's loads in flight while it works on the
+// one before.  It quantizes the super-groups that begin in its channels.  These begin at another pixel in every channel
+// (first_pixel), so a chunk completes one group of each channel whose head came with the chunk before: LDS holds two groups
+// per channel, in turn.  A super-group that runs past its channel's last pixel ends in the next channel: past the end the walk
+// goes on at the first pixels with every column belonging to the channel before it.  A strip can be cut into segments of
+// whole super-groups, for more workgroups than there are strips; a segment reads up to a super-group of pixels beyond its own.
+// Bound by its steps: half [64,256,56,56] at 4 bit 43 us, vector instructions issued in 53 % of the cycles at two waves per SIMD and
+// in 63 % at four, which more segments give and their extra reading takes back (44 us).
+#define STRIP_PIECES 4    /* 16-byte pieces of a memory row in a strip (8: half [2,64,128,128] 4 bit 7.6 -> 9.5 us, large tensors equal) */
+#define STRIP_CHUNK 256   /* pixels: a thread takes four of one piece */
+#define STRIP_THREADS (STRIP_PIECES * STRIP_CHUNK / 4)
+struct StripShape {
+  int64_t sb, sk;
+  uint32_t M, K, strips;   // strips of a batch entry
+  uint32_t batch, segments, segment;   // segment: super-groups of a channel in a segment
+};
+template <typename T, int BITS, int NOISE>
+__global__ void __launch_bounds__(STRIP_THREADS, 4)
+quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_t N, uint8_t* __restrict__ packed,
+                       typename Elem<T>::Stat* __restrict__ scale_out, T* __restrict__ mn_out, T* __restrict__ mx_out, StripShape g) {
+  typedef typename Elem<T>::Stat Stat;
+  constexpr int CH = Elem<T>::kQChunks, W = Elem<T>::kQWidth, WPT = 8 / BITS, QMAX = (1 << BITS) - 1;
+  constexpr uint32_t ES = sizeof(T), SGE = WPT * GROUP;
+  constexpr int STRIP = STRIP_PIECES * W;             // channels of a strip
+  constexpr int OWN = STRIP / (STRIP_THREADS / 16);   // channels of a row of 16 lanes: 2 (16-bit types), 1 (float)
+  // LDS: two groups per channel; 16 bytes behind every channel and 64 behind every 8 half channels keep the channels, and the
+  // pieces, that a wave writes at once out of each other's banks
+  constexpr uint32_t SLOT = GROUP * ES, CHANNEL = 2 * SLOT + 16, PIECE = W * CHANNEL + (ES == 2 ? 64 : 0);
+  __shared__ u32x4 ring_lds[STRIP_PIECES * PIECE / 16];
+  uint8_t* const ring = reinterpret_cast<uint8_t*>(ring_lds);
+  const uint32_t id = xcd_tile<GACT_XCD_RUN_TR>(blockIdx.x, gridDim.x);
+  const uint32_t seg = id / (g.strips * g.batch), strip = id - seg * (g.strips * g.batch);
+  const uint32_t b = strip / g.strips, m0 = (strip - b * g.strips) * STRIP;
+  const uint32_t width = g.M - m0 < (uint32_t)STRIP ? g.M - m0 : (uint32_t)STRIP;   // a multiple of W
+  const T* const entry = x + (int64_t)b * g.sb;
+  const uint32_t K = g.K;
+  // the column behind the strip's last one, where that channel's super-groups may end: the next channel, perhaps of the next entry
+  const T* const behind = m0 + width < g.M ? entry + m0 + width : b + 1 < g.batch ? x + (int64_t)(b + 1) * g.sb : nullptr;
+
+  // this thread's part of a chunk: four pixels of one piece
+  const uint32_t piece = threadIdx.x % STRIP_PIECES, quad = threadIdx.x / STRIP_PIECES;
+  const bool has_piece = piece * W < width;
+  const bool last_piece = (piece + 1) * W == width;
+  const T* const from = entry + m0 + piece * W;
+  const uint32_t P0 = (uint32_t)(((uint64_t)b * g.M + m0) * K);   // element index of the strip's first channel, low bits
+  const auto first_pixel = [&](uint32_t channel) { return (0u - (P0 + channel * K)) & (SGE - 1); };   // of its first super-group
+  uint32_t first_of[W];
+#pragma unroll
+  for (int e = 0; e < W; e++) first_of[e] = first_pixel(piece * W + e);
+  struct Chunk { u32x4 v[4]; T beyond[4]; };
+  const uint32_t g_first = seg * g.segment * WPT;                  // first group of the segment within a channel
+  const uint32_t g_end = g_first + g.segment * WPT;
+  auto load = [&](uint32_t chunk, Chunk& q) {
+    const uint32_t at = chunk * STRIP_CHUNK + 4 * quad;            // four pixels on one side of K: both are multiples of four
+    const uint32_t k = at < K ? at : at - K;
+    if (has_piece && at < K + SGE) {
+      const T* const p = from + (int64_t)k * g.sk;
+#pragma unroll
+      for (int j = 0; j < 4; j++) q.v[j] = *reinterpret_cast<const u32x4*>(p + j * g.sk);
+      if (at >= K && last_piece) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) q.beyond[j] = behind ? behind[(int64_t)(k + j) * g.sk] : (T)0.0f;
+      }
+    }
+  };
+  // four elements of a channel (16-bit types: in lo) to their place in the channel's two groups.  A chunk holds 256 consecutive
+  // elements of a channel, so what comes before the first super-group cannot reach a group that is being filled.
+  auto put = [&](uint32_t base, uint32_t pos, u32x2 lo, u32x2 hi) {
+    uint8_t* const to = ring + base + (pos & (2 * GROUP - 1)) * ES;
+    if constexpr (ES == 4) *reinterpret_cast<u32x4*>(to) = u32x4{lo.x, lo.y, hi.x, hi.y};
+    else *reinterpret_cast<u32x2*>(to) = lo;
+  };
+  auto column = [&](const Chunk& q, int e, u32x2& lo, u32x2& hi) {   // channel e of the piece: its four pixels side by side
+    if constexpr (ES == 4) {
+      lo = u32x2{q.v[0][e], q.v[1][e]};
+      hi = u32x2{q.v[2][e], q.v[3][e]};
+    } else {
+      const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
+      lo = u32x2{__builtin_amdgcn_perm(q.v[1][e / 2], q.v[0][e / 2], sel), __builtin_amdgcn_perm(q.v[3][e / 2], q.v[2][e / 2], sel)};
+      hi = u32x2{0u, 0u};
+    }
+  };
+  auto scatter = [&](uint32_t chunk, const Chunk& q) {
+    const uint32_t at = chunk * STRIP_CHUNK + 4 * quad;
+    if (!has_piece) return;
+    u32x2 lo, hi;
+    if (at < K) {
+#pragma unroll
+      for (int e = 0; e < W; e++) {
+        column(q, e, lo, hi);
+        put(piece * PIECE + e * CHANNEL, at - first_of[e], lo, hi);
+      }
+    } else if (at < K + SGE) {   // past the end: a column belongs to the channel before it
+#pragma unroll
+      for (int e = 0; e < W; e++) {
+        column(q, e, lo, hi);
+        if (e > 0) put(piece * PIECE + (e - 1) * CHANNEL, at - first_of[e > 0 ? e - 1 : 0], lo, hi);
+        else if (piece > 0) put((piece - 1) * PIECE + (W - 1) * CHANNEL, at - first_pixel(piece * W - 1), lo, hi);
+      }
+      if (last_piece) {
+        hi = u32x2{0u, 0u};
+        if constexpr (ES == 4) {
+          lo = u32x2{__builtin_bit_cast(uint32_t, q.beyond[0]), __builtin_bit_cast(uint32_t, q.beyond[1])};
+          hi = u32x2{__builtin_bit_cast(uint32_t, q.beyond[2]), __builtin_bit_cast(uint32_t, q.beyond[3])};
+        } else {
+          const auto half = [&](int j) { return (uint32_t)__builtin_bit_cast(uint16_t, q.beyond[j]); };
+          lo = u32x2{half(0) | half(1) << 16, half(2) | half(3) << 16};
+        }
+        put(piece * PIECE + (W - 1) * CHANNEL, at - first_of[W - 1], lo, hi);
+      }
+    }
+  };
+
+  // this row's channels
+  const uint64_t seed = seed_arg.value();
+  const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+  const int row = threadIdx.x >> 4, i = threadIdx.x & 15;
+  uint32_t delay[OWN], groups[OWN];   // chunk c completes group c - delay of the channel; end of the segment's groups
+  int64_t n_first[OWN];
+#pragma unroll
+  for (int c = 0; c < OWN; c++) {
+    const uint32_t m = row * OWN + c, first = first_pixel(m);
+    groups[c] = m < width ? (K - first + SGE - 1) / SGE * WPT : 0u;
+    groups[c] = groups[c] < g_end ? groups[c] : g_end;
+    delay[c] = (first + 255) >> 8;
+    n_first[c] = (((int64_t)b * g.M + m0 + m) * K + first) / GROUP;
+  }
+  uint32_t bytes[OWN][4];   // the lane's 16 bytes of each channel's super-group, in the order of their addresses
+
+  const uint32_t most = (K + SGE - 1) / STRIP_CHUNK + 1;   // no channel has anything left after so many chunks
+  const uint32_t end = g_end + WPT < most ? g_end + WPT : most;
+  auto step = [&](uint32_t chunk, Chunk& q) {
+    scatter(chunk, q);
+    if (chunk + 2 < end) load(chunk + 2, q);
+    __syncthreads();
+    uint32_t j[OWN];
+    bool due[OWN], any = false;
+#pragma unroll
+    for (int c = 0; c < OWN; c++) {
+      j[c] = chunk - delay[c];
+      due[c] = chunk >= delay[c] && j[c] < groups[c] && j[c] >= g_first;
+      any |= due[c];
+    }
+    if (__builtin_amdgcn_ballot_w64(any) == 0) {
+      __syncthreads();
+      return;
+    }
+    typename Elem<T>::Store st[OWN];
+    Stat lo[OWN], hi[OWN], sc[OWN];
+#pragma unroll
+    for (int c = 0; c < OWN; c++) {
+      lo[c] = hi[c] = (Stat)0.0f;
+      const uint32_t m = row * OWN + c;
+      const uint8_t* p = ring + (m / W) * PIECE + (m % W) * CHANNEL + (j[c] & 1) * SLOT;
+#pragma unroll
+      for (int k = 0; k < CH; k++) Elem<T>::load_chunk(reinterpret_cast<const T*>(p) + chunk_col<T>(k, i), st[c], k);
+    }
+#pragma unroll
+    for (int c = 0; c < OWN; c++) Elem<T>::group_minmax(st[c], lo[c], hi[c]);
+    {
+      const int mine = i & (OWN - 1);
+      const Stat lo_m = mine ? lo[OWN - 1] : lo[0], hi_m = mine ? hi[OWN - 1] : hi[0];
+      const Stat s_m = Elem<T>::make_scale(lo_m, hi_m, QMAX);
+      const int64_t n = (mine ? n_first[OWN - 1] + j[OWN - 1] : n_first[0] + j[0]);
+      if (i < OWN && (mine ? due[OWN - 1] : due[0]) && n < N) {
+        scale_out[n] = s_m;
+        mn_out[n] = Elem<T>::elem_of(lo_m);
+        if (mx_out) mx_out[n] = Elem<T>::elem_of(hi_m);
+      }
+      sc[0] = OWN == 1 ? s_m : row_bcast<0>(s_m);
+      if (OWN > 1) sc[OWN - 1] = row_bcast<1>(s_m);
+    }
+#pragma unroll
+    for (int c = 0; c < OWN; c++) {
+      if (due[c]) {
+        const int64_t n = n_first[c] + j[c];
+        const uint32_t ni = j[c] % WPT, shift = ni * BITS;
+        const uint32_t field = 0x01010101u * ((0xffu << shift) & 0xffu);   // what a code may reach of its byte
+        float cd[CH / 2][W];
+        if (NOISE == GACT_NOISE_FAST) {
+          FastRow<T, 1> fast;
+          fast.draws(0, n, i, k0, k1, cd);
+        }
+#pragma unroll
+        for (int k = 0; k < CH; k++) {
+          uint32_t code[W];
+          if (NOISE == GACT_NOISE_FAST) {
+            if (k < CH / 2) Elem<T>::template codes<false, false, true, false>(st[c], k, lo[c], sc[c], cd[k % (CH / 2)], code);
+            else Elem<T>::template codes<false, false, true, true>(st[c], k, lo[c], sc[c], cd[k % (CH / 2)], code);
+          } else {
+            float u[W];
+#pragma unroll
+            for (int e = 0; e < W; e++) u[e] = 0.5f;
+            Elem<T>::template codes<true, false>(st[c], k, lo[c], sc[c], u, code);
+          }
+          if (Elem<T>::kRepairsInfiniteScale && Elem<T>::scale_is_inf(sc[c])) {   // rare, see Elem<T>::kRepairsInfiniteScale
+#pragma unroll
+            for (int e = 0; e < W; e++)
+              if (Elem<T>::above(st[c], k, e, lo[c])) code[e] = 0xffu;
+          }
+#pragma unroll
+          for (int q = 0; q < W / 4; q++) {
+            const uint32_t w = (pack4(code + 4 * q) << shift) & field;
+            uint32_t& byte4 = bytes[c][k * (W / 4) + q];
+            byte4 = ni == 0 ? w : byte4 | w;
+          }
+        }
+        if (ni == WPT - 1) {
+#pragma unroll
+          for (int k = 0; k < CH; k++) {
+            uint8_t* const to = packed + n / WPT * GROUP + chunk_col<T>(k, i);
+            if constexpr (W == 4) stream_store(bytes[c][k], reinterpret_cast<uint32_t*>(to));
+            else stream_store(u32x2{bytes[c][2 * k], bytes[c][2 * k + 1]}, reinterpret_cast<u32x2*>(to));
+          }
+        }
+      }
+    }
+    __syncthreads();
+  };
+  Chunk even, odd;   // two chunks' loads in flight
+  load(g_first, even);
+  if (g_first + 1 < end) load(g_first + 1, odd);
+  for (uint32_t chunk = g_first; chunk < end; chunk += 2) {
+    step(chunk, even);
+    if (chunk + 1 < end) step(chunk + 1, odd);
+  }
 }
 
 template <typename T, int BITS, bool LARGE = false>
@@ -2936,6 +3364,171 @@ int dispatch_dequantize_groups(int64_t group, int bits, const uint8_t* packed, c
   return hipLaunchKernel(p.kernel, p.grid, p.block, args, p.lds, stream) == hipSuccess ? GACT_OK : GACT_ELAUNCH;
 }
 
+// ---- tensors that are not contiguous ----
+inline Divisor divisor(uint32_t d) {   // for numerators below 2^31
+  Divisor r{d, 0u, 0u};
+  if (d > 1) {
+    uint32_t l = 0;
+    while ((1ull << l) < d) l++;
+    r.m = (uint32_t)((1ull << (31 + l)) / d + 1);
+    r.s = l - 1;
+  }
+  return r;
+}
+// sizes and strides with dimensions of one element dropped and dimensions that lie one inside the other joined
+inline int joined_dims(int ndim, const int64_t* sizes, const int64_t* strides, int64_t (&size)[8], int64_t (&stride)[8]) {
+  int n = 0;
+  for (int d = 0; d < ndim; d++) {
+    if (sizes[d] == 1) continue;
+    if (n > 0 && stride[n - 1] == sizes[d] * strides[d]) {
+      size[n - 1] *= sizes[d];
+      stride[n - 1] = strides[d];
+    } else {
+      if (n == 8) return -1;
+      size[n] = sizes[d];
+      stride[n] = strides[d];
+      n++;
+    }
+  }
+  return n;
+}
+// Strips or tiles.  A tile's workgroup reads a piece of its own of every memory row: the longer the channels (K pixels), the
+// narrower that piece; a strip's always reads 64 bytes, but it walks its pixels in steps of about 1.5 us each, at least
+// twice the 8/bits steps of a super-group, and reads up to a super-group of pixels beyond its own.  us, tiles / strips:
+//   half [64,256,56,56] 8 bit 57 / 41  4 bit 55 / 43  2 bit 52 / 45  1 bit 54 / 52    float 4 bit 80 / 61  1 bit 155 / 89
+//   half [64,64,112,112] 8 bit 101 / 38  4 bit 99 / 36  1 bit 94 / 52    half [64,512,28,28] 8 bit 26 / 26  4 bit 23 / 31
+//   half [33,128,52,52] 8 bit 18 / 14  4 bit 18 / 18  2 bit 18 / 22  1 bit 19 / 34
+//   half [2,256,56,56]  8 bit 9 / 6  4 bit 9 / 9  2 bit 9 / 16  1 bit 11 / 26
+inline bool takes_strips(int bits, int64_t numel, int64_t K) {
+  if (K % 4 != 0) return false;
+  return bits >= 4 ? K >= 4 * (8 / bits * GROUP) : K >= 3 * (8 / bits * GROUP) / 2 && numel >= (1 << 24);
+}
+#define STRIP_WORKGROUPS 512   /* at least so many, by cutting strips into segments: more would read more beyond their own */
+// Elements of a workgroup's tile: 64 KB, two workgroups to a CU, where that leaves a tile 16 channels and more (half
+// [64,512,28,28] 4 bit 23 us against 28 with one of 144 KB), else one of up to 144 KB (half [64,256,56,56] 1 bit 54 against 64;
+// [2,256,56,56] 9 against 13); as many tiles as the workgroups that the GPU holds, or a multiple of that.
+inline int transposed_tile(size_t elem_size, int64_t numel, int64_t K) {
+  int64_t slots = 512, most = 65536 / (int64_t)elem_size;
+  if ((most < numel / slots ? most : numel / slots) < 16 * K) {
+    slots = 256;
+    most = 147456 / (int64_t)elem_size;
+  }
+  const int64_t rounds = (numel + slots * most - 1) / (slots * most);
+  return (int)(((numel + slots * rounds - 1) / (slots * rounds) + 2047) / 2048 * 2048);
+}
+template <typename T, int BITS>
+const void* quantize_gather_of(int noise_mode) {
+  return noise_mode == GACT_NOISE_CONST ? (const void*)quantize_gather_kernel<T, BITS, GACT_NOISE_CONST>
+                                        : (const void*)quantize_gather_kernel<T, BITS, GACT_NOISE_FAST>;
+}
+template <typename T, int BITS, int ROWS>
+const void* quantize_transposed_rows_of(int noise_mode) {
+  return noise_mode == GACT_NOISE_CONST ? (const void*)quantize_transposed_kernel<T, BITS, GACT_NOISE_CONST, ROWS>
+                                        : (const void*)quantize_transposed_kernel<T, BITS, GACT_NOISE_FAST, ROWS>;
+}
+template <typename T, int BITS>
+const void* quantize_transposed_of(int noise_mode, uint32_t K) {
+  if constexpr (sizeof(T) == 2)
+    if (K % 8 == 0) return quantize_transposed_rows_of<T, BITS, 8>(noise_mode);
+  if (K % 4 == 0) return quantize_transposed_rows_of<T, BITS, 4>(noise_mode);
+  return quantize_transposed_rows_of<T, BITS, 1>(noise_mode);
+}
+template <typename T, int BITS>
+const void* quantize_strips_of(int noise_mode) {
+  return noise_mode == GACT_NOISE_CONST ? (const void*)quantize_strips_kernel<T, BITS, GACT_NOISE_CONST>
+                                        : (const void*)quantize_strips_kernel<T, BITS, GACT_NOISE_FAST>;
+}
+template <typename T>
+int dispatch_quantize_strided(int n, const int64_t (&size)[8], const int64_t (&stride)[8], const T* x, int64_t numel, int bits,
+                              int noise_mode, SeedArg seed, uint8_t* packed, typename Elem<T>::Stat* scale, T* mn, T* mx,
+                              hipStream_t stream) {
+  constexpr int W = Elem<T>::kQWidth;
+  const int64_t N = (numel + GROUP - 1) / GROUP;
+  LaunchPlan p;
+  GatherShape gs;
+  TransposedShape ts;
+  StripShape ss;
+  void* shape = nullptr;
+  bool pieces = true;   // every stride but the 1 in whole pieces
+  for (int d = 0; d < n; d++) pieces = pieces && (stride[d] == 1 || stride[d] % W == 0);
+  if (!pieces || !aligned16(x) || n < 2) return GACT_ESHAPE;
+  if (stride[n - 1] == 1 && n <= 4 && size[n - 1] % W == 0 && numel / W < 0x7fffffffLL) {
+    int64_t sz[3] = {1, 1, 1}, st[3] = {0, 0, 0};   // the outer dimensions, right-aligned
+    for (int d = 0; d < n - 1; d++) {
+      if (stride[d] == 1) return GACT_ESHAPE;
+      sz[3 - (n - 1) + d] = size[d];
+      st[3 - (n - 1) + d] = stride[d] / W;
+    }
+    gs.run = divisor((uint32_t)(size[n - 1] / W));
+    gs.n2 = divisor((uint32_t)sz[2]);
+    gs.n1 = divisor((uint32_t)sz[1]);
+    gs.s0 = st[0];
+    gs.s1 = st[1];
+    gs.s2 = st[2];
+    shape = &gs;
+    row_grid(supergroups(N, bits) * (bits <= 2 ? 4 : 1), &p.grid, &p.block, bits <= 2 ? GACT_W8_THREADS : 64);
+    switch (bits) {
+      case 1: p.kernel = quantize_gather_of<T, 1>(noise_mode); break;
+      case 2: p.kernel = quantize_gather_of<T, 2>(noise_mode); break;
+      case 4: p.kernel = quantize_gather_of<T, 4>(noise_mode); break;
+      case 8: p.kernel = quantize_gather_of<T, 8>(noise_mode); break;
+    }
+  } else if (stride[n - 2] == 1 && stride[n - 1] != 1 && n <= 3 && (n == 2 || stride[0] != 1) && size[n - 2] % W == 0 &&
+             size[n - 1] < (1 << 24) && numel / size[n - 1] < 0x7fffffffLL) {
+    const int64_t sge = 8 / bits * GROUP;
+    if (takes_strips(bits, numel, size[n - 1])) {
+      ss.M = (uint32_t)size[n - 2];
+      ss.K = (uint32_t)size[n - 1];
+      ss.sk = stride[n - 1];
+      ss.sb = n == 3 ? stride[0] : 0;
+      ss.batch = n == 3 ? (uint32_t)size[0] : 1;
+      ss.strips = (ss.M + STRIP_PIECES * W - 1) / (STRIP_PIECES * W);
+      const int64_t strips = (int64_t)ss.strips * ss.batch, per_channel = (ss.K + sge - 1) / sge;
+      int64_t segments = (STRIP_WORKGROUPS + strips - 1) / strips;
+      segments = segments < per_channel ? segments : per_channel;
+      ss.segment = (uint32_t)((per_channel + segments - 1) / segments);
+      ss.segments = (uint32_t)((per_channel + ss.segment - 1) / ss.segment);
+      shape = &ss;
+      p.grid = dim3((unsigned)(strips * ss.segments));
+      p.block = dim3(STRIP_THREADS);
+      switch (bits) {
+        case 1: p.kernel = quantize_strips_of<T, 1>(noise_mode); break;
+        case 2: p.kernel = quantize_strips_of<T, 2>(noise_mode); break;
+        case 4: p.kernel = quantize_strips_of<T, 4>(noise_mode); break;
+        case 8: p.kernel = quantize_strips_of<T, 8>(noise_mode); break;
+      }
+      void* args[] = {(void*)&seed, (void*)&x, (void*)&numel, (void*)&N, (void*)&packed, (void*)&scale, (void*)&mn, (void*)&mx, shape};
+      return hipLaunchKernel(p.kernel, p.grid, p.block, args, p.lds, stream) == hipSuccess ? GACT_OK : GACT_ELAUNCH;
+    }
+    ts.M = (uint32_t)size[n - 2];
+    ts.K = (uint32_t)size[n - 1];
+    ts.sk = stride[n - 1];
+    ts.sb = n == 3 ? stride[0] : 0;
+    ts.channels = numel / size[n - 1];
+    ts.tile = transposed_tile(sizeof(T), numel, size[n - 1]);
+    // a tile's rows and batch entries have to lie within 4 GB of its first entry
+    const int64_t entries = ts.tile / ((int64_t)ts.M * ts.K) + 2;
+    if ((entries * ts.sb + (int64_t)ts.K * ts.sk + ts.M) * (int64_t)sizeof(T) > 0xffffffffLL) return GACT_ESHAPE;
+    shape = &ts;
+    p.lds = tile_bytes<T>(ts.tile);
+    p.grid = dim3((unsigned)((numel + ts.tile - 1) / ts.tile));
+    p.block = dim3(TRANSPOSED_THREADS);
+    switch (bits) {
+      case 1: p.kernel = quantize_transposed_of<T, 1>(noise_mode, ts.K); break;
+      case 2: p.kernel = quantize_transposed_of<T, 2>(noise_mode, ts.K); break;
+      case 4: p.kernel = quantize_transposed_of<T, 4>(noise_mode, ts.K); break;
+      case 8: p.kernel = quantize_transposed_of<T, 8>(noise_mode, ts.K); break;
+    }
+    if (p.lds > 65536 &&
+        hipFuncSetAttribute(p.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds) != hipSuccess)
+      return GACT_ELAUNCH;
+  } else {
+    return GACT_ESHAPE;
+  }
+  void* args[] = {(void*)&seed, (void*)&x, (void*)&numel, (void*)&N, (void*)&packed, (void*)&scale, (void*)&mn, (void*)&mx, shape};
+  return hipLaunchKernel(p.kernel, p.grid, p.block, args, p.lds, stream) == hipSuccess ? GACT_OK : GACT_ELAUNCH;
+}
+
 template <typename T>
 void launch_minimax_any(const T* x, int64_t N, int64_t D, T* mn, T* mx, hipStream_t stream) {
   const bool vec = aligned16(x);  // D % 32 == 0 keeps every row 16-byte aligned once the base is
@@ -3193,6 +3786,35 @@ int gact_dequantize_groups(const void* packed, int bits, const void* scale, cons
   if (dtype == GACT_F32)
     return dispatch_dequantize_groups<float>(group, bits, (const uint8_t*)packed, (const float*)scale, (const float*)mn, numel, N, (float*)out, s);
   return dispatch_dequantize_groups<f16>(group, bits, (const uint8_t*)packed, (const f16*)scale, (const f16*)mn, numel, N, (f16*)out, s);
+}
+
+int gact_quantize_strided(const void* x, int dtype, int ndim, const int64_t* sizes, const int64_t* strides, int bits, int noise_mode,
+                          uint64_t seed, const uint64_t* seed_add, void* packed, void* scale, void* mn, void* mx, void* stream) {
+  if (dtype != GACT_F32 && dtype != GACT_F16 && dtype != GACT_BF16) return GACT_EINVAL;
+  if (!valid_bits(bits) || ndim < 0 || (ndim > 0 && (!sizes || !strides))) return GACT_EINVAL;
+  if (noise_mode < GACT_NOISE_CONST || noise_mode > GACT_NOISE_FAST) return GACT_EINVAL;
+  if (noise_mode != GACT_NOISE_CONST && noise_mode != GACT_NOISE_FAST) return GACT_ESHAPE;
+  int64_t numel = 1;
+  for (int d = 0; d < ndim; d++) {
+    if (sizes[d] < 0 || strides[d] < 0) return GACT_EINVAL;
+    numel *= sizes[d];
+  }
+  if (numel == 0) return GACT_OK;
+  int64_t size[8], stride[8];
+  const int n = joined_dims(ndim, sizes, strides, size, stride);
+  if (n < 0) return GACT_ESHAPE;
+  if (n == 0 || (n == 1 && stride[0] == 1))
+    return gact_quantize_seeded(x, dtype, numel, bits, noise_mode, seed, seed_add, nullptr, packed, scale, mn, mx, stream);
+  if (!x || !packed || !scale || !mn) return GACT_EINVAL;
+  if (!aligned16(packed) || (reinterpret_cast<uintptr_t>(seed_add) & 7u)) return GACT_EALIGN;
+  hipStream_t s = (hipStream_t)stream;
+  fresh_launch();
+  const SeedArg sa{seed, seed_add};
+  if (dtype == GACT_F32)
+    return dispatch_quantize_strided<float>(n, size, stride, (const float*)x, numel, bits, noise_mode, sa, (uint8_t*)packed, (float*)scale, (float*)mn, (float*)mx, s);
+  if (dtype == GACT_BF16)
+    return dispatch_quantize_strided<bf16>(n, size, stride, (const bf16*)x, numel, bits, noise_mode, sa, (uint8_t*)packed, (float*)scale, (bf16*)mn, (bf16*)mx, s);
+  return dispatch_quantize_strided<f16>(n, size, stride, (const f16*)x, numel, bits, noise_mode, sa, (uint8_t*)packed, (f16*)scale, (f16*)mn, (f16*)mx, s);
 }
 
 int gact_launch_geometry(int kind, int dtype, int bits, int64_t N, int* threads, int* lds_bytes, int* workgroups_per_cu) {

@@ -12,6 +12,7 @@ _LIB = None
 LIB_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "lib", "libgact_hip.so")
 
 F32, F16, BF16 = 0, 1, 2
+ESHAPE = -3
 NOISE_CONST, NOISE_INJECT, NOISE_REF, NOISE_FAST = 0, 1, 2, 3
 NOISE_MODES = {"deterministic": NOISE_CONST, "inject": NOISE_INJECT, "reference": NOISE_REF, "fast": NOISE_FAST}
 GROUP = 256
@@ -49,6 +50,7 @@ SIGNATURES = {
     "gact_dequantize": (_i32, [_vp, _i32, _vp, _vp, _i32, _i64, _vp, _vp]),
     "gact_quantize_groups": (_i32, [_vp, _i32, _i64, _i32, _i32, _i32, _u64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "gact_dequantize_groups": (_i32, [_vp, _i32, _vp, _vp, _i32, _i64, _i32, _vp, _vp]),
+    "gact_quantize_strided": (_i32, [_vp, _i32, _i32, _vp, _vp, _i32, _i32, _u64, _vp, _vp, _vp, _vp, _vp, _vp]),
     "gact_launch_geometry": (_i32, [_i32, _i32, _i32, _i64, _vp, _vp, _vp]),
     "gact_mask_pack": (_i32, [_vp, _i64, _vp, _vp]),
     "gact_mask_unpack": (_i32, [_vp, _i64, _vp, _vp]),

@@ -7,7 +7,9 @@ instead of a concatenated copy.  ``op_dequantize`` writes straight into a tensor
 shape.  The extension-style entry points (minimax, pack_single_precision, unpack_single_precision)
 stay available in gact.cpp_extension for callers that use them directly.
 """
+import ctypes
 import math
+
 import torch
 
 from .conf import config
@@ -24,11 +26,10 @@ def _num_groups(numel):
     return (numel + config.group_size - 1) // config.group_size
 
 
-def _fused(dtype):
+def _one_pass(group, dtype):
     """The single-pass kernels are built for groups of 256, and 64, 128 and 512 for float and half; any other
     config.group_size takes the extension-style sequence minimax -> pack / unpack on the zero-padded tensor, as the
     reference does."""
-    group = config.group_size
     return group == _abi.GROUP or (group in _abi.ONE_PASS_GROUPS and dtype is not torch.bfloat16)
 
 
@@ -52,8 +53,9 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
         q_scale = input_groups.max(dim=-1, keepdim=True).values - q_min
         return input_groups, q_scale, q_min
 
-    if not _fused(input.dtype) or (config.group_size != _abi.GROUP and noise is None
-                                   and (rng_stream or config.rng_stream) == "reference"):
+    group = config.group_size
+    if group != _abi.GROUP and (not _one_pass(group, input.dtype)
+                                or (noise is None and (rng_stream or config.rng_stream) == "reference")):
         if seed_offset is not None:
             raise RuntimeError("seed_offset needs the single-pass kernels (config.group_size 64, 128, 256 or 512)")
         from .cpp_extension import minimax as ext_minimax
@@ -71,10 +73,6 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
         raise RuntimeError("The type of data is not correct!")
     ext_quantization._check_bits(q_bit)
     seed = ext_quantization._seed_u64(seed)
-    # the reference's reshape copies a non-contiguous input as well
-    x = input if input.is_contiguous() else input.contiguous()
-    if x.data_ptr() & 15:
-        x = x.clone()
     if noise is None and rng_stream is None:
         mode = _abi.NOISE_MODES.get(config.rng_stream)
         if mode is None:
@@ -85,8 +83,7 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
             if (not noise.is_cuda) or noise.dtype != torch.float32 or noise.numel() != N * config.group_size \
                     or not noise.is_contiguous():
                 raise RuntimeError("noise must be a contiguous float32 CUDA tensor with one value per padded element")
-    device = x.device
-    group = config.group_size
+    device = input.device
     q_input = torch.empty(ext_quantization.packed_numel(q_bit, N, 1, group), dtype=torch.int8, device=device)
     # bfloat16 (not in the reference) is quantized as the float values it holds: float scale, bfloat16 min
     q_scale = torch.empty((N, 1, 1), dtype=torch.float32 if dtype is torch.bfloat16 else dtype, device=device)
@@ -94,10 +91,37 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
     if seed_offset is not None:
         if seed_offset.dtype is not torch.int64 or seed_offset.numel() != 1 or seed_offset.device != device:
             raise RuntimeError("seed_offset must be one int64 on the device of the data")
+    if input.is_contiguous():
+        x = input
+    elif group == _abi.GROUP and mode in (_abi.NOISE_FAST, _abi.NOISE_CONST) \
+            and _quantize_strided(input, q_bit, mode, seed, seed_offset, q_input, q_scale, q_min):
+        return q_input, q_scale, q_min
+    else:
+        x = input.contiguous()      # as the reference's reshape does
+    if x.data_ptr() & 15:
+        x = x.clone()
+    if group == _abi.GROUP and seed_offset is None:
+        _abi.call_on(device, _abi.lib().gact_quantize, x.data_ptr(), _abi.dtype_code(dtype), x.numel(), q_bit, mode, seed,
+                     None if noise is None else noise.data_ptr(), q_input.data_ptr(), q_scale.data_ptr(), q_min.data_ptr(), None,
+                     _current_stream(device.index))
+        return q_input, q_scale, q_min
     _abi.call_on(device, _abi.lib().gact_quantize_groups, x.data_ptr(), _abi.dtype_code(dtype), x.numel(), group, q_bit, mode,
-                 seed, _abi.ptr(seed_offset), _abi.ptr(noise), q_input.data_ptr(), q_scale.data_ptr(), q_min.data_ptr(), None,
-                 _current_stream(device.index))
+                 seed, None if seed_offset is None else seed_offset.data_ptr(), None if noise is None else noise.data_ptr(),
+                 q_input.data_ptr(), q_scale.data_ptr(), q_min.data_ptr(), None, _current_stream(device.index))
     return q_input, q_scale, q_min
+
+
+def _quantize_strided(input, q_bit, mode, seed, seed_offset, q_input, q_scale, q_min):
+    """Compress a tensor that is not contiguous where it lies; False where the kernels do not take its layout."""
+    dims = ctypes.c_int64 * input.dim()
+    with torch.cuda.device(input.device):
+        code = _abi.lib().gact_quantize_strided(input.data_ptr(), _abi.dtype_code(input.dtype), input.dim(), dims(*input.shape),
+                                                dims(*input.stride()), q_bit, mode, seed, _abi.ptr(seed_offset), q_input.data_ptr(),
+                                                q_scale.data_ptr(), q_min.data_ptr(), None, _current_stream(input.device.index))
+    if code == _abi.ESHAPE:
+        return False
+    _abi.check(code)
+    return True
 
 
 def dequantize_and_unpack(data, shape, q_bit, scale, mn):
@@ -148,7 +172,8 @@ def op_dequantize(input, input_shape):
     if q_bit == 32:
         return q_input.ravel()[:num_features].reshape(*input_shape).contiguous()
 
-    if not _fused(q_min.dtype):
+    group = config.group_size
+    if group != _abi.GROUP and not _one_pass(group, q_min.dtype):
         groups = dequantize_and_unpack(q_input, input_shape, q_bit, q_scale, q_min)
         return groups.ravel()[:num_features].reshape(*input_shape).contiguous()
 
@@ -157,8 +182,7 @@ def op_dequantize(input, input_shape):
         raise RuntimeError("data must be a CUDA tensor!")
     if q_input.dtype is not torch.int8 or q_input.dim() != 1:
         raise RuntimeError("The type of data is not correct!")
-    group = config.group_size
-    N = _num_groups(num_features)
+    N = (num_features + group - 1) // group
     if q_input.numel() < ext_quantization.packed_numel(q_bit, N, 1, group) - 1 \
             or q_scale.numel() < N or q_min.numel() < N:
         raise RuntimeError("packed data / scale / min are too short for shape %s" % (tuple(input_shape),))
@@ -167,6 +191,10 @@ def op_dequantize(input, input_shape):
         raise RuntimeError("expected scalar type of min to match scale")
     device = q_input.device
     out = torch.empty(tuple(input_shape), dtype=dtype, device=device)
+    if group == _abi.GROUP:
+        _abi.call_on(device, _abi.lib().gact_dequantize, q_input.data_ptr(), q_bit, q_scale.data_ptr(), q_min.data_ptr(),
+                     _abi.dtype_code(dtype), num_features, out.data_ptr(), _current_stream(device.index))
+        return out
     _abi.call_on(device, _abi.lib().gact_dequantize_groups, q_input.data_ptr(), q_bit, q_scale.data_ptr(), q_min.data_ptr(),
                  _abi.dtype_code(dtype), num_features, group, out.data_ptr(), _current_stream(device.index))
     return out

@@ -100,6 +100,16 @@ int gact_quantize_groups(const void* x, int dtype, int64_t numel, int group, int
 int gact_dequantize_groups(const void* packed, int bits, const void* scale, const void* mn, int dtype, int64_t numel, int group,
                            void* out, void* stream);
 
+/* gact_quantize_seeded for a tensor that is not contiguous: `ndim` sizes and strides (in elements), the groups being
+ * consecutive elements in index order, as in a contiguous copy of the tensor - which this entry point saves.  Taken: tensors
+ * whose innermost runs are contiguous and whole 16-byte pieces (at most three more dimensions once those that lie one inside
+ * the other are joined), and tensors whose last but one dimension is the contiguous one (channels-last activations,
+ * transposed matrices; at most one more dimension), both with 16-byte aligned base and strides; streams GACT_NOISE_CONST and
+ * GACT_NOISE_FAST.  Anything else: GACT_ESHAPE and no launch - make a contiguous copy.  No counterpart in the reference, whose
+ * reshape copies (gact/gact/ops.py:12-19). */
+int gact_quantize_strided(const void* x, int dtype, int ndim, const int64_t* sizes, const int64_t* strides, int bits, int noise_mode,
+                          uint64_t seed, const uint64_t* seed_add, void* packed, void* scale, void* mn, void* mx, void* stream);
+
 /* What a gact_quantize (kind 0; fast, deterministic or injected noise) or gact_dequantize (kind 1) launch of a tensor of
  * N groups is made of, without launching anything: the threads of a workgroup, the dynamic LDS the launch asks for -
  * on large tensors some kernels ask for LDS they never touch, which is how the library caps their occupancy - and

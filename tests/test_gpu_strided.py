@@ -1,0 +1,92 @@
+"""Tensors that are not contiguous, quantized where they lie, against the same tensor made contiguous first (whose kernels
+the oracle pins): codes, scale and minimum bit for bit.  Layouts the kernels take (contiguous runs; the last but one dimension
+contiguous) at sizes that end inside a group, a super-group and a tile, and layouts they decline."""
+import ctypes
+
+import pytest
+import torch
+
+from gact import ops
+from gact.cpp_extension import _abi
+
+pytestmark = pytest.mark.gpu
+
+
+def channels_last(n, c, h, w):
+    return lambda g: torch.randn((n, c, h, w), generator=g).contiguous(memory_format=torch.channels_last)
+
+
+def heads(b, s, h, d):
+    return lambda g: torch.randn((b, s, h, d), generator=g).permute(0, 2, 1, 3)
+
+
+def keys(b, s, h, d):
+    return lambda g: torch.randn((b, s, h, d), generator=g).permute(0, 2, 3, 1)
+
+
+# name -> (tensor on the CPU, whether the kernels take it at 16-byte pieces of 8 elements)
+LAYOUTS = {
+    "channels_last_7x7": (channels_last(3, 512, 7, 7), True),
+    "channels_last_14x14": (channels_last(2, 256, 14, 14), True),
+    "channels_last_28x28": (channels_last(1, 72, 28, 28), True),
+    "channels_last_56x56": (channels_last(2, 64, 56, 56), True),
+    "channels_last_45x45": (channels_last(5, 24, 45, 45), True),       # an odd number of pixels
+    "channels_last_224x224": (channels_last(1, 8, 224, 224), True),     # a channel of more than a tile
+    "channels_last_one_group": (channels_last(1, 8, 3, 3), True),
+    "channels_last_rgb": (channels_last(4, 3, 32, 32), False),
+    "matrix_transposed": (lambda g: torch.randn((1000, 328), generator=g).t(), True),
+    "matrix_transposed_tall": (lambda g: torch.randn((24, 5000), generator=g).t(), True),
+    "matrix_columns": (lambda g: torch.randn((777, 4 * 136), generator=g)[:, 136:2 * 136], True),
+    "matrix_odd_columns": (lambda g: torch.randn((777, 500), generator=g)[:, 3:100], False),
+    "heads_64": (heads(4, 197, 12, 64), True),
+    "heads_80": (heads(2, 100, 4, 80), True),
+    "heads_8": (heads(1, 3, 2, 8), True),
+    "heads_20": (heads(2, 33, 3, 20), False),                           # 20 halves are not whole pieces (20 floats are)
+    "qkv_query": (lambda g: torch.randn((3, 65, 3, 4, 32), generator=g).permute(2, 0, 3, 1, 4)[0], True),
+    "keys_transposed": (keys(3, 77, 4, 32), True),
+    "keys_transposed_sliced": (lambda g: torch.randn((3, 77, 8, 32), generator=g)[:, :, 2:6].permute(0, 2, 3, 1), True),
+    "expanded": (lambda g: torch.randn((5, 1, 256), generator=g).expand(5, 7, 256), True),
+    "rows_of_every_other": (lambda g: torch.randn((64, 300), generator=g)[:, ::2], False),
+}
+
+
+@pytest.mark.parametrize("layout", sorted(LAYOUTS))
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["f32", "f16", "bf16"])
+def test_strided_equals_contiguous(layout, dtype):
+    make, taken = LAYOUTS[layout]
+    x_cpu = make(torch.Generator().manual_seed(len(layout)))
+    # convert in the layout's own storage, so that the tensor on the GPU has the same strides
+    x = torch.empty(0)
+    base = x_cpu._base if x_cpu._base is not None else x_cpu
+    x = base.to(dtype).cuda().as_strided(x_cpu.shape, x_cpu.stride(), x_cpu.storage_offset()) \
+        if base is not x_cpu else x_cpu.to(dtype).cuda()
+    assert x.stride() == x_cpu.stride() and not x.is_contiguous()
+    y = x.contiguous()
+    N = -(-x.numel() // 256)
+    for bits in (1, 2, 4, 8):
+        for stream in ("fast", "deterministic", "reference"):
+            a, b = ops.op_quantize(x, bits, 11, rng_stream=stream), ops.op_quantize(y, bits, 11, rng_stream=stream)
+            where = "%s %d bit %s" % (layout, bits, stream)
+            assert torch.equal(a[0][:-1], b[0][:-1]), where
+            assert torch.equal(a[2], b[2]) and torch.equal(a[3], b[3]), where
+            assert torch.equal(ops.op_dequantize(a, x.shape), ops.op_dequantize(b, x.shape)), where
+        if dtype != torch.float32:      # and the launch was not declined (or was, and fell back to the copy)
+            dims = ctypes.c_int64 * x.dim()
+            rc = _abi.lib().gact_quantize_strided(x.data_ptr(), _abi.dtype_code(dtype), x.dim(), dims(*x.shape), dims(*x.stride()), bits,
+                                                  _abi.NOISE_FAST, 11, None, a[0].data_ptr(), a[2].data_ptr(), a[3].data_ptr(), None,
+                                                  torch.cuda.current_stream().cuda_stream)
+            assert rc == (0 if taken else _abi.ESHAPE), layout
+    assert a[2].numel() == N
+
+
+def test_strided_large_tensors():
+    """Sizes at which a workgroup's tile is the largest, with every XCD's runs of tiles and a ragged last one."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    for shape in ((5, 256, 112, 112), (40, 1000, 28, 28), (31, 64, 56, 56), (300, 2048, 7, 7)):
+        x = torch.randn(shape, generator=g, device="cuda").to(torch.float16).contiguous(memory_format=torch.channels_last)
+        for y in (x, x.float()):
+            a, b = ops.op_quantize(y, 4, 3), ops.op_quantize(y.contiguous(), 4, 3)
+            assert torch.equal(a[0][:-1], b[0][:-1]) and torch.equal(a[2], b[2]) and torch.equal(a[3], b[3]), shape
+    x = torch.randn((64, 197, 12, 64), generator=g, device="cuda").to(torch.bfloat16).permute(0, 2, 1, 3)
+    a, b = ops.op_quantize(x, 2, 3), ops.op_quantize(x.contiguous(), 2, 3)
+    assert torch.equal(a[0][:-1], b[0][:-1]) and torch.equal(a[2], b[2]) and torch.equal(a[3], b[3])
