@@ -31,7 +31,7 @@ def build(force=False):
 
 def build_ref(reference="/root/reference"):
     """Compile oracle/_ref from the reference checkout; returns False when it is absent."""
-    if not os.path.isdir(reference):
+    if not os.path.exists(os.path.join(reference, "gact", "gact", "cpp_extension", "calc_precision.cc")):
         return False
     subprocess.run(["make", "-C", _HERE, "ref", "REFERENCE=" + reference], check=True)
     return True
