@@ -1,5 +1,6 @@
 """Build libgact_hip.so (the C-ABI library of HIP kernels) and libgact_probe.so (compute-free traffic probes that
-bench.py measures beside the kernels) for gfx950 with hipcc.
+bench.py measures beside the kernels) for gfx950 with hipcc, and gact_torch.so (the operators' host side on torch tensors,
+which calls libgact_hip.so) with the host compiler.
 
     python gact-icml_amd/build.py            # build if the sources are newer than the library
     python gact-icml_amd/build.py --force
@@ -19,6 +20,8 @@ PROBE_SRC = os.path.join(HERE, "csrc", "stream_probe.hip")   # compute-free traf
 HDR = os.path.join(ROOT, "include", "gact_hip.h")
 OUT_DIR = os.path.join(HERE, "gact", "lib")
 OUT = os.path.join(OUT_DIR, "libgact_hip.so")
+TORCH_SRC = os.path.join(HERE, "csrc", "torch_ops.cpp")
+TORCH_OUT = os.path.join(OUT_DIR, "gact_torch.so")
 PROBE_OUT = os.path.join(OUT_DIR, "libgact_probe.so")
 
 HIPCC_FLAGS = [
@@ -49,10 +52,28 @@ def hipcc():
 
 
 def up_to_date():
-    if not os.path.exists(OUT) or not os.path.exists(PROBE_OUT):
+    built = (OUT, PROBE_OUT, TORCH_OUT)
+    if not all(os.path.exists(p) for p in built):
         return False
-    t = min(os.path.getmtime(OUT), os.path.getmtime(PROBE_OUT))
-    return all(os.path.getmtime(p) <= t for p in (SRC, PROBE_SRC, HDR, os.path.abspath(__file__)))
+    t = min(os.path.getmtime(p) for p in built)
+    return all(os.path.getmtime(p) <= t for p in (SRC, PROBE_SRC, TORCH_SRC, HDR, os.path.abspath(__file__)))
+
+
+def torch_command():
+    """The host compiler's line for gact_torch.so: torch's headers and libraries, ROCm's headers, Python's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-I", os.path.join(ROOT, "include")]
+    for path in cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", path]
+    # libtorch.so itself stays out: it would pull in every library torch was built with
+    return cmd + ["-o", TORCH_OUT, TORCH_SRC, "-L", OUT_DIR, "-l:libgact_hip.so", "-L", libs, "-ltorch_python", "-ltorch_cpu", "-lc10",
+                  "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
 
 
 def build(force=False, extra=()):
@@ -62,6 +83,7 @@ def build(force=False, extra=()):
     cmd = [hipcc()] + HIPCC_FLAGS + list(extra) + ["-I", os.path.join(ROOT, "include"), "-o", OUT, SRC]
     subprocess.run(cmd, check=True)
     subprocess.run([hipcc()] + HIPCC_FLAGS + ["-o", PROBE_OUT, PROBE_SRC], check=True)
+    subprocess.run(torch_command(), check=True)
     return OUT
 
 

@@ -1,0 +1,321 @@
+// The host side of the operators: what Python did for every saved tensor - look at the arguments, allocate the results
+// with torch, find the stream, call the library - in one native call.
+//
+// Every function answers the ordinary call: plain tensors on the GPU, contiguous and aligned as the kernels need, no mode or
+// transform of torch's active.  Anything else, an argument that has to be refused included, gets None and nothing is
+// launched: the Python operator then takes its general path, which accepts or raises as it always did.
+//
+// Arguments come through the C API's fast call and tensors through torch's own wrap / unpack (no pybind11).
+#include <torch/csrc/python_headers.h>
+
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/core/Tensor.h>
+#include <ATen/ops/empty.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstdint>
+#include <cstring>
+
+#include "gact_hip.h"
+
+namespace {
+
+constexpr int64_t kGroup = 256;
+
+// torch.empty, called below, would mean something else: a mode that looks at every call, a transform, a trace
+bool ordinary_call() {
+  static const c10::DispatchKeySet special({c10::DispatchKey::Python, c10::DispatchKey::Functionalize, c10::DispatchKey::Tracer,
+                                            c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::FuncTorchVmapMode});
+  return !c10::impl::tls_local_dispatch_key_set().included_.has_any(special) && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+         !at::impl::torch_function_mode_enabled();
+}
+
+// a tensor (or parameter) itself, no subclass and no wrapper, dense on the GPU
+const at::Tensor* plain(PyObject* o) {
+  if (!THPVariable_CheckExact(o)) return nullptr;
+  const at::Tensor& t = THPVariable_Unpack(o);
+  static const c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::Functionalize, c10::DispatchKey::ZeroTensor,
+                                            c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper});
+  if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || !t.has_storage() || t.key_set().has_any(wrapped)) return nullptr;
+  return &t;
+}
+
+int dtype_code(at::ScalarType t) {
+  switch (t) {
+    case at::kFloat: return GACT_F32;
+    case at::kHalf: return GACT_F16;
+    case at::kBFloat16: return GACT_BF16;
+    default: return -1;
+  }
+}
+bool float_or_half(const at::Tensor& t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kHalf; }
+
+bool integer(PyObject* o, int64_t* v) {   // an int and nothing else (no bool)
+  if (!PyLong_CheckExact(o)) return false;
+  int overflow = 0;
+  *v = PyLong_AsLongLongAndOverflow(o, &overflow);
+  return overflow == 0;
+}
+bool width(PyObject* o, int* bits) {
+  int64_t v;
+  if (!integer(o, &v) || (v != 1 && v != 2 && v != 4 && v != 8)) return false;
+  *bits = (int)v;
+  return true;
+}
+bool seed_of(PyObject* o, uint64_t* seed) {   // the reference's binding takes an int and widens it
+  int64_t v;
+  if (!integer(o, &v) || v < INT32_MIN || v > INT32_MAX) return false;
+  *seed = (uint64_t)v;
+  return true;
+}
+// what the kernels draw without further inputs; a stream's name that is not known arrives as -1
+bool noise_mode(PyObject* o, int* mode) {
+  int64_t v;
+  if (!integer(o, &v) || (v != GACT_NOISE_CONST && v != GACT_NOISE_REF && v != GACT_NOISE_FAST)) return false;
+  *mode = (int)v;
+  return true;
+}
+// elements of the packed tensor: the reference allocates one byte more than is ever written
+int64_t packed_numel(int bits, int64_t N, int64_t row) {
+  const int64_t wpt = 8 / bits;
+  return (bits * ((N + wpt - 1) / wpt * wpt) * row + 8) / 8;
+}
+
+at::Tensor make(c10::IntArrayRef shape, at::ScalarType dtype, c10::Device device) {
+  return at::empty(shape, at::TensorOptions().dtype(dtype).device(device));
+}
+void* stream_on(c10::Device device) { return c10::hip::getCurrentHIPStream(device.index()).stream(); }
+const void* in(const at::Tensor& t) { return t.const_data_ptr(); }
+void* out(const at::Tensor& t) { return t.mutable_data_ptr(); }
+
+// The library's call with the GIL released and the data's device current
+template <typename F>
+int on(c10::Device device, const F& call) {
+  const c10::DeviceGuard guard(device);
+  void* const stream = stream_on(device);
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = call(stream);
+  Py_END_ALLOW_THREADS
+  return rc;
+}
+
+PyObject* tuple_of(std::initializer_list<at::Tensor> tensors) {
+  PyObject* const t = PyTuple_New((Py_ssize_t)tensors.size());
+  if (!t) return nullptr;
+  Py_ssize_t i = 0;
+  for (const at::Tensor& e : tensors) {
+    PyObject* const w = THPVariable_Wrap(e);
+    if (!w) {
+      Py_DECREF(t);
+      return nullptr;
+    }
+    PyTuple_SET_ITEM(t, i++, w);
+  }
+  return t;
+}
+
+bool one_pass(int64_t group, int dtype) { return group == kGroup || ((group == 64 || group == 128 || group == 512) && dtype != GACT_BF16); }
+
+// quantize(x, bits, seed, noise mode, group size) -> (codes, scale, min); False: the layout is not one that is taken in place
+PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  int bits, mode;
+  uint64_t seed;
+  int64_t group;
+  const at::Tensor* x;
+  if (n != 5 || !(x = plain(args[0])) || !width(args[1], &bits) || !seed_of(args[2], &seed) || !noise_mode(args[3], &mode) ||
+      !integer(args[4], &group) || !ordinary_call())
+    Py_RETURN_NONE;
+  const int dtype = dtype_code(x->scalar_type());
+  const int64_t numel = x->numel();
+  if (dtype < 0 || numel == 0 || !one_pass(group, dtype) || (group != kGroup && mode == GACT_NOISE_REF)) Py_RETURN_NONE;
+  const bool contiguous = x->is_contiguous();
+  if (contiguous ? (reinterpret_cast<uintptr_t>(in(*x)) & 15u) != 0 : (group != kGroup || mode == GACT_NOISE_REF)) Py_RETURN_NONE;
+  const int64_t N = (numel + group - 1) / group;
+  const c10::Device device = x->device();
+  const at::Tensor codes = make({packed_numel(bits, N, group)}, at::kChar, device);
+  const at::Tensor scale = make({N, 1, 1}, dtype == GACT_BF16 ? at::kFloat : x->scalar_type(), device);
+  const at::Tensor mn = make({N, 1, 1}, x->scalar_type(), device);
+  const int rc = on(device, [&](void* stream) {
+    if (!contiguous)
+      return gact_quantize_strided(in(*x), dtype, (int)x->dim(), x->sizes().data(), x->strides().data(), bits, mode, seed, nullptr,
+                                   out(codes), out(scale), out(mn), nullptr, stream);
+    if (group == kGroup)
+      return gact_quantize(in(*x), dtype, numel, bits, mode, seed, nullptr, out(codes), out(scale), out(mn), nullptr, stream);
+    return gact_quantize_groups(in(*x), dtype, numel, (int)group, bits, mode, seed, nullptr, nullptr, out(codes), out(scale), out(mn),
+                                nullptr, stream);
+  });
+  if (rc == GACT_OK) return tuple_of({codes, scale, mn});
+  if (!contiguous && rc == GACT_ESHAPE) Py_RETURN_FALSE;
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// dequantize(codes, shape, bits, scale, min, group size) -> tensor of that shape
+PyObject* dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  int bits;
+  int64_t group;
+  const at::Tensor *codes, *scale, *mn;
+  if (n != 6 || !(codes = plain(args[0])) || !PyTuple_Check(args[1]) || !width(args[2], &bits) || !(scale = plain(args[3])) ||
+      !(mn = plain(args[4])) || !integer(args[5], &group) || !ordinary_call())
+    Py_RETURN_NONE;
+  const int dtype = dtype_code(mn->scalar_type());
+  const c10::Device device = codes->device();
+  if (dtype < 0 || !one_pass(group, dtype) || codes->scalar_type() != at::kChar || codes->dim() != 1 || scale->device() != device ||
+      mn->device() != device || scale->scalar_type() != (dtype == GACT_BF16 ? at::kFloat : mn->scalar_type()))
+    Py_RETURN_NONE;
+  const Py_ssize_t dims = PyTuple_GET_SIZE(args[1]);
+  int64_t numel = 1;
+  c10::SmallVector<int64_t, 8> shape;
+  for (Py_ssize_t d = 0; d < dims; d++) {
+    int64_t size;
+    if (!integer(PyTuple_GET_ITEM(args[1], d), &size) || size <= 0 || __builtin_mul_overflow(numel, size, &numel)) Py_RETURN_NONE;
+    shape.push_back(size);
+  }
+  if (numel > INT64_MAX / 2) Py_RETURN_NONE;
+  const int64_t N = (numel + group - 1) / group;
+  if (codes->numel() < packed_numel(bits, N, group) - 1 || scale->numel() < N || mn->numel() < N) Py_RETURN_NONE;
+  const at::Tensor data = make(shape, mn->scalar_type(), device);
+  const int rc = on(device, [&](void* stream) {
+    if (group == kGroup) return gact_dequantize(in(*codes), bits, in(*scale), in(*mn), dtype, numel, out(data), stream);
+    return gact_dequantize_groups(in(*codes), bits, in(*scale), in(*mn), dtype, numel, (int)group, out(data), stream);
+  });
+  if (rc == GACT_OK) return THPVariable_Wrap(data);
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// minimax(data[N, D]) -> (min[N], max[N])
+PyObject* minimax(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  const at::Tensor* x;
+  if (n != 1 || !(x = plain(args[0])) || !x->is_contiguous() || !float_or_half(*x) || x->dim() != 2 || x->numel() == 0 || !ordinary_call())
+    Py_RETURN_NONE;
+  const int64_t N = x->size(0), D = x->size(1);
+  if (D % 32 != 0 || D <= 32) Py_RETURN_NONE;
+  const c10::Device device = x->device();
+  const at::Tensor mn = make({N}, x->scalar_type(), device), mx = make({N}, x->scalar_type(), device);
+  const int rc = on(device, [&](void* stream) { return gact_minimax(in(*x), dtype_code(x->scalar_type()), N, D, out(mn), out(mx), stream); });
+  if (rc == GACT_OK) return tuple_of({mn, mx});
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// pack(data[N, G, D], min, max, bits, seed, noise mode) -> (codes, scale[N, G, 1])
+PyObject* pack(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  int bits, mode;
+  uint64_t seed;
+  const at::Tensor *x, *mn, *mx;
+  if (n != 6 || !(x = plain(args[0])) || !(mn = plain(args[1])) || !(mx = plain(args[2])) || !width(args[3], &bits) ||
+      !seed_of(args[4], &seed) || !noise_mode(args[5], &mode) || !ordinary_call())
+    Py_RETURN_NONE;
+  const c10::Device device = x->device();
+  for (const at::Tensor* t : {x, mn, mx})
+    if (!t->is_contiguous() || t->dim() != 3 || t->scalar_type() != x->scalar_type() || t->device() != device) Py_RETURN_NONE;
+  const int64_t N = x->size(0), G = x->size(1), D = x->size(2);
+  if (!float_or_half(*x) || x->numel() == 0 || mn->numel() != N * G || mx->numel() != N * G) Py_RETURN_NONE;
+  const at::Tensor codes = make({packed_numel(bits, N, G * D)}, at::kChar, device), scale = make({N, G, 1}, x->scalar_type(), device);
+  const int rc = on(device, [&](void* stream) {
+    return gact_pack(in(*x), in(*mn), in(*mx), dtype_code(x->scalar_type()), bits, N, G, D, mode, seed, nullptr, out(codes), out(scale), stream);
+  });
+  if (rc == GACT_OK) return tuple_of({codes, scale});
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// unpack(codes, bits, scale, min, N, groups, group size) -> tensor[N, groups, group size]
+PyObject* unpack(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  int bits;
+  int64_t N, G, D;
+  const at::Tensor *codes, *scale, *mn;
+  if (n != 7 || !(codes = plain(args[0])) || !width(args[1], &bits) || !(scale = plain(args[2])) || !(mn = plain(args[3])) ||
+      !integer(args[4], &N) || !integer(args[5], &G) || !integer(args[6], &D) || !ordinary_call())
+    Py_RETURN_NONE;
+  const c10::Device device = codes->device();
+  if (!codes->is_contiguous() || codes->dim() != 1 || codes->scalar_type() != at::kChar) Py_RETURN_NONE;
+  for (const at::Tensor* t : {scale, mn})
+    if (!t->is_contiguous() || t->dim() != 3 || !float_or_half(*t) || t->scalar_type() != scale->scalar_type() || t->device() != device)
+      Py_RETURN_NONE;
+  int64_t rows, numel;
+  if (N <= 0 || G <= 0 || D <= 0 || __builtin_mul_overflow(N, G, &rows) || __builtin_mul_overflow(rows, D, &numel) ||
+      numel > INT64_MAX / 16 || codes->numel() < packed_numel(bits, N, G * D) - 1 || scale->numel() < rows || mn->numel() < rows)
+    Py_RETURN_NONE;
+  const at::Tensor data = make({N, G, D}, scale->scalar_type(), device);
+  const int rc = on(device, [&](void* stream) {
+    return gact_unpack(in(*codes), bits, in(*scale), in(*mn), dtype_code(scale->scalar_type()), N, G, D, out(data), stream);
+  });
+  if (rc == GACT_OK) return THPVariable_Wrap(data);
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// mask_pack(0/1 bytes) -> int32[ceil(n/32)]
+PyObject* mask_pack(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  const at::Tensor* x;
+  if (n != 1 || !(x = plain(args[0])) || !x->is_contiguous() || x->scalar_type() != at::kByte || x->numel() == 0 || !ordinary_call())
+    Py_RETURN_NONE;
+  const c10::Device device = x->device();
+  const at::Tensor mask = make({(x->numel() + 31) / 32}, at::kInt, device);
+  const int rc = on(device, [&](void* stream) { return gact_mask_pack((const uint8_t*)in(*x), x->numel(), (int32_t*)out(mask), stream); });
+  if (rc == GACT_OK) return THPVariable_Wrap(mask);
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// mask_unpack(mask, n) -> uint8[n]
+PyObject* mask_unpack(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  const at::Tensor* mask;
+  int64_t numel;
+  if (n != 2 || !(mask = plain(args[0])) || !integer(args[1], &numel) || mask->scalar_type() != at::kInt || numel <= 0 ||
+      numel > INT64_MAX / 2 || mask->numel() < (numel + 31) / 32 || !ordinary_call())
+    Py_RETURN_NONE;
+  const c10::Device device = mask->device();
+  const at::Tensor data = make({numel}, at::kByte, device);
+  const int rc = on(device, [&](void* stream) { return gact_mask_unpack((const int32_t*)in(*mask), numel, (uint8_t*)out(data), stream); });
+  if (rc == GACT_OK) return THPVariable_Wrap(data);
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// batch_table(entries, tensors, seeds) -> the table as bytes on the host, in pinned memory: `entries` (bytes, one
+// gact_batch_entry per tensor) with each tensor's address and seed filled in
+PyObject* batch_table(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 3 || !PyBytes_CheckExact(args[0]) || !PyList_CheckExact(args[1]) || !PyList_CheckExact(args[2]) || !ordinary_call()) Py_RETURN_NONE;
+  const Py_ssize_t count = PyList_GET_SIZE(args[1]), bytes = PyBytes_GET_SIZE(args[0]);
+  if (count == 0 || PyList_GET_SIZE(args[2]) != count || bytes != count * (Py_ssize_t)sizeof(gact_batch_entry)) Py_RETURN_NONE;
+  const at::Tensor table = at::empty({(int64_t)bytes}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
+  gact_batch_entry* const entry = (gact_batch_entry*)out(table);
+  std::memcpy(entry, PyBytes_AS_STRING(args[0]), (size_t)bytes);
+  for (Py_ssize_t i = 0; i < count; i++) {
+    const at::Tensor* const t = plain(PyList_GET_ITEM(args[1], i));
+    int64_t seed;
+    if (!t || !integer(PyList_GET_ITEM(args[2], i), &seed) || t->numel() != entry[i].numel ||
+        dtype_code(t->scalar_type()) != entry[i].dtype || !t->is_contiguous() || (reinterpret_cast<uintptr_t>(in(*t)) & 15u) != 0)
+      Py_RETURN_NONE;
+    entry[i].x = in(*t);
+    entry[i].seed = (uint64_t)seed;
+  }
+  return THPVariable_Wrap(table);
+  END_HANDLE_TH_ERRORS
+}
+
+#define FASTCALL(f) {#f, (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {FASTCALL(quantize), FASTCALL(dequantize), FASTCALL(minimax),     FASTCALL(pack),        FASTCALL(unpack),
+                         FASTCALL(mask_pack), FASTCALL(mask_unpack), FASTCALL(batch_table), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "gact_torch", "The operators' host side.", -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_gact_torch(void) { return PyModule_Create(&module); }

@@ -24,22 +24,40 @@ class BatchedPacked:
     The widths come from device memory, so whether they were all valid (1, 2, 4 or 8 - a tensor that
     calc_precision left at 32 is not) and whether the arena was large enough is only known on the
     device: when either fails the kernels write nothing.  ``ok()`` reads that verdict back (it
-    synchronises); ``per_tensor`` and ``BatchedQuantizer.dequantize`` call it and raise."""
+    synchronises); ``per_tensor`` calls it and raises.  ``BatchedQuantizer.dequantize`` raises by the copy of the
+    verdict that left for the host right behind the plan, so that it does not wait for the quantize kernels."""
 
-    def __init__(self, owner, packed, scale, mn, table, bits, workspace, shapes, dtypes, seeds):
+    _verdict = None     # (event behind the copy, the workspace's first two words in pinned memory); none in a pickled one
+
+    def __init__(self, owner, packed, scale, mn, table, bits, workspace, shapes, dtypes, seeds, verdict=None):
         self.owner = owner
+        self._verdict = verdict
         self.seeds = list(seeds)
         self.packed, self.scale, self.min = packed, scale, mn
         self.table, self.bits, self.workspace = table, bits, workspace
         self.shapes, self.dtypes = shapes, dtypes
+
+    def __getstate__(self):
+        state = dict(self.__dict__)
+        state.pop("_verdict", None)
+        return state
 
     def ok(self):
         """(plan succeeded, arena bytes the table needs); synchronises."""
         vals = self.workspace[:16].view(torch.int64).tolist()
         return bool(vals[1]), vals[0]
 
-    def require_ok(self):
-        good, need = self.ok()
+    def _planned(self):
+        """What ok() returns, as of the plan of the quantize call; waits for that plan and its copy only."""
+        if self._verdict is None:
+            return self.ok()
+        done, words = self._verdict
+        done.synchronize()
+        need, good = words.tolist()
+        return bool(good), need
+
+    def require_ok(self, verdict=None):
+        good, need = self.ok() if verdict is None else verdict
         if not good:
             raise RuntimeError("gact: the batched launch was void - a width outside {1, 2, 4, 8} or a packed arena "
                                "of %d bytes where %d are needed; nothing was quantized" % (self.packed.numel(), need))
@@ -64,6 +82,8 @@ class BatchedPacked:
 
 class BatchedQuantizer:
     """Geometry of a fixed list of saved tensors (element counts and dtypes), reusable every iteration."""
+
+    _entries = None     # the table's bytes but for what changes from call to call, a tensor's address and its seed
 
     def __init__(self, numels, dtypes, device):
         if len(numels) != len(dtypes):
@@ -109,7 +129,18 @@ class BatchedQuantizer:
         """Whether the last plan written to this workspace succeeded; synchronises."""
         return bool(workspace[8:16].view(torch.int64).item())
 
-    def _table(self, tensors, seeds):
+    def _table(self, tensors, seeds, wait=True):
+        """The table on the GPU.  wait = False where it is used on the current stream: it goes there from pinned memory
+        behind the stream's other work."""
+        if self.L and not torch.cuda.is_current_stream_capturing():
+            if self._entries is None:
+                entries = (_abi.BatchEntry * self.L)()
+                for e, n, dt, first, stats in zip(entries, self.numels, self.dtypes, self.first_blocks, self.stats_offsets):
+                    e.numel, e.dtype, e.first_block, e.stats_offset = n, _abi.dtype_code(dt), first, stats
+                self._entries = bytes(entries)
+            host = _abi.native().batch_table(self._entries, list(tensors), list(seeds))
+            if host is not None:
+                return host.to(self.device, non_blocking=not wait)
         arr = (_abi.BatchEntry * self.L)()
         for i, t in enumerate(tensors):
             if t.numel() != self.numels[i] or t.dtype != self.dtypes[i]:
@@ -132,24 +163,26 @@ class BatchedQuantizer:
     # ---- the launches on caller-owned buffers (nothing is allocated, nothing synchronises) ----
     def launch_quantize(self, table, bits, packed, scale, mn, workspace, mode):
         """Plan into `workspace` from the device-resident `bits`, then quantize every tensor of `table`."""
-        lib = _abi.lib()
-        st = torch.cuda.current_stream(self.device).cuda_stream
-        _abi.check(lib.gact_batch_plan(table.data_ptr(), bits.data_ptr(), self.L, self.total_blocks, packed.numel(),
-                                       workspace.data_ptr(), st))
-        _abi.check(lib.gact_quantize_batched(table.data_ptr(), bits.data_ptr(), self.L, self.total_blocks, mode,
-                                             self.dtype_mask, workspace.data_ptr(), packed.data_ptr(),
-                                             scale.data_ptr(), mn.data_ptr(), st))
+        self._launch_plan(table, bits, packed, workspace)
+        self._launch_quantize(table, bits, packed, scale, mn, workspace, mode)
+
+    def _launch_plan(self, table, bits, packed, workspace):
+        _abi.check(_abi.lib().gact_batch_plan(table.data_ptr(), bits.data_ptr(), self.L, self.total_blocks, packed.numel(),
+                                              workspace.data_ptr(), torch.cuda.current_stream(self.device).cuda_stream))
+
+    def _launch_quantize(self, table, bits, packed, scale, mn, workspace, mode):
+        _abi.check(_abi.lib().gact_quantize_batched(table.data_ptr(), bits.data_ptr(), self.L, self.total_blocks, mode,
+                                                    self.dtype_mask, workspace.data_ptr(), packed.data_ptr(),
+                                                    scale.data_ptr(), mn.data_ptr(),
+                                                    torch.cuda.current_stream(self.device).cuda_stream))
 
     def launch_dequantize(self, table, bits, packed, scale, mn, workspace):
         """Plan into `workspace` (the table's x point at the outputs; planning again from the same widths gives
         the same offsets without reading anything back), then dequantize every tensor."""
-        lib = _abi.lib()
-        st = torch.cuda.current_stream(self.device).cuda_stream
-        _abi.check(lib.gact_batch_plan(table.data_ptr(), bits.data_ptr(), self.L, self.total_blocks, packed.numel(),
-                                       workspace.data_ptr(), st))
-        _abi.check(lib.gact_dequantize_batched(table.data_ptr(), bits.data_ptr(), self.L, self.total_blocks,
-                                               workspace.data_ptr(), packed.data_ptr(), scale.data_ptr(),
-                                               mn.data_ptr(), st))
+        self._launch_plan(table, bits, packed, workspace)
+        _abi.check(_abi.lib().gact_dequantize_batched(table.data_ptr(), bits.data_ptr(), self.L, self.total_blocks,
+                                                      workspace.data_ptr(), packed.data_ptr(), scale.data_ptr(),
+                                                      mn.data_ptr(), torch.cuda.current_stream(self.device).cuda_stream))
 
     def quantize(self, tensors, bits, seeds, arena_bytes=None, rng_stream=None):
         """Quantize all tensors in one batched launch.  `bits` is an int32 tensor on the device (e.g. the output
@@ -162,28 +195,34 @@ class BatchedQuantizer:
         if arena_bytes is None:
             arena_bytes = self.arena_bytes_worst_case()
         with torch.cuda.device(self.device):
-            table = self._table(tensors, seeds)
+            table = self._table(tensors, seeds, wait=False)
             packed = torch.empty((int(arena_bytes),), dtype=torch.uint8, device=self.device)
             scale = torch.empty((self.total_groups * 4,), dtype=torch.uint8, device=self.device)
             mn = torch.empty((self.total_groups * 4,), dtype=torch.uint8, device=self.device)
             ws = self.new_workspace()
             # the widths are kept as they were at quantize time: the caller may refresh its own copy
             kept = bits.clone()
-            self.launch_quantize(table, kept, packed, scale, mn, ws, mode)
+            self._launch_plan(table, kept, packed, ws)
+            verdict = None
+            if not torch.cuda.is_current_stream_capturing():
+                words = torch.empty(2, dtype=torch.int64, pin_memory=True)
+                words.copy_(ws[:16].view(torch.int64), non_blocking=True)
+                verdict = (torch.cuda.current_stream().record_event(), words)
+            self._launch_quantize(table, kept, packed, scale, mn, ws, mode)
         return BatchedPacked(self, packed, scale, mn, table, kept, ws, [t.shape for t in tensors],
-                             list(self.dtypes), seeds)
+                             list(self.dtypes), seeds, verdict)
 
     def dequantize(self, q, outs=None, check=True):
         """Dequantize every tensor of a BatchedPacked in one launch into fresh tensors (or `outs`).
-        check = True reads the plan's verdict back first (one synchronisation) and raises when the quantize
+        check = True waits for the plan's verdict first and raises when the quantize
         launch was void; pass False where nothing may synchronise (stream capture) and the caller has
         checked ``q.ok()`` itself."""
         if check:
-            q.require_ok()
+            q.require_ok(q._planned())
         with torch.cuda.device(self.device):
             if outs is None:
                 outs = [torch.empty(s, dtype=d, device=self.device) for s, d in zip(q.shapes, q.dtypes)]
-            table = self._table(outs, q.seeds)
+            table = self._table(outs, q.seeds, wait=False)
             ws = self.new_workspace()
             self.launch_dequantize(table, q.bits, q.packed, q.scale, q.min, ws)
             # keep the table alive until the stream has consumed it

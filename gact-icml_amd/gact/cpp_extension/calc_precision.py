@@ -35,7 +35,6 @@ def calc_precision_device(b, C, w, target, status=None):
             raise RuntimeError(name + " must be contiguous!")
     if b.dtype != torch.int32 or C.dtype != torch.float32 or w.dtype != torch.int64:
         raise RuntimeError("expected b int32, C float32, w int64")
-    with torch.cuda.device(b.device):
-        _abi.check(_abi.lib().gact_calc_precision_device(b.data_ptr(), C.data_ptr(), w.data_ptr(), b.numel(),
-                                                         float(target), _abi.ptr(status), _abi.stream_of(b)))
+    _abi.call_on(b.device, _abi.lib().gact_calc_precision_device, b.data_ptr(), C.data_ptr(), w.data_ptr(), b.numel(),
+                 float(target), _abi.ptr(status), _abi.stream_of(b))
     return b

@@ -16,6 +16,9 @@ def _check_cuda_float(t, name):
 
 def minimax(data):
     """Per-row (min, max) of a contiguous [N, D] float32/float16 tensor on the GPU."""
+    both = _abi.native().minimax(data)
+    if both is not None:
+        return both
     _check_cuda_float(data, "data")
     if data.dim() != 2:
         raise RuntimeError("The dimension of data is not correct!")

@@ -70,6 +70,15 @@ def pack_single_precision(data, min, max, bits, stochastic, seed, *, noise=None,
     rounding noise (quantization_cuda_kernel.cu:65-66).  `noise` (float32, same number of elements as
     data) injects the uniforms instead of drawing them; `rng_stream` overrides gact.conf.config.rng_stream.
     """
+    if noise is None:
+        if rng_stream is None:
+            from ..conf import config
+            stream = config.rng_stream
+        else:
+            stream = rng_stream
+        q = _abi.native().pack(data, min, max, bits, seed, _abi.NOISE_MODES.get(stream, -1))
+        if q is not None:
+            return q
     _check_cuda_dim_float(data, "data", 3)
     _check_cuda_dim_float(min, "min", 3)
     _check_cuda_dim_float(max, "max", 3)
@@ -96,6 +105,9 @@ def pack_single_precision(data, min, max, bits, stochastic, seed, *, noise=None,
 
 def unpack_single_precision(data, bits, scale, min, N, num_groups, group_size):
     """Inverse of pack_single_precision -> [N, num_groups, group_size] of scale.dtype."""
+    out = _abi.native().unpack(data, bits, scale, min, N, num_groups, group_size)
+    if out is not None:
+        return out
     # CHECK_CUDA_TENSOR_DIM_TYPE(data, 1, kInt8), quantization.cc:43
     _check_cuda(data, "data")
     if data.dim() != 1:
@@ -121,6 +133,9 @@ def unpack_single_precision(data, bits, scale, min, N, num_groups, group_size):
 
 def act_quantize_dropout_mask(data):
     """uint8 0/1 mask of any shape -> int32[ceil(n/32)] bit mask."""
+    mask = _abi.native().mask_pack(data)
+    if mask is not None:
+        return mask
     # CHECK_CUDA_TENSOR_TYPE(data, kUInt8), quantization.cc:27
     _check_cuda(data, "data")
     if data.dtype != torch.uint8:
@@ -134,6 +149,9 @@ def act_quantize_dropout_mask(data):
 
 def act_dequantize_dropout_mask(mask, N):
     """int32 bit mask -> uint8[N] of 0/1."""
+    out = _abi.native().mask_unpack(mask, N)
+    if out is not None:
+        return out
     N = int(N)
     if not mask.is_cuda:
         raise RuntimeError("mask must be a CUDA tensor!")

@@ -26,6 +26,11 @@ def _num_groups(numel):
     return (numel + config.group_size - 1) // config.group_size
 
 
+def _mode_of(rng_stream):
+    """What the native calls take for a noise stream's name; -1, which they refuse, for one that is not known."""
+    return _abi.NOISE_MODES.get(config.rng_stream if rng_stream is None else rng_stream, -1)
+
+
 def _one_pass(group, dtype):
     """The single-pass kernels are built for groups of 256, and 64, 128 and 512 for float and half; any other
     config.group_size takes the extension-style sequence minimax -> pack / unpack on the zero-padded tensor, as the
@@ -45,6 +50,12 @@ def _padded_groups(input):
 def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, seed_offset=None):
     """gact/gact/ops.py:11-32 -> (q_input, q_scale, q_min).  `seed_offset` (one int64 on the GPU, optional) is added
     to `seed` when the kernel runs, for launches recorded in a HIP graph."""
+    in_place = True     # whether a layout that is not contiguous is worth asking the kernels for
+    if noise is None and seed_offset is None:
+        q = _abi.native().quantize(input, q_bit, seed, _mode_of(rng_stream), config.group_size)
+        if q:
+            return q
+        in_place = q is not False
     N = _num_groups(input.numel())
     if q_bit == 32:
         # the passthrough of ops.py:21-24: the padded [N, group] view itself, max - min, min
@@ -93,7 +104,7 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
             raise RuntimeError("seed_offset must be one int64 on the device of the data")
     if input.is_contiguous():
         x = input
-    elif group == _abi.GROUP and mode in (_abi.NOISE_FAST, _abi.NOISE_CONST) \
+    elif in_place and group == _abi.GROUP and mode in (_abi.NOISE_FAST, _abi.NOISE_CONST) \
             and _quantize_strided(input, q_bit, mode, seed, seed_offset, q_input, q_scale, q_min):
         return q_input, q_scale, q_min
     else:
@@ -165,6 +176,9 @@ def op_quantize(input, q_bit, seed, *, noise=None, rng_stream=None, seed_offset=
 def op_dequantize(input, input_shape):
     """gact/gact/ops.py:61-69 -> tensor of `input_shape`, contiguous, dtype of the scale."""
     q_input, q_bit, q_scale, q_min = input
+    out = _abi.native().dequantize(q_input, input_shape, q_bit, q_scale, q_min, config.group_size)
+    if out is not None:
+        return out
     if not isinstance(q_bit, int):
         print("bits must be intergers, now bits ", q_bit)
         assert(False)
