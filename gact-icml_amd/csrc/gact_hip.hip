@@ -1801,35 +1801,40 @@ quantize_transposed_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t nu
                                                (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
 }
 
-// The same layout where channels are long (K pixels hold a super-group and more): a workgroup owns a strip of channels, 128 bytes
-// of every memory row, and walks along the pixels in chunks of 256, the next chunk's loads in flight while it works on the
-// one before.  It quantizes the super-groups that begin in its channels.  These begin at another pixel in every channel
-// (first_pixel), so a chunk completes one group of each channel whose head came with the chunk before: LDS holds two groups
-// per channel, in turn.  A super-group that runs past its channel's last pixel ends in the next channel: past the end the walk
-// goes on at the first pixels with every column belonging to the channel before it.  A strip can be cut into segments of
-// whole super-groups, for more workgroups than there are strips; a segment reads up to a super-group of pixels beyond its own.
-// Bound by its steps: half [64,256,56,56] at 4 bit 43 us, vector instructions issued in 53 % of the cycles at two waves per SIMD and
-// in 63 % at four, which more segments give and their extra reading takes back (44 us).
+// The same layout where channels are long (K pixels hold a super-group and more): a workgroup owns a strip of channels, 64 bytes
+// of every memory row, and walks along the pixels in steps of GS chunks of 256, the next step's loads in flight while it works on
+// the one before.  It quantizes the units - a super-group, or GS groups where that is more - that begin in its channels.  These
+// begin at another pixel in every channel (first_pixel), so a step completes GS groups of each channel whose head came with
+// the step before: LDS holds two steps' groups per channel, in turn.  A unit that runs past its channel's last pixel ends in
+// the next channel: past the end the walk goes on at the first pixels with every column belonging to the channel before it.  A
+// strip can be cut into segments of whole units, for more workgroups than there are strips; a segment reads up to a unit of
+// pixels beyond its own.
+// Bound by its instructions with few waves to overlap them: half [64,256,56,56] at 4 bit 37 us (256 CUs hold its 512 workgroups
+// at once; of the two on a CU the one dispatched second takes a fifth longer).  With GS = 1, 477 vector instructions per
+// 256 pixels and wave, it took 42; more waves through more segments cost more reading than they hide (44), and dropping
+// one of the two barriers by a ring of four slots changed nothing (41.8).
 #define STRIP_PIECES 4    /* 16-byte pieces of a memory row in a strip (8: half [2,64,128,128] 4 bit 7.6 -> 9.5 us, large tensors equal) */
 #define STRIP_CHUNK 256   /* pixels: a thread takes four of one piece */
 #define STRIP_THREADS (STRIP_PIECES * STRIP_CHUNK / 4)
 struct StripShape {
   int64_t sb, sk;
   uint32_t M, K, strips;   // strips of a batch entry
-  uint32_t batch, segments, segment;   // segment: super-groups of a channel in a segment
+  uint32_t batch, segments, segment;   // segment: units of a channel in a segment
 };
-template <typename T, int BITS, int NOISE>
-__global__ void __launch_bounds__(STRIP_THREADS, 4)
+// whole super-groups, and whole steps of GS groups
+template <int BITS, int GS> struct StripUnit { static constexpr int value = 8 / BITS > GS ? 8 / BITS * GROUP : GS * GROUP; };
+template <typename T, int BITS, int NOISE, int GS>
+__global__ void __launch_bounds__(STRIP_THREADS, 4 / GS)
 quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_t N, uint8_t* __restrict__ packed,
                        typename Elem<T>::Stat* __restrict__ scale_out, T* __restrict__ mn_out, T* __restrict__ mx_out, StripShape g) {
   typedef typename Elem<T>::Stat Stat;
   constexpr int CH = Elem<T>::kQChunks, W = Elem<T>::kQWidth, WPT = 8 / BITS, QMAX = (1 << BITS) - 1;
-  constexpr uint32_t ES = sizeof(T), SGE = WPT * GROUP;
+  constexpr uint32_t ES = sizeof(T), UNIT = StripUnit<BITS, GS>::value, STEP = GS * GROUP;
   constexpr int STRIP = STRIP_PIECES * W;             // channels of a strip
   constexpr int OWN = STRIP / (STRIP_THREADS / 16);   // channels of a row of 16 lanes: 2 (16-bit types), 1 (float)
-  // LDS: two groups per channel; 16 bytes behind every channel and 64 behind every 8 half channels keep the channels, and the
+  // LDS: two steps' groups per channel; 16 bytes behind every channel and 64 behind every 8 half channels keep the channels, and the
   // pieces, that a wave writes at once out of each other's banks
-  constexpr uint32_t SLOT = GROUP * ES, CHANNEL = 2 * SLOT + 16, PIECE = W * CHANNEL + (ES == 2 ? 64 : 0);
+  constexpr uint32_t SLOT = STEP * ES, CHANNEL = 2 * SLOT + 16, PIECE = W * CHANNEL + (ES == 2 ? 64 : 0);
   __shared__ u32x4 ring_lds[STRIP_PIECES * PIECE / 16];
   uint8_t* const ring = reinterpret_cast<uint8_t*>(ring_lds);
   const uint32_t id = xcd_tile<GACT_XCD_RUN_TR>(blockIdx.x, gridDim.x);
@@ -1838,26 +1843,26 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
   const uint32_t width = g.M - m0 < (uint32_t)STRIP ? g.M - m0 : (uint32_t)STRIP;   // a multiple of W
   const T* const entry = x + (int64_t)b * g.sb;
   const uint32_t K = g.K;
-  // the column behind the strip's last one, where that channel's super-groups may end: the next channel, perhaps of the next entry
+  // the column behind the strip's last one, where that channel's units may end: the next channel, perhaps of the next entry
   const T* const behind = m0 + width < g.M ? entry + m0 + width : b + 1 < g.batch ? x + (int64_t)(b + 1) * g.sb : nullptr;
 
-  // this thread's part of a chunk: four pixels of one piece
+  // this thread's part of a step: four pixels of one piece in each of its chunks
   const uint32_t piece = threadIdx.x % STRIP_PIECES, quad = threadIdx.x / STRIP_PIECES;
   const bool has_piece = piece * W < width;
   const bool last_piece = (piece + 1) * W == width;
   const T* const from = entry + m0 + piece * W;
   const uint32_t P0 = (uint32_t)(((uint64_t)b * g.M + m0) * K);   // element index of the strip's first channel, low bits
-  const auto first_pixel = [&](uint32_t channel) { return (0u - (P0 + channel * K)) & (SGE - 1); };   // of its first super-group
+  const auto first_pixel = [&](uint32_t channel) { return (0u - (P0 + channel * K)) & (UNIT - 1); };   // of its first unit
   uint32_t first_of[W];
 #pragma unroll
   for (int e = 0; e < W; e++) first_of[e] = first_pixel(piece * W + e);
   struct Chunk { u32x4 v[4]; T beyond[4]; };
-  const uint32_t g_first = seg * g.segment * WPT;                  // first group of the segment within a channel
-  const uint32_t g_end = g_first + g.segment * WPT;
+  const uint32_t j_first = seg * g.segment * (UNIT / STEP);        // first step's groups of the segment within a channel
+  const uint32_t j_end = j_first + g.segment * (UNIT / STEP);
   auto load = [&](uint32_t chunk, Chunk& q) {
     const uint32_t at = chunk * STRIP_CHUNK + 4 * quad;            // four pixels on one side of K: both are multiples of four
     const uint32_t k = at < K ? at : at - K;
-    if (has_piece && at < K + SGE) {
+    if (has_piece && at < K + UNIT) {
       const T* const p = from + (int64_t)k * g.sk;
 #pragma unroll
       for (int j = 0; j < 4; j++) q.v[j] = *reinterpret_cast<const u32x4*>(p + j * g.sk);
@@ -1867,10 +1872,10 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
       }
     }
   };
-  // four elements of a channel (16-bit types: in lo) to their place in the channel's two groups.  A chunk holds 256 consecutive
-  // elements of a channel, so what comes before the first super-group cannot reach a group that is being filled.
+  // four elements of a channel (16-bit types: in lo) to their place in the channel's two slots.  A step holds a slot's number of
+  // consecutive elements of a channel, so what comes before the first unit cannot reach a slot that is being filled.
   auto put = [&](uint32_t base, uint32_t pos, u32x2 lo, u32x2 hi) {
-    uint8_t* const to = ring + base + (pos & (2 * GROUP - 1)) * ES;
+    uint8_t* const to = ring + base + (pos & (2 * STEP - 1)) * ES;
     if constexpr (ES == 4) *reinterpret_cast<u32x4*>(to) = u32x4{lo.x, lo.y, hi.x, hi.y};
     else *reinterpret_cast<u32x2*>(to) = lo;
   };
@@ -1894,7 +1899,7 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
         column(q, e, lo, hi);
         put(piece * PIECE + e * CHANNEL, at - first_of[e], lo, hi);
       }
-    } else if (at < K + SGE) {   // past the end: a column belongs to the channel before it
+    } else if (at < K + UNIT) {   // past the end: a column belongs to the channel before it
 #pragma unroll
       for (int e = 0; e < W; e++) {
         column(q, e, lo, hi);
@@ -1915,118 +1920,162 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
     }
   };
 
+  // this lane's 16 bytes of the super-group that group n belongs to
+  auto store_bytes = [&](int64_t n, const uint32_t (&b4)[4]) {
+#pragma unroll
+    for (int k = 0; k < CH; k++) {
+      uint8_t* const to = packed + n / WPT * GROUP + chunk_col<T>(k, threadIdx.x & 15);
+      if constexpr (W == 4) stream_store(b4[k], reinterpret_cast<uint32_t*>(to));
+      else stream_store(u32x2{b4[2 * k], b4[2 * k + 1]}, reinterpret_cast<u32x2*>(to));
+    }
+  };
   // this row's channels
   const uint64_t seed = seed_arg.value();
   const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
   const int row = threadIdx.x >> 4, i = threadIdx.x & 15;
-  uint32_t delay[OWN], groups[OWN];   // chunk c completes group c - delay of the channel; end of the segment's groups
+  uint32_t delay[OWN], last[OWN];   // step t completes groups (t - delay) * GS .. of the channel; end of the segment's (t - delay)
   int64_t n_first[OWN];
 #pragma unroll
   for (int c = 0; c < OWN; c++) {
     const uint32_t m = row * OWN + c, first = first_pixel(m);
-    groups[c] = m < width ? (K - first + SGE - 1) / SGE * WPT : 0u;
-    groups[c] = groups[c] < g_end ? groups[c] : g_end;
-    delay[c] = (first + 255) >> 8;
+    last[c] = m < width ? (K - first + UNIT - 1) / UNIT * (UNIT / STEP) : 0u;
+    last[c] = last[c] < j_end ? last[c] : j_end;
+    delay[c] = (first + STEP - 1) / STEP;
     n_first[c] = (((int64_t)b * g.M + m0 + m) * K + first) / GROUP;
   }
   uint32_t bytes[OWN][4];   // the lane's 16 bytes of each channel's super-group, in the order of their addresses
 
-  const uint32_t most = (K + SGE - 1) / STRIP_CHUNK + 1;   // no channel has anything left after so many chunks
-  const uint32_t end = g_end + WPT < most ? g_end + WPT : most;
-  auto step = [&](uint32_t chunk, Chunk& q) {
-    scatter(chunk, q);
-    if (chunk + 2 < end) load(chunk + 2, q);
+  const uint32_t most = (K + UNIT - 1) / STEP + 1;   // no channel has anything left after so many steps
+  const uint32_t end = j_end + UNIT / STEP < most ? j_end + UNIT / STEP : most;
+  // `ahead` steps further on the same registers are loaded again
+  auto step = [&](uint32_t t, Chunk (&q)[GS], uint32_t ahead) {
+#pragma unroll
+    for (int h = 0; h < GS; h++) {
+      scatter(t * GS + h, q[h]);
+      if (t + ahead < end) load((t + ahead) * GS + h, q[h]);
+    }
     __syncthreads();
     uint32_t j[OWN];
     bool due[OWN], any = false;
 #pragma unroll
     for (int c = 0; c < OWN; c++) {
-      j[c] = chunk - delay[c];
-      due[c] = chunk >= delay[c] && j[c] < groups[c] && j[c] >= g_first;
+      j[c] = t - delay[c];
+      due[c] = t >= delay[c] && j[c] < last[c] && j[c] >= j_first;
       any |= due[c];
     }
     if (__builtin_amdgcn_ballot_w64(any) == 0) {
       __syncthreads();
       return;
     }
-    typename Elem<T>::Store st[OWN];
-    Stat lo[OWN], hi[OWN], sc[OWN];
+    constexpr int G = OWN * GS;   // groups of the row: group s of channel c is number c * GS + s
+    typename Elem<T>::Store st[G];
+    Stat lo[G], hi[G], sc[G];
 #pragma unroll
-    for (int c = 0; c < OWN; c++) {
-      lo[c] = hi[c] = (Stat)0.0f;
-      const uint32_t m = row * OWN + c;
-      const uint8_t* p = ring + (m / W) * PIECE + (m % W) * CHANNEL + (j[c] & 1) * SLOT;
+    for (int r = 0; r < G; r++) {
+      lo[r] = hi[r] = (Stat)0.0f;
+      const uint32_t m = row * OWN + r / GS;
+      const uint8_t* p = ring + (m / W) * PIECE + (m % W) * CHANNEL + (j[r / GS] & 1) * SLOT + (r % GS) * (GROUP * ES);
 #pragma unroll
-      for (int k = 0; k < CH; k++) Elem<T>::load_chunk(reinterpret_cast<const T*>(p) + chunk_col<T>(k, i), st[c], k);
+      for (int k = 0; k < CH; k++) Elem<T>::load_chunk(reinterpret_cast<const T*>(p) + chunk_col<T>(k, i), st[r], k);
     }
 #pragma unroll
-    for (int c = 0; c < OWN; c++) Elem<T>::group_minmax(st[c], lo[c], hi[c]);
+    for (int r = 0; r < G; r++) Elem<T>::group_minmax(st[r], lo[r], hi[r]);
     {
-      const int mine = i & (OWN - 1);
-      const Stat lo_m = mine ? lo[OWN - 1] : lo[0], hi_m = mine ? hi[OWN - 1] : hi[0];
+      // one division per lane: lane r of the row takes group r % G
+      const int mine = i & (G - 1);
+      Stat lo_m = lo[0], hi_m = hi[0];
+      int64_t n = n_first[0] + j[0] * GS;
+      bool mine_due = due[0];
+#pragma unroll
+      for (int r = 1; r < G; r++) {
+        lo_m = mine == r ? lo[r] : lo_m;
+        hi_m = mine == r ? hi[r] : hi_m;
+      }
+      if (OWN > 1 && mine >= GS) {
+        n = n_first[OWN - 1] + j[OWN - 1] * GS;
+        mine_due = due[OWN - 1];
+      }
+      n += mine % GS;
       const Stat s_m = Elem<T>::make_scale(lo_m, hi_m, QMAX);
-      const int64_t n = (mine ? n_first[OWN - 1] + j[OWN - 1] : n_first[0] + j[0]);
-      if (i < OWN && (mine ? due[OWN - 1] : due[0]) && n < N) {
+      if (i < G && mine_due && n < N) {
         scale_out[n] = s_m;
         mn_out[n] = Elem<T>::elem_of(lo_m);
         if (mx_out) mx_out[n] = Elem<T>::elem_of(hi_m);
       }
-      sc[0] = OWN == 1 ? s_m : row_bcast<0>(s_m);
-      if (OWN > 1) sc[OWN - 1] = row_bcast<1>(s_m);
+      sc[0] = G == 1 ? s_m : row_bcast<0>(s_m);
+      if (G > 1) sc[1 % G] = row_bcast<1>(s_m);
+      if (G > 2) {
+        sc[2 % G] = row_bcast<2>(s_m);
+        sc[3 % G] = row_bcast<3>(s_m);
+      }
     }
 #pragma unroll
     for (int c = 0; c < OWN; c++) {
       if (due[c]) {
-        const int64_t n = n_first[c] + j[c];
-        const uint32_t ni = j[c] % WPT, shift = ni * BITS;
-        const uint32_t field = 0x01010101u * ((0xffu << shift) & 0xffu);   // what a code may reach of its byte
-        float cd[CH / 2][W];
-        if (NOISE == GACT_NOISE_FAST) {
-          FastRow<T, 1> fast;
-          fast.draws(0, n, i, k0, k1, cd);
-        }
+        const int64_t n0 = n_first[c] + j[c] * GS;
+        constexpr bool WHOLE = WPT <= GS;                                   // a step completes its super-groups
+        const uint32_t before = WHOLE ? 0u : (j[c] * GS) % WPT;             // groups of the super-group before this step's
+        FastRow<T, GS> fast;
+        uint32_t sum[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int k = 0; k < CH; k++) {
-          uint32_t code[W];
-          if (NOISE == GACT_NOISE_FAST) {
-            if (k < CH / 2) Elem<T>::template codes<false, false, true, false>(st[c], k, lo[c], sc[c], cd[k % (CH / 2)], code);
-            else Elem<T>::template codes<false, false, true, true>(st[c], k, lo[c], sc[c], cd[k % (CH / 2)], code);
-          } else {
-            float u[W];
-#pragma unroll
-            for (int e = 0; e < W; e++) u[e] = 0.5f;
-            Elem<T>::template codes<true, false>(st[c], k, lo[c], sc[c], u, code);
-          }
-          if (Elem<T>::kRepairsInfiniteScale && Elem<T>::scale_is_inf(sc[c])) {   // rare, see Elem<T>::kRepairsInfiniteScale
-#pragma unroll
-            for (int e = 0; e < W; e++)
-              if (Elem<T>::above(st[c], k, e, lo[c])) code[e] = 0xffu;
-          }
-#pragma unroll
-          for (int q = 0; q < W / 4; q++) {
-            const uint32_t w = (pack4(code + 4 * q) << shift) & field;
-            uint32_t& byte4 = bytes[c][k * (W / 4) + q];
-            byte4 = ni == 0 ? w : byte4 | w;
-          }
-        }
-        if (ni == WPT - 1) {
+        for (int s = 0; s < GS; s++) {
+          const int r = c * GS + s;
+          const uint32_t field_shift = (s % WPT) * BITS;
+          float cd[CH / 2][W];
+          if (NOISE == GACT_NOISE_FAST) fast.draws(s, n0, i, k0, k1, cd);
 #pragma unroll
           for (int k = 0; k < CH; k++) {
-            uint8_t* const to = packed + n / WPT * GROUP + chunk_col<T>(k, i);
-            if constexpr (W == 4) stream_store(bytes[c][k], reinterpret_cast<uint32_t*>(to));
-            else stream_store(u32x2{bytes[c][2 * k], bytes[c][2 * k + 1]}, reinterpret_cast<u32x2*>(to));
+            uint32_t code[W];
+            if (NOISE == GACT_NOISE_FAST) {
+              if (k < CH / 2) Elem<T>::template codes<false, false, true, false>(st[r], k, lo[r], sc[r], cd[k % (CH / 2)], code);
+              else Elem<T>::template codes<false, false, true, true>(st[r], k, lo[r], sc[r], cd[k % (CH / 2)], code);
+            } else {
+              float u[W];
+#pragma unroll
+              for (int e = 0; e < W; e++) u[e] = 0.5f;
+              Elem<T>::template codes<true, false>(st[r], k, lo[r], sc[r], u, code);
+            }
+            if (Elem<T>::kRepairsInfiniteScale && Elem<T>::scale_is_inf(sc[r])) {   // rare, see Elem<T>::kRepairsInfiniteScale
+#pragma unroll
+              for (int e = 0; e < W; e++)
+                if (Elem<T>::above(st[r], k, e, lo[r])) code[e] = 0xffu;
+            }
+#pragma unroll
+            for (int d = 0; d < W / 4; d++) {
+              // what a shifted code may reach of its byte: it can have a bit more than its field
+              const uint32_t w = (pack4(code + 4 * d) << field_shift) & (0x01010101u * ((0xffu << field_shift) & 0xffu));
+              uint32_t& byte4 = sum[k * (W / 4) + d];
+              byte4 = s % WPT == 0 ? w : byte4 | w;
+            }
           }
+          if (WHOLE && s % WPT == WPT - 1 && (WPT > 1 || GS == 1 || n0 + s < N)) store_bytes(n0 + s, sum);
+        }
+        if (!WHOLE) {
+          const uint32_t shift = before * BITS, field = 0x01010101u * ((0xffu << shift) & 0xffu);
+#pragma unroll
+          for (int d = 0; d < 4; d++) {
+            const uint32_t w = (sum[d] << shift) & field;
+            bytes[c][d] = before == 0 ? w : bytes[c][d] | w;
+          }
+          if (before == WPT - GS) store_bytes(n0, bytes[c]);
         }
       }
     }
     __syncthreads();
   };
-  Chunk even, odd;   // two chunks' loads in flight
-  load(g_first, even);
-  if (g_first + 1 < end) load(g_first + 1, odd);
-  for (uint32_t chunk = g_first; chunk < end; chunk += 2) {
-    step(chunk, even);
-    if (chunk + 1 < end) step(chunk + 1, odd);
+  if constexpr (GS == 1) {   // two steps' loads in flight
+    Chunk even[1], odd[1];
+    load(j_first, even[0]);
+    if (j_first + 1 < end) load(j_first + 1, odd[0]);
+    for (uint32_t t = j_first; t < end; t += 2) {
+      step(t, even, 2);
+      if (t + 1 < end) step(t + 1, odd, 2);
+    }
+  } else {                   // one step's, as many bytes
+    Chunk q[GS];
+#pragma unroll
+    for (int h = 0; h < GS; h++) load(j_first * GS + h, q[h]);
+    for (uint32_t t = j_first; t < end; t++) step(t, q, 1);
   }
 }
 
@@ -3393,17 +3442,47 @@ inline int joined_dims(int ndim, const int64_t* sizes, const int64_t* strides, i
   return n;
 }
 // Strips or tiles.  A tile's workgroup reads a piece of its own of every memory row: the longer the channels (K pixels), the
-// narrower that piece; a strip's always reads 64 bytes, but it walks its pixels in steps of about 1.5 us each, at least
-// twice the 8/bits steps of a super-group, and reads up to a super-group of pixels beyond its own.  us, tiles / strips:
-//   half [64,256,56,56] 8 bit 57 / 41  4 bit 55 / 43  2 bit 52 / 45  1 bit 54 / 52    float 4 bit 80 / 61  1 bit 155 / 89
-//   half [64,64,112,112] 8 bit 101 / 38  4 bit 99 / 36  1 bit 94 / 52    half [64,512,28,28] 8 bit 26 / 26  4 bit 23 / 31
-//   half [33,128,52,52] 8 bit 18 / 14  4 bit 18 / 18  2 bit 18 / 22  1 bit 19 / 34
-//   half [2,256,56,56]  8 bit 9 / 6  4 bit 9 / 9  2 bit 9 / 16  1 bit 11 / 26
-inline bool takes_strips(int bits, int64_t numel, int64_t K) {
+// narrower that piece; a strip's always reads 64 bytes, but it walks its pixels one step after the other, at least twice
+// the groups of a super-group, and reads up to a super-group of pixels beyond its own.  us, tiles / strips:
+//   half [64,256,56,56] 8 bit 57 / 41  4 bit 55 / 37  2 bit 52 / 40  1 bit 54 / 48    float 4 bit 80 / 63  1 bit 155 / 78
+//   half [64,64,112,112] 8 bit 101 / 37  4 bit 99 / 35  1 bit 94 / 52    half [64,512,28,28] 8 bit 26 / 26  4 bit 23 / 31
+//   half [33,128,52,52] 8 bit 18 / 13  4 bit 18 / 14  2 bit 17 / 19    [40,96,64,64] 2 bit 16 / 19    [2,256,56,56] 2 bit 10 / 14
+//   half [8,64,112,112] 2 bit 31 / 14  1 bit 32 / 26    [1,64,112,112] 2 bit 9 / 13
+//   float [16,256,56,56] 2 bit 28 / 21  1 bit 30 / 28    [2,256,56,56] 2 bit 14 / 10  1 bit 15 / 16    [8,64,112,112] 1 bit 39 / 20
+inline bool takes_strips(size_t elem_size, int bits, int64_t numel, int64_t K) {
   if (K % 4 != 0) return false;
-  return bits >= 4 ? K >= 4 * (8 / bits * GROUP) : K >= 3 * (8 / bits * GROUP) / 2 && numel >= (1 << 24);
+  const int64_t sge = 8 / bits * GROUP;
+  if (bits >= 4) return K >= 4 * sge;
+  if (K < 3 * sge / 2) return false;
+  if (elem_size == 4) return bits == 2 || numel >= (1 << 22);
+  return numel >= (K >= 8192 ? 1 << 22 : 1 << 24);
 }
-#define STRIP_WORKGROUPS 512   /* at least so many, by cutting strips into segments: more would read more beyond their own */
+// How strips are worked through: GS groups of a channel per step, and the segments they are cut into.  Two groups share a Philox
+// block and a division sequence and have half the barriers, in 66 KB of LDS, two workgroups to a CU: half [64,256,56,56] 4 bit
+// 42 -> 37 us, 2 bit 45 -> 40, float 4 bit 69 -> 63, half [16,256,56,56] 4 bit 16.4 -> 14.2.  At 8 bit, whose super-group is one
+// group, there is nothing in it and smaller tensors lose half their segments (half [2,256,56,56] 5.8 -> 7.5), so it keeps one
+// group.  So do strips that two to a CU would leave a quarter of the CUs' places empty (float [33,128,52,52] 4 bit,
+// 264 strips: 19.1 against 19.8).
+#define STRIP_WORKGROUPS 512
+struct StripCut { int gs; int64_t segment, segments; };   // segment: units
+inline StripCut strip_cut(int bits, int64_t strips, int64_t K) {
+  StripCut c;
+  c.gs = bits == 8 ? 1 : 2;
+  for (;;) {
+    const int64_t unit = 8 / bits > c.gs ? 8 / bits * GROUP : c.gs * GROUP, per_channel = (K + unit - 1) / unit;
+    // one group: at least so many workgroups (more would read more beyond their own); two: what the CUs hold at once
+    int64_t segments = c.gs == 1 ? (STRIP_WORKGROUPS + strips - 1) / strips : STRIP_WORKGROUPS / strips;
+    segments = segments < 1 ? 1 : segments;
+    if (c.gs == 2 && segments <= per_channel && strips * segments < STRIP_WORKGROUPS * 3 / 4) {
+      c.gs = 1;
+      continue;
+    }
+    segments = segments < per_channel ? segments : per_channel;
+    c.segment = (per_channel + segments - 1) / segments;
+    c.segments = (per_channel + c.segment - 1) / c.segment;
+    return c;
+  }
+}
 // Elements of a workgroup's tile: 64 KB, two workgroups to a CU, where that leaves a tile 16 channels and more (half
 // [64,512,28,28] 4 bit 23 us against 28 with one of 144 KB), else one of up to 144 KB (half [64,256,56,56] 1 bit 54 against 64;
 // [2,256,56,56] 9 against 13); as many tiles as the workgroups that the GPU holds, or a multiple of that.
@@ -3433,10 +3512,10 @@ const void* quantize_transposed_of(int noise_mode, uint32_t K) {
   if (K % 4 == 0) return quantize_transposed_rows_of<T, BITS, 4>(noise_mode);
   return quantize_transposed_rows_of<T, BITS, 1>(noise_mode);
 }
-template <typename T, int BITS>
+template <typename T, int BITS, int GS>
 const void* quantize_strips_of(int noise_mode) {
-  return noise_mode == GACT_NOISE_CONST ? (const void*)quantize_strips_kernel<T, BITS, GACT_NOISE_CONST>
-                                        : (const void*)quantize_strips_kernel<T, BITS, GACT_NOISE_FAST>;
+  return noise_mode == GACT_NOISE_CONST ? (const void*)quantize_strips_kernel<T, BITS, GACT_NOISE_CONST, GS>
+                                        : (const void*)quantize_strips_kernel<T, BITS, GACT_NOISE_FAST, GS>;
 }
 template <typename T>
 int dispatch_quantize_strided(int n, const int64_t (&size)[8], const int64_t (&stride)[8], const T* x, int64_t numel, int bits,
@@ -3475,27 +3554,25 @@ int dispatch_quantize_strided(int n, const int64_t (&size)[8], const int64_t (&s
     }
   } else if (stride[n - 2] == 1 && stride[n - 1] != 1 && n <= 3 && (n == 2 || stride[0] != 1) && size[n - 2] % W == 0 &&
              size[n - 1] < (1 << 24) && numel / size[n - 1] < 0x7fffffffLL) {
-    const int64_t sge = 8 / bits * GROUP;
-    if (takes_strips(bits, numel, size[n - 1])) {
+    if (takes_strips(sizeof(T), bits, numel, size[n - 1])) {
       ss.M = (uint32_t)size[n - 2];
       ss.K = (uint32_t)size[n - 1];
       ss.sk = stride[n - 1];
       ss.sb = n == 3 ? stride[0] : 0;
       ss.batch = n == 3 ? (uint32_t)size[0] : 1;
       ss.strips = (ss.M + STRIP_PIECES * W - 1) / (STRIP_PIECES * W);
-      const int64_t strips = (int64_t)ss.strips * ss.batch, per_channel = (ss.K + sge - 1) / sge;
-      int64_t segments = (STRIP_WORKGROUPS + strips - 1) / strips;
-      segments = segments < per_channel ? segments : per_channel;
-      ss.segment = (uint32_t)((per_channel + segments - 1) / segments);
-      ss.segments = (uint32_t)((per_channel + ss.segment - 1) / ss.segment);
+      const int64_t strips = (int64_t)ss.strips * ss.batch;
+      const StripCut cut = strip_cut(bits, strips, ss.K);
+      ss.segment = (uint32_t)cut.segment;
+      ss.segments = (uint32_t)cut.segments;
       shape = &ss;
       p.grid = dim3((unsigned)(strips * ss.segments));
       p.block = dim3(STRIP_THREADS);
       switch (bits) {
-        case 1: p.kernel = quantize_strips_of<T, 1>(noise_mode); break;
-        case 2: p.kernel = quantize_strips_of<T, 2>(noise_mode); break;
-        case 4: p.kernel = quantize_strips_of<T, 4>(noise_mode); break;
-        case 8: p.kernel = quantize_strips_of<T, 8>(noise_mode); break;
+        case 1: p.kernel = cut.gs == 1 ? quantize_strips_of<T, 1, 1>(noise_mode) : quantize_strips_of<T, 1, 2>(noise_mode); break;
+        case 2: p.kernel = cut.gs == 1 ? quantize_strips_of<T, 2, 1>(noise_mode) : quantize_strips_of<T, 2, 2>(noise_mode); break;
+        case 4: p.kernel = cut.gs == 1 ? quantize_strips_of<T, 4, 1>(noise_mode) : quantize_strips_of<T, 4, 2>(noise_mode); break;
+        case 8: p.kernel = quantize_strips_of<T, 8, 1>(noise_mode); break;
       }
       void* args[] = {(void*)&seed, (void*)&x, (void*)&numel, (void*)&N, (void*)&packed, (void*)&scale, (void*)&mn, (void*)&mx, shape};
       return hipLaunchKernel(p.kernel, p.grid, p.block, args, p.lds, stream) == hipSuccess ? GACT_OK : GACT_ELAUNCH;

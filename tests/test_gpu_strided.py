@@ -90,3 +90,21 @@ def test_strided_large_tensors():
     x = torch.randn((64, 197, 12, 64), generator=g, device="cuda").to(torch.bfloat16).permute(0, 2, 1, 3)
     a, b = ops.op_quantize(x, 2, 3), ops.op_quantize(x.contiguous(), 2, 3)
     assert torch.equal(a[0][:-1], b[0][:-1]) and torch.equal(a[2], b[2]) and torch.equal(a[3], b[3])
+
+
+# batch, channels, pixels: channels that do not fill a strip, first super-groups at every offset, a ragged last group; strips cut
+# into segments and not, more of them than the GPU holds at once, and (270) a number for which a step takes one group
+@pytest.mark.parametrize("shape", [(3, 40, 2052), (1, 8, 1540), (9, 40, 12292), (270, 32, 2048), (530, 32, 2060), (70, 256, 3076)],
+                         ids=lambda s: "%dx%dx%d" % s)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["f32", "f16"])
+def test_strips_of_long_channels(shape, dtype):
+    b, c, k = shape
+    x = torch.randn((b, k, c), generator=torch.Generator(device="cuda").manual_seed(k), device="cuda").to(dtype)
+    x[0, :600] = 0.0        # groups of equal values: the largest scale there is (half: infinite in the first)
+    x[0, 5, 0] = 6e-8
+    x = x.transpose(1, 2)
+    y = x.contiguous()
+    for bits in (1, 2, 4, 8):
+        for stream in ("fast", "deterministic"):
+            p, q = ops.op_quantize(x, bits, 5, rng_stream=stream), ops.op_quantize(y, bits, 5, rng_stream=stream)
+            assert torch.equal(p[0][:-1], q[0][:-1]) and torch.equal(p[2], q[2]) and torch.equal(p[3], q[3]), (bits, stream)
