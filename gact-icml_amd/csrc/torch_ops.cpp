@@ -35,12 +35,12 @@ bool ordinary_call() {
          !at::impl::torch_function_mode_enabled();
 }
 
-// a tensor (or parameter) itself, no subclass and no wrapper, dense on the GPU
+// a tensor (or parameter) itself, no subclass and no wrapper, no lazily negated view, dense on the GPU
 const at::Tensor* plain(PyObject* o) {
   if (!THPVariable_CheckExact(o)) return nullptr;
   const at::Tensor& t = THPVariable_Unpack(o);
   static const c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::Functionalize, c10::DispatchKey::ZeroTensor,
-                                            c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper});
+                                            c10::DispatchKey::Negative, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper});
   if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || !t.has_storage() || t.key_set().has_any(wrapped)) return nullptr;
   return &t;
 }

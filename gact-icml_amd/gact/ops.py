@@ -104,7 +104,7 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
             raise RuntimeError("seed_offset must be one int64 on the device of the data")
     if input.is_contiguous():
         x = input
-    elif in_place and group == _abi.GROUP and mode in (_abi.NOISE_FAST, _abi.NOISE_CONST) \
+    elif in_place and not input.is_neg() and group == _abi.GROUP and mode in (_abi.NOISE_FAST, _abi.NOISE_CONST) \
             and _quantize_strided(input, q_bit, mode, seed, seed_offset, q_input, q_scale, q_min):
         return q_input, q_scale, q_min
     else:
