@@ -2071,7 +2071,8 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
       step(t, even, 2);
       if (t + 1 < end) step(t + 1, odd, 2);
     }
-  } else {                   // one step's, as many bytes
+  } else {                   // one step's, as many bytes (two steps': half [64,256,56,56] 4 bit 37.8 -> 39.9 us, 2 bit 40.4 -> 44.5,
+                             // float 4 bit 63.9 -> 66.5, half [16,256,56,56] 15.9 -> 17.4; nothing gained)
     Chunk q[GS];
 #pragma unroll
     for (int h = 0; h < GS; h++) load(j_first * GS + h, q[h]);
