@@ -169,7 +169,9 @@ PyObject* dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int dtype = dtype_code(mn->scalar_type());
   const c10::Device device = codes->device();
   if (dtype < 0 || !one_pass(group, dtype) || codes->scalar_type() != at::kChar || codes->dim() != 1 || scale->device() != device ||
-      mn->device() != device || scale->scalar_type() != (dtype == GACT_BF16 ? at::kFloat : mn->scalar_type()))
+      mn->device() != device || scale->scalar_type() != (dtype == GACT_BF16 ? at::kFloat : mn->scalar_type()) ||
+      !codes->is_contiguous() || !scale->is_contiguous() || !mn->is_contiguous() ||
+      (group != kGroup && (scale->dim() != 3 || mn->dim() != 3)))
     Py_RETURN_NONE;
   const Py_ssize_t dims = PyTuple_GET_SIZE(args[1]);
   int64_t numel = 1;
@@ -277,7 +279,7 @@ PyObject* mask_unpack(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   const at::Tensor* mask;
   int64_t numel;
-  if (n != 2 || !(mask = plain(args[0])) || !integer(args[1], &numel) || mask->scalar_type() != at::kInt || numel <= 0 ||
+  if (n != 2 || !(mask = plain(args[0])) || !integer(args[1], &numel) || mask->scalar_type() != at::kInt || !mask->is_contiguous() || numel <= 0 ||
       numel > INT64_MAX / 2 || mask->numel() < (numel + 31) / 32 || !ordinary_call())
     Py_RETURN_NONE;
   const c10::Device device = mask->device();

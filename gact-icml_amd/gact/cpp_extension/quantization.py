@@ -153,8 +153,7 @@ def act_dequantize_dropout_mask(mask, N):
     if out is not None:
         return out
     N = int(N)
-    if not mask.is_cuda:
-        raise RuntimeError("mask must be a CUDA tensor!")
+    _check_cuda(mask, "mask")
     if mask.dtype != torch.int32 or mask.numel() < (N + 31) // 32:
         raise RuntimeError("mask must be int32 with ceil(N/32) words")
     out = torch.empty((N,), dtype=torch.uint8, device=mask.device)

@@ -192,10 +192,15 @@ def op_dequantize(input, input_shape):
         return groups.ravel()[:num_features].reshape(*input_shape).contiguous()
 
     ext_quantization._check_bits(q_bit)
-    if not q_input.is_cuda:
-        raise RuntimeError("data must be a CUDA tensor!")
+    # the kernels index dense memory of the GPU
+    ext_quantization._check_cuda(q_input, "data")
     if q_input.dtype is not torch.int8 or q_input.dim() != 1:
         raise RuntimeError("The type of data is not correct!")
+    for t, name in ((q_scale, "scale"), (q_min, "min")):
+        if group == _abi.GROUP:
+            ext_quantization._check_cuda(t, name)
+        else:       # as unpack_single_precision, which serves the group sizes without a single-pass kernel
+            ext_quantization._check_cuda_dim_float(t, name, 3)
     N = (num_features + group - 1) // group
     if q_input.numel() < ext_quantization.packed_numel(q_bit, N, 1, group) - 1 \
             or q_scale.numel() < N or q_min.numel() < N:

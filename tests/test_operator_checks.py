@@ -1,0 +1,115 @@
+"""What the operators' Python path refuses, copies and hands on, without a GPU: tensors in host memory that say they are on the
+GPU, and a library that only writes down which entry point was called."""
+import pytest
+import torch
+
+from gact import ops
+from gact.conf import config
+from gact.cpp_extension import _abi, quantization
+
+
+class _SaysGpu(torch.Tensor):
+    is_cuda = property(lambda self: True)
+
+
+class _Library:
+    """Every entry point succeeds and is noted with its arguments."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.calls.append((name, args))
+            return 0
+        return call
+
+
+@pytest.fixture
+def library(monkeypatch):
+    lib = _Library()
+    _abi.native()       # the real one: it leaves tensors that are not plain GPU tensors to Python
+    monkeypatch.setattr(_abi, "lib", lambda: lib)
+    monkeypatch.setattr(_abi, "call_on", lambda device, fn, *args: fn(*args))
+    monkeypatch.setattr(_abi, "stream_of", lambda t: 0)
+    monkeypatch.setattr(ops, "_current_stream", lambda index: 0)
+    monkeypatch.setattr(torch.cuda, "device", lambda device: _Nothing())
+    saved = config.group_size
+    yield lib
+    config.group_size = saved
+
+
+class _Nothing:
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *args):
+        return False
+
+
+def gpu(t):
+    return t.as_subclass(_SaysGpu)
+
+
+def _compressed(group, bits=4, groups=6):
+    codes = gpu(torch.zeros(quantization.packed_numel(bits, groups, 1, group), dtype=torch.int8))
+    return [codes, bits, gpu(torch.ones(groups, 1, 1)), gpu(torch.zeros(groups, 1, 1))]
+
+
+@pytest.mark.parametrize("group", [64, 128, 256, 512])
+def test_dequantize_takes_dense_gpu_memory_only(library, group):
+    config.group_size = group
+    shape = (6, group)
+    ops.op_dequantize(_compressed(group), shape)
+    assert len(library.calls) == 1
+    n = _compressed(group)[0].numel()
+    bad = [(0, torch.zeros(n, dtype=torch.int8), "data must be a CUDA tensor"),
+           (0, gpu(torch.zeros(2 * n, dtype=torch.int8)[::2]), "data must be contiguous"),
+           (0, gpu(torch.zeros(1, dtype=torch.int8).expand(n)), "data must be contiguous")]
+    for i, name in ((2, "scale"), (3, "min")):
+        bad += [(i, torch.ones(6, 1, 1), name + " must be a CUDA tensor"),
+                (i, gpu(torch.ones(1, 1, 1).expand(6, 1, 1)), name + " must be contiguous"),
+                (i, gpu(torch.ones(12, 1, 1)[::2]), name + " must be contiguous")]
+        if group != 256:
+            bad.append((i, gpu(torch.ones(6)), "dimension of %s" % name))
+    for i, t, message in bad:
+        q = _compressed(group)
+        q[i] = t
+        with pytest.raises(RuntimeError, match=message):
+            ops.op_dequantize(q, shape)
+    assert len(library.calls) == 1
+
+
+def test_mask_is_dense_gpu_memory(library):
+    for t, message in ((torch.zeros(4, dtype=torch.int32), "mask must be a CUDA tensor"),
+                       (gpu(torch.zeros(8, dtype=torch.int32)[::2]), "mask must be contiguous"),
+                       (gpu(torch.zeros(1, dtype=torch.int32).expand(4)), "mask must be contiguous")):
+        with pytest.raises(RuntimeError, match=message):
+            quantization.act_dequantize_dropout_mask(t, 128)
+    assert not library.calls
+    quantization.act_dequantize_dropout_mask(gpu(torch.zeros(4, dtype=torch.int32)), 128)
+    assert len(library.calls) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("group", [64, 128, 256, 512])
+def test_strided_statistics_codes_and_masks_are_refused_on_the_gpu(group, monkeypatch):
+    """The native calls leave them to Python, which raises; nothing is launched."""
+    monkeypatch.setattr(config, "group_size", group)
+    x = torch.randn(6, group, device="cuda")
+    q = ops.op_quantize(x, 4, 1)
+    native = _abi.native()
+    assert native.dequantize(q[0], x.shape, 4, q[2], q[3], group) is not None
+    bad = [(0, torch.cat([q[0], q[0]])[::2], "data"), (0, q[0][:1].expand(q[0].numel()), "data"), (0, q[0].cpu(), "data"),
+           (2, torch.cat([q[2], q[2]])[::2], "scale"), (2, q[2][:1].expand(6, 1, 1), "scale"), (2, q[2].cpu(), "scale"),
+           (3, torch.cat([q[3], q[3]])[::2], "min"), (3, q[3][:1].expand(6, 1, 1), "min"), (3, q[3].cpu(), "min")]
+    for i, t, name in bad:
+        args = [t if k == i else v for k, v in enumerate(q)]
+        assert native.dequantize(args[0], x.shape, 4, args[2], args[3], group) is None, (i, name)
+        with pytest.raises(RuntimeError, match=name + " must be"):
+            ops.op_dequantize(args, x.shape)
+    mask = torch.zeros(8, dtype=torch.int32, device="cuda")
+    for t in (mask[::2], mask[:1].expand(4)):
+        assert native.mask_unpack(t, 128) is None
+        with pytest.raises(RuntimeError, match="mask must be contiguous"):
+            quantization.act_dequantize_dropout_mask(t, 128)
