@@ -94,6 +94,8 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
             if (not noise.is_cuda) or noise.dtype != torch.float32 or noise.numel() != N * config.group_size \
                     or not noise.is_contiguous():
                 raise RuntimeError("noise must be a contiguous float32 CUDA tensor with one value per padded element")
+            if group != _abi.GROUP and not _abi.aligned(noise):
+                noise = noise.clone()       # the launches of the extension-style sequence took it as it was
     device = input.device
     q_input = torch.empty(ext_quantization.packed_numel(q_bit, N, 1, group), dtype=torch.int8, device=device)
     # bfloat16 (not in the reference) is quantized as the float values it holds: float scale, bfloat16 min
@@ -187,7 +189,8 @@ def op_dequantize(input, input_shape):
         return q_input.ravel()[:num_features].reshape(*input_shape).contiguous()
 
     group = config.group_size
-    if group != _abi.GROUP and not _one_pass(group, q_min.dtype):
+    # codes at any address: the one-pass kernels load 16 bytes at a time, unpack takes what they do not
+    if group != _abi.GROUP and not (_one_pass(group, q_min.dtype) and _abi.aligned(q_input)):
         groups = dequantize_and_unpack(q_input, input_shape, q_bit, q_scale, q_min)
         return groups.ravel()[:num_features].reshape(*input_shape).contiguous()
 

@@ -91,6 +91,41 @@ def test_mask_is_dense_gpu_memory(library):
     assert len(library.calls) == 1
 
 
+@pytest.mark.parametrize("group", [64, 128, 512])
+def test_codes_and_noise_at_any_address(library, group):
+    """The one-pass kernels are for 16-byte aligned memory: other codes take unpack, other noise is copied first."""
+    config.group_size = group
+    q = _compressed(group)
+    for offset, entry in ((0, "gact_dequantize_groups"), (1, "gact_unpack"), (16, "gact_dequantize_groups")):
+        buffer = torch.zeros(q[0].numel() + 16, dtype=torch.int8)
+        assert buffer.data_ptr() % 16 == 0
+        library.calls.clear()
+        ops.op_dequantize([gpu(buffer[offset:offset + q[0].numel()])] + q[1:], (6, group))
+        assert [name for name, _ in library.calls] == [entry], offset
+    x, noise = gpu(torch.zeros(6, group)), gpu(torch.zeros(6 * group + 1))
+    for part in (noise[:-1], noise[1:]):
+        library.calls.clear()
+        ops.op_quantize(x, 4, 1, noise=part)
+        (name, args), = library.calls
+        assert name == "gact_quantize_groups" and args[8] % 16 == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("group", [64, 128, 512])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["f32", "f16"])
+def test_codes_and_noise_at_any_address_on_the_gpu(group, dtype, monkeypatch):
+    monkeypatch.setattr(config, "group_size", group)
+    x = torch.randn(5 * group + 3, device="cuda").to(dtype)
+    noise = torch.rand(6 * group + 1, device="cuda")
+    for bits in (1, 2, 4, 8):
+        p, q = ops.op_quantize(x, bits, 1, noise=noise[1:]), ops.op_quantize(x, bits, 1, noise=noise[1:].clone())
+        want = ops.op_dequantize(q, x.shape)
+        assert torch.equal(p[0][:-1], q[0][:-1])
+        codes = torch.cat([q[0][:1], q[0]])[1:]
+        assert codes.data_ptr() % 16 == 1
+        assert torch.equal(ops.op_dequantize([codes] + q[1:], x.shape), want)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("group", [64, 128, 256, 512])
 def test_strided_statistics_codes_and_masks_are_refused_on_the_gpu(group, monkeypatch):
