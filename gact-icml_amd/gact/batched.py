@@ -147,6 +147,8 @@ class BatchedQuantizer:
                 raise RuntimeError("tensor %d does not match the geometry this batch was built for" % i)
             if not t.is_cuda or not t.is_contiguous():
                 raise RuntimeError("tensor %d must be a contiguous CUDA tensor" % i)
+            if t.is_neg():      # an output as well as an input
+                raise RuntimeError("tensor %d is a lazily negated view: resolve_neg() it first" % i)
             if not _abi.aligned(t):
                 raise RuntimeError("tensor %d is not 16-byte aligned" % i)
             e = arr[i]

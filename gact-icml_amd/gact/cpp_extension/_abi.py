@@ -150,3 +150,9 @@ def ptr(t):
 def aligned(t):
     """The kernels use 16-byte loads; fresh torch allocations always qualify, offset views may not."""
     return t.data_ptr() % 16 == 0
+
+
+def stored(t):
+    """t, or a copy of it where its memory does not hold its values (a lazily negated view: torch reads it through a
+    sign flip, a kernel would not)."""
+    return t.resolve_neg() if t.is_neg() else t

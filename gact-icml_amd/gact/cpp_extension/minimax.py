@@ -19,6 +19,7 @@ def minimax(data):
     both = _abi.native().minimax(data)
     if both is not None:
         return both
+    data = _abi.stored(data)
     _check_cuda_float(data, "data")
     if data.dim() != 2:
         raise RuntimeError("The dimension of data is not correct!")

@@ -79,6 +79,7 @@ def pack_single_precision(data, min, max, bits, stochastic, seed, *, noise=None,
         q = _abi.native().pack(data, min, max, bits, seed, _abi.NOISE_MODES.get(stream, -1))
         if q is not None:
             return q
+    data, min, max = _abi.stored(data), _abi.stored(min), _abi.stored(max)
     _check_cuda_dim_float(data, "data", 3)
     _check_cuda_dim_float(min, "min", 3)
     _check_cuda_dim_float(max, "max", 3)
@@ -108,6 +109,7 @@ def unpack_single_precision(data, bits, scale, min, N, num_groups, group_size):
     out = _abi.native().unpack(data, bits, scale, min, N, num_groups, group_size)
     if out is not None:
         return out
+    data, scale, min = _abi.stored(data), _abi.stored(scale), _abi.stored(min)
     # CHECK_CUDA_TENSOR_DIM_TYPE(data, 1, kInt8), quantization.cc:43
     _check_cuda(data, "data")
     if data.dim() != 1:

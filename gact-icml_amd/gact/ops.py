@@ -56,6 +56,7 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
         if q:
             return q
         in_place = q is not False
+    input = _abi.stored(input)
     N = _num_groups(input.numel())
     if q_bit == 32:
         # the passthrough of ops.py:21-24: the padded [N, group] view itself, max - min, min
@@ -106,7 +107,7 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
             raise RuntimeError("seed_offset must be one int64 on the device of the data")
     if input.is_contiguous():
         x = input
-    elif in_place and not input.is_neg() and group == _abi.GROUP and mode in (_abi.NOISE_FAST, _abi.NOISE_CONST) \
+    elif in_place and group == _abi.GROUP and mode in (_abi.NOISE_FAST, _abi.NOISE_CONST) \
             and _quantize_strided(input, q_bit, mode, seed, seed_offset, q_input, q_scale, q_min):
         return q_input, q_scale, q_min
     else:
@@ -195,6 +196,7 @@ def op_dequantize(input, input_shape):
         return groups.ravel()[:num_features].reshape(*input_shape).contiguous()
 
     ext_quantization._check_bits(q_bit)
+    q_input, q_scale, q_min = _abi.stored(q_input), _abi.stored(q_scale), _abi.stored(q_min)
     # the kernels index dense memory of the GPU
     ext_quantization._check_cuda(q_input, "data")
     if q_input.dtype is not torch.int8 or q_input.dim() != 1:

@@ -79,10 +79,12 @@ def test_strided_equals_contiguous(layout, dtype):
     assert a[2].numel() == N
 
 
-def test_lazily_negated_view():
-    """Memory holds the values before the negation: the contiguous copy resolves it, the kernels in place would not."""
+@pytest.mark.parametrize("dense", [False, True], ids=["transposed", "dense"])
+def test_lazily_negated_view(dense):
+    """Memory holds the values before the negation: it is resolved first."""
     x = torch.randn((1000, 328), generator=torch.Generator().manual_seed(2)).cuda()
-    a, b = ops.op_quantize(torch._neg_view(x.t()), 4, 3), ops.op_quantize((-x).t().contiguous(), 4, 3)
+    x = x if dense else x.t()
+    a, b = ops.op_quantize(torch._neg_view(x), 4, 3), ops.op_quantize((-x).contiguous(), 4, 3)
     assert torch.equal(a[0][:-1], b[0][:-1]) and torch.equal(a[2], b[2]) and torch.equal(a[3], b[3])
 
 

@@ -1,11 +1,14 @@
 """What the operators' Python path refuses, copies and hands on, without a GPU: tensors in host memory that say they are on the
 GPU, and a library that only writes down which entry point was called."""
+import ctypes
+
 import pytest
 import torch
 
 from gact import ops
+from gact.batched import BatchedQuantizer
 from gact.conf import config
-from gact.cpp_extension import _abi, quantization
+from gact.cpp_extension import _abi, minimax, quantization
 
 
 class _SaysGpu(torch.Tensor):
@@ -34,6 +37,7 @@ def library(monkeypatch):
     monkeypatch.setattr(_abi, "stream_of", lambda t: 0)
     monkeypatch.setattr(ops, "_current_stream", lambda index: 0)
     monkeypatch.setattr(torch.cuda, "device", lambda device: _Nothing())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     saved = config.group_size
     yield lib
     config.group_size = saved
@@ -45,6 +49,11 @@ class _Nothing:
 
     def __exit__(self, *args):
         return False
+
+
+class _NoTables:
+    def batch_table(self, *args):
+        return None
 
 
 def gpu(t):
@@ -89,6 +98,49 @@ def test_mask_is_dense_gpu_memory(library):
     assert not library.calls
     quantization.act_dequantize_dropout_mask(gpu(torch.zeros(4, dtype=torch.int32)), 128)
     assert len(library.calls) == 1
+
+
+def _floats(address, n):
+    return list((ctypes.c_float * n).from_address(address))
+
+
+def _negated(t):
+    return gpu(torch._neg_view(-t))
+
+
+@pytest.mark.parametrize("group", [128, 256])
+def test_lazily_negated_views_are_resolved(library, group, monkeypatch):
+    """A dense one is contiguous: what goes to the library is its values, not its memory, which holds them with the other sign."""
+    config.group_size = group
+    seen = []
+
+    def entry(*indices):
+        def call(*args):
+            seen.append([_floats(args[i], n) for i, n in indices])
+            return 0
+        return call
+
+    n = 2 * group
+    x, stats = torch.arange(1.0, n + 1).view(2, group), torch.tensor([3.0, 5.0]).view(2, 1, 1)
+    values, two = x.flatten().tolist(), [3.0, 5.0]
+    library.gact_quantize = library.gact_quantize_groups = entry((0, n))
+    ops.op_quantize(_negated(x), 4, 0)
+    library.gact_dequantize = library.gact_dequantize_groups = entry((2, 2), (3, 2))
+    q = _compressed(group, groups=2)
+    ops.op_dequantize([q[0], 4, _negated(stats), _negated(stats)], (2, group))
+    library.gact_minimax = entry((0, n))
+    minimax.minimax(_negated(x))
+    library.gact_pack = entry((0, n), (1, 2), (2, 2))
+    quantization.pack_single_precision(_negated(x.view(2, 1, group)), _negated(stats), _negated(stats), 4, True, 0)
+    library.gact_unpack = entry((2, 2), (3, 2))
+    quantization.unpack_single_precision(q[0], 4, _negated(stats), _negated(stats), 2, 1, group)
+    assert seen == [[values], [two, two], [values], [values, two, two], [two, two]]
+    library.gact_batch_workspace_bytes = lambda *args: 4096
+    batch = BatchedQuantizer([n], [torch.float32], "cpu")
+    monkeypatch.setattr(_abi, "native", lambda: _NoTables())       # the native one asks for pinned memory first
+    batch._table([gpu(x)], [0])
+    with pytest.raises(RuntimeError, match="resolve_neg"):
+        batch._table([_negated(x)], [0])
 
 
 @pytest.mark.parametrize("group", [64, 128, 512])
