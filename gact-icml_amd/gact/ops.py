@@ -51,7 +51,7 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
     """gact/gact/ops.py:11-32 -> (q_input, q_scale, q_min).  `seed_offset` (one int64 on the GPU, optional) is added
     to `seed` when the kernel runs, for launches recorded in a HIP graph."""
     in_place = True     # whether a layout that is not contiguous is worth asking the kernels for
-    if noise is None and seed_offset is None:
+    if noise is None and seed_offset is None and q_bit != 32:     # the passthrough needs no library
         q = _abi.native().quantize(input, q_bit, seed, _mode_of(rng_stream), config.group_size)
         if q:
             return q
@@ -179,16 +179,16 @@ def op_quantize(input, q_bit, seed, *, noise=None, rng_stream=None, seed_offset=
 def op_dequantize(input, input_shape):
     """gact/gact/ops.py:61-69 -> tensor of `input_shape`, contiguous, dtype of the scale."""
     q_input, q_bit, q_scale, q_min = input
-    out = _abi.native().dequantize(q_input, input_shape, q_bit, q_scale, q_min, config.group_size)
-    if out is not None:
-        return out
     if not isinstance(q_bit, int):
         print("bits must be intergers, now bits ", q_bit)
         assert(False)
-    num_features = math.prod(input_shape)
-    if q_bit == 32:
-        return q_input.ravel()[:num_features].reshape(*input_shape).contiguous()
+    if q_bit == 32:         # the passthrough needs no library
+        return q_input.ravel()[:math.prod(input_shape)].reshape(*input_shape).contiguous()
+    out = _abi.native().dequantize(q_input, input_shape, q_bit, q_scale, q_min, config.group_size)
+    if out is not None:
+        return out
 
+    num_features = math.prod(input_shape)
     group = config.group_size
     # codes at any address: the one-pass kernels load 16 bytes at a time, unpack takes what they do not
     if group != _abi.GROUP and not (_one_pass(group, q_min.dtype) and _abi.aligned(q_input)):

@@ -117,6 +117,18 @@ def test_32_bit_passthrough_needs_no_kernel():
     assert torch.equal(ops.op_dequantize(q, x.shape), x)
 
 
+def test_32_bit_passthrough_needs_no_library(monkeypatch):
+    def missing():
+        raise RuntimeError("not built")
+
+    monkeypatch.setattr(_abi, "native", missing)
+    monkeypatch.setattr(_abi, "lib", missing)
+    x = torch.rand(7, 100)
+    assert torch.equal(ops.op_dequantize(ops.op_quantize(x, 32, 0), x.shape), x)
+    with pytest.raises(AssertionError):
+        ops.op_dequantize([torch.zeros(1), 2.0, torch.zeros(1), torch.zeros(1)], (1,))
+
+
 def test_dequantize_rejects_non_int_bits():
     with pytest.raises(AssertionError):
         ops.op_dequantize([torch.zeros(1), 2.0, torch.zeros(1), torch.zeros(1)], (1,))
