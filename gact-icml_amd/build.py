@@ -55,8 +55,18 @@ def up_to_date():
     built = (OUT, PROBE_OUT, TORCH_OUT)
     if not all(os.path.exists(p) for p in built):
         return False
+    with open(TORCH_OUT, "rb") as f:
+        if torch_mark() not in f.read():     # built for another torch
+            return False
     t = min(os.path.getmtime(p) for p in built)
     return all(os.path.getmtime(p) <= t for p in (SRC, PROBE_SRC, TORCH_SRC, HDR, os.path.abspath(__file__)))
+
+
+def torch_mark():
+    """What gact_torch.so holds of the torch whose headers and libraries it was built with (gact_torch.torch_version)."""
+    import torch
+
+    return b"torch " + torch.__version__.encode() + b"\0"
 
 
 def torch_command():
@@ -68,7 +78,8 @@ def torch_command():
 
     libs = os.path.join(os.path.dirname(torch.__file__), "lib")
     cmd = [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-I", os.path.join(ROOT, "include")]
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
+           '-DGACT_TORCH_VERSION="%s"' % torch.__version__, "-I", os.path.join(ROOT, "include")]
     for path in cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]]:
         cmd += ["-isystem", path]
     # libtorch.so itself stays out: it would pull in every library torch was built with

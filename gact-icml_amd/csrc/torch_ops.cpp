@@ -320,4 +320,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "gact_torch", "The operators' host 
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_gact_torch(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit_gact_torch(void) {
+  static const char built_with[] = "torch " GACT_TORCH_VERSION;   // the build looks for it in the library
+  PyObject* const m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", built_with + 6) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

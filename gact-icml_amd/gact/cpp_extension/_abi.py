@@ -100,6 +100,9 @@ def native():
         loader = importlib.machinery.ExtensionFileLoader("gact_torch", NATIVE_PATH)
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("gact_torch", loader))
         loader.exec_module(module)
+        if module.torch_version != torch.__version__:
+            raise RuntimeError("gact_torch.so was built with torch %s, this is %s: run `python gact-icml_amd/build.py`"
+                               % (module.torch_version, torch.__version__))
         _NATIVE = module
     return _NATIVE
 

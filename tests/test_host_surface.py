@@ -129,6 +129,20 @@ def test_32_bit_passthrough_needs_no_library(monkeypatch):
         ops.op_dequantize([torch.zeros(1), 2.0, torch.zeros(1), torch.zeros(1)], (1,))
 
 
+def test_native_host_side_belongs_to_the_torch_it_was_built_with(monkeypatch):
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("gact_build", os.path.join(ROOT, "gact-icml_amd", "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    monkeypatch.setattr(build.os.path, "getmtime", lambda path: 0.0)
+    assert _abi.native().torch_version == torch.__version__ and build.up_to_date()
+    monkeypatch.setattr(torch, "__version__", "0.1")
+    monkeypatch.setattr(_abi, "_NATIVE", None)
+    with pytest.raises(RuntimeError, match="built with torch"):
+        _abi.native()
+    assert not build.up_to_date()
+
+
 def test_dequantize_rejects_non_int_bits():
     with pytest.raises(AssertionError):
         ops.op_dequantize([torch.zeros(1), 2.0, torch.zeros(1), torch.zeros(1)], (1,))
