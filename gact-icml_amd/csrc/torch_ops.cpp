@@ -1,8 +1,8 @@
 // The host side of the operators: what Python did for every saved tensor - look at the arguments, allocate the results
 // with torch, find the stream, call the library - in one native call.
 //
-// Every function answers the ordinary call: plain tensors on the GPU, contiguous and aligned as the kernels need, no mode or
-// transform of torch's active.  Anything else, an argument that has to be refused included, gets None and nothing is
+// Every function answers the ordinary call: plain tensors on the GPU, contiguous and aligned as the kernels need (quantize: of
+// any strides, in place or through a contiguous copy), no mode or transform of torch's active.  Anything else, an argument that has to be refused included, gets None and nothing is
 // launched: the Python operator then takes its general path, which accepts or raises as it always did.
 //
 // Arguments come through the C API's fast call and tensors through torch's own wrap / unpack (no pybind11).
@@ -122,7 +122,7 @@ PyObject* tuple_of(std::initializer_list<at::Tensor> tensors) {
 
 bool one_pass(int64_t group, int dtype) { return group == kGroup || ((group == 64 || group == 128 || group == 512) && dtype != GACT_BF16); }
 
-// quantize(x, bits, seed, noise mode, group size) -> (codes, scale, min); False: the layout is not one that is taken in place
+// quantize(x, bits, seed, noise mode, group size) -> (codes, scale, min)
 PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   int bits, mode;
@@ -136,23 +136,29 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int64_t numel = x->numel();
   if (dtype < 0 || numel == 0 || !one_pass(group, dtype) || (group != kGroup && mode == GACT_NOISE_REF)) Py_RETURN_NONE;
   const bool contiguous = x->is_contiguous();
-  if (contiguous ? (reinterpret_cast<uintptr_t>(in(*x)) & 15u) != 0 : (group != kGroup || mode == GACT_NOISE_REF)) Py_RETURN_NONE;
+  if (contiguous && (reinterpret_cast<uintptr_t>(in(*x)) & 15u) != 0) Py_RETURN_NONE;
   const int64_t N = (numel + group - 1) / group;
   const c10::Device device = x->device();
   const at::Tensor codes = make({packed_numel(bits, N, group)}, at::kChar, device);
   const at::Tensor scale = make({N, 1, 1}, dtype == GACT_BF16 ? at::kFloat : x->scalar_type(), device);
   const at::Tensor mn = make({N, 1, 1}, x->scalar_type(), device);
-  const int rc = on(device, [&](void* stream) {
-    if (!contiguous)
+  int rc = GACT_ESHAPE;
+  if (!contiguous && group == kGroup && mode != GACT_NOISE_REF) {
+    rc = on(device, [&](void* stream) {
       return gact_quantize_strided(in(*x), dtype, (int)x->dim(), x->sizes().data(), x->strides().data(), bits, mode, seed, nullptr,
                                    out(codes), out(scale), out(mn), nullptr, stream);
-    if (group == kGroup)
-      return gact_quantize(in(*x), dtype, numel, bits, mode, seed, nullptr, out(codes), out(scale), out(mn), nullptr, stream);
-    return gact_quantize_groups(in(*x), dtype, numel, (int)group, bits, mode, seed, nullptr, nullptr, out(codes), out(scale), out(mn),
-                                nullptr, stream);
-  });
+    });
+  }
+  if (rc == GACT_ESHAPE) {   // contiguous, or a layout that is copied first
+    const at::Tensor dense = x->contiguous();
+    rc = on(device, [&](void* stream) {
+      if (group == kGroup)
+        return gact_quantize(in(dense), dtype, numel, bits, mode, seed, nullptr, out(codes), out(scale), out(mn), nullptr, stream);
+      return gact_quantize_groups(in(dense), dtype, numel, (int)group, bits, mode, seed, nullptr, nullptr, out(codes), out(scale),
+                                  out(mn), nullptr, stream);
+    });
+  }
   if (rc == GACT_OK) return tuple_of({codes, scale, mn});
-  if (!contiguous && rc == GACT_ESHAPE) Py_RETURN_FALSE;
   Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS
 }

@@ -50,12 +50,10 @@ def _padded_groups(input):
 def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, seed_offset=None):
     """gact/gact/ops.py:11-32 -> (q_input, q_scale, q_min).  `seed_offset` (one int64 on the GPU, optional) is added
     to `seed` when the kernel runs, for launches recorded in a HIP graph."""
-    in_place = True     # whether a layout that is not contiguous is worth asking the kernels for
     if noise is None and seed_offset is None and q_bit != 32:     # the passthrough needs no library
         q = _abi.native().quantize(input, q_bit, seed, _mode_of(rng_stream), config.group_size)
-        if q:
+        if q is not None:
             return q
-        in_place = q is not False
     input = _abi.stored(input)
     N = _num_groups(input.numel())
     if q_bit == 32:
@@ -107,7 +105,7 @@ def no_scheme_quantize_pack(input, q_bit, seed, *, noise=None, rng_stream=None, 
             raise RuntimeError("seed_offset must be one int64 on the device of the data")
     if input.is_contiguous():
         x = input
-    elif in_place and group == _abi.GROUP and mode in (_abi.NOISE_FAST, _abi.NOISE_CONST) \
+    elif group == _abi.GROUP and mode in (_abi.NOISE_FAST, _abi.NOISE_CONST) \
             and _quantize_strided(input, q_bit, mode, seed, seed_offset, q_input, q_scale, q_min):
         return q_input, q_scale, q_min
     else:

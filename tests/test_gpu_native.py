@@ -75,6 +75,17 @@ def test_round_trips_equal_the_python_path(monkeypatch, dtype, shape, layout):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("group,stream", [(256, "fast"), (256, "reference"), (128, "fast")])
+def test_layouts_without_a_kernel_are_copied_in_the_native_call(group, stream):
+    for x in (torch.randn(4, 3, 16, 16, device="cuda").contiguous(memory_format=torch.channels_last),
+              torch.randn(33, 50, device="cuda")[:, 3:20], torch.randn(6, 40, device="cuda").t()[::2]):
+        assert not x.is_contiguous()
+        mode = _abi.NOISE_MODES[stream]
+        p, q = (_abi.native().quantize(t, 4, 7, mode, group) for t in (x, x.contiguous()))
+        assert _equal(_written([p[0], 4, p[1], p[2]], x.numel(), 4, group), _written([q[0], 4, q[1], q[2]], x.numel(), 4, group))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("group", [64, 96, 128, 256, 512])
 def test_group_sizes_and_extension_calls_equal_the_python_path(monkeypatch, group):
     monkeypatch.setattr(config, "group_size", group)
