@@ -3496,6 +3496,35 @@ inline int transposed_tile(size_t elem_size, int64_t numel, int64_t K) {
   const int64_t rounds = (numel + slots * most - 1) / (slots * most);
   return (int)(((numel + slots * rounds - 1) / (slots * rounds) + 2047) / 2048 * 2048);
 }
+// Where the tile kernel gains over the contiguous copy before quantize_kernel; elsewhere the caller makes that copy.  us, in place
+// / copy and quantize:
+//   Few pixels: a step of the walk is wider than a channel, most lanes idle, and at 1 bit float few super-groups are in flight:
+//     33 M elements of 2 pixels, half 4 bit 72 / 60  1 bit 109 / 60  float 4 bit 115 / 75  1 bit 206 / 75
+//     of 3, half 1 bit 77 / 62  float 4 bit 84 / 76  1 bit 152 / 77;  of 8, float 1 bit 1.16-1.19 times;  of 12, 0.95
+//   Long channels: a tile of c channels reads (c + W - 1) / c times its bytes (W elements of a piece), the copy always once.  4 bit:
+//     half [1,64,50257] 35 / 39  [5,64,12321] 34 / 25  [42,64,12321] 75 / 148  [3,64,20001] 50 / 27  [26,64,20001] 101 / 168
+//     [3,64,169343] 553 / 453  [42,8,12321] 29 / 15  [24,8,169343] 245 / 65    float [1,256,50257] 220 / 165  [26,64,20001] 167 / 233
+//     [340,8,12321] 94 / 110  [10,64,50257] 504 / 403
+//   Below about a million elements both are bound by their launches, of which this is one less.
+// Of 4851 layouts of 2 to 1000004 pixels, 8 to 1024 channels and 2^15 to 2^26 elements, at the four widths each, 2220 were slower in
+// place by 3 % and more without these lines and the one on channels of one piece in dispatch_quantize_strided; with them fewer than
+// 200 are, 45 of these by more than a tenth.
+inline bool tiles_pay(size_t elem_size, int bits, int64_t numel, int64_t M, int64_t K, int64_t tile) {
+  const bool word = elem_size == 4;
+  int fewest = 0;   // pixels
+  if (numel >= 1 << 24) fewest = bits == 1 ? (word ? 10 : 5) : (word ? 4 : 3);
+  else if (numel >= (bits == 1 ? 1 << 21 : 1 << 23)) fewest = bits == 1 ? (word ? 6 : 3) : (word ? 3 : 0);
+  if (K < fewest) return false;
+  if (numel < (K % 4 != 0 ? (bits == 1 ? 3 << 17 : 1 << 20) : (bits == 1 ? 1 << 20 : 1 << 21))) return true;
+  // the longest channel, in sixteenths of a tile; the copy of narrow memory rows is the faster one (one piece: M is W)
+  int longest = word ? (numel < 1 << 24 ? 11 : 14) : M < 64 ? 6 : numel < 3 << 22 ? 11 : 16;
+  if (!word && M == 8) longest = K % 4 == 0 ? 6 : 3;
+  if (numel < 3 << 20) {
+    if (K % 4 == 0) longest = 17;
+    else if (M == 8) longest = 11;
+  }
+  return 16 * K <= longest * tile;
+}
 template <typename T, int BITS>
 const void* quantize_gather_of(int noise_mode) {
   return noise_mode == GACT_NOISE_CONST ? (const void*)quantize_gather_kernel<T, BITS, GACT_NOISE_CONST>
@@ -3555,7 +3584,13 @@ int dispatch_quantize_strided(int n, const int64_t (&size)[8], const int64_t (&s
     }
   } else if (stride[n - 2] == 1 && stride[n - 1] != 1 && n <= 3 && (n == 2 || stride[0] != 1) && size[n - 2] % W == 0 &&
              size[n - 1] < (1 << 24) && numel / size[n - 1] < 0x7fffffffLL) {
-    if (takes_strips(sizeof(T), bits, numel, size[n - 1])) {
+    const int tile = transposed_tile(sizeof(T), numel, size[n - 1]);
+    const bool tiles = tiles_pay(sizeof(T), bits, numel, size[n - 2], size[n - 1], tile);
+    // channels of one piece leave three quarters of a strip's lanes without work: half [1091,8,3844] 4 bit strips 77, copy 68 us,
+    // [1551,8,2704] 2 bit 90, 63, where tiles (as odd numbers of pixels take) need half of the copy's time
+    const bool one_piece = size[n - 2] == W && bits < 8;
+    if (takes_strips(sizeof(T), bits, numel, size[n - 1]) && !(one_piece && tiles)) {
+      if (one_piece && bits == 1 && size[n - 1] < 32768) return GACT_ESHAPE;   // half [83,8,12544] 36, copy 24; [83,8,50176] 68, 102
       ss.M = (uint32_t)size[n - 2];
       ss.K = (uint32_t)size[n - 1];
       ss.sk = stride[n - 1];
@@ -3578,12 +3613,13 @@ int dispatch_quantize_strided(int n, const int64_t (&size)[8], const int64_t (&s
       void* args[] = {(void*)&seed, (void*)&x, (void*)&numel, (void*)&N, (void*)&packed, (void*)&scale, (void*)&mn, (void*)&mx, shape};
       return hipLaunchKernel(p.kernel, p.grid, p.block, args, p.lds, stream) == hipSuccess ? GACT_OK : GACT_ELAUNCH;
     }
+    if (!tiles) return GACT_ESHAPE;
     ts.M = (uint32_t)size[n - 2];
     ts.K = (uint32_t)size[n - 1];
     ts.sk = stride[n - 1];
     ts.sb = n == 3 ? stride[0] : 0;
     ts.channels = numel / size[n - 1];
-    ts.tile = transposed_tile(sizeof(T), numel, size[n - 1]);
+    ts.tile = tile;
     // a tile's rows and batch entries have to lie within 4 GB of its first entry
     const int64_t entries = ts.tile / ((int64_t)ts.M * ts.K) + 2;
     if ((entries * ts.sb + (int64_t)ts.K * ts.sk + ts.M) * (int64_t)sizeof(T) > 0xffffffffLL) return GACT_ESHAPE;

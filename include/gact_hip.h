@@ -105,8 +105,9 @@ int gact_dequantize_groups(const void* packed, int bits, const void* scale, cons
  * whose innermost runs are contiguous and whole 16-byte pieces (at most three more dimensions once those that lie one inside
  * the other are joined), and tensors whose last but one dimension is the contiguous one (channels-last activations,
  * transposed matrices; at most one more dimension), both with 16-byte aligned base and strides; streams GACT_NOISE_CONST and
- * GACT_NOISE_FAST.  Anything else: GACT_ESHAPE and no launch - make a contiguous copy.  No counterpart in the reference, whose
- * reshape copies (gact/gact/ops.py:12-19). */
+ * GACT_NOISE_FAST.  Anything else, and layouts of the second kind of which a contiguous copy is the faster way (one or a few
+ * of the strided dimension's elements per channel; channels far longer than what a workgroup holds): GACT_ESHAPE and no
+ * launch - make a contiguous copy.  No counterpart in the reference, whose reshape copies (gact/gact/ops.py:12-19). */
 int gact_quantize_strided(const void* x, int dtype, int ndim, const int64_t* sizes, const int64_t* strides, int bits, int noise_mode,
                           uint64_t seed, const uint64_t* seed_add, void* packed, void* scale, void* mn, void* mx, void* stream);
 

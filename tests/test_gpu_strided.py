@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from gact import ops
-from gact.cpp_extension import _abi
+from gact.cpp_extension import _abi, quantization
 
 pytestmark = pytest.mark.gpu
 
@@ -117,3 +117,39 @@ def test_strips_of_long_channels(shape, dtype):
         for stream in ("fast", "deterministic"):
             p, q = ops.op_quantize(x, bits, 5, rng_stream=stream), ops.op_quantize(y, bits, 5, rng_stream=stream)
             assert torch.equal(p[0][:-1], q[0][:-1]) and torch.equal(p[2], q[2]) and torch.equal(p[3], q[3]), (bits, stream)
+
+
+def _rc(x, bits, stream="fast"):
+    """What the entry point answers for the layout, and its outputs."""
+    n = -(-x.numel() // 256)
+    codes = torch.empty(quantization.packed_numel(bits, n, 1, 256), dtype=torch.int8, device="cuda")
+    scale = torch.empty(n, dtype=torch.float32 if x.dtype == torch.bfloat16 else x.dtype, device="cuda")
+    mn = torch.empty(n, dtype=x.dtype, device="cuda")
+    dims = ctypes.c_int64 * x.dim()
+    rc = _abi.lib().gact_quantize_strided(x.data_ptr(), _abi.dtype_code(x.dtype), x.dim(), dims(*x.shape), dims(*x.stride()), bits,
+                                          _abi.NOISE_MODES[stream], 5, None, codes.data_ptr(), scale.data_ptr(), mn.data_ptr(), None,
+                                          torch.cuda.current_stream().cuda_stream)
+    return rc, codes, scale, mn
+
+
+# [batch, channels, pixels], dtype, widths the kernels take in place, widths left to the contiguous copy, which is the faster way there
+@pytest.mark.parametrize("shape,dtype,taken,declined", [
+    ((4096, 8, 2), torch.float32, (1, 2, 4, 8), ()), ((1 << 19, 8, 2), torch.float32, (), (1, 2, 4, 8)),        # few pixels
+    ((1 << 18, 64, 3), torch.float16, (2, 4, 8), (1,)), ((1 << 16, 64, 9), torch.float32, (2, 4, 8), (1,)),
+    ((1 << 14, 64, 17), torch.float32, (1, 2, 4, 8), ()),
+    ((1, 8, 20001), torch.float16, (1, 2, 4, 8), ()), ((3, 64, 20001), torch.float16, (), (1, 2, 4, 8)),        # long channels
+    ((13, 64, 20001), torch.bfloat16, (1, 2, 4, 8), ()), ((7, 64, 20001), torch.float32, (1, 2, 4, 8), ()),
+    ((1, 256, 50257), torch.float32, (), (1, 2, 4, 8)), ((42, 8, 12321), torch.float16, (), (1, 2, 4, 8)),
+    ((83, 8, 12544), torch.float16, (2, 4, 8), (1,)), ((83, 8, 50176), torch.float16, (1, 2, 4, 8), ()),        # channels of one piece
+    ((545, 8, 3844), torch.bfloat16, (1, 2, 4, 8), ()), ((700, 4, 3136), torch.float32, (1, 2, 4, 8), ()),
+], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v)[6:])
+def test_where_the_contiguous_copy_is_faster_it_is_made(shape, dtype, taken, declined):
+    b, c, k = shape
+    x = torch.randn((b, k, c), generator=torch.Generator(device="cuda").manual_seed(k), device="cuda").to(dtype).transpose(1, 2)
+    for bits in taken + declined:
+        q = ops.op_quantize(x.contiguous(), bits, 5)
+        rc, codes, scale, mn = _rc(x, bits)
+        assert rc == (_abi.ESHAPE if bits in declined else 0), bits
+        p = ops.op_quantize(x, bits, 5)
+        for codes, scale, mn in [(p[0], p[2], p[3])] + ([(codes, scale, mn)] if bits in taken else []):
+            assert torch.equal(codes[:-1], q[0][:-1]) and torch.equal(scale.view(-1), q[2].view(-1)) and torch.equal(mn.view(-1), q[3].view(-1)), bits
