@@ -18,8 +18,30 @@ class _NoNative:
         return lambda *args: None
 
 
-def _both(monkeypatch, call):
-    taken = call()
+class _Recorder:
+    """The native functions, and which of them gave an answer."""
+
+    def __init__(self):
+        self.answers = {}
+
+    def __getattr__(self, name):
+        def call(*args):
+            out = getattr(_NATIVE, name)(*args)
+            self.answers.setdefault(name, []).append(out is not None)
+            return out
+        return call
+
+
+_NATIVE = _abi.native()
+
+
+def _both(monkeypatch, call, function, answers=True):
+    """What the call gives by the native function of that name - which answers, or leaves it to Python - and without it."""
+    recorder = _Recorder()
+    with monkeypatch.context() as m:
+        m.setattr(_abi, "native", lambda: recorder)
+        taken = call()
+    assert recorder.answers[function] == [answers]
     with monkeypatch.context() as m:
         m.setattr(_abi, "native", lambda: _NoNative())
         general = call()
@@ -69,9 +91,9 @@ def test_round_trips_equal_the_python_path(monkeypatch, dtype, shape, layout):
         x = x.flatten()[1:]     # not aligned
     for bits in (1, 2, 4, 8):
         for stream in ("fast", "deterministic", "reference"):
-            q, want = _both(monkeypatch, lambda: ops.op_quantize(x, bits, -5, rng_stream=stream))
+            q, want = _both(monkeypatch, lambda: ops.op_quantize(x, bits, -5, rng_stream=stream), "quantize", layout != "sliced")
             assert _equal(_written(q, x.numel(), bits, 256), _written(want, x.numel(), bits, 256)), (bits, stream)
-            assert _equal(*_both(monkeypatch, lambda: ops.op_dequantize(q, x.shape))), (bits, stream)
+            assert _equal(*_both(monkeypatch, lambda: ops.op_dequantize(q, x.shape), "dequantize")), (bits, stream)
 
 
 @pytest.mark.gpu
@@ -90,25 +112,25 @@ def test_layouts_without_a_kernel_are_copied_in_the_native_call(group, stream):
 def test_group_sizes_and_extension_calls_equal_the_python_path(monkeypatch, group):
     monkeypatch.setattr(config, "group_size", group)
     x = torch.randn(5, group * 3 // 2, device="cuda")
-    q, want = _both(monkeypatch, lambda: ops.op_quantize(x, 2, 3))
+    q, want = _both(monkeypatch, lambda: ops.op_quantize(x, 2, 3), "quantize", group != 96)
     assert _equal(_written(q, x.numel(), 2, group), _written(want, x.numel(), 2, group))
-    assert _equal(*_both(monkeypatch, lambda: ops.op_dequantize(q, x.shape)))
+    assert _equal(*_both(monkeypatch, lambda: ops.op_dequantize(q, x.shape), "dequantize", group != 96))
     rows = torch.randn(6, group, device="cuda", dtype=torch.float16)
     mn, mx = minimax.minimax(rows)
-    assert _equal(*_both(monkeypatch, lambda: minimax.minimax(rows)))
+    assert _equal(*_both(monkeypatch, lambda: minimax.minimax(rows), "minimax"))
     args = (rows.view(3, 2, group), mn.view(3, 2, 1), mx.view(3, 2, 1), 4, True, 9)
-    (codes, scale), want = _both(monkeypatch, lambda: quantization.pack_single_precision(*args))
+    (codes, scale), want = _both(monkeypatch, lambda: quantization.pack_single_precision(*args), "pack")
     assert _equal([codes[:-1], scale], [want[0][:-1], want[1]])
-    assert _equal(*_both(monkeypatch, lambda: quantization.unpack_single_precision(codes, 4, scale, args[1], 3, 2, group)))
+    assert _equal(*_both(monkeypatch, lambda: quantization.unpack_single_precision(codes, 4, scale, args[1], 3, 2, group), "unpack"))
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 31, 512, 5000])
 def test_masks_equal_the_python_path(monkeypatch, n):
     x = (torch.rand(n, device="cuda") < 0.5).to(torch.uint8)
-    q, want = _both(monkeypatch, lambda: ops.op_quantize_mask(x))
+    q, want = _both(monkeypatch, lambda: ops.op_quantize_mask(x), "mask_pack")
     assert _equal(q, want)
-    assert _equal(*_both(monkeypatch, lambda: ops.op_dequantize_mask(q)))
+    assert _equal(*_both(monkeypatch, lambda: ops.op_dequantize_mask(q), "mask_unpack"))
 
 
 @pytest.mark.gpu
@@ -146,7 +168,7 @@ def test_batched_tables_and_verdicts(monkeypatch):
     xs = [torch.randn(n, device="cuda").to(dt) for n, dt in ((300, torch.float32), (70000, torch.float16), (256, torch.bfloat16))]
     batch = BatchedQuantizer([x.numel() for x in xs], [x.dtype for x in xs], "cuda")
     bits = torch.tensor([1, 4, 8], dtype=torch.int32, device="cuda")
-    assert _equal(*_both(monkeypatch, lambda: batch._table(xs, [1, -2, 1 << 40])))
+    assert _equal(*_both(monkeypatch, lambda: batch._table(xs, [1, -2, 1 << 40]), "batch_table"))
     outs = {}
     side = torch.cuda.Stream()
     for name in ("here", "elsewhere"):
