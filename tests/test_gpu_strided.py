@@ -12,6 +12,19 @@ from gact.cpp_extension import _abi, quantization
 pytestmark = pytest.mark.gpu
 
 
+def _rc(x, bits, stream="fast"):
+    """What the entry point answers for the layout, and its outputs."""
+    n = -(-x.numel() // 256)
+    codes = torch.empty(quantization.packed_numel(bits, n, 1, 256), dtype=torch.int8, device="cuda")
+    scale = torch.empty(n, dtype=torch.float32 if x.dtype == torch.bfloat16 else x.dtype, device="cuda")
+    mn = torch.empty(n, dtype=x.dtype, device="cuda")
+    dims = ctypes.c_int64 * x.dim()
+    rc = _abi.lib().gact_quantize_strided(x.data_ptr(), _abi.dtype_code(x.dtype), x.dim(), dims(*x.shape), dims(*x.stride()), bits,
+                                          _abi.NOISE_MODES[stream], 5, None, codes.data_ptr(), scale.data_ptr(), mn.data_ptr(), None,
+                                          torch.cuda.current_stream().cuda_stream)
+    return rc, codes, scale, mn
+
+
 def channels_last(n, c, h, w):
     return lambda g: torch.randn((n, c, h, w), generator=g).contiguous(memory_format=torch.channels_last)
 
@@ -70,12 +83,8 @@ def test_strided_equals_contiguous(layout, dtype):
             assert torch.equal(a[0][:-1], b[0][:-1]), where
             assert torch.equal(a[2], b[2]) and torch.equal(a[3], b[3]), where
             assert torch.equal(ops.op_dequantize(a, x.shape), ops.op_dequantize(b, x.shape)), where
-        if dtype != torch.float32:      # and the launch was not declined (or was, and fell back to the copy)
-            dims = ctypes.c_int64 * x.dim()
-            rc = _abi.lib().gact_quantize_strided(x.data_ptr(), _abi.dtype_code(dtype), x.dim(), dims(*x.shape), dims(*x.stride()), bits,
-                                                  _abi.NOISE_FAST, 11, None, a[0].data_ptr(), a[2].data_ptr(), a[3].data_ptr(), None,
-                                                  torch.cuda.current_stream().cuda_stream)
-            assert rc == (0 if taken else _abi.ESHAPE), layout
+        # and the launch was not declined (or was, and fell back to the copy)
+        assert _rc(x, bits)[0] == (0 if taken or (layout == "heads_20" and dtype == torch.float32) else _abi.ESHAPE), layout
     assert a[2].numel() == N
 
 
@@ -95,17 +104,20 @@ def test_strided_large_tensors():
         x = torch.randn(shape, generator=g, device="cuda").to(torch.float16).contiguous(memory_format=torch.channels_last)
         for y in (x, x.float()):
             a, b = ops.op_quantize(y, 4, 3), ops.op_quantize(y.contiguous(), 4, 3)
+            assert _rc(y, 4)[0] == 0, shape
             assert torch.equal(a[0][:-1], b[0][:-1]) and torch.equal(a[2], b[2]) and torch.equal(a[3], b[3]), shape
     x = torch.randn((64, 197, 12, 64), generator=g, device="cuda").to(torch.bfloat16).permute(0, 2, 1, 3)
     a, b = ops.op_quantize(x, 2, 3), ops.op_quantize(x.contiguous(), 2, 3)
+    assert _rc(x, 2)[0] == 0
     assert torch.equal(a[0][:-1], b[0][:-1]) and torch.equal(a[2], b[2]) and torch.equal(a[3], b[3])
 
 
 # batch, channels, pixels: channels that do not fill a strip, first super-groups at every offset, a ragged last group; strips cut
-# into segments and not, more of them than the GPU holds at once, and (270) a number for which a step takes one group
-@pytest.mark.parametrize("shape", [(3, 40, 2052), (1, 8, 1540), (9, 40, 12292), (270, 32, 2048), (530, 32, 2060), (70, 256, 3076)],
-                         ids=lambda s: "%dx%dx%d" % s)
-@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["f32", "f16"])
+# into segments and not, more of them than the GPU holds at once, and numbers for which a step takes one group (half: 270 and, in
+# three segments, 180 of 32 channels; float: 264 and 180 of 16)
+@pytest.mark.parametrize("shape", [(3, 40, 2052), (1, 8, 1540), (9, 40, 12292), (270, 32, 2048), (530, 32, 2060), (70, 256, 3076),
+                                   (270, 32, 3076), (180, 32, 3076), (264, 16, 3076), (180, 16, 3076)], ids=lambda s: "%dx%dx%d" % s)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["f32", "f16", "bf16"])
 def test_strips_of_long_channels(shape, dtype):
     b, c, k = shape
     x = torch.randn((b, k, c), generator=torch.Generator(device="cuda").manual_seed(k), device="cuda").to(dtype)
@@ -116,20 +128,8 @@ def test_strips_of_long_channels(shape, dtype):
     for bits in (1, 2, 4, 8):
         for stream in ("fast", "deterministic"):
             p, q = ops.op_quantize(x, bits, 5, rng_stream=stream), ops.op_quantize(y, bits, 5, rng_stream=stream)
+            assert _rc(x, bits, stream)[0] == 0
             assert torch.equal(p[0][:-1], q[0][:-1]) and torch.equal(p[2], q[2]) and torch.equal(p[3], q[3]), (bits, stream)
-
-
-def _rc(x, bits, stream="fast"):
-    """What the entry point answers for the layout, and its outputs."""
-    n = -(-x.numel() // 256)
-    codes = torch.empty(quantization.packed_numel(bits, n, 1, 256), dtype=torch.int8, device="cuda")
-    scale = torch.empty(n, dtype=torch.float32 if x.dtype == torch.bfloat16 else x.dtype, device="cuda")
-    mn = torch.empty(n, dtype=x.dtype, device="cuda")
-    dims = ctypes.c_int64 * x.dim()
-    rc = _abi.lib().gact_quantize_strided(x.data_ptr(), _abi.dtype_code(x.dtype), x.dim(), dims(*x.shape), dims(*x.stride()), bits,
-                                          _abi.NOISE_MODES[stream], 5, None, codes.data_ptr(), scale.data_ptr(), mn.data_ptr(), None,
-                                          torch.cuda.current_stream().cuda_stream)
-    return rc, codes, scale, mn
 
 
 # [batch, channels, pixels], dtype, widths the kernels take in place, widths left to the contiguous copy, which is the faster way there
@@ -153,3 +153,29 @@ def test_where_the_contiguous_copy_is_faster_it_is_made(shape, dtype, taken, dec
         p = ops.op_quantize(x, bits, 5)
         for codes, scale, mn in [(p[0], p[2], p[3])] + ([(codes, scale, mn)] if bits in taken else []):
             assert torch.equal(codes[:-1], q[0][:-1]) and torch.equal(scale.view(-1), q[2].view(-1)) and torch.equal(mn.view(-1), q[3].view(-1)), bits
+
+
+# one shape per kernel: pieces with addresses of their own, a tile, strips of one and of two groups per step (half, float)
+@pytest.mark.parametrize("shape", [(40, 8, 784), (3, 40, 2052), (9, 40, 12292), (270, 32, 3076), (257, 16, 3076), (33, 12, 197, 64)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["f32", "f16", "bf16"])
+def test_special_values(shape, dtype):
+    """NaN, infinities and the largest values in single elements, in runs along the memory and along a channel, and in whole
+    groups."""
+    g = torch.Generator(device="cuda").manual_seed(sum(shape))
+    x = torch.randn([shape[0], shape[2], shape[1]] + list(shape[3:]), generator=g, device="cuda").to(dtype).transpose(1, 2)
+    big = torch.finfo(dtype).max
+    for i, v in enumerate((float("nan"), float("inf"), -float("inf"), big, -big, 2e30 if dtype != torch.float16 else 6e-8, -0.0)):
+        flat = torch.randint(0, x.numel(), (12,), generator=g, device="cuda")
+        y = x.reshape(-1)               # a copy in index order
+        y[flat] = v
+        y[4096 * i + 1024:4096 * i + 1024 + 512] = v
+        y[4096 * i + 2048:4096 * i + 2048 + 512:2] = v
+        x.copy_(y.view(x.shape))
+        x[0, i % shape[1], :40] = v
+    y = x.contiguous()
+    for bits in (1, 2, 4, 8):
+        for stream in ("fast", "deterministic"):
+            p, q = ops.op_quantize(x, bits, 5, rng_stream=stream), ops.op_quantize(y, bits, 5, rng_stream=stream)
+            for a, b in ((p[0][:-1], q[0][:-1]), (p[2], q[2]), (p[3], q[3])):
+                assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8)), (bits, stream)
