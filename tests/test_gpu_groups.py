@@ -9,6 +9,7 @@ import torch
 import oracle
 from gact import ops
 from gact.conf import config
+from gact.cpp_extension import minimax, quantization
 
 pytestmark = pytest.mark.gpu
 
@@ -73,3 +74,43 @@ def test_one_pass_groups_past_the_lines_of_the_launch(group, dtype):
     x = torch.randn((1 << 26) + 77, generator=torch.Generator().manual_seed(group)).to(dtype)
     for bits in BITS:
         check(x, group, bits, "fast", 5)
+
+
+def _special(numel, group, dtype, gen):
+    """Groups with NaN, infinities and the type's largest values in them, at the first and last element and everywhere, between
+    ordinary ones."""
+    big = torch.finfo(dtype).max
+    x = torch.randn(numel, generator=gen)
+    for i, v in enumerate((float("nan"), float("inf"), -float("inf"), big, -big, 2e30, -2e30, -0.0, 1e-45)):
+        for j, at in enumerate((slice(0, 1), slice(group - 1, group), slice(0, group), slice(0, group, 2), slice(group // 2, group // 2 + 8))):
+            x[(9 * j + i) * group + at.start:(9 * j + i) * group + at.stop:at.step or 1] = v
+    x[45 * group:45 * group + 2] = torch.tensor([float("inf"), -float("inf")])
+    x[46 * group:46 * group + 2] = torch.tensor([big, -big])
+    x[47 * group:48 * group] = float("nan")
+    x[47 * group + 3] = 1.0
+    return x.to(dtype).cuda()
+
+
+def _bits(t):
+    return t.contiguous().view(-1).view(torch.uint8)
+
+
+@pytest.mark.parametrize("group", [64, 128, 512])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=["f32", "f16"])
+@pytest.mark.parametrize("bits", BITS)
+def test_special_values_equal_the_extension_calls(group, dtype, bits):
+    """Bit for bit what minimax, pack and unpack, which serve every group size, make of the zero-padded tensor."""
+    config.group_size = group
+    x = _special(50 * group + 7, group, dtype, torch.Generator().manual_seed(bits))
+    groups = torch.cat([x, x.new_zeros(group - 7)]).view(51, group)
+    mn, mx = minimax.minimax(groups)
+    for stream in ("fast", "deterministic"):
+        q = ops.op_quantize(x, bits, 3, rng_stream=stream)
+        codes, scale = quantization.pack_single_precision(groups.view(51, 1, group), mn.view(51, 1, 1), mx.view(51, 1, 1), bits, True, 3,
+                                                          rng_stream=stream)
+        assert torch.equal(q[0][:-1], codes[:-1]), stream
+        assert torch.equal(_bits(q[2]), _bits(scale)) and torch.equal(_bits(q[3]), _bits(mn)), stream
+        want = quantization.unpack_single_precision(codes, bits, scale, mn.view(51, 1, 1), 51, 1, group).view(-1)[:x.numel()]
+        out = ops.op_dequantize(q, x.shape)
+        assert torch.equal(_bits(out), _bits(want)) or torch.equal(torch.isnan(out), torch.isnan(want)) \
+            and torch.equal(out[~out.isnan()], want[~want.isnan()]), stream
