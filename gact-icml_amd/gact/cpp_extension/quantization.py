@@ -138,6 +138,7 @@ def act_quantize_dropout_mask(data):
     mask = _abi.native().mask_pack(data)
     if mask is not None:
         return mask
+    data = _abi.stored(data)
     # CHECK_CUDA_TENSOR_TYPE(data, kUInt8), quantization.cc:27
     _check_cuda(data, "data")
     if data.dtype != torch.uint8:
@@ -155,6 +156,7 @@ def act_dequantize_dropout_mask(mask, N):
     if out is not None:
         return out
     N = int(N)
+    mask = _abi.stored(mask)
     _check_cuda(mask, "mask")
     if mask.dtype != torch.int32 or mask.numel() < (N + 31) // 32:
         raise RuntimeError("mask must be int32 with ceil(N/32) words")

@@ -104,6 +104,10 @@ def _floats(address, n):
     return list((ctypes.c_float * n).from_address(address))
 
 
+def _words(address, n):
+    return list((ctypes.c_int32 * n).from_address(address))
+
+
 def _negated(t):
     return gpu(torch._neg_view(-t))
 
@@ -141,6 +145,15 @@ def test_lazily_negated_views_are_resolved(library, group, monkeypatch):
     batch._table([gpu(x)], [0])
     with pytest.raises(RuntimeError, match="resolve_neg"):
         batch._table([_negated(x)], [0])
+
+
+def test_lazily_negated_masks_are_resolved(library):
+    seen = []
+    library.gact_mask_pack = lambda x, n, *args: seen.append((ctypes.c_uint8 * n).from_address(x)[:]) or 0
+    library.gact_mask_unpack = lambda x, n, *args: seen.append(_words(x, 2)) or 0
+    ops.op_quantize_mask(gpu(torch._neg_view(torch.tensor([0, 255, 255, 0], dtype=torch.uint8))))
+    ops.op_dequantize_mask([_negated(torch.tensor([5, 9], dtype=torch.int32)), (64,)])
+    assert seen == [[0, 1, 1, 0], [5, 9]]
 
 
 @pytest.mark.parametrize("group", [64, 128, 512])
