@@ -1827,6 +1827,7 @@ template <typename T, int BITS, int NOISE, int GS>
 __global__ void __launch_bounds__(STRIP_THREADS, 4 / GS)
 quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_t N, uint8_t* __restrict__ packed,
                        typename Elem<T>::Stat* __restrict__ scale_out, T* __restrict__ mn_out, T* __restrict__ mx_out, StripShape g) {
+  static_assert(GS <= 8 / BITS, "a super-group holds a step's groups: past the tensor's last group there may be none to store");
   typedef typename Elem<T>::Stat Stat;
   constexpr int CH = Elem<T>::kQChunks, W = Elem<T>::kQWidth, WPT = 8 / BITS, QMAX = (1 << BITS) - 1;
   constexpr uint32_t ES = sizeof(T), UNIT = StripUnit<BITS, GS>::value, STEP = GS * GROUP;
@@ -2048,7 +2049,7 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
               byte4 = s % WPT == 0 ? w : byte4 | w;
             }
           }
-          if (WHOLE && s % WPT == WPT - 1 && (WPT > 1 || GS == 1 || n0 + s < N)) store_bytes(n0 + s, sum);
+          if (WHOLE && s % WPT == WPT - 1) store_bytes(n0 + s, sum);
         }
         if (!WHOLE) {
           const uint32_t shift = before * BITS, field = 0x01010101u * ((0xffu << shift) & 0xffu);
