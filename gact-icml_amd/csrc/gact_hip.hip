@@ -1661,7 +1661,7 @@ quantize_wave8_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, 
 // ------------------------------------------------------------------------------------------------
 // Quantize a tensor that is not contiguous, without a contiguous copy of it: groups are consecutive elements in the order of
 // the tensor's indices, wherever they lie.  The copy these kernels replace is torch's element-wise one, 0.5-2 TB/s: half
-// channels-last [64,256,56,56], 4 bit, 223 us of copy and 20 of quantize -> 43; [64,512,28,28] 107 + 12 -> 23; half heads
+// channels-last [64,256,56,56], 4 bit, 223 us of copy and 20 of quantize -> 37; [64,512,28,28] 107 + 12 -> 23; half heads
 // [64,12,197,64] 14 + 7 -> 8; small tensors lose a launch ([2,12,197,64] 3.6 + 3.5 -> 4.6).
 // ------------------------------------------------------------------------------------------------
 // Innermost runs contiguous (GatherSource): quantize_kernel - at 1 and 2 bit quantize_wave8_kernel, whatever the size: a row
@@ -1690,8 +1690,11 @@ quantize_gather_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
 // them in 16-byte pieces and scatters each piece's elements, one channel each, to where they belong.  Rows of 16 lanes then
 // quantize super-groups out of LDS.  Neighbouring tiles read other channels of the same memory rows; they run on one XCD at about
 // the same time (xcd_tile), so a line that several of them share comes from HBM once and from that XCD's L2 afterwards.
-// Bound by its two phases standing one behind the other: half [64,256,56,56] at 4 bit 54 us, of which reading and scattering
-// alone take 33 and quantizing out of LDS alone 27 (with more, smaller workgroups 41 and 21, together 51).
+// Bound by its two phases standing one behind the other: half [64,256,56,56] at 4 bit (which takes strips) 54 us, of which reading
+// and scattering alone take 33 and quantizing out of LDS alone 27 (with more, smaller workgroups 41 and 21, together 51).  Half
+// [64,512,28,28] at 4 bit, 21 us on one buffer, 32 from HBM: 2.1 waves per SIMD on average, which wait for memory and barriers 0.39
+// and for their turn to issue 0.35 of their lives; the vector units issue 0.37 of the cycles, LDS conflicts take 0.09; it reads 1.24
+// times its bytes from HBM.
 struct TransposedShape {
   int64_t sb, sk;          // strides of batch and pixel, in elements
   uint32_t M, K;           // channels of a batch entry, pixels
@@ -1809,10 +1812,12 @@ quantize_transposed_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t nu
 // the next channel: past the end the walk goes on at the first pixels with every column belonging to the channel before it.  A
 // strip can be cut into segments of whole units, for more workgroups than there are strips; a segment reads up to a unit of
 // pixels beyond its own.
-// Bound by its instructions with few waves to overlap them: half [64,256,56,56] at 4 bit 37 us (256 CUs hold its 512 workgroups
-// at once; of the two on a CU the one dispatched second takes a fifth longer).  With GS = 1, 477 vector instructions per
-// 256 pixels and wave, it took 42; more waves through more segments cost more reading than they hide (44), and dropping
-// one of the two barriers by a ring of four slots changed nothing (41.8).
+// Bound by the chain of a step - loads, scatter, barrier, quantize, barrier - with few waves to overlap it: half [64,256,56,56] at
+// 4 bit 37 us with inputs in rotation, 32 on one buffer, 56 from HBM.  256 CUs hold its 512 workgroups at once (of the two on a CU
+// the one dispatched second takes a fifth longer): 1.4 waves per SIMD on average, waiting 0.46 of their lives (from HBM 0.63), with
+// 0.44 of the cycles issuing vector instructions and LDS conflicts 0.06; it reads 1.18 times its bytes from HBM.  With GS = 1 it
+// took 42; more waves through more segments cost more reading than they hide (44), and dropping one of the two barriers by a
+// ring of four slots changed nothing (41.8).
 #define STRIP_PIECES 4    /* 16-byte pieces of a memory row in a strip (8: half [2,64,128,128] 4 bit 7.6 -> 9.5 us, large tensors equal) */
 #define STRIP_CHUNK 256   /* pixels: a thread takes four of one piece */
 #define STRIP_THREADS (STRIP_PIECES * STRIP_CHUNK / 4)
@@ -3444,8 +3449,8 @@ inline int joined_dims(int ndim, const int64_t* sizes, const int64_t* strides, i
   return n;
 }
 // Strips or tiles.  A tile's workgroup reads a piece of its own of every memory row: the longer the channels (K pixels), the
-// narrower that piece; a strip's always reads 64 bytes, but it walks its pixels one step after the other, at least twice
-// the groups of a super-group, and reads up to a super-group of pixels beyond its own.  us, tiles / strips:
+// narrower that piece; a strip's always reads 64 bytes, but it walks its pixels one step after the other - of a channel at least
+// four super-groups, at 1 and 2 bit one and a half - and reads up to a super-group of pixels beyond its own.  us, tiles / strips:
 //   half [64,256,56,56] 8 bit 57 / 41  4 bit 55 / 37  2 bit 52 / 40  1 bit 54 / 48    float 4 bit 80 / 63  1 bit 155 / 78
 //   half [64,64,112,112] 8 bit 101 / 37  4 bit 99 / 35  1 bit 94 / 52    half [64,512,28,28] 8 bit 26 / 26  4 bit 23 / 31
 //   half [33,128,52,52] 8 bit 18 / 13  4 bit 18 / 14  2 bit 17 / 19    [40,96,64,64] 2 bit 16 / 19    [2,256,56,56] 2 bit 10 / 14
