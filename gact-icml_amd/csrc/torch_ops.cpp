@@ -9,11 +9,13 @@
 #include <torch/csrc/python_headers.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/core/CachingHostAllocator.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -319,9 +321,150 @@ PyObject* batch_table(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// What both batched calls take first: entries (bytes, one gact_batch_entry per tensor) and the same on the GPU, the tensors, their seeds and
+// the widths; false where anything is not as the launch needs it
+struct Batch {
+  int64_t count;
+  const at::Tensor *geometry, *bits;
+  c10::SmallVector<const void*, GACT_BATCH_ARGS> x;
+  c10::SmallVector<uint64_t, GACT_BATCH_ARGS> seeds;
+};
+bool batch_of(PyObject* const* args, Batch* b) {
+  if (!PyBytes_CheckExact(args[0]) || !(b->geometry = plain(args[1])) || !PyList_CheckExact(args[2]) || !PyList_CheckExact(args[3]) ||
+      !(b->bits = plain(args[4])) || !ordinary_call())
+    return false;
+  const Py_ssize_t count = PyList_GET_SIZE(args[2]), bytes = PyBytes_GET_SIZE(args[0]);
+  const c10::Device device = b->geometry->device();
+  if (count == 0 || count > GACT_BATCH_ARGS || PyList_GET_SIZE(args[3]) != count || bytes != count * (Py_ssize_t)sizeof(gact_batch_entry) ||
+      b->geometry->numel() != bytes || !b->geometry->is_contiguous() || b->bits->scalar_type() != at::kInt || b->bits->numel() != count ||
+      !b->bits->is_contiguous() || b->bits->device() != device)
+    return false;
+  b->count = count;
+  for (Py_ssize_t i = 0; i < count; i++) {
+    gact_batch_entry entry;   // a bytes object promises no alignment
+    std::memcpy(&entry, PyBytes_AS_STRING(args[0]) + i * sizeof entry, sizeof entry);
+    const at::Tensor* const t = plain(PyList_GET_ITEM(args[2], i));
+    int64_t seed;
+    if (!t || !integer(PyList_GET_ITEM(args[3], i), &seed) || t->device() != device || t->numel() != entry.numel ||
+        dtype_code(t->scalar_type()) != entry.dtype || !t->is_contiguous() || (reinterpret_cast<uintptr_t>(in(*t)) & 15u) != 0)
+      return false;
+    b->x.push_back(in(*t));
+    b->seeds.push_back((uint64_t)seed);
+  }
+  return true;
+}
+// The geometry outlives one call and may be used on a stream other than the one it was made on: its memory waits for that stream too
+void used_on(const at::Tensor& t, c10::hip::HIPStream stream) { c10::hip::HIPCachingAllocator::recordStream(t.storage().data_ptr(), stream); }
+bool capturing(c10::Device device) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing((hipStream_t)stream_on(device), &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+}
+void drop_event(PyObject* capsule) { (void)hipEventDestroy((hipEvent_t)PyCapsule_GetPointer(capsule, "hipEvent_t")); }
+
+// batch_quantize(entries, geometry, tensors, seeds, bits, (blocks, groups, workspace bytes, arena bytes, noise mode, element types)) ->
+// (codes, scale, min, table, widths kept, workspace, the plan's verdict in pinned memory, an event behind the plan for event_wait)
+PyObject* batch_quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Batch b;
+  int64_t blocks, groups, ws_bytes, arena, mode, dtypes;
+  if (n != 6 || !PyTuple_CheckExact(args[5]) || PyTuple_GET_SIZE(args[5]) != 6 || !integer(PyTuple_GET_ITEM(args[5], 0), &blocks) ||
+      !integer(PyTuple_GET_ITEM(args[5], 1), &groups) || !integer(PyTuple_GET_ITEM(args[5], 2), &ws_bytes) ||
+      !integer(PyTuple_GET_ITEM(args[5], 3), &arena) || !integer(PyTuple_GET_ITEM(args[5], 4), &mode) ||
+      !integer(PyTuple_GET_ITEM(args[5], 5), &dtypes) || blocks <= 0 || arena <= 0 || !batch_of(args, &b))
+    Py_RETURN_NONE;
+  const c10::Device device = b.geometry->device();
+  const c10::DeviceGuard guard(device);
+  if (capturing(device)) Py_RETURN_NONE;
+  const at::Tensor packed = make({arena}, at::kByte, device), scale = make({groups * 4}, at::kByte, device), mn = make({groups * 4}, at::kByte, device);
+  const at::Tensor table = make({b.geometry->numel()}, at::kByte, device), kept = make(b.bits->sizes(), at::kInt, device), ws = make({ws_bytes}, at::kByte, device);
+  const at::Tensor words = at::empty({2}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+  const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(device.index());
+  used_on(*b.geometry, stream);
+  hipEvent_t event;
+  if (hipEventCreateWithFlags(&event, hipEventDisableTiming) != hipSuccess) Py_RETURN_NONE;
+  PyObject* const capsule = PyCapsule_New(event, "hipEvent_t", drop_event);
+  if (!capsule) {
+    (void)hipEventDestroy(event);
+    return nullptr;
+  }
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = gact_batch_plan_args((const gact_batch_entry*)in(*b.geometry), b.x.data(), b.seeds.data(), (gact_batch_entry*)out(table),
+                            (const int32_t*)in(*b.bits), (int32_t*)out(kept), b.count, blocks, arena, out(ws), (int64_t*)out(words), stream.stream());
+  if (rc == GACT_OK && hipEventRecord(event, stream.stream()) != hipSuccess) rc = GACT_ELAUNCH;
+  if (rc == GACT_OK)
+    rc = gact_quantize_batched((const gact_batch_entry*)out(table), (const int32_t*)out(kept), b.count, blocks, (int)mode, (int)dtypes, out(ws),
+                               out(packed), out(scale), out(mn), stream.stream());
+  Py_END_ALLOW_THREADS
+  // the words' memory is not handed out again before the plan has written them, also where nobody waits for the event
+  (void)at::getHostAllocator(at::kCUDA)->record_event(words.mutable_data_ptr(), words.storage().data_ptr().get_context(),
+                                                        c10::Stream(c10::Stream::UNSAFE, device, stream.id()));
+  PyObject* const tensors = rc == GACT_OK ? tuple_of({packed, scale, mn, table, kept, ws, words}) : nullptr;
+  if (rc != GACT_OK || !tensors) {
+    Py_DECREF(capsule);
+    if (rc == GACT_OK) return nullptr;
+    Py_RETURN_NONE;
+  }
+  PyObject* const result = PyTuple_Pack(2, tensors, capsule);
+  Py_DECREF(tensors);
+  Py_DECREF(capsule);
+  return result;
+  END_HANDLE_TH_ERRORS
+}
+
+// event_wait(event of batch_quantize)
+PyObject* event_wait(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  void* const event = n == 1 ? PyCapsule_GetPointer(args[0], "hipEvent_t") : nullptr;
+  if (!event) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "event_wait takes one event");
+    return nullptr;
+  }
+  hipError_t rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = hipEventSynchronize((hipEvent_t)event);
+  Py_END_ALLOW_THREADS
+  if (rc != hipSuccess) {
+    PyErr_SetString(PyExc_RuntimeError, hipGetErrorString(rc));
+    return nullptr;
+  }
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
+// batch_dequantize(entries, geometry, outputs, seeds, widths, codes, scale, min, (blocks, workspace bytes)) -> (table, workspace)
+PyObject* batch_dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Batch b;
+  int64_t blocks, ws_bytes;
+  const at::Tensor *packed, *scale, *mn;
+  if (n != 9 || !(packed = plain(args[5])) || !(scale = plain(args[6])) || !(mn = plain(args[7])) || !PyTuple_CheckExact(args[8]) ||
+      PyTuple_GET_SIZE(args[8]) != 2 || !integer(PyTuple_GET_ITEM(args[8], 0), &blocks) || !integer(PyTuple_GET_ITEM(args[8], 1), &ws_bytes) ||
+      blocks <= 0 || !batch_of(args, &b))
+    Py_RETURN_NONE;
+  const c10::Device device = b.geometry->device();
+  for (const at::Tensor* t : {packed, scale, mn})
+    if (t->scalar_type() != at::kByte || !t->is_contiguous() || t->device() != device) Py_RETURN_NONE;
+  const c10::DeviceGuard guard(device);
+  if (capturing(device)) Py_RETURN_NONE;
+  used_on(*b.geometry, c10::hip::getCurrentHIPStream(device.index()));
+  const at::Tensor table = make({b.geometry->numel()}, at::kByte, device), ws = make({ws_bytes}, at::kByte, device);
+  const int rc = on(device, [&](void* stream) {
+    const int planned = gact_batch_plan_args((const gact_batch_entry*)in(*b.geometry), b.x.data(), b.seeds.data(), (gact_batch_entry*)out(table),
+                                             (const int32_t*)in(*b.bits), nullptr, b.count, blocks, packed->numel(), out(ws), nullptr, stream);
+    if (planned != GACT_OK) return planned;
+    return gact_dequantize_batched((const gact_batch_entry*)out(table), (const int32_t*)in(*b.bits), b.count, blocks, out(ws), in(*packed), in(*scale),
+                                   in(*mn), stream);
+  });
+  if (rc == GACT_OK) return tuple_of({table, ws});
+  Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
+}
+
 #define FASTCALL(f) {#f, (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {FASTCALL(quantize), FASTCALL(dequantize), FASTCALL(minimax),     FASTCALL(pack),        FASTCALL(unpack),
-                         FASTCALL(mask_pack), FASTCALL(mask_unpack), FASTCALL(batch_table), {nullptr, nullptr, 0, nullptr}};
+                         FASTCALL(mask_pack), FASTCALL(mask_unpack), FASTCALL(batch_table),
+                         FASTCALL(batch_quantize), FASTCALL(batch_dequantize), FASTCALL(event_wait), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "gact_torch", "The operators' host side.", -1, methods};
 
 }  // namespace

@@ -52,7 +52,7 @@ class BatchedPacked:
         if self._verdict is None:
             return self.ok()
         done, words = self._verdict
-        done.synchronize()
+        done.synchronize() if isinstance(done, torch.cuda.Event) else _abi.native().event_wait(done)
         need, good = words.tolist()
         return bool(good), need
 
@@ -84,6 +84,7 @@ class BatchedQuantizer:
     """Geometry of a fixed list of saved tensors (element counts and dtypes), reusable every iteration."""
 
     _entries = None     # the table's bytes but for what changes from call to call, a tensor's address and its seed
+    _geometry = None    # the same on the GPU, kept for the launches that bring the rest in their arguments
 
     def __init__(self, numels, dtypes, device):
         if len(numels) != len(dtypes):
@@ -109,6 +110,11 @@ class BatchedQuantizer:
         self.total_groups = groups
         self.workspace_bytes = int(_abi.lib().gact_batch_workspace_bytes(self.L, self.total_blocks))
 
+    def __getstate__(self):
+        state = dict(self.__dict__)
+        state.pop("_geometry", None)
+        return state
+
     # ---- arena sizing (host-side bounds; the exact need is computed on the device) ----
     def arena_bytes_for_budget(self, target_bits):
         """Upper bound of the packed bytes when the widths come from calc_precision with this bit
@@ -129,16 +135,26 @@ class BatchedQuantizer:
         """Whether the last plan written to this workspace succeeded; synchronises."""
         return bool(workspace[8:16].view(torch.int64).item())
 
+    def _entry_bytes(self):
+        if self._entries is None:
+            entries = (_abi.BatchEntry * self.L)()
+            for e, n, dt, first, stats in zip(entries, self.numels, self.dtypes, self.first_blocks, self.stats_offsets):
+                e.numel, e.dtype, e.first_block, e.stats_offset = n, _abi.dtype_code(dt), first, stats
+            self._entries = bytes(entries)
+        return self._entries
+
+    def _on_gpu(self):
+        """The entries on the GPU, for the native calls; None where those do not apply."""
+        if self._geometry is None and 0 < self.L <= _abi.BATCH_ARGS and not torch.cuda.is_current_stream_capturing():
+            # a copy that has arrived when this returns, whatever stream uses it
+            self._geometry = torch.frombuffer(bytearray(self._entry_bytes()), dtype=torch.uint8).to(self.device)
+        return self._geometry
+
     def _table(self, tensors, seeds, wait=True):
         """The table on the GPU.  wait = False where it is used on the current stream: it goes there from pinned memory
         behind the stream's other work."""
         if self.L and not torch.cuda.is_current_stream_capturing():
-            if self._entries is None:
-                entries = (_abi.BatchEntry * self.L)()
-                for e, n, dt, first, stats in zip(entries, self.numels, self.dtypes, self.first_blocks, self.stats_offsets):
-                    e.numel, e.dtype, e.first_block, e.stats_offset = n, _abi.dtype_code(dt), first, stats
-                self._entries = bytes(entries)
-            host = _abi.native().batch_table(self._entries, list(tensors), list(seeds))
+            host = _abi.native().batch_table(self._entry_bytes(), list(tensors), list(seeds))
             if host is not None:
                 return host.to(self.device, non_blocking=not wait)
         arr = (_abi.BatchEntry * self.L)()
@@ -196,6 +212,14 @@ class BatchedQuantizer:
         mode = _noise_mode(None, rng_stream)
         if arena_bytes is None:
             arena_bytes = self.arena_bytes_worst_case()
+        geometry = self._on_gpu()
+        if geometry is not None:
+            done = _abi.native().batch_quantize(self._entries, geometry, list(tensors), list(seeds), bits,
+                                                (self.total_blocks, self.total_groups, self.workspace_bytes, int(arena_bytes), mode, self.dtype_mask))
+            if done is not None:
+                (packed, scale, mn, table, kept, ws, words), event = done
+                return BatchedPacked(self, packed, scale, mn, table, kept, ws, [t.shape for t in tensors],
+                                     list(self.dtypes), seeds, (event, words))
         with torch.cuda.device(self.device):
             table = self._table(tensors, seeds, wait=False)
             packed = torch.empty((int(arena_bytes),), dtype=torch.uint8, device=self.device)
@@ -224,6 +248,13 @@ class BatchedQuantizer:
         with torch.cuda.device(self.device):
             if outs is None:
                 outs = [torch.empty(s, dtype=d, device=self.device) for s, d in zip(q.shapes, q.dtypes)]
+            geometry = self._on_gpu()
+            if geometry is not None:
+                done = _abi.native().batch_dequantize(self._entries, geometry, list(outs), list(q.seeds), q.bits, q.packed, q.scale, q.min,
+                                                      (self.total_blocks, self.workspace_bytes))
+                if done is not None:
+                    q._dq_table = done
+                    return outs
             table = self._table(outs, q.seeds, wait=False)
             ws = self.new_workspace()
             self.launch_dequantize(table, q.bits, q.packed, q.scale, q.min, ws)

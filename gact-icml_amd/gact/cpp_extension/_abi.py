@@ -23,6 +23,7 @@ NOISE_MODES = {"deterministic": NOISE_CONST, "inject": NOISE_INJECT, "reference"
 GROUP = 256
 ONE_PASS_GROUPS = (64, 128, 256, 512)     # group sizes with single-pass kernels (other than 256: float and half only)
 ABI_VERSION = 7
+BATCH_ARGS = 192        # tensors of a batch whose addresses and seeds fit a launch's arguments
 
 
 class BatchEntry(ctypes.Structure):
@@ -63,6 +64,7 @@ SIGNATURES = {
     "gact_calc_precision_device": (_i32, [_vp, _vp, _vp, _i64, _f64, _vp, _vp]),
     "gact_batch_workspace_bytes": (_i64, [_i64, _i64]),
     "gact_batch_plan": (_i32, [_vp, _vp, _i64, _i64, _i64, _vp, _vp]),
+    "gact_batch_plan_args": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp]),
     "gact_quantize_batched": (_i32, [_vp, _vp, _i64, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp]),
     "gact_dequantize_batched": (_i32, [_vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp]),
     "gact_quantize_batched_static": (_i32, [_vp, _vp, _i64, _i64, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp]),

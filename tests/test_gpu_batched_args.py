@@ -1,0 +1,80 @@
+"""A batch whose addresses and seeds travel in the plan's launch (up to 192 tensors) and one that is a tensor too long for it, against
+the tensors one by one: codes, scales, minima, widths kept and restored values bit for bit, and the plan's header."""
+import pickle
+import random
+
+import pytest
+import torch
+
+from gact import ops
+from gact.batched import BatchedQuantizer
+from gact.cpp_extension import _abi
+
+pytestmark = pytest.mark.gpu
+
+
+def make(count):
+    rng = random.Random(count)
+    g = torch.Generator(device="cuda").manual_seed(count)
+    sizes = [rng.choice([1, 255, 256, 257, 2048, 32768, 32769, rng.randint(1, 100000)]) for _ in range(count)]
+    dtypes = [rng.choice([torch.float32, torch.float16, torch.bfloat16]) for _ in range(count)]
+    xs = [torch.randn(n, generator=g, device="cuda").to(d) for n, d in zip(sizes, dtypes)]
+    widths = [rng.choice([1, 2, 4, 8]) for _ in range(count)]
+    return xs, widths, [rng.randint(-5, 1 << 20) for _ in range(count)], BatchedQuantizer(sizes, dtypes, "cuda")
+
+
+@pytest.mark.parametrize("count", [1, 63, 64, 65, 192, 193])     # a wave's share of the plan, its end, the longest, one more
+def test_batch_equals_its_tensors(count):
+    assert _abi.BATCH_ARGS == 192
+    xs, widths, seeds, batch = make(count)
+    bits = torch.tensor(widths, dtype=torch.int32, device="cuda")
+    native = _abi.native().batch_quantize(batch._entry_bytes(), batch._on_gpu(), xs, seeds, bits,
+                                          (batch.total_blocks, batch.total_groups, batch.workspace_bytes, batch.arena_bytes_worst_case(), _abi.NOISE_FAST,
+                                           batch.dtype_mask)) if count <= 192 else None
+    assert (native is not None) == (count <= 192)
+    q = batch.quantize(xs, bits, seeds)
+    bits.fill_(32)     # the widths are kept as they were
+    outs = batch.dequantize(q)
+    assert q.ok() == (True, q.ok()[1]) and q.workspace[16:48].view(torch.int64).tolist() == [widths.count(b) for b in (1, 2, 4, 8)]
+    for i, x in enumerate(xs):
+        want = ops.op_quantize(x, widths[i], seeds[i])
+        codes, b, scale, mn = q.per_tensor(i)
+        assert b == widths[i] and torch.equal(codes, want[0][: codes.numel()])
+        assert torch.equal(scale, want[2]) and torch.equal(mn, want[3])
+        assert torch.equal(outs[i], ops.op_dequantize(want, x.shape))
+    later = pickle.loads(pickle.dumps(q))
+    assert all(torch.equal(a, b) for a, b in zip(later.owner.dequantize(later), outs))
+
+
+def test_void_plans_and_dropped_batches():
+    xs, widths, seeds, batch = make(40)
+    bits = torch.tensor(widths, dtype=torch.int32, device="cuda")
+    for _ in range(30):       # nobody waits for these
+        batch.quantize(xs, bits, seeds)
+    small = batch.quantize(xs, bits, seeds, arena_bytes=512)
+    with pytest.raises(RuntimeError, match="void"):
+        batch.dequantize(small)
+    bad = bits.clone()
+    bad[-1] = 32
+    with pytest.raises(RuntimeError, match="void"):
+        batch.dequantize(batch.quantize(xs, bad, seeds))
+    with pytest.raises(RuntimeError, match="geometry"):
+        batch.quantize([x[:1] for x in xs], bits, seeds)
+    q = batch.quantize(xs, bits, seeds)
+    assert q.ok()[0] and all(torch.equal(a, ops.op_dequantize(ops.op_quantize(x, b, s), x.shape))
+                             for a, x, b, s in zip(batch.dequantize(q), xs, widths, seeds))
+
+
+def test_batches_on_streams_of_their_own():
+    xs, widths, seeds, batch = make(20)
+    bits = torch.tensor(widths, dtype=torch.int32, device="cuda")
+    want = batch.dequantize(batch.quantize(xs, bits, seeds))
+    torch.cuda.synchronize()
+    outs = []
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    for s in streams:
+        with torch.cuda.stream(s):
+            outs.append(batch.dequantize(batch.quantize(xs, bits, seeds)))
+    del batch
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for o in outs for a, b in zip(o, want))
