@@ -3393,7 +3393,7 @@ __device__ __forceinline__ void dequantize_batched_block(const gact_batch_entry&
   else
     dequantize_block128<bf16, BITS>(packed, (const float*)sc, (const bf16*)mn, ent.numel, N, lb, quarter, (bf16*)ent.x);
 }
-// grid: four workgroups per block of 128 groups
+// grid: four workgroups per block of 128 groups; workgroups on a CU: BATCHED_CAP_LDS
 __global__ void __launch_bounds__(256)
 dequantize_batched_kernel(const gact_batch_entry* __restrict__ table, const int32_t* __restrict__ bits,
                           BatchWorkspace ws, const uint8_t* __restrict__ packed_arena,
@@ -4291,6 +4291,15 @@ int64_t gact_batch_workspace_bytes(int64_t L, int64_t total_blocks) {
 }
 
 namespace {
+// Three workgroups on a CU, by a request for dynamic LDS that nobody touches (see quantize_lds_cap), for two of the batched kernels:
+//   quantize, half: its registers admit four.  120 half tensors, four / three / two workgroups, us: 1.83 G elements, 1, 2 and 4 bit mixed
+//     696 / 676 / 665, all at 1 bit 634 / 606 / 638, 2 bit 674 / 655 / 661, 4 bit 769 / 758 / 718, 8 bit 870 / 843 / 893;
+//     0.23 G mixed 88.5 / 84.7 / 88.5, 57 M 25.1 / 25.2 / 27.5.  Three never loses whatever the widths, which the host does not know.
+//     Float and bfloat16 hold two by their registers.
+//   dequantize, float: eight / four / three workgroups, 0.69 G elements mixed 539 / 492 / 475, 1 bit 517 / 484 / 444, 8 bit 586 / 551 / 585;
+//     0.23 G mixed 180 / 166 / 162, 57 M 46.9 / 43.4 / 44.3.  Half and bfloat16 lose by any cap (mixed 673 / 856 / 1010), so it goes
+//     with batches that are known to hold float tensors only.
+#define BATCHED_CAP_LDS 53000u
 int batch_plan_on(gact_batch_entry* table, const int32_t* bits, int64_t L, int64_t total_blocks, int64_t capacity,
                   void* workspace, int64_t* verdict, hipStream_t s) {
   const BatchWorkspace ws = batch_workspace(workspace);
@@ -4305,7 +4314,7 @@ int quantize_batched_on(const gact_batch_entry* table, const int32_t* bits, int6
   const BatchWorkspace ws = batch_workspace(workspace);
   const dim3 grid((unsigned)total_blocks), block(256);
 #define GACT_LAUNCH_QB(T, M)                                                                                  \
-  hipLaunchKernelGGL((quantize_batched_kernel<T, M>), grid, block, 0, s, table, bits, ws, (uint8_t*)packed_arena, \
+  hipLaunchKernelGGL((quantize_batched_kernel<T, M>), grid, block, (Elem<T>::kDtype == GACT_F16 ? BATCHED_CAP_LDS : 0u), s, table, bits, ws, (uint8_t*)packed_arena, \
                      (uint8_t*)scale_arena, (uint8_t*)min_arena)
 #define GACT_LAUNCH_QB_ALL(M)                                                                                 \
   do {                                                                                                        \
@@ -4375,13 +4384,18 @@ int gact_quantize_batched(const gact_batch_entry* table, const int32_t* bits, in
 int gact_dequantize_batched(const gact_batch_entry* table, const int32_t* bits, int64_t L, int64_t total_blocks,
                             const void* workspace, const void* packed_arena, const void* scale_arena,
                             const void* min_arena, void* stream) {
-  if (!batched_args_ok(L, total_blocks)) return GACT_EINVAL;
+  return gact_dequantize_batched_types(table, bits, L, total_blocks, GACT_DTYPES_ALL, workspace, packed_arena, scale_arena, min_arena, stream);
+}
+int gact_dequantize_batched_types(const gact_batch_entry* table, const int32_t* bits, int64_t L, int64_t total_blocks, int dtypes,
+                                  const void* workspace, const void* packed_arena, const void* scale_arena, const void* min_arena,
+                                  void* stream) {
+  if (!batched_args_ok(L, total_blocks) || dtypes < 0 || dtypes > GACT_DTYPES_ALL) return GACT_EINVAL;
   if (L == 0 || total_blocks == 0) return GACT_OK;
   if (!table || !bits || !workspace || !packed_arena || !scale_arena || !min_arena) return GACT_EINVAL;
   if (!aligned16(packed_arena) || !aligned16(workspace)) return GACT_EALIGN;
   fresh_launch();
   const dim3 grid((unsigned)(4 * total_blocks)), block(256);
-  hipLaunchKernelGGL(dequantize_batched_kernel, grid, block, 0, (hipStream_t)stream, table, bits,
+  hipLaunchKernelGGL(dequantize_batched_kernel, grid, block, (dtypes == GACT_DTYPES_F32 ? BATCHED_CAP_LDS : 0u), (hipStream_t)stream, table, bits,
                      batch_workspace(const_cast<void*>(workspace)), (const uint8_t*)packed_arena,
                      (const uint8_t*)scale_arena, (const uint8_t*)min_arena);
   return launch_status();

@@ -432,15 +432,15 @@ PyObject* event_wait(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// batch_dequantize(entries, geometry, outputs, seeds, widths, codes, scale, min, (blocks, workspace bytes)) -> (table, workspace)
+// batch_dequantize(entries, geometry, outputs, seeds, widths, codes, scale, min, (blocks, workspace bytes, element types)) -> (table, workspace)
 PyObject* batch_dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Batch b;
-  int64_t blocks, ws_bytes;
+  int64_t blocks, ws_bytes, dtypes;
   const at::Tensor *packed, *scale, *mn;
   if (n != 9 || !(packed = plain(args[5])) || !(scale = plain(args[6])) || !(mn = plain(args[7])) || !PyTuple_CheckExact(args[8]) ||
-      PyTuple_GET_SIZE(args[8]) != 2 || !integer(PyTuple_GET_ITEM(args[8], 0), &blocks) || !integer(PyTuple_GET_ITEM(args[8], 1), &ws_bytes) ||
-      blocks <= 0 || !batch_of(args, &b))
+      PyTuple_GET_SIZE(args[8]) != 3 || !integer(PyTuple_GET_ITEM(args[8], 0), &blocks) || !integer(PyTuple_GET_ITEM(args[8], 1), &ws_bytes) ||
+      !integer(PyTuple_GET_ITEM(args[8], 2), &dtypes) || blocks <= 0 || !batch_of(args, &b))
     Py_RETURN_NONE;
   const c10::Device device = b.geometry->device();
   for (const at::Tensor* t : {packed, scale, mn})
@@ -453,8 +453,8 @@ PyObject* batch_dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int planned = gact_batch_plan_args((const gact_batch_entry*)in(*b.geometry), b.x.data(), b.seeds.data(), (gact_batch_entry*)out(table),
                                              (const int32_t*)in(*b.bits), nullptr, b.count, blocks, packed->numel(), out(ws), nullptr, stream);
     if (planned != GACT_OK) return planned;
-    return gact_dequantize_batched((const gact_batch_entry*)out(table), (const int32_t*)in(*b.bits), b.count, blocks, out(ws), in(*packed), in(*scale),
-                                   in(*mn), stream);
+    return gact_dequantize_batched_types((const gact_batch_entry*)out(table), (const int32_t*)in(*b.bits), b.count, blocks, (int)dtypes, out(ws),
+                                         in(*packed), in(*scale), in(*mn), stream);
   });
   if (rc == GACT_OK) return tuple_of({table, ws});
   Py_RETURN_NONE;

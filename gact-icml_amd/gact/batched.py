@@ -198,9 +198,9 @@ class BatchedQuantizer:
         """Plan into `workspace` (the table's x point at the outputs; planning again from the same widths gives
         the same offsets without reading anything back), then dequantize every tensor."""
         self._launch_plan(table, bits, packed, workspace)
-        _abi.check(_abi.lib().gact_dequantize_batched(table.data_ptr(), bits.data_ptr(), self.L, self.total_blocks,
-                                                      workspace.data_ptr(), packed.data_ptr(), scale.data_ptr(),
-                                                      mn.data_ptr(), torch.cuda.current_stream(self.device).cuda_stream))
+        _abi.check(_abi.lib().gact_dequantize_batched_types(table.data_ptr(), bits.data_ptr(), self.L, self.total_blocks, self.dtype_mask,
+                                                            workspace.data_ptr(), packed.data_ptr(), scale.data_ptr(),
+                                                            mn.data_ptr(), torch.cuda.current_stream(self.device).cuda_stream))
 
     def quantize(self, tensors, bits, seeds, arena_bytes=None, rng_stream=None):
         """Quantize all tensors in one batched launch.  `bits` is an int32 tensor on the device (e.g. the output
@@ -251,7 +251,7 @@ class BatchedQuantizer:
             geometry = self._on_gpu()
             if geometry is not None:
                 done = _abi.native().batch_dequantize(self._entries, geometry, list(outs), list(q.seeds), q.bits, q.packed, q.scale, q.min,
-                                                      (self.total_blocks, self.workspace_bytes))
+                                                      (self.total_blocks, self.workspace_bytes, self.dtype_mask))
                 if done is not None:
                     q._dq_table = done
                     return outs

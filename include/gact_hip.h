@@ -191,6 +191,12 @@ int gact_dequantize_batched(const gact_batch_entry* table, const int32_t* bits, 
                             int64_t total_blocks, const void* workspace, const void* packed_arena,
                             const void* scale_arena, const void* min_arena, void* stream);
 
+/* gact_dequantize_batched where the host knows which element types the table holds (the same mask; 0 or GACT_DTYPES_ALL: any): the
+ * launch is shaped for them, the results are the same. */
+int gact_dequantize_batched_types(const gact_batch_entry* table, const int32_t* bits, int64_t L, int64_t total_blocks, int dtypes,
+                                  const void* workspace, const void* packed_arena, const void* scale_arena, const void* min_arena,
+                                  void* stream);
+
 /* gact_batch_plan followed by gact_quantize_batched, with the workspace in a device array that is part of
  * the library (1 MB per GPU the library runs on, held until the process ends) instead of memory the
  * caller brings: nothing is allocated, by the library or on its behalf.  No counterpart in the reference; it

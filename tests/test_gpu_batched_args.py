@@ -46,6 +46,19 @@ def test_batch_equals_its_tensors(count):
     assert all(torch.equal(a, b) for a, b in zip(later.owner.dequantize(later), outs))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["f32", "f16", "bf16"])
+def test_batches_of_one_type_whatever_is_said_of_it(dtype):
+    """The launch of a batch of one type is shaped for it; told of any type it gives the same bytes."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    sizes = [70000, 513, 256 * 128 * 9, 3]
+    xs = [torch.randn(n, generator=g, device="cuda").to(dtype) for n in sizes]
+    batch = BatchedQuantizer(sizes, [dtype] * 4, "cuda")
+    q = batch.quantize(xs, torch.tensor([1, 2, 4, 8], dtype=torch.int32, device="cuda"), [1, 2, 3, 4])
+    outs = batch.dequantize(q)
+    batch.dtype_mask = 7
+    assert all(torch.equal(a, b) for a, b in zip(outs, batch.dequantize(q)))
+
+
 def test_void_plans_and_dropped_batches():
     xs, widths, seeds, batch = make(40)
     bits = torch.tensor(widths, dtype=torch.int32, device="cuda")
