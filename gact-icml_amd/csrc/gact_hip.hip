@@ -2962,6 +2962,7 @@ __host__ __device__ inline bool prec_valid_bits(int b) { return b == 1 || b == 2
 #define PREC_MAX_L 4096      /* tensors the device kernel handles (LDS tables) */
 #define PREC_SORT_MAX_L 4096 /* tensors the sorting path handles (4 candidate steps each, 8 bytes per candidate) */
 #define PREC_THREADS 1024    /* largest workgroup the kernel is launched with */
+#define PREC_LDS_L 1024      /* tensors whose sizes the kernel keeps in LDS */
 
 // The sequential restatement of the heap loop by one wave: each step is a 64-lane argmax.  Used when a
 // tensor's step keys do not decrease (never the case for the finite positive sensitivities the callers
@@ -3012,9 +3013,23 @@ __device__ __forceinline__ uint32_t sortable_key(float k) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
+// The value of lane ^ J: within a row by DPP moves (a few cycles), across rows through the LDS crossbar
+template <int J>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+  if constexpr (J == 1) return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xB1, 0xf, 0xf, false);         // quad_perm [1,0,3,2]
+  else if constexpr (J == 2) return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x4E, 0xf, 0xf, false);    // quad_perm [2,3,0,1]
+  else if constexpr (J == 8) return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x128, 0xf, 0xf, false);   // row_ror:8
+  else if constexpr (J == 4) {   // four lanes up for the even quads (row_ror:12), four down for the odd ones (row_ror:4)
+    const int up = __builtin_amdgcn_update_dpp((int)v, (int)v, 0x12C, 0xf, 0xf, false);
+    return (uint32_t)__builtin_amdgcn_update_dpp(up, (int)v, 0x124, 0xf, 0xa, false);
+  } else {
+    return (uint32_t)__shfl_xor((int)v, J, 64);
+  }
+}
+
 // Bitonic sort of M = R * NT candidate slots, descending, by a workgroup of NT threads (M and NT powers of two,
 // NT >= 64).  Thread t keeps slots t, NT + t, ... in registers: partners NT or more apart are its own registers,
-// partners less than a wave apart are reached with a shuffle, and only the passes in between go through LDS and
+// partners less than a wave apart are reached by lane_xor, and only the passes in between go through LDS and
 // a barrier (512 slots by 512 threads: 6 of 45 passes).
 template <int R, int JR>
 __device__ __forceinline__ void prec_exchange_own(uint64_t (&v)[R], int tid, int NT, int k) {
@@ -3029,13 +3044,32 @@ __device__ __forceinline__ void prec_exchange_own(uint64_t (&v)[R], int tid, int
     }
   }
 }
+// the lower slot of a pair keeps the larger key where the run descends, the smaller where it ascends
+template <int R>
+__device__ __forceinline__ void prec_keep(uint64_t (&v)[R], const uint64_t (&o)[R], int tid, int NT, int j, int k) {
+  const bool lower = (tid & j) == 0;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const bool descending = ((r * NT + tid) & k) == 0;
+    const uint64_t larger = v[r] > o[r] ? v[r] : o[r], smaller = v[r] > o[r] ? o[r] : v[r];
+    v[r] = (descending == lower) ? larger : smaller;
+  }
+}
+template <int R, int J>
+__device__ __forceinline__ void prec_exchange_lanes(uint64_t (&v)[R], int tid, int NT, int k) {
+  if (J >= k) return;   // not a pass of this run length
+  uint64_t o[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) o[r] = ((uint64_t)lane_xor<J>((uint32_t)(v[r] >> 32)) << 32) | lane_xor<J>((uint32_t)v[r]);
+  prec_keep<R>(v, o, tid, NT, J, k);
+}
 template <int R>
 __device__ __forceinline__ void prec_sort_slots(uint64_t* cand, int tid, int NT, int M) {
   uint64_t v[R];
 #pragma unroll
-  for (int r = 0; r < R; r++) v[r] = cand[r * NT + tid];
+  for (int r = 0; r < R; r++) v[r] = r * NT + tid < M ? cand[r * NT + tid] : 0;   // fewer slots than a wave has lanes: the others idle
   for (int k = 2; k <= M; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
+    for (int j = k >> 1; j >= 64; j >>= 1) {
       if (j >= NT) {
         switch (j / NT) {
           case 1: prec_exchange_own<R, 1>(v, tid, NT, k); break;
@@ -3046,34 +3080,36 @@ __device__ __forceinline__ void prec_sort_slots(uint64_t* cand, int tid, int NT,
         continue;
       }
       uint64_t o[R];
-      if (j >= 64) {
 #pragma unroll
-        for (int r = 0; r < R; r++) cand[r * NT + tid] = v[r];
-        __syncthreads();
+      for (int r = 0; r < R; r++) cand[r * NT + tid] = v[r];
+      __syncthreads();
 #pragma unroll
-        for (int r = 0; r < R; r++) o[r] = cand[(r * NT + tid) ^ j];
-        __syncthreads();
-      } else {
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          const uint32_t lo32 = (uint32_t)__shfl_xor((int)(uint32_t)v[r], j, 64);
-          const uint32_t hi32 = (uint32_t)__shfl_xor((int)(uint32_t)(v[r] >> 32), j, 64);
-          o[r] = ((uint64_t)hi32 << 32) | lo32;
-        }
-      }
-      // the lower slot of a pair keeps the larger key where the run descends, the smaller where it ascends
-      const bool lower = (tid & j) == 0;
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        const bool descending = ((r * NT + tid) & k) == 0;
-        const uint64_t larger = v[r] > o[r] ? v[r] : o[r], smaller = v[r] > o[r] ? o[r] : v[r];
-        v[r] = (descending == lower) ? larger : smaller;
-      }
+      for (int r = 0; r < R; r++) o[r] = cand[(r * NT + tid) ^ j];
+      __syncthreads();
+      prec_keep<R>(v, o, tid, NT, j, k);
     }
+    prec_exchange_lanes<R, 32>(v, tid, NT, k);
+    prec_exchange_lanes<R, 16>(v, tid, NT, k);
+    prec_exchange_lanes<R, 8>(v, tid, NT, k);
+    prec_exchange_lanes<R, 4>(v, tid, NT, k);
+    prec_exchange_lanes<R, 2>(v, tid, NT, k);
+    prec_exchange_lanes<R, 1>(v, tid, NT, k);
   }
 #pragma unroll
-  for (int r = 0; r < R; r++) cand[r * NT + tid] = v[r];
+  for (int r = 0; r < R; r++)
+    if (r * NT + tid < M) cand[r * NT + tid] = v[r];
   __syncthreads();
+}
+// A candidate's low word: index, earlier steps above later ones, and the width the step ends at (its logarithm), which
+// orders nothing: index and step are unique.
+__device__ __forceinline__ uint32_t prec_candidate(int idx, int step, int to) {
+  return ((uint32_t)idx << 4) | ((uint32_t)(3 - step) << 2) | (to == 8 ? 3u : to == 4 ? 2u : to == 2 ? 1u : 0u);
+}
+__device__ __forceinline__ int prec_index(uint64_t c) { return (int)((uint32_t)c >> 4); }
+__device__ __forceinline__ int prec_to(uint64_t c) { return 1 << ((uint32_t)c & 3u); }
+__device__ __forceinline__ int64_t prec_saving(uint64_t c, int64_t w) {
+  const int to = prec_to(c);
+  return w * (int64_t)(to == 8 ? 24 : to);   // 32 -> 8, or halved
 }
 
 // The greedy pops candidates (tensor i, step s) in descending (key, i) order.  A tensor's steps have
@@ -3082,6 +3118,9 @@ __device__ __forceinline__ void prec_sort_slots(uint64_t* cand, int tid, int NT,
 // One workgroup, one thread per candidate slot up to 1024: build up to 4 candidates per tensor, bitonic-sort them,
 // prefix-sum the savings (integers, exact in double), apply the prefix.  Falls back to the sequential
 // loop when that order argument does not hold.
+// Bound by its chain of latencies, one workgroup that waits for loads, lane exchanges and barriers: a thread asks for a tensor's three
+// values at once, the sizes (up to PREC_LDS_L tensors) stay in LDS for the savings, which need nothing else - a candidate says what
+// width its step ends at - and the exchanges within a row are DPP moves.
 __global__ void __launch_bounds__(PREC_THREADS)
 calc_precision_kernel(int32_t* __restrict__ b, const float* __restrict__ C, const int64_t* __restrict__ w,
                       int L, double target, int32_t* __restrict__ status) {
@@ -3089,12 +3128,13 @@ calc_precision_kernel(int32_t* __restrict__ b, const float* __restrict__ C, cons
   // tensors); the sequential path reuses it for its float keys
   extern __shared__ uint64_t cand[];
   __shared__ int32_t b_s[PREC_MAX_L];
-  __shared__ double part_s[PREC_THREADS];
+  __shared__ double part_s[PREC_THREADS / 64];
   __shared__ int flag_s;
   const int tid = threadIdx.x, NT = blockDim.x;
   const bool sortable = L <= PREC_SORT_MAX_L;
   int M = 4;
   while (M < 4 * L) M <<= 1;
+  int64_t* const w_s = L <= PREC_LDS_L ? reinterpret_cast<int64_t*>(cand + M) : nullptr;   // behind the candidates
   if (tid == 0) flag_s = 0;
   if (sortable)
     for (int t = tid; t < M; t += NT) cand[t] = 0;  // 0 sorts after every real candidate
@@ -3104,29 +3144,34 @@ calc_precision_kernel(int32_t* __restrict__ b, const float* __restrict__ C, cons
   bool bad_order = false, bad_width = false;
   for (int idx = tid; idx < L; idx += NT) {
     const int bi = b[idx];
+    const int64_t wi = w[idx];
+    const float Ci = C[idx];
     b_s[idx] = bi;
+    if (w_s) w_s[idx] = wi;
     if (!prec_valid_bits(bi)) {
       bad_width = true;
     } else if (bi > 1) {
-      const int64_t wi = w[idx];
       part += (double)((int64_t)bi * wi);
       if (sortable) {
-        const float Ci = C[idx];
         float prev = __builtin_inff();
         int cur = bi, st = 0;
         while (cur > 1 && st < 4) {
+          const int to = prec_next_bits(cur);
           const float k = prec_key(Ci, cur, wi);
           if (!(k < prev) && !(k == prev && k == 0.0f)) bad_order = true;  // also catches NaN
-          cand[idx * 4 + st] = ((uint64_t)sortable_key(k) << 32) | ((uint32_t)idx << 2) | (uint32_t)(3 - st);
+          cand[idx * 4 + st] = ((uint64_t)sortable_key(k) << 32) | prec_candidate(idx, st, to);
           prev = k;
-          cur = prec_next_bits(cur);
+          cur = to;
           st++;
         }
         if (cur > 1) bad_order = true;  // a width the 4-step descent does not know
       }
     }
   }
-  part_s[tid] = part;
+  // every term is an integer; the sum is exact (and order-free) below 2^53
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
+  if ((tid & 63) == 0) part_s[tid >> 6] = part;   // at most 16 waves
   if (bad_order) flag_s = 1;
   __syncthreads();
   if (bad_width) flag_s = 3;
@@ -3135,12 +3180,8 @@ calc_precision_kernel(int32_t* __restrict__ b, const float* __restrict__ C, cons
     if (status && tid == 0) *status = GACT_EINVAL;
     return;
   }
-  // every term is an integer; the sum is exact (and order-free) below 2^53
-  for (int off = NT >> 1; off >= 1; off >>= 1) {
-    if (tid < off) part_s[tid] += part_s[tid + off];
-    __syncthreads();
-  }
-  const double b_sum0 = part_s[0];
+  double b_sum0 = 0.0;
+  for (int wv = 0; wv < (NT + 63) >> 6; wv++) b_sum0 += part_s[wv];
   const bool sequential = !sortable || flag_s != 0;
   __syncthreads();
 
@@ -3150,6 +3191,7 @@ calc_precision_kernel(int32_t* __restrict__ b, const float* __restrict__ C, cons
   } else {
     // bitonic sort, descending
     switch (M / NT) {
+      case 0:
       case 1: prec_sort_slots<1>(cand, tid, NT, M); break;
       case 2: prec_sort_slots<2>(cand, tid, NT, M); break;
       case 4: prec_sort_slots<4>(cand, tid, NT, M); break;
@@ -3163,10 +3205,7 @@ calc_precision_kernel(int32_t* __restrict__ b, const float* __restrict__ C, cons
     for (int t = lo; t < hi && t < M; t++) {
       const uint64_t c = cand[t];
       if (c == 0) break;
-      const int idx = (int)((uint32_t)c >> 2), st = 3 - (int)(c & 3u);
-      int cur = b[idx];
-      for (int q = 0; q < st; q++) cur = prec_next_bits(cur);
-      mine += (double)(w[idx] * (int64_t)(cur - prec_next_bits(cur)));
+      mine += (double)prec_saving(c, w_s ? w_s[prec_index(c)] : w[prec_index(c)]);
     }
     // exclusive prefix of the threads' savings: a scan inside every wave, then the waves' totals (the terms are
     // integers below 2^53, so the sums are exact in any order)
@@ -3186,17 +3225,13 @@ calc_precision_kernel(int32_t* __restrict__ b, const float* __restrict__ C, cons
       total += v;
     }
     if (tid == 0 && b_sum0 - total > target) flag_s = 2;  // every step taken and still over budget
-    __syncthreads();
     double running = b_sum0 - (before + incl - mine);
     for (int t = lo; t < hi && t < M; t++) {
       const uint64_t c = cand[t];
       if (c == 0 || !(running > target)) break;
-      const int idx = (int)((uint32_t)c >> 2), st = 3 - (int)(c & 3u);
-      int cur = b[idx];
-      for (int q = 0; q < st; q++) cur = prec_next_bits(cur);
-      const int nb = prec_next_bits(cur);
-      atomicMin(&b_s[idx], nb);
-      running -= (double)(w[idx] * (int64_t)(cur - nb));
+      const int idx = prec_index(c);
+      atomicMin(&b_s[idx], prec_to(c));
+      running -= (double)prec_saving(c, w_s ? w_s[idx] : w[idx]);
     }
     __syncthreads();
     if (flag_s == 2) rc = GACT_EBUDGET;
@@ -4272,7 +4307,7 @@ int gact_calc_precision_device(int32_t* b, const float* C, const int64_t* w, int
   fresh_launch();
   int64_t M = 4;
   while (M < 4 * L) M <<= 1;
-  const size_t lds = (size_t)M * sizeof(uint64_t);
+  const size_t lds = (size_t)(M + (L <= PREC_LDS_L ? L : 0)) * sizeof(uint64_t);
   if (lds > 48 * 1024 &&
       hipFuncSetAttribute((const void*)calc_precision_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
           hipSuccess)
