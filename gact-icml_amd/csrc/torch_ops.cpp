@@ -8,9 +8,12 @@
 // Arguments come through the C API's fast call and tensors through torch's own wrap / unpack (no pybind11).
 #include <torch/csrc/python_headers.h>
 
+#include <ATen/Context.h>
+#include <ATen/EmptyTensor.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/CachingHostAllocator.h>
 #include <ATen/core/Tensor.h>
+#include <ATen/detail/CUDAHooksInterface.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -88,8 +91,13 @@ int64_t packed_numel(int bits, int64_t N, int64_t row) {
   return (bits * ((N + wpt - 1) / wpt * wpt) * row + 8) / 8;
 }
 
+// torch.empty on the GPU without the dispatcher's way there, half of what an allocation costs: every caller has looked whether anything
+// listens to that (ordinary_call).  torch's deterministic mode fills new memory, so it goes through torch.
 at::Tensor make(c10::IntArrayRef shape, at::ScalarType dtype, c10::Device device) {
-  return at::empty(shape, at::TensorOptions().dtype(dtype).device(device));
+  if (at::globalContext().deterministicAlgorithms() && at::globalContext().deterministicFillUninitializedMemory())
+    return at::empty(shape, at::TensorOptions().dtype(dtype).device(device));
+  const c10::DeviceGuard guard(device);
+  return at::detail::empty_generic(shape, at::detail::getCUDAHooks().getCUDADeviceAllocator(), c10::DispatchKeySet(c10::DispatchKey::CUDA), dtype, std::nullopt);
 }
 void* stream_on(c10::Device device) { return c10::hip::getCurrentHIPStream(device.index()).stream(); }
 const void* in(const at::Tensor& t) { return t.const_data_ptr(); }

@@ -186,3 +186,28 @@ def test_batched_tables_and_verdicts(monkeypatch):
         batch.quantize(xs[::-1], bits, [4, 5, 6])
     assert "_verdict" not in void.__getstate__()
     assert pickle.loads(pickle.dumps(batch))._table(xs, [1, 2, 3]).numel() == 3 * 56
+
+
+@pytest.mark.gpu
+def test_results_are_allocated_as_torch_allocates_them():
+    """Device, storage and inference marks of the native calls' results, and the byte nobody writes under deterministic mode, which
+    fills new memory."""
+    x = torch.randn(16, 512, device="cuda")
+    q = ops.op_quantize(x, 4, 0)
+    out = ops.op_dequantize(q, x.shape)
+    for t in (q[0], q[2], q[3], out):
+        like = torch.empty(t.shape, dtype=t.dtype, device="cuda")
+        assert t.device == like.device and t.is_cuda and t.stride() == like.stride() and not t.requires_grad
+        assert t.untyped_storage().nbytes() == like.untyped_storage().nbytes() and t.untyped_storage().resizable()
+    assert not q[0].is_inference()
+    with torch.inference_mode():
+        assert ops.op_quantize(x, 4, 0)[0].is_inference()
+    before = torch.cuda.memory_allocated()
+    kept = ops.op_quantize(x, 8, 0)[0]
+    assert torch.cuda.memory_allocated() > before
+    del kept
+    torch.use_deterministic_algorithms(True)
+    try:
+        assert ops.op_quantize(x, 4, 0)[0][-1].item() == torch.empty(1, dtype=torch.int8, device="cuda").item()
+    finally:
+        torch.use_deterministic_algorithms(False)
