@@ -434,3 +434,19 @@ def test_fused_quantize_also_writes_the_maxima_when_asked(dtype, bits):
         ref = oracle.op_quantize(x.numpy(), bits, oracle.NOISE_FAST, 5)
         np.testing.assert_array_equal(packed.cpu().numpy().view(np.uint8)[:ref[0].size], ref[0])
         np.testing.assert_array_equal(sc.cpu().numpy(), ref[2].reshape(-1))
+
+
+@pytest.mark.parametrize("full", [0, 1, 2, 7, 8, 9])
+def test_mask_ends_at_every_element_of_a_block(full):
+    # the partial block: bytes written are the elements', none behind them, and its words are the plain sequence of bits
+    for tail in list(range(0, 70)) + [95, 96, 97, 127, 128, 129, 255, 256, 257, 383, 479, 480, 481, 508, 509, 510, 511]:
+        n = 512 * full + tail
+        if n == 0:
+            continue
+        x = torch.randint(0, 3, (n,), generator=torch.Generator().manual_seed(n), dtype=torch.uint8)     # 2 counts as 1
+        want = oracle.mask_pack((x.numpy() != 0).astype(np.uint8))
+        mask = ext_quantization.act_quantize_dropout_mask(x.cuda())
+        np.testing.assert_array_equal(mask.cpu().numpy().view(np.uint32), want.view(np.uint32), err_msg=str(n))
+        buffer = torch.full((n + 16,), 7, dtype=torch.uint8, device="cuda")
+        assert _abi.lib().gact_mask_unpack(mask.data_ptr(), n, buffer.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(buffer[:n].cpu(), (x != 0).to(torch.uint8)) and buffer[n:].eq(7).all(), n
