@@ -3380,8 +3380,8 @@ batch_plan_kernel(gact_batch_entry* table, const int32_t* __restrict__ bits, int
 // The plan of a table that the launch itself brings: what changes from call to call - a tensor's address and its seed - arrives in the
 // kernel's arguments, everything else of the entries is read from `geometry` on the GPU.  The table, a copy of the widths and the
 // verdict (which may lie in pinned host memory) are written by the same launch, where three copies stood around it, four launches and the
-// Python between them.  69 half tensors of 3.9 M elements together: host time of a quantize call 68 -> 26 us, of a dequantize call 34 -> 14,
-// allocation, quantize and dequantize together 116 -> 62; 142 float tensors, 36 M elements, 165 -> 144.
+// Python between them.  69 half tensors, 16 M elements together: host time of a quantize call 68 -> 26 us; with the dequantize call's plan
+// brought the same way calc_precision, quantize and dequantize together 116 -> 62; 142 float tensors, 67 M elements, 165 -> 144.
 struct BatchArgs {
   const void* x[GACT_BATCH_ARGS];
   uint64_t seed[GACT_BATCH_ARGS];
@@ -3448,17 +3448,18 @@ __device__ __forceinline__ void dequantize_batched_block(const gact_batch_entry&
     dequantize_block128<bf16, BITS>(packed, (const float*)sc, (const bf16*)mn, ent.numel, N, lb, quarter, (bf16*)ent.x);
 }
 // grid: four workgroups per block of 128 groups; workgroups on a CU: BATCHED_CAP_LDS
-__global__ void __launch_bounds__(256)
-dequantize_batched_kernel(const gact_batch_entry* __restrict__ table, const int32_t* __restrict__ bits,
-                          BatchWorkspace ws, const uint8_t* __restrict__ packed_arena,
-                          const uint8_t* __restrict__ scale_arena, const uint8_t* __restrict__ min_arena) {
+__device__ __forceinline__ void dequantize_batched(const gact_batch_entry* __restrict__ table, const void* const* outs,
+                                                   const int32_t* __restrict__ bits, const BatchWorkspace& ws,
+                                                   const uint8_t* __restrict__ packed_arena, const uint8_t* __restrict__ scale_arena,
+                                                   const uint8_t* __restrict__ min_arena) {
   if (ws.hdr->ok == 0) return;
   // the XCD-aware order of the single-tensor kernel (715 -> 709 us on 120 half tensors)
   const uint32_t tile = xcd_tile<GACT_XCD_RUN_DQB>(blockIdx.x, gridDim.x);
   const int64_t block = tile >> 2;
   const int quarter = tile & 3;   // which quarter of the block
   const int t = ws.block_tensor[block];
-  const gact_batch_entry ent = table[t];
+  gact_batch_entry ent = table[t];
+  if (outs) ent.x = outs[t];
   const int64_t lb = block - ent.first_block;
   const uint8_t* packed = packed_arena + ent.packed_offset;
   const uint8_t* sc = scale_arena + ent.stats_offset * 4;
@@ -3469,6 +3470,25 @@ dequantize_batched_kernel(const gact_batch_entry* __restrict__ table, const int3
     case 4: dequantize_batched_block<4>(ent, lb, quarter, packed, sc, mn); break;
     default: dequantize_batched_block<8>(ent, lb, quarter, packed, sc, mn); break;
   }
+}
+__global__ void __launch_bounds__(256)
+dequantize_batched_kernel(const gact_batch_entry* __restrict__ table, const int32_t* __restrict__ bits,
+                          BatchWorkspace ws, const uint8_t* __restrict__ packed_arena,
+                          const uint8_t* __restrict__ scale_arena, const uint8_t* __restrict__ min_arena) {
+  dequantize_batched(table, nullptr, bits, ws, packed_arena, scale_arena, min_arena);
+}
+// With the outputs' addresses in the launch's arguments: the table and the plan of the quantize call serve as they are, where a plan of
+// the outputs' own table stood before this launch (3.8 us on the GPU and a launch).  A block's address is one more scalar load beside its
+// entry.  69 half tensors, 16 M elements: calc_precision, quantize and dequantize 61.5 -> 53.7 us, 142 float tensors 140 -> 131; 120 half
+// tensors, 1.83 G elements, 1360 -> 1351.
+struct BatchOutputs {
+  const void* x[GACT_BATCH_ARGS];
+};
+__global__ void __launch_bounds__(256)
+dequantize_batched_to_kernel(const gact_batch_entry* __restrict__ table, const int32_t* __restrict__ bits,
+                             BatchWorkspace ws, const uint8_t* __restrict__ packed_arena,
+                             const uint8_t* __restrict__ scale_arena, const uint8_t* __restrict__ min_arena, BatchOutputs outs) {
+  dequantize_batched(table, outs.x, bits, ws, packed_arena, scale_arena, min_arena);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -4452,6 +4472,24 @@ int gact_dequantize_batched_types(const gact_batch_entry* table, const int32_t* 
   hipLaunchKernelGGL(dequantize_batched_kernel, grid, block, (dtypes == GACT_DTYPES_F32 ? BATCHED_CAP_LDS : 0u), (hipStream_t)stream, table, bits,
                      batch_workspace(const_cast<void*>(workspace)), (const uint8_t*)packed_arena,
                      (const uint8_t*)scale_arena, (const uint8_t*)min_arena);
+  return launch_status();
+}
+
+int gact_dequantize_batched_to(const gact_batch_entry* table, void* const* x, const int32_t* bits, int64_t L, int64_t total_blocks, int dtypes,
+                               const void* workspace, const void* packed_arena, const void* scale_arena, const void* min_arena,
+                               void* stream) {
+  if (!batched_args_ok(L, total_blocks) || dtypes < 0 || dtypes > GACT_DTYPES_ALL) return GACT_EINVAL;
+  if (L > GACT_BATCH_ARGS) return GACT_ELIMIT;
+  if (L == 0 || total_blocks == 0) return GACT_OK;
+  if (!table || !x || !bits || !workspace || !packed_arena || !scale_arena || !min_arena) return GACT_EINVAL;
+  if (!aligned16(packed_arena) || !aligned16(workspace)) return GACT_EALIGN;
+  BatchOutputs outs = {};
+  for (int64_t t = 0; t < L; t++) outs.x[t] = x[t];
+  fresh_launch();
+  const dim3 grid((unsigned)(4 * total_blocks)), block(256);
+  hipLaunchKernelGGL(dequantize_batched_to_kernel, grid, block, (dtypes == GACT_DTYPES_F32 ? BATCHED_CAP_LDS : 0u), (hipStream_t)stream, table,
+                     bits, batch_workspace(const_cast<void*>(workspace)), (const uint8_t*)packed_arena, (const uint8_t*)scale_arena,
+                     (const uint8_t*)min_arena, outs);
   return launch_status();
 }
 

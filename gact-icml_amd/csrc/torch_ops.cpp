@@ -440,31 +440,28 @@ PyObject* event_wait(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// batch_dequantize(entries, geometry, outputs, seeds, widths, codes, scale, min, (blocks, workspace bytes, element types)) -> (table, workspace)
+// batch_dequantize(entries, geometry, outputs, seeds, widths, codes, scale, min, table, workspace, (blocks, workspace bytes, element types)) -> True
 PyObject* batch_dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Batch b;
   int64_t blocks, ws_bytes, dtypes;
-  const at::Tensor *packed, *scale, *mn;
-  if (n != 9 || !(packed = plain(args[5])) || !(scale = plain(args[6])) || !(mn = plain(args[7])) || !PyTuple_CheckExact(args[8]) ||
-      PyTuple_GET_SIZE(args[8]) != 3 || !integer(PyTuple_GET_ITEM(args[8], 0), &blocks) || !integer(PyTuple_GET_ITEM(args[8], 1), &ws_bytes) ||
-      !integer(PyTuple_GET_ITEM(args[8], 2), &dtypes) || blocks <= 0 || !batch_of(args, &b))
+  const at::Tensor *packed, *scale, *mn, *table, *ws;
+  if (n != 11 || !(packed = plain(args[5])) || !(scale = plain(args[6])) || !(mn = plain(args[7])) || !(table = plain(args[8])) ||
+      !(ws = plain(args[9])) || !PyTuple_CheckExact(args[10]) || PyTuple_GET_SIZE(args[10]) != 3 ||
+      !integer(PyTuple_GET_ITEM(args[10], 0), &blocks) || !integer(PyTuple_GET_ITEM(args[10], 1), &ws_bytes) ||
+      !integer(PyTuple_GET_ITEM(args[10], 2), &dtypes) || blocks <= 0 || !batch_of(args, &b))
     Py_RETURN_NONE;
   const c10::Device device = b.geometry->device();
-  for (const at::Tensor* t : {packed, scale, mn})
+  for (const at::Tensor* t : {packed, scale, mn, table, ws})
     if (t->scalar_type() != at::kByte || !t->is_contiguous() || t->device() != device) Py_RETURN_NONE;
-  const c10::DeviceGuard guard(device);
-  if (capturing(device)) Py_RETURN_NONE;
-  used_on(*b.geometry, c10::hip::getCurrentHIPStream(device.index()));
-  const at::Tensor table = make({b.geometry->numel()}, at::kByte, device), ws = make({ws_bytes}, at::kByte, device);
+  if (table->numel() != b.geometry->numel() || ws->numel() != ws_bytes || capturing(device)) Py_RETURN_NONE;
+  void* x[GACT_BATCH_ARGS];
+  for (int64_t i = 0; i < b.count; i++) x[i] = const_cast<void*>(b.x[i]);
   const int rc = on(device, [&](void* stream) {
-    const int planned = gact_batch_plan_args((const gact_batch_entry*)in(*b.geometry), b.x.data(), b.seeds.data(), (gact_batch_entry*)out(table),
-                                             (const int32_t*)in(*b.bits), nullptr, b.count, blocks, packed->numel(), out(ws), nullptr, stream);
-    if (planned != GACT_OK) return planned;
-    return gact_dequantize_batched_types((const gact_batch_entry*)out(table), (const int32_t*)in(*b.bits), b.count, blocks, (int)dtypes, out(ws),
-                                         in(*packed), in(*scale), in(*mn), stream);
+    return gact_dequantize_batched_to((const gact_batch_entry*)in(*table), x, (const int32_t*)in(*b.bits), b.count, blocks, (int)dtypes, in(*ws),
+                                      in(*packed), in(*scale), in(*mn), stream);
   });
-  if (rc == GACT_OK) return tuple_of({table, ws});
+  if (rc == GACT_OK) Py_RETURN_TRUE;
   Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS
 }

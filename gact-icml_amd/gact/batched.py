@@ -250,10 +250,8 @@ class BatchedQuantizer:
                 outs = [torch.empty(s, dtype=d, device=self.device) for s, d in zip(q.shapes, q.dtypes)]
             geometry = self._on_gpu()
             if geometry is not None:
-                done = _abi.native().batch_dequantize(self._entries, geometry, list(outs), list(q.seeds), q.bits, q.packed, q.scale, q.min,
-                                                      (self.total_blocks, self.workspace_bytes, self.dtype_mask))
-                if done is not None:
-                    q._dq_table = done
+                if _abi.native().batch_dequantize(self._entries, geometry, list(outs), list(q.seeds), q.bits, q.packed, q.scale, q.min,
+                                                  q.table, q.workspace, (self.total_blocks, self.workspace_bytes, self.dtype_mask)):
                     return outs
             table = self._table(outs, q.seeds, wait=False)
             ws = self.new_workspace()

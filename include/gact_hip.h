@@ -197,6 +197,12 @@ int gact_dequantize_batched_types(const gact_batch_entry* table, const int32_t* 
                                   const void* workspace, const void* packed_arena, const void* scale_arena, const void* min_arena,
                                   void* stream);
 
+/* The same for up to GACT_BATCH_ARGS tensors into x[L] (host array of device addresses, 16-byte aligned), with the table and the workspace
+ * of the batch's quantize call: no plan of its own.  GACT_ELIMIT beyond GACT_BATCH_ARGS tensors. */
+int gact_dequantize_batched_to(const gact_batch_entry* table, void* const* x, const int32_t* bits, int64_t L, int64_t total_blocks, int dtypes,
+                               const void* workspace, const void* packed_arena, const void* scale_arena, const void* min_arena,
+                               void* stream);
+
 /* gact_batch_plan followed by gact_quantize_batched, with the workspace in a device array that is part of
  * the library (1 MB per GPU the library runs on, held until the process ends) instead of memory the
  * caller brings: nothing is allocated, by the library or on its behalf.  No counterpart in the reference; it

@@ -78,6 +78,23 @@ def test_void_plans_and_dropped_batches():
                              for a, x, b, s in zip(batch.dequantize(q), xs, widths, seeds))
 
 
+def test_outputs_of_the_caller():
+    xs, widths, seeds, batch = make(33)
+    q = batch.quantize(xs, torch.tensor(widths, dtype=torch.int32, device="cuda"), seeds)
+    want = batch.dequantize(q)
+    flat = torch.zeros(sum((x.numel() + 7) // 8 * 8 * x.element_size() for x in xs) + 16 * len(xs), dtype=torch.uint8, device="cuda")
+    outs, at = [], 0
+    for x in xs:      # side by side in one buffer, each on a 16-byte boundary
+        outs.append(flat[at:at + x.numel() * x.element_size()].view(x.dtype))
+        at += (x.numel() * x.element_size() + 15) // 16 * 16
+    assert all(torch.equal(a, b) for a, b in zip(batch.dequantize(q, outs), want))
+    with pytest.raises(RuntimeError, match="geometry"):
+        batch.dequantize(q, outs[::-1])
+    with pytest.raises(RuntimeError, match="aligned"):
+        batch.dequantize(q, [flat[1:1 + x.numel() * x.element_size()].view(x.dtype) if x.element_size() == 1 else
+                             flat[4:4 + x.numel() * x.element_size()].view(x.dtype) for x in xs])
+
+
 def test_batches_on_streams_of_their_own():
     xs, widths, seeds, batch = make(20)
     bits = torch.tensor(widths, dtype=torch.int32, device="cuda")
