@@ -892,7 +892,7 @@ __device__ __forceinline__ void chunk_words(const typename Elem<T>::Store& st, i
 //   GIVEN = true : min/max are read from mn_io / mx_io (the pack entry point's contract).
 // Codes follow quantization_cuda_kernel.cu:38-71; see Elem<T>::code1 for the arithmetic.
 // ------------------------------------------------------------------------------------------------
-template <typename T, int BITS, int NOISE, bool GIVEN, int SGR = 1, int STAGE = 0, bool LAZY = false, typename SRC>
+template <typename T, int BITS, int NOISE, bool GIVEN, int SGR = 1, int STAGE = 0, bool LAZY = false, bool PACKS = true, typename SRC>
 __device__ __forceinline__ void quantize_supergroup(const SRC& src, int64_t N, int64_t sg0,
                                                     int i, uint8_t* __restrict__ packed,
                                                     typename Elem<T>::Stat* __restrict__ scale_out,
@@ -903,7 +903,7 @@ __device__ __forceinline__ void quantize_supergroup(const SRC& src, int64_t N, i
   static_assert(GPR == 1 || GPR == 2 || GPR == 4 || GPR == 8, "a row holds 1, 2, 4 or 8 groups");
   constexpr int QMAX = (1 << BITS) - 1;
   constexpr int CH = Elem<T>::kQChunks, W = Elem<T>::kQWidth;
-  constexpr bool PK = packs_bytes<T, BITS, NOISE, GIVEN>();
+  constexpr bool PK = PACKS && packs_bytes<T, BITS, NOISE, GIVEN>();
   const int64_t n0 = sg0 * WPT;
 
   typename Elem<T>::Store v[GPR];
@@ -1619,7 +1619,7 @@ struct SeedArg {
 // (-DGACT_QGEOM_F32=..., _F16, _BF16) for experiments.
 struct QGeom { int sgr, threads, run, stage, stage_small, small_below; bool lazy, lazy_small; };
 #ifndef GACT_QGEOM_F16
-#define GACT_QGEOM_F16 {{1, 64, 0, 4, 4, 1 << 15, true, false}, {1, 64, 128, 2, 2, 0, true, true}, {1, 64, 128, 1, 1, 0, true, true}, {1, 64, 128, 0, 0, 0, false, false}}
+#define GACT_QGEOM_F16 {{1, 64, 0, 4, 4, 1 << 15, true, false}, {1, 64, 128, 2, 2, 1 << 17, true, true}, {1, 64, 128, 1, 1, 0, true, true}, {1, 64, 128, 0, 0, 0, false, false}}
 #endif
 #ifndef GACT_QGEOM_BF16
 #define GACT_QGEOM_BF16 {{1, 64, 0, 4, 4, 1 << 15, true, false}, {1, 64, 128, 2, 2, 0, true, true}, {1, 64, 128, 1, 1, 0, true, true}, {1, 64, 128, 0, 0, 0, false, false}}
@@ -1697,7 +1697,11 @@ quantize_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_
   const int64_t sg0 = ((int64_t)tile * (blockDim.x >> 4) + (threadIdx.x >> 4)) * SGR;
   if (sg0 * (8 / BITS) >= N) return;
   const uint64_t seed = seed_arg.value();
-  quantize_supergroup<T, BITS, NOISE, GIVEN, SGR, STAGE, LAZY>(ContiguousSource<T>{x, numel}, N, sg0, threadIdx.x & 15, packed, scale_out, mn_io, mx_io,
+  // half at 2 bit: packed bytes leave registers for seven waves on a SIMD instead of five, which helps while a tensor does not fill the
+  // chip for long and costs bandwidth on large ones (4 M elements 4.53 -> 4.35 us, 17 M 8.7 -> 8.4, 51 M and 72 M equal, 134 M 49.7 -> 51.3, 268 M 96 -> 100; a cap
+  // by dynamic LDS at five or four waves gets half of that back)
+  constexpr bool PACKS = SMALL || !(std::is_same<T, f16>::value && BITS == 2 && NOISE != GACT_NOISE_REF);
+  quantize_supergroup<T, BITS, NOISE, GIVEN, SGR, STAGE, LAZY, PACKS>(ContiguousSource<T>{x, numel}, N, sg0, threadIdx.x & 15, packed, scale_out, mn_io, mx_io,
                                                   (uint32_t)seed, (uint32_t)(seed >> 32), noise);
 }
 
@@ -1995,7 +1999,12 @@ quantize_transposed_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t nu
 // the one dispatched second takes a fifth longer): 1.4 waves per SIMD on average, waiting 0.46 of their lives (from HBM 0.63), with
 // 0.44 of the cycles issuing vector instructions and LDS conflicts 0.06; it reads 1.18 times its bytes from HBM.  With GS = 1 it
 // took 42; more waves through more segments cost more reading than they hide (44), and dropping one of the two barriers by a
-// ring of four slots changed nothing (41.8).
+// ring of four slots changed nothing (41.8).  (36.8 since codes are packed by conversions, [64,64,112,112] 1 bit 53.0 -> 48.8.)
+// What its 37 us are made of, each part taken out of a copy: the walk's reads alone 24.7 (a linear read of the tensor 16.5), with the
+// scatter 26.6, with everything but the stores 31 to 33.  Of the two workgroups on a CU the first takes 2.8 us a step and the
+// second 6, until the first has ended at 22 us and leaves the second 3.1 us a step and the CU half empty.  None of these changed it by more than 1 %:
+// twice the waves (512 threads), strips of 128 bytes (one workgroup of 1024), no reading beyond the channel's end (the first step's
+// pixels kept in registers), the stores held back until the next loads have arrived, priorities by progress.
 #define STRIP_PIECES 4    /* 16-byte pieces of a memory row in a strip (8: half [2,64,128,128] 4 bit 7.6 -> 9.5 us, large tensors equal) */
 #define STRIP_CHUNK 256   /* pixels: a thread takes four of one piece */
 #define STRIP_THREADS (STRIP_PIECES * STRIP_CHUNK / 4)
@@ -3572,7 +3581,9 @@ struct LaunchPlan {
 template <typename T, int BITS, int NOISE, bool GIVEN>
 const void* quantize_kernel_of(bool small) {
   constexpr QGeom G = q_geom<T>(BITS);
-  if constexpr (!GIVEN && NOISE != GACT_NOISE_REF && (G.stage_small != G.stage || G.lazy_small != G.lazy)) {
+  // small tensors have a kernel of their own where it differs: in its stages, or (half at 2 bit) in how it packs
+  constexpr bool PACKS_WHEN_SMALL = std::is_same<T, f16>::value && BITS == 2 && NOISE != GACT_NOISE_INJECT;
+  if constexpr (!GIVEN && NOISE != GACT_NOISE_REF && (G.stage_small != G.stage || G.lazy_small != G.lazy || PACKS_WHEN_SMALL)) {
     if (small) return (const void*)quantize_kernel<T, BITS, NOISE, GIVEN, true>;
   }
   return (const void*)quantize_kernel<T, BITS, NOISE, GIVEN, false>;
