@@ -238,6 +238,12 @@ class BatchedQuantizer:
         return BatchedPacked(self, packed, scale, mn, table, kept, ws, [t.shape for t in tensors],
                              list(self.dtypes), seeds, verdict)
 
+    def _plan_serves(self, q):
+        """Whether the table and plan q holds may be launched from as they are: they say how much is written where, so the quantizer that
+        made them has to have this one's tensors.  Any other batch is planned again by this quantizer's own table."""
+        owner = q.owner
+        return owner is self or (isinstance(owner, BatchedQuantizer) and owner._entry_bytes() == self._entry_bytes())
+
     def dequantize(self, q, outs=None, check=True):
         """Dequantize every tensor of a BatchedPacked in one launch into fresh tensors (or `outs`).
         check = True waits for the plan's verdict first and raises when the quantize
@@ -248,7 +254,7 @@ class BatchedQuantizer:
         with torch.cuda.device(self.device):
             if outs is None:
                 outs = [torch.empty(s, dtype=d, device=self.device) for s, d in zip(q.shapes, q.dtypes)]
-            geometry = self._on_gpu()
+            geometry = self._on_gpu() if self._plan_serves(q) else None
             if geometry is not None:
                 if _abi.native().batch_dequantize(self._entries, geometry, list(outs), list(q.seeds), q.bits, q.packed, q.scale, q.min,
                                                   q.table, q.workspace, (self.total_blocks, self.workspace_bytes, self.dtype_mask)):

@@ -108,3 +108,16 @@ def test_batches_on_streams_of_their_own():
     del batch
     torch.cuda.synchronize()
     assert all(torch.equal(a, b) for o in outs for a, b in zip(o, want))
+
+
+def test_a_batch_of_another_quantizer_fills_the_outputs_it_was_given():
+    """Fewer elements in as many blocks: the beginning of the tensor, and not a byte behind it."""
+    g = torch.Generator(device="cuda").manual_seed(2)
+    xs = [torch.randn(n, generator=g, device="cuda") for n in (300, 40000)]
+    q = BatchedQuantizer([300, 40000], [torch.float32] * 2, "cuda").quantize(xs, torch.tensor([4, 8], dtype=torch.int32, device="cuda"), [1, 2])
+    want = q.owner.dequantize(q)
+    flat = torch.full((64 * 1024,), 7.0, device="cuda")
+    fewer = [flat[:100], flat[1024:1024 + 33000]]
+    BatchedQuantizer([100, 33000], [torch.float32] * 2, "cuda").dequantize(q, fewer)
+    assert torch.equal(fewer[0], want[0][:100]) and torch.equal(fewer[1], want[1][:33000])
+    assert bool((flat[100:1024] == 7.0).all()) and bool((flat[1024 + 33000:] == 7.0).all())
