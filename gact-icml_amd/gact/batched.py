@@ -27,6 +27,7 @@ class BatchedPacked:
     synchronises); ``per_tensor`` calls it and raises.  ``BatchedQuantizer.dequantize`` raises by the copy of the
     verdict that left for the host right behind the plan, so that it does not wait for the quantize kernels."""
 
+    _arena_bytes = None     # of `packed` when the plan was made
     _verdict = None     # (event behind the copy, the workspace's first two words in pinned memory); none in a pickled one
 
     def __init__(self, owner, packed, scale, mn, table, bits, workspace, shapes, dtypes, seeds, verdict=None):
@@ -34,6 +35,7 @@ class BatchedPacked:
         self._verdict = verdict
         self.seeds = list(seeds)
         self.packed, self.scale, self.min = packed, scale, mn
+        self._arena_bytes = packed.numel()
         self.table, self.bits, self.workspace = table, bits, workspace
         self.shapes, self.dtypes = shapes, dtypes
 
@@ -240,8 +242,11 @@ class BatchedQuantizer:
 
     def _plan_serves(self, q):
         """Whether the table and plan q holds may be launched from as they are: they say how much is written where, so the quantizer that
-        made them has to have this one's tensors.  Any other batch is planned again by this quantizer's own table."""
+        made them has to have this one's tensors, and how far the codes are read, so the arena must not have been cut since.  Any other
+        batch is planned again by this quantizer's own table."""
         owner = q.owner
+        if q._arena_bytes is None or q.packed.numel() < q._arena_bytes:
+            return False
         return owner is self or (isinstance(owner, BatchedQuantizer) and owner._entry_bytes() == self._entry_bytes())
 
     def dequantize(self, q, outs=None, check=True):

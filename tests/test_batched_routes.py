@@ -68,3 +68,18 @@ def test_a_batch_of_another_quantizer(routes, numels, dtypes, same):
     q.owner = None      # a batch put together by hand
     other.dequantize(q, outs, check=False)
     assert routes == ["kept plan" if same else "own plan"] * 2 + ["kept plan", "own plan"]
+
+
+def test_an_arena_cut_after_the_call(routes):
+    """The plan vouches for the bytes there were when it was made; with fewer the next plan decides whether they are enough."""
+    batch = BatchedQuantizer([300, 70], [F32, F16], "cpu")
+    q = packed_by(batch)
+    q.packed = torch.cat([q.packed, q.packed])      # a copy with room behind it
+    batch.dequantize(q, check=False)
+    q.packed = q.packed[:512].clone()
+    batch.dequantize(q, check=False)
+    batch.dequantize(pickle.loads(pickle.dumps(q)), check=False)
+    older = packed_by(batch)
+    del older._arena_bytes      # as unpickled from a file that does not say
+    batch.dequantize(older, check=False)
+    assert routes == ["kept plan", "own plan", "own plan", "own plan"]
