@@ -3307,6 +3307,13 @@ __device__ __forceinline__ int batch_find(const gact_batch_entry* __restrict__ t
   return lo;
 }
 
+// Bytes of the arena a tensor of N groups takes at a width, as the plan counts them
+__device__ __forceinline__ int64_t batch_span(int width, int64_t N) {
+  const int wpt = 8 / width;
+  const int64_t n_round = (N + wpt - 1) / wpt * wpt;
+  return ((int64_t)width * n_round * (GROUP / 8) + 255) / 256 * 256;
+}
+
 // What the plan's workgroup 0 does: thread t sizes tensors t, t + 256, ...; the running packed-arena offset is carried across rounds of
 // 256 with an inclusive scan of each wave and the waves' totals.  One round, with the loads of all tensors under way at once, where a
 // wave alone took two (65 to 128 tensors).  entry(t) gives a tensor's size and type, place(t, width, offset) takes what the plan
@@ -3334,10 +3341,7 @@ __device__ __forceinline__ void batch_plan_sizes(const int32_t* __restrict__ bit
       width = valid ? given : 8;
       if (!valid || e.dtype < 0 || e.dtype > 2) bad_s = 1;
       atomicAdd(&count_s[width_index(width)], 1);
-      const int wpt = 8 / width;
-      const int64_t N = (e.numel + GROUP - 1) / GROUP;
-      const int64_t n_round = (N + wpt - 1) / wpt * wpt;
-      bytes = ((int64_t)width * n_round * (GROUP / 8) + 255) / 256 * 256;
+      bytes = batch_span(width, (e.numel + GROUP - 1) / GROUP);
     }
     int64_t incl = bytes;
 #pragma unroll
@@ -3469,11 +3473,18 @@ __device__ __forceinline__ void dequantize_batched(const gact_batch_entry* __res
   const int t = ws.block_tensor[block];
   gact_batch_entry ent = table[t];
   if (outs) ent.x = outs[t];
+  const int width = bits[t];
+  // the plan may be older than this launch: a width written over since must not lead past the codes
+  if (outs) {
+    const int64_t N = (ent.numel + GROUP - 1) / GROUP;
+    const int64_t span = width == 1 ? batch_span(1, N) : width == 2 ? batch_span(2, N) : width == 4 ? batch_span(4, N) : batch_span(8, N);
+    if (ent.packed_offset + span > ws.hdr->need) return;
+  }
   const int64_t lb = block - ent.first_block;
   const uint8_t* packed = packed_arena + ent.packed_offset;
   const uint8_t* sc = scale_arena + ent.stats_offset * 4;
   const uint8_t* mn = min_arena + ent.stats_offset * 4;
-  switch (bits[t]) {
+  switch (width) {
     case 1: dequantize_batched_block<1>(ent, lb, quarter, packed, sc, mn); break;
     case 2: dequantize_batched_block<2>(ent, lb, quarter, packed, sc, mn); break;
     case 4: dequantize_batched_block<4>(ent, lb, quarter, packed, sc, mn); break;

@@ -198,7 +198,8 @@ int gact_dequantize_batched_types(const gact_batch_entry* table, const int32_t* 
                                   void* stream);
 
 /* The same for up to GACT_BATCH_ARGS tensors into x[L] (host array of device addresses, 16-byte aligned), with the table and the workspace
- * of the batch's quantize call: no plan of its own.  GACT_ELIMIT beyond GACT_BATCH_ARGS tensors. */
+ * of the batch's quantize call: no plan of its own.  A width written over since then is looked at: a tensor whose codes would end past
+ * the plan's bytes is left out.  GACT_ELIMIT beyond GACT_BATCH_ARGS tensors. */
 int gact_dequantize_batched_to(const gact_batch_entry* table, void* const* x, const int32_t* bits, int64_t L, int64_t total_blocks, int dtypes,
                                const void* workspace, const void* packed_arena, const void* scale_arena, const void* min_arena,
                                void* stream);

@@ -121,3 +121,19 @@ def test_a_batch_of_another_quantizer_fills_the_outputs_it_was_given():
     BatchedQuantizer([100, 33000], [torch.float32] * 2, "cuda").dequantize(q, fewer)
     assert torch.equal(fewer[0], want[0][:100]) and torch.equal(fewer[1], want[1][:33000])
     assert bool((flat[100:1024] == 7.0).all()) and bool((flat[1024 + 33000:] == 7.0).all())
+
+
+def test_widths_written_over_after_the_call():
+    """Codes end where the plan says: a tensor that its new width would take further is left as it is, the others keep to their codes."""
+    sizes = [257, 256 * 128 * 3 + 5, 9]
+    g = torch.Generator(device="cuda").manual_seed(3)
+    xs = [torch.randn(n, generator=g, device="cuda") for n in sizes]
+    batch = BatchedQuantizer(sizes, [torch.float32] * 3, "cuda")
+    q = batch.quantize(xs, torch.tensor([1, 2, 4], dtype=torch.int32, device="cuda"), [1, 2, 3])
+    want = batch.dequantize(q)
+    for widths, untouched in [([1, 2, 4], []), ([1, 4, 4], [1]), ([8, 8, 8], [1]), ([1, 2, 8], []), ([2, 1, 32], [])]:
+        q.bits.copy_(torch.tensor(widths, dtype=torch.int32))
+        outs = batch.dequantize(q, [torch.full((n,), 7.0, device="cuda") for n in sizes])
+        for i, (a, b) in enumerate(zip(outs, want)):
+            assert bool((a == 7.0).all()) == (i in untouched), (widths, i)
+            assert widths[i] != (1, 2, 4)[i] or torch.equal(a, b)
