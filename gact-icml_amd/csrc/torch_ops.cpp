@@ -361,7 +361,8 @@ bool batch_of(PyObject* const* args, Batch* b) {
   }
   return true;
 }
-// The geometry outlives one call and may be used on a stream other than the one it was made on: its memory waits for that stream too
+// What outlives the call that made it - the geometry, all that a compressed batch holds - may be used on another stream and dropped before
+// that stream gets to it: its memory waits for that stream too (the allocator passes over its own stream)
 void used_on(const at::Tensor& t, c10::hip::HIPStream stream) { c10::hip::HIPCachingAllocator::recordStream(t.storage().data_ptr(), stream); }
 bool capturing(c10::Device device) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
@@ -455,6 +456,8 @@ PyObject* batch_dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   for (const at::Tensor* t : {packed, scale, mn, table, ws})
     if (t->scalar_type() != at::kByte || !t->is_contiguous() || t->device() != device) Py_RETURN_NONE;
   if (table->numel() != b.geometry->numel() || ws->numel() != ws_bytes || capturing(device)) Py_RETURN_NONE;
+  const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(device.index());
+  for (const at::Tensor* t : {packed, scale, mn, table, ws, b.bits}) used_on(*t, stream);
   void* x[GACT_BATCH_ARGS];
   for (int64_t i = 0; i < b.count; i++) x[i] = const_cast<void*>(b.x[i]);
   const int rc = on(device, [&](void* stream) {

@@ -137,3 +137,24 @@ def test_widths_written_over_after_the_call():
         for i, (a, b) in enumerate(zip(outs, want)):
             assert bool((a == 7.0).all()) == (i in untouched), (widths, i)
             assert widths[i] != (1, 2, 4)[i] or torch.equal(a, b)
+
+
+def test_a_batch_dropped_while_another_stream_waits_to_restore_it():
+    """Nothing of it is handed out again before that stream has read it."""
+    xs, widths, seeds, batch = make(24)
+    bits = torch.tensor(widths, dtype=torch.int32, device="cuda")
+    want = batch.dequantize(batch.quantize(xs, bits, seeds))
+    q = batch.quantize(xs, bits, seeds)
+    torch.cuda.synchronize()
+    held = [q.packed, q.scale, q.min, q.table, q.workspace, q.bits]
+    spans = [(t.data_ptr(), t.numel() * t.element_size()) for t in held]
+    late = torch.cuda.Stream()
+    with torch.cuda.stream(late):
+        torch.cuda._sleep(100_000_000)      # 0.05 s at least
+        outs = batch.dequantize(q)
+    del held, q
+    fresh = [torch.full((n,), 255, dtype=torch.uint8, device="cuda") for _, n in spans]
+    assert not late.query()
+    assert not any(t.data_ptr() < at + n and at < t.data_ptr() + t.numel() for t in fresh for at, n in spans)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(outs, want))
