@@ -469,10 +469,17 @@ PyObject* batch_dequantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// ordinary() -> whether what is made now is what it will be later: no mode, transform or trace around the call
+PyObject* ordinary(PyObject*, PyObject* const*, Py_ssize_t) {
+  if (ordinary_call()) Py_RETURN_TRUE;
+  Py_RETURN_FALSE;
+}
+
 #define FASTCALL(f) {#f, (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {FASTCALL(quantize), FASTCALL(dequantize), FASTCALL(minimax),     FASTCALL(pack),        FASTCALL(unpack),
                          FASTCALL(mask_pack), FASTCALL(mask_unpack), FASTCALL(batch_table),
-                         FASTCALL(batch_quantize), FASTCALL(batch_dequantize), FASTCALL(event_wait), {nullptr, nullptr, 0, nullptr}};
+                         FASTCALL(batch_quantize), FASTCALL(batch_dequantize), FASTCALL(event_wait),
+                         FASTCALL(ordinary), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "gact_torch", "The operators' host side.", -1, methods};
 
 }  // namespace

@@ -147,7 +147,8 @@ class BatchedQuantizer:
 
     def _on_gpu(self):
         """The entries on the GPU, for the native calls; None where those do not apply."""
-        if self._geometry is None and 0 < self.L <= _abi.BATCH_ARGS and not torch.cuda.is_current_stream_capturing():
+        if (self._geometry is None and 0 < self.L <= _abi.BATCH_ARGS and not torch.cuda.is_current_stream_capturing()
+                and _abi.native().ordinary()):      # inside a transform or a mode it would be a wrapper, kept past its time
             # a copy that has arrived when this returns, whatever stream uses it
             self._geometry = torch.frombuffer(bytearray(self._entry_bytes()), dtype=torch.uint8).to(self.device)
         return self._geometry

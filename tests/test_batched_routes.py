@@ -83,3 +83,29 @@ def test_an_arena_cut_after_the_call(routes):
     del older._arena_bytes      # as unpickled from a file that does not say
     batch.dequantize(older, check=False)
     assert routes == ["kept plan", "own plan", "own plan", "own plan"]
+
+
+@pytest.mark.parametrize("around", ["functionalize", "jvp", "fake"])
+def test_the_geometry_is_not_made_inside_a_transform_or_a_mode(around, monkeypatch):
+    """It is kept for later calls, so it must not be a wrapper that only means something there."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    batch = BatchedQuantizer([300], [F32], "cpu")
+    batch.device = torch.device("meta")     # a copy to another device, which a transform wraps
+    seen = []
+
+    def inside(x):
+        seen.append(batch._on_gpu())
+        return x
+
+    x = torch.ones(2)
+    if around == "fake":
+        with FakeTensorMode(allow_non_fake_inputs=True):
+            inside(x)
+    elif around == "functionalize":
+        torch.func.functionalize(inside)(x)
+    else:
+        torch.func.jvp(inside, (x,), (x,))
+    assert seen == [None] and batch._geometry is None
+    assert batch._on_gpu() is batch._geometry and type(batch._geometry) is torch.Tensor
