@@ -1490,7 +1490,7 @@ __device__ __forceinline__ void dequantize_unit(const uint8_t* __restrict__ pack
 #ifndef GACT_QB_STAGE
 #define GACT_QB_STAGE 0 /* groups at a time in the batched quantize rows (0: all 8 at once) */
 #endif
-template <typename T, int BITS, int NOISE>
+template <typename T, int BITS, int NOISE, bool PACKS = true>
 __device__ __forceinline__ void quantize_block128(const T* __restrict__ x, int64_t numel, int64_t N, int64_t lb,
                                                   uint8_t* __restrict__ packed,
                                                   typename Elem<T>::Stat* __restrict__ scale_out,
@@ -1506,8 +1506,8 @@ __device__ __forceinline__ void quantize_block128(const T* __restrict__ x, int64
         quantize_supergroup<T, BITS, NOISE, false, 1>(ContiguousSource<T>{x, numel}, N, sg0 + q, i, packed, scale_out, mn_out, (T*)nullptr,
                                                       (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
   } else if (sg0 * WPT < N) {
-    quantize_supergroup<T, BITS, NOISE, false, BITS, GACT_QB_STAGE>(ContiguousSource<T>{x, numel}, N, sg0, i, packed, scale_out, mn_out, (T*)nullptr,
-                                                                    (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
+    quantize_supergroup<T, BITS, NOISE, false, BITS, GACT_QB_STAGE, false, PACKS>(ContiguousSource<T>{x, numel}, N, sg0, i, packed, scale_out, mn_out,
+                                                                                  (T*)nullptr, (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
   }
 }
 // Dequantize: four workgroups share a block of 128 groups, 32 groups each - 4 units of 8 groups for float (a wave
@@ -3422,8 +3422,9 @@ batch_plan_args_kernel(BatchArgs args, const gact_batch_entry* __restrict__ geom
 
 // Quantize, one launch per element type over all blocks of the grid: the width of a block's tensor is read from
 // device memory and selects the code path (a row takes 8 groups whatever the width, so every path holds the same
-// amount of data in registers); blocks of tensors of another element type leave at once.
-template <typename T, int NOISE>
+// amount of data in registers); blocks of tensors of another element type leave at once.  PACKED: the sum of the widths below 8 whose
+// codes are packed as bytes where packs_bytes allows it (see batch_packs).
+template <typename T, int NOISE, int PACKED>
 __global__ void __launch_bounds__(256)
 quantize_batched_kernel(const gact_batch_entry* __restrict__ table, const int32_t* __restrict__ bits,
                         BatchWorkspace ws, uint8_t* __restrict__ packed_arena, uint8_t* __restrict__ scale_arena,
@@ -3440,9 +3441,9 @@ quantize_batched_kernel(const gact_batch_entry* __restrict__ table, const int32_
   typename Elem<T>::Stat* sc = (typename Elem<T>::Stat*)(scale_arena + ent.stats_offset * 4);
   T* mn = (T*)(min_arena + ent.stats_offset * 4);
   switch (bits[t]) {
-    case 1: quantize_block128<T, 1, NOISE>(x, ent.numel, N, lb, packed, sc, mn, ent.seed); break;
-    case 2: quantize_block128<T, 2, NOISE>(x, ent.numel, N, lb, packed, sc, mn, ent.seed); break;
-    case 4: quantize_block128<T, 4, NOISE>(x, ent.numel, N, lb, packed, sc, mn, ent.seed); break;
+    case 1: quantize_block128<T, 1, NOISE, (PACKED & 1) != 0>(x, ent.numel, N, lb, packed, sc, mn, ent.seed); break;
+    case 2: quantize_block128<T, 2, NOISE, (PACKED & 2) != 0>(x, ent.numel, N, lb, packed, sc, mn, ent.seed); break;
+    case 4: quantize_block128<T, 4, NOISE, (PACKED & 4) != 0>(x, ent.numel, N, lb, packed, sc, mn, ent.seed); break;
     default: quantize_block128<T, 8, NOISE>(x, ent.numel, N, lb, packed, sc, mn, ent.seed); break;
   }
 }
@@ -4388,14 +4389,27 @@ int64_t gact_batch_workspace_bytes(int64_t L, int64_t total_blocks) {
 
 namespace {
 // Three workgroups on a CU, by a request for dynamic LDS that nobody touches (see quantize_lds_cap), for two of the batched kernels:
-//   quantize, half: its registers admit four.  120 half tensors, four / three / two workgroups, us: 1.83 G elements, 1, 2 and 4 bit mixed
-//     696 / 676 / 665, all at 1 bit 634 / 606 / 638, 2 bit 674 / 655 / 661, 4 bit 769 / 758 / 718, 8 bit 870 / 843 / 893;
-//     0.23 G mixed 88.5 / 84.7 / 88.5, 57 M 25.1 / 25.2 / 27.5.  Three never loses whatever the widths, which the host does not know.
-//     Float and bfloat16 hold two by their registers.
+//   quantize, half: where codes are packed as bytes (batch_packs) its registers admit four, which is one too many from 10^8 elements on.
+//     120 half tensors, four / three workgroups, us: 29 M elements, 1, 2 and 4 bit mixed 15.1 / 14.9, 114 M 46.3 / 44.9, 229 M 89.0 / 84.7,
+//     343 M 132 / 126;  at 4 bit 15.7 / 15.4, 50.3 / 48.9, 97.8 / 94.3, 145 / 141;  57 M at 1 bit 23.8 / 24.6, the one loss seen.  Two
+//     lose 5 % up to 0.23 G.  Without packed bytes three or four make no difference (1.83 G mixed 669 / 666).  Float and bfloat16 hold
+//     two by their registers.
 //   dequantize, float: eight / four / three workgroups, 0.69 G elements mixed 539 / 492 / 475, 1 bit 517 / 484 / 444, 8 bit 586 / 551 / 585;
 //     0.23 G mixed 180 / 166 / 162, 57 M 46.9 / 43.4 / 44.3.  Half and bfloat16 lose by any cap (mixed 673 / 856 / 1010), so it goes
 //     with batches that are known to hold float tensors only.
 #define BATCHED_CAP_LDS 53000u
+// Whose codes the batched quantize of half tensors packs as bytes (fast stream), a sum of widths.  Bytes are fewer instructions and
+// registers, which pays while a batch does not fill the chip for long and costs bandwidth where HBM bounds it, at 4 bit first; whatever
+// the widths turn out to be, the line lies where the form taken loses to neither of the others.  120 tensors, us, all packed / all but
+// 4 bit / none:
+//   14 M elements  1 bit 11.2 / 11.2 / 11.8, 2 bit 11.4 / 11.4 / 12.1, 4 bit 11.4 / 12.5 / 12.5, the three mixed 11.3 / 11.7 / 12.1
+//   57 M           24.6 / 24.6 / 25.2, 25.7 / 25.7 / 26.5, 27.3 / 28.6 / 28.5, 25.9 / 26.6 / 27.0
+//   114 M          42.2 / 42.1 / 42.7, 44.2 / 44.1 / 45.1, 49.1 / 48.8 / 48.8, 45.1 / 45.7 / 45.8     -> all up to 2^12 blocks (134 M)
+//   229 M          77.1 / 77.7 / 78.4, 82.1 / 82.3 / 83.3, 93.8 / 92.1 / 92.1, 84.9 / 85.0 / 85.6
+//   343 M          113 / 113 / 115, 122.2 / 121.6 / 122.5, 141.7 / 134.8 / 134.8, 124.8 / 124.3 / 124.1  -> all but 4 bit below 12 * 2^10 (403 M)
+//   458 M          149 / 150 / 153, 162.0 / 161.3 / 160.6, 187.6 / 179.6 / 179.1, 168.4 / 166.8 / 165.1  -> none from there on
+//   1.83 G         600 / 610 / 602, 657 / 657 / 640, 757 / 739 / 743, 677 / 671 / 661
+int batch_packs(int64_t total_blocks) { return total_blocks < (1 << 12) ? 7 : total_blocks < 12 << 10 ? 3 : 0; }
 int batch_plan_on(gact_batch_entry* table, const int32_t* bits, int64_t L, int64_t total_blocks, int64_t capacity,
                   void* workspace, int64_t* verdict, hipStream_t s) {
   const BatchWorkspace ws = batch_workspace(workspace);
@@ -4409,19 +4423,25 @@ int quantize_batched_on(const gact_batch_entry* table, const int32_t* bits, int6
                         hipStream_t s) {
   const BatchWorkspace ws = batch_workspace(workspace);
   const dim3 grid((unsigned)total_blocks), block(256);
-#define GACT_LAUNCH_QB(T, M)                                                                                  \
-  hipLaunchKernelGGL((quantize_batched_kernel<T, M>), grid, block, (Elem<T>::kDtype == GACT_F16 ? BATCHED_CAP_LDS : 0u), s, table, bits, ws, (uint8_t*)packed_arena, \
-                     (uint8_t*)scale_arena, (uint8_t*)min_arena)
-#define GACT_LAUNCH_QB_ALL(M)                                                                                 \
+#define GACT_LAUNCH_QB(T, M, PACKED)                                                                          \
+  hipLaunchKernelGGL((quantize_batched_kernel<T, M, PACKED>), grid, block, (Elem<T>::kDtype == GACT_F16 ? BATCHED_CAP_LDS : 0u), s, table, bits, ws, \
+                     (uint8_t*)packed_arena, (uint8_t*)scale_arena, (uint8_t*)min_arena)
+#define GACT_LAUNCH_QB_ALL(M, LAUNCH_F16)                                                                     \
   do {                                                                                                        \
-    if (dtypes & GACT_DTYPES_F32) GACT_LAUNCH_QB(float, M);                                                   \
-    if (dtypes & GACT_DTYPES_F16) GACT_LAUNCH_QB(f16, M);                                                     \
-    if (dtypes & GACT_DTYPES_BF16) GACT_LAUNCH_QB(bf16, M);                                                   \
+    if (dtypes & GACT_DTYPES_F32) GACT_LAUNCH_QB(float, M, 7);                                                \
+    if (dtypes & GACT_DTYPES_F16) LAUNCH_F16;                                                                 \
+    if (dtypes & GACT_DTYPES_BF16) GACT_LAUNCH_QB(bf16, M, 7);                                                \
   } while (0)
   switch (noise_mode) {
-    case GACT_NOISE_CONST: GACT_LAUNCH_QB_ALL(GACT_NOISE_CONST); break;
-    case GACT_NOISE_REF: GACT_LAUNCH_QB_ALL(GACT_NOISE_REF); break;
-    default: GACT_LAUNCH_QB_ALL(GACT_NOISE_FAST); break;
+    case GACT_NOISE_CONST: GACT_LAUNCH_QB_ALL(GACT_NOISE_CONST, GACT_LAUNCH_QB(f16, GACT_NOISE_CONST, 7)); break;
+    case GACT_NOISE_REF: GACT_LAUNCH_QB_ALL(GACT_NOISE_REF, GACT_LAUNCH_QB(f16, GACT_NOISE_REF, 7)); break;
+    default:
+      GACT_LAUNCH_QB_ALL(GACT_NOISE_FAST, switch (batch_packs(total_blocks)) {
+        case 7: GACT_LAUNCH_QB(f16, GACT_NOISE_FAST, 7); break;
+        case 3: GACT_LAUNCH_QB(f16, GACT_NOISE_FAST, 3); break;
+        default: GACT_LAUNCH_QB(f16, GACT_NOISE_FAST, 0); break;
+      });
+      break;
   }
 #undef GACT_LAUNCH_QB_ALL
 #undef GACT_LAUNCH_QB

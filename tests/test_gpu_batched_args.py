@@ -158,3 +158,25 @@ def test_a_batch_dropped_while_another_stream_waits_to_restore_it():
     assert not any(t.data_ptr() < at + n and at < t.data_ptr() + t.numel() for t in fresh for at, n in spans)
     torch.cuda.synchronize()
     assert all(torch.equal(a, b) for a, b in zip(outs, want))
+
+
+@pytest.mark.parametrize("blocks", [(1 << 12) - 1, 1 << 12, (12 << 10) - 1, 12 << 10])
+def test_half_batches_where_another_kernel_takes_over(blocks):
+    """On either side of the sizes from which fewer widths pack their codes as bytes: every width, ragged ends, a long tensor at each width
+    below 8."""
+    sizes = [1, 257, 32769, 100003] * 4
+    long = (blocks - sum(-(-n // 32768) for n in sizes)) // 3
+    ends = [long, long, blocks - sum(-(-n // 32768) for n in sizes) - 2 * long]
+    sizes += [n * 32768 - 5 for n in ends]
+    widths = [b for b in (1, 2, 4, 8) for _ in range(4)] + [1, 2, 4]
+    g = torch.Generator(device="cuda").manual_seed(blocks)
+    xs = [torch.randn(n, generator=g, device="cuda", dtype=torch.float16) for n in sizes]
+    xs[2][5], xs[6][300], xs[10][7] = float("nan"), float("inf"), 60000.0
+    batch = BatchedQuantizer(sizes, [torch.float16] * len(xs), "cuda")
+    assert batch.total_blocks == blocks
+    q = batch.quantize(xs, torch.tensor(widths, dtype=torch.int32, device="cuda"), list(range(len(xs))))
+    for i, x in enumerate(xs):
+        want = ops.op_quantize(x, widths[i], i)
+        codes, b, scale, mn = q.per_tensor(i)
+        assert b == widths[i] and torch.equal(codes, want[0][: codes.numel()]), i
+        assert torch.equal(scale.view(torch.int16), want[2].view(torch.int16)) and torch.equal(mn.view(torch.int16), want[3].view(torch.int16))
