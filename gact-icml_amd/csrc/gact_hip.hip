@@ -2370,7 +2370,7 @@ __device__ __forceinline__ void groups_share_scale(T mine, T (&sc)[GroupsShape<T
   }
 }
 
-template <typename T, int D, int BITS, int NOISE>
+template <typename T, int D, int BITS, int NOISE, bool PACKS = true>
 __global__ void __launch_bounds__(64)
 quantize_groups_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_t N, uint8_t* __restrict__ packed,
                        T* __restrict__ scale_out, T* __restrict__ mn_out, T* __restrict__ mx_out,
@@ -2387,7 +2387,7 @@ quantize_groups_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
   const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
   const int half = S::HALF ? i >> 3 : 0;
 
-  constexpr bool PK = packs_bytes<T, BITS, NOISE, false>();
+  constexpr bool PK = PACKS && packs_bytes<T, BITS, NOISE, false>();
   typename Elem<T>::Store v[2];
   uint32_t acc[S::CPG][W];
   uint32_t words_of[S::CPG][W / 4];   // PK: the same bytes, packed
@@ -3696,7 +3696,15 @@ LaunchPlan plan_quantize_groups(int64_t N, int noise_mode) {
   LaunchPlan p;
   row_grid((N + S::UNIT_GROUPS - 1) / S::UNIT_GROUPS * S::ROWS, &p.grid, &p.block, 64);
   switch (noise_mode) {
-    case GACT_NOISE_CONST: p.kernel = (const void*)quantize_groups_kernel<T, D, BITS, GACT_NOISE_CONST>; break;
+    case GACT_NOISE_CONST:
+      p.kernel = (const void*)quantize_groups_kernel<T, D, BITS, GACT_NOISE_CONST>;
+      // half at 1 bit in groups of 512: packed bytes take 80 registers instead of 94, six waves on a SIMD instead of five, which costs
+      // bandwidth from 16 M elements on (a cap at five or four waves does not help).  Joined per byte / packed, us: 2 M 4.31 / 4.02,
+      // 4 M 4.57 / 4.30, 8 M 5.50 / 5.53, 12 M 6.96 / 7.22, 17 M 8.3 / 8.9, 34 M 14.6 / 15.0, 67 M 25.1 / 26.0, 134 M 46.7 / 48.1
+      if constexpr (std::is_same<T, f16>::value && D == 512 && BITS == 1) {
+        if (N >= 1 << 14) p.kernel = (const void*)quantize_groups_kernel<T, D, BITS, GACT_NOISE_CONST, false>;
+      }
+      break;
     case GACT_NOISE_INJECT: p.kernel = (const void*)quantize_groups_kernel<T, D, BITS, GACT_NOISE_INJECT>; break;
     case GACT_NOISE_FAST: p.kernel = (const void*)quantize_groups_kernel<T, D, BITS, GACT_NOISE_FAST>; break;
   }

@@ -114,3 +114,14 @@ def test_special_values_equal_the_extension_calls(group, dtype, bits):
         out = ops.op_dequantize(q, x.shape)
         assert torch.equal(_bits(out), _bits(want)) or torch.equal(torch.isnan(out), torch.isnan(want)) \
             and torch.equal(out[~out.isnan()], want[~want.isnan()]), stream
+
+
+@pytest.mark.parametrize("groups", [(1 << 14) - 1, 1 << 14, (1 << 14) + 1])
+def test_long_deterministic_half_tensors_at_one_bit_in_groups_of_512(groups):
+    """On either side of the size from which their codes are joined byte by byte, the last group short."""
+    g = torch.Generator().manual_seed(groups)
+    x = torch.randn(groups * 512 - 3, generator=g)
+    x[:512] = 0.25                                     # constant
+    x[512:1024] *= 2e-7                                # subnormal, the scale overflows
+    x[1024], x[2048], x[3000] = float("nan"), float("inf"), -65504.0
+    check(x.half(), 512, 1, "deterministic", 3)
