@@ -3461,7 +3461,7 @@ __device__ __forceinline__ void dequantize_batched_block(const gact_batch_entry&
   else
     dequantize_block128<bf16, BITS>(packed, (const float*)sc, (const bf16*)mn, ent.numel, N, lb, quarter, (bf16*)ent.x);
 }
-// grid: four workgroups per block of 128 groups; workgroups on a CU: BATCHED_CAP_LDS
+// grid: four workgroups per block of 128 groups; workgroups on a CU: batch_dequantize_lds
 __device__ __forceinline__ void dequantize_batched(const gact_batch_entry* __restrict__ table, const void* const* outs,
                                                    const int32_t* __restrict__ bits, const BatchWorkspace& ws,
                                                    const uint8_t* __restrict__ packed_arena, const uint8_t* __restrict__ scale_arena,
@@ -4396,16 +4396,27 @@ int64_t gact_batch_workspace_bytes(int64_t L, int64_t total_blocks) {
 }
 
 namespace {
-// Three workgroups on a CU, by a request for dynamic LDS that nobody touches (see quantize_lds_cap), for two of the batched kernels:
-//   quantize, half: where codes are packed as bytes (batch_packs) its registers admit four, which is one too many from 10^8 elements on.
-//     120 half tensors, four / three workgroups, us: 29 M elements, 1, 2 and 4 bit mixed 15.1 / 14.9, 114 M 46.3 / 44.9, 229 M 89.0 / 84.7,
-//     343 M 132 / 126;  at 4 bit 15.7 / 15.4, 50.3 / 48.9, 97.8 / 94.3, 145 / 141;  57 M at 1 bit 23.8 / 24.6, the one loss seen.  Two
-//     lose 5 % up to 0.23 G.  Without packed bytes three or four make no difference (1.83 G mixed 669 / 666).  Float and bfloat16 hold
-//     two by their registers.
-//   dequantize, float: eight / four / three workgroups, 0.69 G elements mixed 539 / 492 / 475, 1 bit 517 / 484 / 444, 8 bit 586 / 551 / 585;
-//     0.23 G mixed 180 / 166 / 162, 57 M 46.9 / 43.4 / 44.3.  Half and bfloat16 lose by any cap (mixed 673 / 856 / 1010), so it goes
-//     with batches that are known to hold float tensors only.
+// Fewer workgroups on a CU, by a request for dynamic LDS that nobody touches (see quantize_lds_cap), for two of the batched kernels.
+// Quantize, half: three.  Where codes are packed as bytes (batch_packs) its registers admit four, which is one too many from 10^8 elements
+// on.  120 half tensors, four / three workgroups, us: 29 M elements, 1, 2 and 4 bit mixed 15.1 / 14.9, 114 M 46.3 / 44.9, 229 M 89.0 / 84.7,
+// 343 M 132 / 126;  at 4 bit 15.7 / 15.4, 50.3 / 48.9, 97.8 / 94.3, 145 / 141;  57 M at 1 bit 23.8 / 24.6, the one loss seen.  Two
+// lose 5 % up to 0.23 G.  Without packed bytes three or four make no difference (1.83 G mixed 669 / 666).  Float and bfloat16 hold
+// two by their registers.
 #define BATCHED_CAP_LDS 53000u
+// Dequantize: batches that are known to hold float tensors only, by their size; half and bfloat16 lose by any cap (mixed 673 us, four on a
+// CU 856, three 1010).  Whatever the widths, which the host does not know: the cap taken is one that loses at none of them.
+// us with eight (no cap) / four / three workgroups, at 1 bit, 2 bit, 4 bit, 8 bit, and 1, 2 and 4 mixed:
+//   8 M elements  7.6 / 8.4 / 7.7   7.6 / 8.3 / 8.7   7.9 / 8.8 / 9.4   9.2 / 10.6 / 11.0   8.1 / 9.3 / 9.9
+//   14 M  13.1 / 12.7 / 12.0   13.0 / 13.2 / 13.8   13.7 / 13.7 / 14.1   16.3 / 16.6 / 16.4   13.7 / 14.4 / 14.6
+//   29 M  23.4 / 22.0 / 22.2   23.3 / 22.2 / 23.3   24.3 / 23.3 / 24.3   28.1 / 27.5 / 29.0 (in 12 tensors 26.6 / 27.1 / 27.8)   24.5 / 23.1 / 24.1
+//   43 M  33.9 / 32.3 / 32.6   33.9 / 32.4 / 33.7   35.5 / 33.6 / 34.5   39.4 / 39.4 / 41.5   36.2 / 33.8 / 34.8    -> four from 2^10 blocks (34 M) on
+//   114 M  89.4 / 81.9 / 79.5   88.0 / 79.6 / 81.7   92.6 / 84.6 / 84.3   96.8 / 94.7 / 102.1   92.8 / 84.1 / 84.7
+//   286 M, 8 bit 238 / 229 / 246, all four widths mixed 233 / 212 / 222
+//   343 M  262 / 240 / 229   265 / 239 / 241   276 / 251 / 243   296 / 276 / 296   277 / 251 / 245    -> three from 10 * 2^10 (336 M)
+//   915 M  689 / 639 / 603   697 / 639 / 633   737 / 671 / 641   813 / 744 / 793   730 / 663 / 634
+unsigned batch_dequantize_lds(int dtypes, int64_t total_blocks) {
+  return dtypes != GACT_DTYPES_F32 || total_blocks < 1 << 10 ? 0u : total_blocks < 10 << 10 ? 40000u : BATCHED_CAP_LDS;
+}
 // Whose codes the batched quantize of half tensors packs as bytes (fast stream), a sum of widths.  Bytes are fewer instructions and
 // registers, which pays while a batch does not fill the chip for long and costs bandwidth where HBM bounds it, at 4 bit first; whatever
 // the widths turn out to be, the line lies where the form taken loses to neither of the others.  120 tensors, us, all packed / all but
@@ -4519,7 +4530,7 @@ int gact_dequantize_batched_types(const gact_batch_entry* table, const int32_t* 
   if (!aligned16(packed_arena) || !aligned16(workspace)) return GACT_EALIGN;
   fresh_launch();
   const dim3 grid((unsigned)(4 * total_blocks)), block(256);
-  hipLaunchKernelGGL(dequantize_batched_kernel, grid, block, (dtypes == GACT_DTYPES_F32 ? BATCHED_CAP_LDS : 0u), (hipStream_t)stream, table, bits,
+  hipLaunchKernelGGL(dequantize_batched_kernel, grid, block, batch_dequantize_lds(dtypes, total_blocks), (hipStream_t)stream, table, bits,
                      batch_workspace(const_cast<void*>(workspace)), (const uint8_t*)packed_arena,
                      (const uint8_t*)scale_arena, (const uint8_t*)min_arena);
   return launch_status();
@@ -4537,7 +4548,7 @@ int gact_dequantize_batched_to(const gact_batch_entry* table, void* const* x, co
   for (int64_t t = 0; t < L; t++) outs.x[t] = x[t];
   fresh_launch();
   const dim3 grid((unsigned)(4 * total_blocks)), block(256);
-  hipLaunchKernelGGL(dequantize_batched_to_kernel, grid, block, (dtypes == GACT_DTYPES_F32 ? BATCHED_CAP_LDS : 0u), (hipStream_t)stream, table,
+  hipLaunchKernelGGL(dequantize_batched_to_kernel, grid, block, batch_dequantize_lds(dtypes, total_blocks), (hipStream_t)stream, table,
                      bits, batch_workspace(const_cast<void*>(workspace)), (const uint8_t*)packed_arena, (const uint8_t*)scale_arena,
                      (const uint8_t*)min_arena, outs);
   return launch_status();

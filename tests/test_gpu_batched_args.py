@@ -180,3 +180,22 @@ def test_half_batches_where_another_kernel_takes_over(blocks):
         codes, b, scale, mn = q.per_tensor(i)
         assert b == widths[i] and torch.equal(codes, want[0][: codes.numel()]), i
         assert torch.equal(scale.view(torch.int16), want[2].view(torch.int16)) and torch.equal(mn.view(torch.int16), want[3].view(torch.int16))
+
+
+@pytest.mark.parametrize("blocks", [(1 << 10) - 1, 1 << 10, (10 << 10) - 1, 10 << 10])
+def test_float_batches_where_the_launch_of_dequantize_changes(blocks):
+    """On either side of the sizes from which fewer workgroups share a CU: by the quantize call's plan and by one of the outputs' own."""
+    sizes = [1, 257, 32769, 100003]
+    sizes.append((blocks - sum(-(-n // 32768) for n in sizes)) * 32768 - 5)
+    widths = [8, 4, 2, 1, 4]
+    g = torch.Generator(device="cuda").manual_seed(blocks)
+    xs = [torch.randn(n, generator=g, device="cuda") for n in sizes]
+    batch = BatchedQuantizer(sizes, [torch.float32] * len(xs), "cuda")
+    assert batch.total_blocks == blocks
+    q = batch.quantize(xs, torch.tensor(widths, dtype=torch.int32, device="cuda"), list(range(len(xs))))
+    outs = batch.dequantize(q)
+    table, again = batch._table(xs, q.seeds), [x.clone() for x in xs]
+    batch.launch_dequantize(table, q.bits, q.packed, q.scale, q.min, batch.new_workspace())      # over the inputs
+    for i, x in enumerate(again):
+        want = ops.op_dequantize(ops.op_quantize(x, widths[i], i), x.shape)
+        assert torch.equal(outs[i], want) and torch.equal(xs[i], want), i
