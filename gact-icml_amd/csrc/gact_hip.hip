@@ -237,7 +237,8 @@ __device__ __forceinline__ uint32_t centred_code_bits_of_any(float z) { return c
 // float's mantissa takes an addition (and a median) of its own, a shift-or into its byte's register and the joining of four registers.
 // Fields of one to four bits then join word by word.  It differs from the reference from 256 on, which truncates to the byte: the
 // 8-bit code of a half tensor (whose scale, rounded to half, can put the largest element at 256), injected noise and a caller's min and
-// max stay with the forms above - and so does float under the reference stream, which a Philox block per byte bounds: 1 % faster to 4 %
+// max stay with the forms above - and so do half kernels that the registers saved let hold more waves than HBM bears (2 bit from 2^17 groups
+// on, batches by batch_packs, deterministic 1 bit in long tensors of groups of 512), and float under the reference stream, which a Philox block per byte bounds: 1 % faster to 4 %
 // slower with packed bytes (103 M elements, 2 bit 74.2 -> 76.9 us) where half is 2-4 % faster (134 M, 4 bit 105.5 -> 101.0).
 // Quantize alone, before -> after: 4 M elements float 1 bit 5.73 -> 5.45 us, 2 bit 5.40 -> 5.21, bfloat16 4 bit 4.11 -> 4.02; half in groups of 128
 // [16384,1024] 4 bit 9.57 -> 9.28; large contiguous tensors are bound by HBM and gain 0-3 %.  A half scale that overflowed to +inf makes
@@ -4383,7 +4384,8 @@ int gact_calc_precision_device(int32_t* b, const float* C, const int64_t* w, int
           hipSuccess)
     return GACT_ELAUNCH;
   // one thread per candidate slot up to the largest workgroup: the sort's passes are what the kernel spends its time
-  // on (120 tensors: 65.7 us with 64 threads, 25.5 with 256, 22.6 with 512; 24 tensors: 12.0 with 128, 14.1 with 256)
+  // on (250 tensors: 47.3 us with 64 threads, 17.3 with 256, 13.9 with 1024; 120 tensors: 21.4 with 64, 11.3 with 256, 9.7 with 512;
+  // 24 tensors: 8.3 with 64, 7.4 with 128)
   const unsigned threads = (unsigned)(M < 64 ? 64 : M > PREC_THREADS ? PREC_THREADS : M);
   hipLaunchKernelGGL(calc_precision_kernel, dim3(1), dim3(threads), lds, (hipStream_t)stream, b, C, w,
                      (int)L, target, status);

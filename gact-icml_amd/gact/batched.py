@@ -208,7 +208,7 @@ class BatchedQuantizer:
     def quantize(self, tensors, bits, seeds, arena_bytes=None, rng_stream=None):
         """Quantize all tensors in one batched launch.  `bits` is an int32 tensor on the device (e.g. the output
         of calc_precision_device) holding 1, 2, 4 or 8 for every tensor.  Returns a BatchedPacked; nothing
-        synchronises, so a void launch (see BatchedPacked) shows when the result is used."""
+        synchronises but a quantizer's first call, which brings its entries to the GPU, so a void launch (see BatchedPacked) shows when the result is used."""
         from .cpp_extension.quantization import _noise_mode
         if bits.dtype != torch.int32 or not bits.is_cuda or bits.numel() != self.L:
             raise RuntimeError("bits must be an int32 CUDA tensor with one entry per tensor")
@@ -251,7 +251,8 @@ class BatchedQuantizer:
         return owner is self or (isinstance(owner, BatchedQuantizer) and owner._entry_bytes() == self._entry_bytes())
 
     def dequantize(self, q, outs=None, check=True):
-        """Dequantize every tensor of a BatchedPacked in one launch into fresh tensors (or `outs`).
+        """Dequantize every tensor of a BatchedPacked in one launch into fresh tensors (or `outs`), by the plan of its quantize call
+        where that serves (_plan_serves) and by one of this quantizer's own otherwise.
         check = True waits for the plan's verdict first and raises when the quantize
         launch was void; pass False where nothing may synchronise (stream capture) and the caller has
         checked ``q.ok()`` itself."""
