@@ -2006,6 +2006,10 @@ quantize_transposed_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t nu
 // second 6, until the first has ended at 22 us and leaves the second 3.1 us a step and the CU half empty.  None of these changed it by more than 1 %:
 // twice the waves (512 threads), strips of 128 bytes (one workgroup of 1024), no reading beyond the channel's end (the first step's
 // pixels kept in registers), the stores held back until the next loads have arrived, priorities by progress.
+// What did: the loads of a step behind all of its scatter, and the four elements of the column behind the strip asked for together
+// (each had a test and a wait of its own: three round trips to memory a chunk, at the end of every strip).  Before -> now, us, inputs in
+// rotation: half [64,256,56,56] 1 bit 47.1 -> 42.8, 2 bit 39.4 -> 37.7, 4 bit 36.8 -> 36.0, 8 bit 42.8 -> 41.8, [64,64,112,112] 1 bit 48.6 -> 45.9,
+// [8,256,56,56] 4 bit 11.5 -> 10.9, [2,64,128,128] 5.8 -> 5.3; float equal, small tensors -2 to +2.5 %.
 #define STRIP_PIECES 4    /* 16-byte pieces of a memory row in a strip (8: half [2,64,128,128] 4 bit 7.6 -> 9.5 us, large tensors equal) */
 #define STRIP_CHUNK 256   /* pixels: a thread takes four of one piece */
 #define STRIP_THREADS (STRIP_PIECES * STRIP_CHUNK / 4)
@@ -2050,7 +2054,7 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
   uint32_t first_of[W];
 #pragma unroll
   for (int e = 0; e < W; e++) first_of[e] = first_pixel(piece * W + e);
-  struct Chunk { u32x4 v[4]; T beyond[4]; };
+  struct Chunk { u32x4 v[4]; uint32_t beyond[4]; };   // beyond: the elements' bits
   const uint32_t j_first = seg * g.segment * (UNIT / STEP);        // first step's groups of the segment within a channel
   const uint32_t j_end = j_first + g.segment * (UNIT / STEP);
   auto load = [&](uint32_t chunk, Chunk& q) {
@@ -2061,8 +2065,16 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
 #pragma unroll
       for (int j = 0; j < 4; j++) q.v[j] = *reinterpret_cast<const u32x4*>(p + j * g.sk);
       if (at >= K && last_piece) {
+        // into registers of their own and under one test, so that all four are asked for before any is waited for
+        if (behind) {
+          typedef typename std::conditional<ES == 4, uint32_t, uint16_t>::type Bits;
+          const Bits* const p1 = reinterpret_cast<const Bits*>(behind) + (int64_t)k * g.sk;
 #pragma unroll
-        for (int j = 0; j < 4; j++) q.beyond[j] = behind ? behind[(int64_t)(k + j) * g.sk] : (T)0.0f;
+          for (int j = 0; j < 4; j++) q.beyond[j] = p1[j * g.sk];
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; j++) q.beyond[j] = 0u;
+        }
       }
     }
   };
@@ -2103,11 +2115,10 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
       if (last_piece) {
         hi = u32x2{0u, 0u};
         if constexpr (ES == 4) {
-          lo = u32x2{__builtin_bit_cast(uint32_t, q.beyond[0]), __builtin_bit_cast(uint32_t, q.beyond[1])};
-          hi = u32x2{__builtin_bit_cast(uint32_t, q.beyond[2]), __builtin_bit_cast(uint32_t, q.beyond[3])};
+          lo = u32x2{q.beyond[0], q.beyond[1]};
+          hi = u32x2{q.beyond[2], q.beyond[3]};
         } else {
-          const auto half = [&](int j) { return (uint32_t)__builtin_bit_cast(uint16_t, q.beyond[j]); };
-          lo = u32x2{half(0) | half(1) << 16, half(2) | half(3) << 16};
+          lo = u32x2{q.beyond[0] | q.beyond[1] << 16, q.beyond[2] | q.beyond[3] << 16};
         }
         put(piece * PIECE + (W - 1) * CHANNEL, at - first_of[W - 1], lo, hi);
       }
@@ -2144,9 +2155,11 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
   // `ahead` steps further on the same registers are loaded again
   auto step = [&](uint32_t t, Chunk (&q)[GS], uint32_t ahead) {
 #pragma unroll
-    for (int h = 0; h < GS; h++) {
-      scatter(t * GS + h, q[h]);
-      if (t + ahead < end) load((t + ahead) * GS + h, q[h]);
+    for (int h = 0; h < GS; h++) scatter(t * GS + h, q[h]);
+    // after the last of the step's registers is read: a wait between two chunks would be one for the loads issued in between
+    if (t + ahead < end) {
+#pragma unroll
+      for (int h = 0; h < GS; h++) load((t + ahead) * GS + h, q[h]);
     }
     __syncthreads();
     uint32_t j[OWN];
