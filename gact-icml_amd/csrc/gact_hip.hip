@@ -319,10 +319,20 @@ template <> struct Elem<float> {
     lo_out = lo;
     hi_out = hi;
   }
-  // min and max of the whole group, in every lane of the row
-  __device__ static __forceinline__ void group_minmax(const Store& st, float& lo_out, float& hi_out) {
-    lane_minmax<0, kQChunks>(st, lo_out, hi_out);
-    row_all_minmax(lo_out, hi_out);
+  // the same, NaN apart: nan says that the lane's elements have to go through lane_minmax instead (see Elem<f16>)
+  template <int K0, int K1>
+  __device__ static __forceinline__ void lane_ordered(const Store& st, float& lo_out, float& hi_out, bool&) { lane_minmax<K0, K1>(st, lo_out, hi_out); }
+  // min and max of the first `there` of G whole groups, in every lane of the row; of the others 0
+  template <int G, bool ORDERED = true>
+  __device__ static __forceinline__ void groups_minmax(const Store* st, float* lo_out, float* hi_out, int64_t there = G) {
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      lo_out[g] = hi_out[g] = 0.0f;
+      if (g < there) {
+        lane_minmax<0, kQChunks>(st[g], lo_out[g], hi_out[g]);
+        row_all_minmax(lo_out[g], hi_out[g]);
+      }
+    }
   }
   __device__ static __forceinline__ void store_codes(uint8_t* p, const uint32_t (&b)[4]) {
     // the reference accumulates in a uint8_t: keep the low 8 bits of every byte
@@ -457,10 +467,50 @@ template <> struct Elem<f16> {
     lo_out = lo;
     hi_out = hi;
   }
-  // min and max of the whole group, in every lane of the row
-  __device__ static __forceinline__ void group_minmax(const Store& st, f16& lo_out, f16& hi_out) {
-    lane_minmax<0, kQChunks>(st, lo_out, hi_out);
-    row_all_minmax(lo_out, hi_out);
+  // The same from the packed three-operand minimum and maximum, half the instructions.  These hand a NaN on where the others ignore it, so
+  // a lane that holds one ends up with NaN, which the callers look for: they then take lane_minmax.  Anything else comes out bit
+  // for bit alike (subnormals, infinities, zeros of either sign: -0 below +0).
+  template <int K0, int K1>
+  __device__ static __forceinline__ void lane_ordered(const Store& st, f16& lo_out, f16& hi_out, bool& nan) {
+    f16x2 l, h;
+    ordered8<K1 - K0 == 2>(st.v[K0], st.v[K1 - 1], l, h);
+    lo_out = l[0];
+    hi_out = h[0];
+    nan |= lo_out != lo_out;
+  }
+  // Over eight or (BOTH) sixteen elements in pairs; the low half of l and h holds the result.  The last but one step takes the last
+  // pair and the two halves of what came before, the last one its own halves.
+  template <bool BOTH, typename V>
+  __device__ static __forceinline__ void ordered8(const V (&a)[4], const V (&b)[4], f16x2& l, f16x2& h) {
+    if constexpr (BOTH)
+      asm("v_pk_minimum3_f16 %0, %2, %3, %4\n\tv_pk_maximum3_f16 %1, %2, %3, %4\n\t"
+          "v_pk_minimum3_f16 %0, %0, %5, %6\n\tv_pk_maximum3_f16 %1, %1, %5, %6\n\t"
+          "v_pk_minimum3_f16 %0, %0, %7, %8\n\tv_pk_maximum3_f16 %1, %1, %7, %8\n\t"
+          "v_pk_minimum3_f16 %0, %0, %9, %0 op_sel:[0,0,1] op_sel_hi:[1,1,0]\n\tv_pk_maximum3_f16 %1, %1, %9, %1 op_sel:[0,0,1] op_sel_hi:[1,1,0]\n\t"
+          "v_pk_minimum3_f16 %0, %0, %0, %0 op_sel:[0,1,1] op_sel_hi:[1,0,0]\n\tv_pk_maximum3_f16 %1, %1, %1, %1 op_sel:[0,1,1] op_sel_hi:[1,0,0]"
+          : "=&v"(l), "=&v"(h) : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]));
+    else
+      asm("v_pk_minimum3_f16 %0, %2, %3, %4\n\tv_pk_maximum3_f16 %1, %2, %3, %4\n\t"
+          "v_pk_minimum3_f16 %0, %0, %5, %0 op_sel:[0,0,1] op_sel_hi:[1,1,0]\n\tv_pk_maximum3_f16 %1, %1, %5, %1 op_sel:[0,0,1] op_sel_hi:[1,1,0]\n\t"
+          "v_pk_minimum3_f16 %0, %0, %0, %0 op_sel:[0,1,1] op_sel_hi:[1,0,0]\n\tv_pk_maximum3_f16 %1, %1, %1, %1 op_sel:[0,1,1] op_sel_hi:[1,0,0]"
+          : "=&v"(l), "=&v"(h) : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]));
+  }
+  // min and max of the first `there` of G whole groups, in every lane of the row; of the others 0
+  template <int G, bool ORDERED = true>
+  __device__ static __forceinline__ void groups_minmax(const Store* st, f16* lo_out, f16* hi_out, int64_t there = G) {
+    bool nan = false;
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      lo_out[g] = hi_out[g] = (f16)0.0f;
+      if (g < there) lane_ordered<0, kQChunks>(st[g], lo_out[g], hi_out[g], nan);
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(nan) != 0, 0)) {
+#pragma unroll
+      for (int g = 0; g < G; g++)
+        if (g < there) lane_minmax<0, kQChunks>(st[g], lo_out[g], hi_out[g]);
+    }
+#pragma unroll
+    for (int g = 0; g < G; g++) row_all_minmax(lo_out[g], hi_out[g]);   // a group is there for the whole row or for none of it
   }
   // range is a half operation; the quotient is a double narrowed to float and then to half
   __device__ static __forceinline__ f16 make_scale(f16 lo, f16 hi, int qmax) {
@@ -638,18 +688,53 @@ template <> struct Elem<bf16> {
     if (e & 1) st.w[k][e >> 1] |= h << 16;   // the callers set a chunk's elements in order: the even one starts the pair
     else st.w[k][e >> 1] = h;
   }
-  __device__ static __forceinline__ void group_minmax(const Store& st, float& lo_out, float& hi_out) {
-    float lo = Elem<float>::init_lo(), hi = Elem<float>::init_hi();
+  // Min and max of the first `there` of G whole groups, in every lane of the row, of the others 0.
+  // ORDERED: two bfloat16 of magnitude up to 2^121 (bits 0x7c00) are ordered as the halves with their bits are, so they take half's packed
+  // instructions, a quarter of what widening every element takes; a larger one, an infinity or a NaN is a half NaN, and then
+  // every element of the wave is widened.  The float path's start values bound the results either way.
+  template <int G, bool ORDERED = true>
+  __device__ static __forceinline__ void groups_minmax(const Store* st, float* lo_out, float* hi_out, int64_t there = G) {
+    f16 lo16[G], hi16[G];
+    bool nan = !ORDERED;
+    if constexpr (ORDERED) {
 #pragma unroll
-    for (int k = 0; k < kQChunks; k++)
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        lo = __builtin_fminf(lo, widen(st, k, e));
-        hi = __builtin_fmaxf(hi, widen(st, k, e));
+      for (int g = 0; g < G; g++) {
+        lo16[g] = hi16[g] = (f16)0.0f;
+        if (g < there) {
+          f16x2 l, h;
+          Elem<f16>::template ordered8<true>(st[g].w[0], st[g].w[1], l, h);
+          lo16[g] = l[0];
+          hi16[g] = h[0];
+          nan |= lo16[g] != lo16[g];
+        }
       }
-    row_all_minmax(lo, hi);
-    lo_out = lo;
-    hi_out = hi;
+    }
+    if (!ORDERED || __builtin_expect(__builtin_amdgcn_ballot_w64(nan) != 0, 0)) {
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        lo_out[g] = hi_out[g] = 0.0f;
+        if (g < there) {
+          float lo = Elem<float>::init_lo(), hi = Elem<float>::init_hi();
+#pragma unroll
+          for (int k = 0; k < kQChunks; k++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+              lo = __builtin_fminf(lo, widen(st[g], k, e));
+              hi = __builtin_fmaxf(hi, widen(st[g], k, e));
+            }
+          row_all_minmax(lo, hi);
+          lo_out[g] = lo;
+          hi_out[g] = hi;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        row_all_minmax(lo16[g], hi16[g]);
+        lo_out[g] = __builtin_fminf(Elem<float>::init_lo(), __builtin_bit_cast(float, (uint32_t)__builtin_bit_cast(uint16_t, lo16[g]) << 16));
+        hi_out[g] = __builtin_fmaxf(Elem<float>::init_hi(), __builtin_bit_cast(float, (uint32_t)__builtin_bit_cast(uint16_t, hi16[g]) << 16));
+      }
+    }
   }
   __device__ static __forceinline__ float make_scale(float lo, float hi, int qmax) {
     return Elem<float>::make_scale(lo, hi, qmax);
@@ -893,7 +978,7 @@ __device__ __forceinline__ void chunk_words(const typename Elem<T>::Store& st, i
 //   GIVEN = true : min/max are read from mn_io / mx_io (the pack entry point's contract).
 // Codes follow quantization_cuda_kernel.cu:38-71; see Elem<T>::code1 for the arithmetic.
 // ------------------------------------------------------------------------------------------------
-template <typename T, int BITS, int NOISE, bool GIVEN, int SGR = 1, int STAGE = 0, bool LAZY = false, bool PACKS = true, typename SRC>
+template <typename T, int BITS, int NOISE, bool GIVEN, int SGR = 1, int STAGE = 0, bool LAZY = false, bool PACKS = true, bool ORDERED = true, typename SRC>
 __device__ __forceinline__ void quantize_supergroup(const SRC& src, int64_t N, int64_t sg0,
                                                     int i, uint8_t* __restrict__ packed,
                                                     typename Elem<T>::Stat* __restrict__ scale_out,
@@ -943,11 +1028,7 @@ __device__ __forceinline__ void quantize_supergroup(const SRC& src, int64_t N, i
           for (int k = 0; k < CH; k++) Elem<T>::load_chunk(x + (n0 + g0 + j) * GROUP + chunk_col<T>(k, i), v[g0 + j], k);
       }
       Stat lo_s[ST], hi_s[ST], sc_s[ST];
-#pragma unroll
-      for (int j = 0; j < ST; j++) {
-        lo_s[j] = hi_s[j] = (Stat)0.0f;
-        Elem<T>::group_minmax(v[g0 + j], lo_s[j], hi_s[j]);
-      }
+      Elem<T>::template groups_minmax<ST, ORDERED>(v + g0, lo_s, hi_s);
       {
         const int mine = i & (ST - 1);
         Stat lo_m = lo_s[0], hi_m = hi_s[0];
@@ -1061,19 +1142,18 @@ __device__ __forceinline__ void quantize_supergroup(const SRC& src, int64_t N, i
   for (int g = 0; g < GPR; g++) {
     if (n0 + g < N) src.load(n0 + g, i, v[g]);
   }
+  if constexpr (GIVEN) {
 #pragma unroll
-  for (int g = 0; g < GPR; g++) {
-    const int64_t n = n0 + g;
-    lo_t[g] = (Stat)0.0f;
-    hi_t[g] = (Stat)0.0f;
-    if (n < N) {
-      if (GIVEN) {
+    for (int g = 0; g < GPR; g++) {
+      const int64_t n = n0 + g;
+      lo_t[g] = hi_t[g] = (Stat)0.0f;
+      if (n < N) {
         lo_t[g] = Elem<T>::stat_of(mn_io[n]);
         hi_t[g] = Elem<T>::stat_of(mx_io[n]);
-      } else {
-        Elem<T>::group_minmax(v[g], lo_t[g], hi_t[g]);
       }
     }
+  } else {
+    Elem<T>::template groups_minmax<GPR, ORDERED>(v, lo_t, hi_t, N - n0);
   }
   // one scale division per lane: lane j of the row takes group j % GPR, then the row shares the results
   {
@@ -1556,7 +1636,7 @@ __device__ __forceinline__ void minimax_row(const T* __restrict__ x, int64_t N, 
   for (int g = 0; g < MINIMAX_ROW_GROUPS; g++) {
     if (n0 + g < N) {
       T lo, hi;
-      Elem<T>::group_minmax(v[g], lo, hi);
+      Elem<T>::template groups_minmax<1>(v + g, &lo, &hi);
       lo_m = i == g ? lo : lo_m;
       hi_m = i == g ? hi : hi_m;
     }
@@ -1702,7 +1782,11 @@ quantize_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_
   // chip for long and costs bandwidth on large ones (4 M elements 4.53 -> 4.35 us, 17 M 8.7 -> 8.4, 51 M and 72 M equal, 134 M 49.7 -> 51.3, 268 M 96 -> 100; a cap
   // by dynamic LDS at five or four waves gets half of that back)
   constexpr bool PACKS = SMALL || !(std::is_same<T, f16>::value && BITS == 2 && NOISE != GACT_NOISE_REF);
-  quantize_supergroup<T, BITS, NOISE, GIVEN, SGR, STAGE, LAZY, PACKS>(ContiguousSource<T>{x, numel}, N, sg0, threadIdx.x & 15, packed, scale_out, mn_io, mx_io,
+  // bfloat16 widens here: ordered minima leave registers for more waves than HBM bears (67 M elements 1 bit 26.7 -> 27.5 us, 2 bit 25.7 -> 26.9,
+  // 8 M 5.58 -> 5.67), where batches (three waves on a SIMD instead of two: 686 M 562 -> 548 us a round trip, 83 M 97.5 -> 95.5) and tensors that
+  // are not contiguous (heads [64,12,512,64] 4 bit 14.1 -> 13.8) gain
+  constexpr bool ORDERED = !std::is_same<T, bf16>::value;
+  quantize_supergroup<T, BITS, NOISE, GIVEN, SGR, STAGE, LAZY, PACKS, ORDERED>(ContiguousSource<T>{x, numel}, N, sg0, threadIdx.x & 15, packed, scale_out, mn_io, mx_io,
                                                   (uint32_t)seed, (uint32_t)(seed >> 32), noise);
 }
 
@@ -1746,11 +1830,8 @@ __device__ __forceinline__ void quantize_wave8(const SeedArg& seed_arg, const SR
   for (int g = 0; g < GR; g++)
     if (na + g < N) src.load(na + g, i, v[g]);
   Stat lo[GR], hi[GR], sc[GR];
-#pragma unroll
-  for (int g = 0; g < GR; g++) {
-    lo[g] = hi[g] = (Stat)0.0f;
-    if (na + g < N) Elem<T>::group_minmax(v[g], lo[g], hi[g]);
-  }
+  constexpr bool ORDERED = !(std::is_same<T, bf16>::value && SRC::kContiguous);   // see quantize_kernel
+  Elem<T>::template groups_minmax<GR, ORDERED>(v, lo, hi, N - na);
   {
     const int mine = i & (GR - 1);   // with two groups a row, odd lanes divide for the second
     const Stat lo_m = mine ? lo[GR - 1] : lo[0], hi_m = mine ? hi[GR - 1] : hi[0];
@@ -2179,14 +2260,12 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
     Stat lo[G], hi[G], sc[G];
 #pragma unroll
     for (int r = 0; r < G; r++) {
-      lo[r] = hi[r] = (Stat)0.0f;
       const uint32_t m = row * OWN + r / GS;
       const uint8_t* p = ring + (m / W) * PIECE + (m % W) * CHANNEL + (j[r / GS] & 1) * SLOT + (r % GS) * (GROUP * ES);
 #pragma unroll
       for (int k = 0; k < CH; k++) Elem<T>::load_chunk(reinterpret_cast<const T*>(p) + chunk_col<T>(k, i), st[r], k);
     }
-#pragma unroll
-    for (int r = 0; r < G; r++) Elem<T>::group_minmax(st[r], lo[r], hi[r]);
+    Elem<T>::template groups_minmax<G>(st, lo, hi);
     {
       // one division per lane: lane r of the row takes group r % G
       const int mine = i & (G - 1);
@@ -2350,29 +2429,36 @@ struct GroupsShape {
   static_assert(D == 64 || D == 128 || D == 512, "group sizes of the one-pass kernels");
 };
 
-template <typename T, int D, int BITS, int G>
-__device__ __forceinline__ void groups_lane_minmax(const typename Elem<T>::Store (&v)[2], T& lo, T& hi) {
+// of the lane's chunks of every group: ORDERED by lane_ordered, which may ask (nan) for the other way
+template <typename T, int D, int BITS, bool ORDERED, int G = 0>
+__device__ __forceinline__ void groups_lane_minmax(const typename Elem<T>::Store (&v)[2], T (&lo)[GroupsShape<T, D, BITS>::GL],
+                                                   T (&hi)[GroupsShape<T, D, BITS>::GL], bool& nan) {
   typedef GroupsShape<T, D, BITS> S;
-  constexpr int C0 = G * S::CPG, CH = S::CH;
-  if constexpr (S::CPG <= CH) {
-    Elem<T>::template lane_minmax<C0 % CH, C0 % CH + S::CPG>(v[C0 / CH], lo, hi);
-  } else {   // a group of 512: both halves
-    T lo2, hi2;
-    Elem<T>::template lane_minmax<0, CH>(v[0], lo, hi);
-    Elem<T>::template lane_minmax<0, CH>(v[1], lo2, hi2);
-    lo = lo2 < lo ? lo2 : lo;   // never NaN: the start values are not
-    hi = hi2 > hi ? hi2 : hi;
+  constexpr int C0 = G * S::CPG, CH = S::CH, CPG = S::CPG <= CH ? S::CPG : CH;
+  if constexpr (G < S::GL) {
+    if constexpr (ORDERED) Elem<T>::template lane_ordered<C0 % CH, C0 % CH + CPG>(v[C0 / CH], lo[G], hi[G], nan);
+    else Elem<T>::template lane_minmax<C0 % CH, C0 % CH + CPG>(v[C0 / CH], lo[G], hi[G]);
+    if constexpr (S::CPG > CH) {   // a group of 512: both halves
+      T lo2, hi2;
+      if constexpr (ORDERED) Elem<T>::template lane_ordered<0, CH>(v[1], lo2, hi2, nan);
+      else Elem<T>::template lane_minmax<0, CH>(v[1], lo2, hi2);
+      lo[G] = lo2 < lo[G] ? lo2 : lo[G];   // no NaN that lane_ordered has not told of; the other way's start values are none
+      hi[G] = hi2 > hi[G] ? hi2 : hi[G];
+    }
+    groups_lane_minmax<T, D, BITS, ORDERED, G + 1>(v, lo, hi, nan);
   }
 }
-template <typename T, int D, int BITS, int G = 0>
+template <typename T, int D, int BITS>
 __device__ __forceinline__ void groups_stats(const typename Elem<T>::Store (&v)[2], T (&lo)[GroupsShape<T, D, BITS>::GL],
                                              T (&hi)[GroupsShape<T, D, BITS>::GL]) {
   typedef GroupsShape<T, D, BITS> S;
-  if constexpr (G < S::GL) {
-    groups_lane_minmax<T, D, BITS, G>(v, lo[G], hi[G]);
-    if constexpr (S::HALF) half_row_all_minmax(lo[G], hi[G]);
-    else row_all_minmax(lo[G], hi[G]);
-    groups_stats<T, D, BITS, G + 1>(v, lo, hi);
+  bool nan = false;
+  groups_lane_minmax<T, D, BITS, true>(v, lo, hi, nan);
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(nan) != 0, 0)) groups_lane_minmax<T, D, BITS, false>(v, lo, hi, nan);
+#pragma unroll
+  for (int g = 0; g < S::GL; g++) {
+    if constexpr (S::HALF) half_row_all_minmax(lo[g], hi[g]);
+    else row_all_minmax(lo[g], hi[g]);
   }
 }
 template <typename T, int D, int BITS, int G = 0>
