@@ -3087,10 +3087,9 @@ __host__ __device__ inline float prec_key(float C, int b, int64_t w) {
 }
 __host__ __device__ inline bool prec_valid_bits(int b) { return b == 1 || b == 2 || b == 4 || b == 8 || b == 32; }
 
-#define PREC_MAX_L 4096      /* tensors the device kernel handles (LDS tables) */
-#define PREC_SORT_MAX_L 4096 /* tensors the sorting path handles (4 candidate steps each, 8 bytes per candidate) */
+#define PREC_MAX_L 4096      /* tensors the device kernel handles (LDS tables, 12 bits of a candidate's key) */
 #define PREC_THREADS 1024    /* largest workgroup the kernel is launched with */
-#define PREC_LDS_L 1024      /* tensors whose sizes the kernel keeps in LDS */
+#define PREC_BINS 256        /* bins of a histogram, four per lane of a wave */
 
 // The sequential restatement of the heap loop by one wave: each step is a 64-lane argmax.  Used when a
 // tensor's step keys do not decrease (never the case for the finite positive sensitivities the callers
@@ -3141,231 +3140,222 @@ __device__ __forceinline__ uint32_t sortable_key(float k) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-// The value of lane ^ J: within a row by DPP moves (a few cycles), across rows through the LDS crossbar
-template <int J>
-__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
-  if constexpr (J == 1) return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xB1, 0xf, 0xf, false);         // quad_perm [1,0,3,2]
-  else if constexpr (J == 2) return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x4E, 0xf, 0xf, false);    // quad_perm [2,3,0,1]
-  else if constexpr (J == 8) return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x128, 0xf, 0xf, false);   // row_ror:8
-  else if constexpr (J == 4) {   // four lanes up for the even quads (row_ror:12), four down for the odd ones (row_ror:4)
-    const int up = __builtin_amdgcn_update_dpp((int)v, (int)v, 0x12C, 0xf, 0xf, false);
-    return (uint32_t)__builtin_amdgcn_update_dpp(up, (int)v, 0x124, 0xf, 0xa, false);
-  } else {
-    return (uint32_t)__shfl_xor((int)v, J, 64);
-  }
+// Over the lanes of a wave by DPP moves (rows, then the last lane of a row into the next ones): a running sum, and the least or
+// greatest value, which ends up in the last lane.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t lane_before(uint32_t v, uint32_t none) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint64_t add_lane_before(uint64_t v) {
+  return v + (((uint64_t)lane_before<CTRL, ROWS>((uint32_t)(v >> 32), 0u) << 32) | lane_before<CTRL, ROWS>((uint32_t)v, 0u));
+}
+__device__ __forceinline__ uint64_t wave_running_sum(uint64_t v) {
+  v = add_lane_before<0x111, 0xf>(v);   // row_shr:1, 2, 4, 8
+  v = add_lane_before<0x112, 0xf>(v);
+  v = add_lane_before<0x114, 0xf>(v);
+  v = add_lane_before<0x118, 0xf>(v);
+  v = add_lane_before<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+  return add_lane_before<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
+}
+template <bool MOST>
+__device__ __forceinline__ uint32_t wave_extreme(uint32_t v) {
+  const auto pick = [](uint32_t a, uint32_t b) { return MOST ? (a > b ? a : b) : (a < b ? a : b); };
+  v = pick(v, lane_before<0x111, 0xf>(v, v));
+  v = pick(v, lane_before<0x112, 0xf>(v, v));
+  v = pick(v, lane_before<0x114, 0xf>(v, v));
+  v = pick(v, lane_before<0x118, 0xf>(v, v));
+  v = pick(v, lane_before<0x142, 0xa>(v, v));
+  v = pick(v, lane_before<0x143, 0xc>(v, v));
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ uint64_t read_lane(uint64_t v, int lane) {
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
 }
 
-// Bitonic sort of M = R * NT candidate slots, descending, by a workgroup of NT threads (M and NT powers of two,
-// NT >= 64).  Thread t keeps slots t, NT + t, ... in registers: partners NT or more apart are its own registers,
-// partners less than a wave apart are reached by lane_xor, and only the passes in between go through LDS and
-// a barrier (512 slots by 512 threads: 6 of 45 passes).
-template <int R, int JR>
-__device__ __forceinline__ void prec_exchange_own(uint64_t (&v)[R], int tid, int NT, int k) {
-#pragma unroll
-  for (int r = 0; r < R; r++) {
-    if ((r & JR) == 0 && (r | JR) < R) {
-      const bool descending = ((r * NT + tid) & k) == 0;
-      const uint64_t a = v[r], b = v[r | JR];
-      const uint64_t larger = a > b ? a : b, smaller = a > b ? b : a;
-      v[r] = descending ? larger : smaller;   // slot r is the lower one of the pair
-      v[r | JR] = descending ? smaller : larger;
-    }
-  }
-}
-// the lower slot of a pair keeps the larger key where the run descends, the smaller where it ascends
-template <int R>
-__device__ __forceinline__ void prec_keep(uint64_t (&v)[R], const uint64_t (&o)[R], int tid, int NT, int j, int k) {
-  const bool lower = (tid & j) == 0;
-#pragma unroll
-  for (int r = 0; r < R; r++) {
-    const bool descending = ((r * NT + tid) & k) == 0;
-    const uint64_t larger = v[r] > o[r] ? v[r] : o[r], smaller = v[r] > o[r] ? o[r] : v[r];
-    v[r] = (descending == lower) ? larger : smaller;
-  }
-}
-template <int R, int J>
-__device__ __forceinline__ void prec_exchange_lanes(uint64_t (&v)[R], int tid, int NT, int k) {
-  if (J >= k) return;   // not a pass of this run length
-  uint64_t o[R];
-#pragma unroll
-  for (int r = 0; r < R; r++) o[r] = ((uint64_t)lane_xor<J>((uint32_t)(v[r] >> 32)) << 32) | lane_xor<J>((uint32_t)v[r]);
-  prec_keep<R>(v, o, tid, NT, J, k);
-}
-template <int R>
-__device__ __forceinline__ void prec_sort_slots(uint64_t* cand, int tid, int NT, int M) {
-  uint64_t v[R];
-#pragma unroll
-  for (int r = 0; r < R; r++) v[r] = r * NT + tid < M ? cand[r * NT + tid] : 0;   // fewer slots than a wave has lanes: the others idle
-  for (int k = 2; k <= M; k <<= 1) {
-    for (int j = k >> 1; j >= 64; j >>= 1) {
-      if (j >= NT) {
-        switch (j / NT) {
-          case 1: prec_exchange_own<R, 1>(v, tid, NT, k); break;
-          case 2: prec_exchange_own<R, 2>(v, tid, NT, k); break;
-          case 4: prec_exchange_own<R, 4>(v, tid, NT, k); break;
-          default: prec_exchange_own<R, 8>(v, tid, NT, k); break;
-        }
-        continue;
-      }
-      uint64_t o[R];
-#pragma unroll
-      for (int r = 0; r < R; r++) cand[r * NT + tid] = v[r];
-      __syncthreads();
-#pragma unroll
-      for (int r = 0; r < R; r++) o[r] = cand[(r * NT + tid) ^ j];
-      __syncthreads();
-      prec_keep<R>(v, o, tid, NT, j, k);
-    }
-    prec_exchange_lanes<R, 32>(v, tid, NT, k);
-    prec_exchange_lanes<R, 16>(v, tid, NT, k);
-    prec_exchange_lanes<R, 8>(v, tid, NT, k);
-    prec_exchange_lanes<R, 4>(v, tid, NT, k);
-    prec_exchange_lanes<R, 2>(v, tid, NT, k);
-    prec_exchange_lanes<R, 1>(v, tid, NT, k);
-  }
-#pragma unroll
-  for (int r = 0; r < R; r++)
-    if (r * NT + tid < M) cand[r * NT + tid] = v[r];
-  __syncthreads();
-}
-// A candidate's low word: index, earlier steps above later ones, and the width the step ends at (its logarithm), which
-// orders nothing: index and step are unique.
-__device__ __forceinline__ uint32_t prec_candidate(int idx, int step, int to) {
-  return ((uint32_t)idx << 4) | ((uint32_t)(3 - step) << 2) | (to == 8 ? 3u : to == 4 ? 2u : to == 2 ? 1u : 0u);
-}
-__device__ __forceinline__ int prec_index(uint64_t c) { return (int)((uint32_t)c >> 4); }
-__device__ __forceinline__ int prec_to(uint64_t c) { return 1 << ((uint32_t)c & 3u); }
-__device__ __forceinline__ int64_t prec_saving(uint64_t c, int64_t w) {
-  const int to = prec_to(c);
-  return w * (int64_t)(to == 8 ? 24 : to);   // 32 -> 8, or halved
+// Widths by level: 1, 2, 4, 8, 32.  The step down from a level and its key, prec_key with the widths' constants worked out beforehand.
+__device__ __forceinline__ int prec_level(int bits) { return bits == 32 ? 4 : bits == 8 ? 3 : bits == 4 ? 2 : bits == 2 ? 1 : 0; }
+__device__ __forceinline__ int prec_width(int level) { return level == 4 ? 32 : 1 << level; }
+__device__ __forceinline__ float prec_level_key(float C, int level, int64_t saving) {
+  double obj;
+  if (level == 4) obj = -(double)C / 65025;
+  else obj = C * (level == 3 ? 1.0 / 65025 - 1.0 / 225 : level == 2 ? 1.0 / 225 - 1.0 / 9 : 1.0 / 9 - 1.0 / 1);
+  return (float)(obj / (double)saving);
 }
 
 // The greedy pops candidates (tensor i, step s) in descending (key, i) order.  A tensor's steps have
-// strictly decreasing keys, so that order is the descending sort of ALL candidate steps by
-// (key, index, earlier step first); the loop `while (b_sum > target) pop` then takes a prefix of it.
-// One workgroup, one thread per candidate slot up to 1024: build up to 4 candidates per tensor, bitonic-sort them,
-// prefix-sum the savings (integers, exact in double), apply the prefix.  Falls back to the sequential
-// loop when that order argument does not hold.
-// Bound by its chain of latencies, one workgroup that waits for loads, lane exchanges and barriers: a thread asks for a tensor's three
-// values at once, the sizes (up to PREC_LDS_L tensors) stay in LDS for the savings, which need nothing else - a candidate says what
-// width its step ends at - and the exchanges within a row are DPP moves.
+// strictly decreasing keys, so that order is the descending order of ALL candidate steps by
+// (key, index, earlier step first); the loop `while (b_sum > target) pop` then takes the candidates down to the one whose saving
+// brings the sum to the target.  One workgroup, a thread per candidate (four a tensor, R a thread beyond 1024), looks for that one: the
+// candidates' savings go into a histogram over the range of the keys left, a running sum over its bins from the top says in which bin the
+// target is met, and that bin is the next range, until it holds one candidate (two or three histograms; six at most, the
+// keys have 48 bits).  Then every candidate with a key not below that one's is taken.  Savings are integers: their
+// sums are exact in any order.  Falls back to the sequential loop where the order argument does not hold.
+// Bound by its chain of latencies - the loads, a double division, and per histogram the additions in LDS, a barrier and a scan that every
+// wave does for itself.  Sorting all candidates (bitonic, slots in registers) and summing along the sorted order took, in graph replay, us, that /
+// this: 3 tensors 5.6 / 2.7, 24 7.0 / 3.3, 69 9.3 / 3.8, 120 9.4 / 3.7, 160 13.4 / 4.5, 300 21.3 / 7.5, 1000 39.7 / 8.8, 4000 176 / 31.
+template <int R>
 __global__ void __launch_bounds__(PREC_THREADS)
 calc_precision_kernel(int32_t* __restrict__ b, const float* __restrict__ C, const int64_t* __restrict__ w,
                       int L, double target, int32_t* __restrict__ status) {
-  // dynamic LDS: one 8-byte slot per candidate, 4 per tensor rounded up to a power of two (128 KB for 4096
-  // tensors); the sequential path reuses it for its float keys
-  extern __shared__ uint64_t cand[];
-  __shared__ int32_t b_s[PREC_MAX_L];
-  __shared__ double part_s[PREC_THREADS / 64];
-  __shared__ int flag_s;
-  const int tid = threadIdx.x, NT = blockDim.x;
-  const bool sortable = L <= PREC_SORT_MAX_L;
-  int M = 4;
-  while (M < 4 * L) M <<= 1;
-  int64_t* const w_s = L <= PREC_LDS_L ? reinterpret_cast<int64_t*>(cand + M) : nullptr;   // behind the candidates
-  if (tid == 0) flag_s = 0;
-  if (sortable)
-    for (int t = tid; t < M; t += NT) cand[t] = 0;  // 0 sorts after every real candidate
-  __syncthreads();
-
-  double part = 0.0;
-  bool bad_order = false, bad_width = false;
-  for (int idx = tid; idx < L; idx += NT) {
-    const int bi = b[idx];
-    const int64_t wi = w[idx];
-    const float Ci = C[idx];
-    b_s[idx] = bi;
-    if (w_s) w_s[idx] = wi;
-    if (!prec_valid_bits(bi)) {
-      bad_width = true;
-    } else if (bi > 1) {
-      part += (double)((int64_t)bi * wi);
-      if (sortable) {
-        float prev = __builtin_inff();
-        int cur = bi, st = 0;
-        while (cur > 1 && st < 4) {
-          const int to = prec_next_bits(cur);
-          const float k = prec_key(Ci, cur, wi);
-          if (!(k < prev) && !(k == prev && k == 0.0f)) bad_order = true;  // also catches NaN
-          cand[idx * 4 + st] = ((uint64_t)sortable_key(k) << 32) | prec_candidate(idx, st, to);
-          prev = k;
-          cur = to;
-          st++;
-        }
-        if (cur > 1) bad_order = true;  // a width the 4-step descent does not know
-      }
+  constexpr int WAVES = PREC_THREADS / 64;
+  __shared__ __align__(16) uint64_t sum_s[3][PREC_BINS];
+  __shared__ __align__(16) uint32_t count_s[3][PREC_BINS];
+  __shared__ int64_t total_s[WAVES];
+  __shared__ uint32_t least_s[WAVES], most_s[WAVES], flag_s[WAVES];   // flags: 1 not in order, 2 a width that is none
+  __shared__ int32_t b_s[PREC_MAX_L];   // the sequential path's
+  __shared__ float key_s[PREC_MAX_L];
+  const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wave = tid >> 6, waves = NT >> 6;
+  const auto clear = [&](int h) {
+    for (int bin = tid; bin < PREC_BINS; bin += NT) {
+      sum_s[h][bin] = 0;
+      count_s[h][bin] = 0;
     }
-  }
-  // every term is an integer; the sum is exact (and order-free) below 2^53
+  };
+
+  uint64_t key[R];      // float key (ordered), index, earlier steps above later ones; 0: no candidate
+  int64_t saving[R];
+  int level[R];         // of the tensor's width
+  int64_t total = 0;    // bits of all tensors that can take a step
+  uint32_t least = 0xffffffffu, most = 0u;
+  bool bad_order = false, bad_width = false;
+  int32_t given[R];
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
-  if ((tid & 63) == 0) part_s[tid >> 6] = part;   // at most 16 waves
-  if (bad_order) flag_s = 1;
+  for (int r = 0; r < R; r++) {
+    const int slot = r * NT + tid, idx = slot >> 2;
+    given[r] = idx < L ? b[idx] : 1;
+    saving[r] = idx < L ? w[idx] : 1;
+  }
+  float Ci[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int idx = (r * NT + tid) >> 2;
+    Ci[r] = idx < L ? C[idx] : 0.0f;
+  }
+  clear(0);
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int slot = r * NT + tid, idx = slot >> 2, st = slot & 3;
+    const int64_t wi = saving[r];
+    bad_width |= !prec_valid_bits(given[r]);
+    level[r] = prec_level(given[r]);
+    const int from = level[r] - st;
+    const bool step = from > 0;
+    if (level[r] > 0 && st == 0) total += (int64_t)given[r] * wi;
+    saving[r] = wi * (int64_t)(prec_width(step ? from : 1) - prec_width(step ? from - 1 : 0));
+    const float k = prec_level_key(Ci[r], step ? from : 1, saving[r]);
+    const float before = __builtin_bit_cast(float, lane_before<0x90, 0xf>(__builtin_bit_cast(uint32_t, k), 0u));   // quad_perm [0,0,1,2]
+    const float prev = st == 0 ? __builtin_inff() : before;
+    const uint32_t order = sortable_key(k);
+    if (step) {
+      // keys that do not decrease (NaN among them), or a size that is no size
+      if ((!(k < prev) && !(k == prev && k == 0.0f)) || wi <= 0) bad_order = true;
+      least = order < least ? order : least;
+      most = order > most ? order : most;
+    }
+    key[r] = step ? ((uint64_t)order << 16) | ((uint32_t)idx << 4) | (uint32_t)(3 - st) : 0;
+  }
+  total = (int64_t)read_lane(wave_running_sum((uint64_t)total), 63);
+  least = wave_extreme<false>(least);
+  most = wave_extreme<true>(most);
+  const uint32_t flags = (__builtin_amdgcn_ballot_w64(bad_order) != 0 ? 1u : 0u) | (__builtin_amdgcn_ballot_w64(bad_width) != 0 ? 2u : 0u);
+  if (lane == 0) {
+    total_s[wave] = total;
+    least_s[wave] = least;
+    most_s[wave] = most;
+    flag_s[wave] = flags;
+  }
   __syncthreads();
-  if (bad_width) flag_s = 3;
-  __syncthreads();
-  if (flag_s == 3) {  // a width outside {1,2,4,8,32}: leave b as it is
+  int64_t b_sum = 0;
+  uint32_t flag = 0;
+  for (int v = 0; v < waves; v++) {
+    b_sum += total_s[v];
+    least = least_s[v] < least ? least_s[v] : least;
+    most = most_s[v] > most ? most_s[v] : most;
+    flag |= flag_s[v];
+  }
+  if (flag & 2) {  // a width outside {1,2,4,8,32}: leave b as it is
     if (status && tid == 0) *status = GACT_EINVAL;
     return;
   }
-  double b_sum0 = 0.0;
-  for (int wv = 0; wv < (NT + 63) >> 6; wv++) b_sum0 += part_s[wv];
-  const bool sequential = !sortable || flag_s != 0;
-  __syncthreads();
-
   int rc = 0;
-  if (sequential) {
-    if (tid < 64) calc_precision_sequential(b_s, reinterpret_cast<float*>(cand), C, w, L, b_sum0, target, &rc);
-  } else {
-    // bitonic sort, descending
-    switch (M / NT) {
-      case 0:
-      case 1: prec_sort_slots<1>(cand, tid, NT, M); break;
-      case 2: prec_sort_slots<2>(cand, tid, NT, M); break;
-      case 4: prec_sort_slots<4>(cand, tid, NT, M); break;
-      case 8: prec_sort_slots<8>(cand, tid, NT, M); break;
-      default: prec_sort_slots<16>(cand, tid, NT, M); break;
-    }
-    // savings of the sorted candidates, chunked over the threads
-    const int per = M / NT > 0 ? M / NT : 1;
-    const int lo = tid * per, hi = lo + per < M ? lo + per : M;
-    double mine = 0.0;
-    for (int t = lo; t < hi && t < M; t++) {
-      const uint64_t c = cand[t];
-      if (c == 0) break;
-      mine += (double)prec_saving(c, w_s ? w_s[prec_index(c)] : w[prec_index(c)]);
-    }
-    // exclusive prefix of the threads' savings: a scan inside every wave, then the waves' totals (the terms are
-    // integers below 2^53, so the sums are exact in any order)
-    if (lo >= M) mine = 0.0;
-    double incl = mine;
+  if (flag) {
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const double up = __shfl_up(incl, off, 64);
-      if ((tid & 63) >= off) incl += up;
-    }
-    if ((tid & 63) == 63) part_s[tid >> 6] = incl;   // at most 16 waves
-    __syncthreads();
-    double before = 0.0, total = 0.0;
-    for (int wv = 0; wv < (NT + 63) >> 6; wv++) {
-      const double v = part_s[wv];
-      if (wv < (tid >> 6)) before += v;
-      total += v;
-    }
-    if (tid == 0 && b_sum0 - total > target) flag_s = 2;  // every step taken and still over budget
-    double running = b_sum0 - (before + incl - mine);
-    for (int t = lo; t < hi && t < M; t++) {
-      const uint64_t c = cand[t];
-      if (c == 0 || !(running > target)) break;
-      const int idx = prec_index(c);
-      atomicMin(&b_s[idx], prec_to(c));
-      running -= (double)prec_saving(c, w_s ? w_s[idx] : w[idx]);
+    for (int r = 0; r < R; r++) {
+      const int slot = r * NT + tid;
+      if ((slot & 3) == 0 && (slot >> 2) < L) b_s[slot >> 2] = given[r];
     }
     __syncthreads();
-    if (flag_s == 2) rc = GACT_EBUDGET;
+    if (tid < 64) calc_precision_sequential(b_s, key_s, C, w, L, (double)b_sum, target, &rc);
+    __syncthreads();
+    for (int idx = tid; idx < L; idx += NT) b[idx] = b_s[idx];
+    if (status && tid == 0) *status = rc;
+    return;
   }
-  __syncthreads();
-  for (int idx = tid; idx < L; idx += NT) b[idx] = b_s[idx];
+
+  uint64_t last = ~0ull;   // candidates from this key on are taken
+  if ((double)b_sum > target) {
+    uint64_t from = (uint64_t)least << 16, span = ((((uint64_t)most << 16) | 0xffffu) - from);   // the keys left: from .. from + span
+    if (most < least) span = 0;                                                                  // no candidate at all
+    int64_t left = b_sum;                                                                        // without what lies above the range
+    // three histograms in turn: the next one is cleared while this one fills, and two levels back everybody has passed a barrier since
+    for (int h = 0;; h = h == 2 ? 0 : h + 1) {
+      const int bits = 64 - __builtin_clzll(span | 1), shift = bits > 8 ? bits - 8 : 0;
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const uint64_t at = key[r] - from;
+        if (key[r] != 0 && at <= span) {
+          const uint32_t bin = (uint32_t)(at >> shift);
+          atomicAdd((unsigned long long*)&sum_s[h][bin], (unsigned long long)saving[r]);
+          atomicAdd(&count_s[h][bin], 1u);
+        }
+      }
+      clear(h == 2 ? 0 : h + 1);
+      __syncthreads();
+      // lane l: bins 255 - 4 l and the three below, the higher ones first
+      int64_t s4[4];
+      uint32_t c4[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        s4[j] = (int64_t)sum_s[h][PREC_BINS - 1 - 4 * lane - j];
+        c4[j] = count_s[h][PREC_BINS - 1 - 4 * lane - j];
+      }
+      const int64_t mine = s4[0] + s4[1] + s4[2] + s4[3];
+      const int64_t incl = (int64_t)wave_running_sum((uint64_t)mine);
+      const uint64_t meets = __builtin_amdgcn_ballot_w64(!((double)(left - incl) > target));
+      if (meets == 0) {   // every step taken and still over budget
+        last = 0;
+        rc = GACT_EBUDGET;
+        break;
+      }
+      const int where = __builtin_ctzll(meets);   // the first lane after whose bins the target is met
+      int64_t running = left - (incl - mine), above = running;
+      int bin = 0;
+      uint32_t count = 0;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        if ((double)running > target) {
+          bin = j;
+          above = running;
+          count = c4[j];
+        }
+        running -= s4[j];
+      }
+      left = (int64_t)read_lane((uint64_t)above, where);
+      from += (uint64_t)(PREC_BINS - 1 - 4 * where - __builtin_amdgcn_readlane(bin, where)) << shift;
+      span = (1ull << shift) - 1;
+      if (__builtin_amdgcn_readlane((int)count, where) <= 1) {
+        last = from;
+        break;
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int slot = r * NT + tid;
+    const uint64_t taken = __builtin_amdgcn_ballot_w64(key[r] != 0 && key[r] >= last);   // a tensor's: its first so many
+    if ((slot & 3) == 0 && (slot >> 2) < L) b[slot >> 2] = prec_width(level[r] - __builtin_popcount((uint32_t)(taken >> lane) & 15u));
+  }
   if (status && tid == 0) *status = rc;
 }
 
@@ -4475,19 +4465,14 @@ int gact_calc_precision_device(int32_t* b, const float* C, const int64_t* w, int
   if (L == 0) return GACT_OK;
   if (!b || !C || !w) return GACT_EINVAL;
   fresh_launch();
-  int64_t M = 4;
-  while (M < 4 * L) M <<= 1;
-  const size_t lds = (size_t)(M + (L <= PREC_LDS_L ? L : 0)) * sizeof(uint64_t);
-  if (lds > 48 * 1024 &&
-      hipFuncSetAttribute((const void*)calc_precision_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
-          hipSuccess)
-    return GACT_ELAUNCH;
-  // one thread per candidate slot up to the largest workgroup: the sort's passes are what the kernel spends its time
-  // on (250 tensors: 47.3 us with 64 threads, 17.3 with 256, 13.9 with 1024; 120 tensors: 21.4 with 64, 11.3 with 256, 9.7 with 512;
-  // 24 tensors: 8.3 with 64, 7.4 with 128)
-  const unsigned threads = (unsigned)(M < 64 ? 64 : M > PREC_THREADS ? PREC_THREADS : M);
-  hipLaunchKernelGGL(calc_precision_kernel, dim3(1), dim3(threads), lds, (hipStream_t)stream, b, C, w,
-                     (int)L, target, status);
+  // one thread per candidate up to the largest workgroup
+  const int64_t candidates = 4 * L;
+  const dim3 threads((unsigned)(candidates >= PREC_THREADS ? PREC_THREADS : (candidates + 63) / 64 * 64));
+  hipStream_t s = (hipStream_t)stream;
+  const int each = (int)((candidates + PREC_THREADS - 1) / PREC_THREADS);
+  if (each <= 1) hipLaunchKernelGGL((calc_precision_kernel<1>), dim3(1), threads, 0, s, b, C, w, (int)L, target, status);
+  else if (each <= 4) hipLaunchKernelGGL((calc_precision_kernel<4>), dim3(1), threads, 0, s, b, C, w, (int)L, target, status);
+  else hipLaunchKernelGGL((calc_precision_kernel<16>), dim3(1), threads, 0, s, b, C, w, (int)L, target, status);
   return launch_status();
 }
 
