@@ -3456,9 +3456,9 @@ __device__ __forceinline__ void batch_plan_sizes(const int32_t* __restrict__ bit
     const int64_t ok = (!bad_s && base <= capacity) ? 1 : 0;
     ws.hdr->need = base;
     ws.hdr->ok = ok;
-    if (verdict) {   // the same two words where the caller can see them
-      verdict[0] = base;
-      verdict[1] = ok;
+    if (verdict) {   // the same two words where the caller can see them: written through, for a host that looks at them before the kernel's end
+      __hip_atomic_store(verdict, base, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(verdict + 1, ok, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 #pragma unroll
     for (int k = 0; k < 4; k++) ws.hdr->tensors_at[k] = count_s[k];

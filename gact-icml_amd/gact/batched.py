@@ -28,7 +28,9 @@ class BatchedPacked:
     verdict that left for the host right behind the plan, so that it does not wait for the quantize kernels."""
 
     _arena_bytes = None     # of `packed` when the plan was made
-    _verdict = None     # (event behind the copy, the workspace's first two words in pinned memory); none in a pickled one
+    # the plan's verdict: of a native call what it waits by, else (event behind the copy, the workspace's first two words in
+    # pinned memory); none in a pickled one
+    _verdict = None
 
     def __init__(self, owner, packed, scale, mn, table, bits, workspace, shapes, dtypes, seeds, verdict=None):
         self.owner = owner
@@ -53,9 +55,12 @@ class BatchedPacked:
         """What ok() returns, as of the plan of the quantize call; waits for that plan and its copy only."""
         if self._verdict is None:
             return self.ok()
-        done, words = self._verdict
-        done.synchronize() if isinstance(done, torch.cuda.Event) else _abi.native().event_wait(done)
-        need, good = words.tolist()
+        if isinstance(self._verdict, tuple):
+            done, words = self._verdict
+            done.synchronize()
+            need, good = words.tolist()
+        else:
+            need, good = _abi.native().verdict_wait(self._verdict)
         return bool(good), need
 
     def require_ok(self, verdict=None):
@@ -220,9 +225,9 @@ class BatchedQuantizer:
             done = _abi.native().batch_quantize(self._entries, geometry, list(tensors), list(seeds), bits,
                                                 (self.total_blocks, self.total_groups, self.workspace_bytes, int(arena_bytes), mode, self.dtype_mask))
             if done is not None:
-                (packed, scale, mn, table, kept, ws, words), event = done
+                (packed, scale, mn, table, kept, ws), verdict = done
                 return BatchedPacked(self, packed, scale, mn, table, kept, ws, [t.shape for t in tensors],
-                                     list(self.dtypes), seeds, (event, words))
+                                     list(self.dtypes), seeds, verdict)
         with torch.cuda.device(self.device):
             table = self._table(tensors, seeds, wait=False)
             packed = torch.empty((int(arena_bytes),), dtype=torch.uint8, device=self.device)

@@ -164,7 +164,8 @@ int gact_batch_plan(gact_batch_entry* table, const int32_t* bits, int64_t L, int
 /* gact_batch_plan for up to GACT_BATCH_ARGS tensors whose addresses and seeds lie on the host (x[L], seeds[L]) and go to the GPU in the
  * launch's own arguments: writes all of `table` - `geometry`, a table in device memory of which x, seed and packed_offset are not
  * looked at, completed by them and by the offsets - and, where they are not null, a copy of the widths to `kept` and header words
- * [0] and [1] to `verdict` (two int64, device memory or pinned host memory, 8-byte aligned).  GACT_ELIMIT beyond GACT_BATCH_ARGS tensors. */
+ * [0] and [1] to `verdict` (two int64, device memory or pinned host memory, 8-byte aligned), each written through as soon as it is
+ * known: a host that has put -1 there before the call may look for the change.  GACT_ELIMIT beyond GACT_BATCH_ARGS tensors. */
 #define GACT_BATCH_ARGS 192
 int gact_batch_plan_args(const gact_batch_entry* geometry, const void* const* x, const uint64_t* seeds, gact_batch_entry* table,
                          const int32_t* bits, int32_t* kept, int64_t L, int64_t total_blocks, int64_t capacity, void* workspace,

@@ -1,0 +1,65 @@
+"""The verdict of a batch's plan, which the plan's kernel writes to the host: it is there while the stream still has later work, waits for
+earlier work, and may be dropped before the plan has run."""
+import pytest
+import torch
+
+from gact.batched import BatchedQuantizer
+from gact.cpp_extension import _abi
+
+pytestmark = pytest.mark.gpu
+
+LONG = 100_000_000      # cycles: 0.04 s at least
+
+
+@pytest.fixture
+def batch():
+    sizes = [70001, 256, 40000]
+    xs = [torch.randn(n, device="cuda") for n in sizes]
+    made = BatchedQuantizer(sizes, [torch.float32] * 3, "cuda")
+    made._on_gpu()
+    bits = torch.tensor([1, 2, 4], dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    return made, xs, bits
+
+
+def test_the_verdict_does_not_wait_for_later_work(batch):
+    made, xs, bits = batch
+    q = made.quantize(xs, bits, [1, 2, 3])
+    torch.cuda._sleep(LONG)
+    assert not isinstance(q._verdict, tuple)
+    planned = q._planned()
+    assert not torch.cuda.current_stream().query()
+    assert planned == q.ok() and planned[0]
+    void = made.quantize(xs, bits, [1, 2, 3], arena_bytes=256)
+    assert void._planned() == (False, planned[1])
+
+
+def test_the_verdict_waits_for_earlier_work(batch):
+    made, xs, bits = batch
+    side = torch.cuda.Stream()
+    for stream in (torch.cuda.current_stream(), side):
+        with torch.cuda.stream(stream):
+            torch.cuda._sleep(LONG)
+            q = made.quantize(xs, bits, [1, 2, 3])
+            assert not stream.query()
+            assert q._planned() == q.ok()
+
+
+def test_verdicts_dropped_before_the_plan_has_run(batch):
+    """Their words are not handed out again before: pinned memory taken meanwhile keeps its values."""
+    made, xs, bits = batch
+    torch.cuda._sleep(LONG)
+    for _ in range(50):
+        made.quantize(xs, bits, [1, 2, 3])
+    words = [torch.full((2,), -7, dtype=torch.int64).pin_memory() for _ in range(100)]
+    assert not torch.cuda.current_stream().query()
+    torch.cuda.synchronize()
+    assert all(w.tolist() == [-7, -7] for w in words)
+    q = made.quantize(xs, bits, [1, 2, 3])
+    assert q._planned() == q.ok()
+
+
+def test_what_is_no_verdict_is_refused():
+    for args in ((), (None,), (1, 2)):
+        with pytest.raises((TypeError, ValueError)):
+            _abi.native().verdict_wait(*args)
