@@ -3388,13 +3388,30 @@ __host__ __device__ inline BatchWorkspace batch_workspace(void* base) {
 }
 __device__ __forceinline__ int width_index(int bits) { return bits == 1 ? 0 : bits == 2 ? 1 : bits == 4 ? 2 : 3; }
 
-__device__ __forceinline__ int batch_find(const gact_batch_entry* __restrict__ table, int L, int64_t block) {
+template <typename FIRST>
+__device__ __forceinline__ int batch_find(const FIRST& first_block, int L, int64_t block) {
   int lo = 0, hi = L - 1;  // last entry with first_block <= block
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (table[mid].first_block <= block) lo = mid; else hi = mid - 1;
+    if (first_block(mid) <= block) lo = mid; else hi = mid - 1;
   }
   return lo;
+}
+// The plan's workgroups behind the first note the tensor of 256 blocks each.  The tensors' first blocks come into LDS at once (up to
+// PLAN_LDS_L of them): a search in memory is a chain of loads, one for every bit of L, and was what the plan's launch took longest for
+// (graph replay, a launch: 3 tensors 4.0 -> 2.6 us, 45 4.0 -> 2.55, 120 4.1 -> 2.7, 190 4.3 -> 2.9, whatever the number of blocks).
+#define PLAN_THREADS 256
+#define PLAN_LDS_L 2048
+__device__ __forceinline__ void batch_plan_blocks(const gact_batch_entry* __restrict__ table, int L, int64_t total_blocks, const BatchWorkspace& ws) {
+  __shared__ int32_t first_s[PLAN_LDS_L];   // a grid has fewer than 2^31 blocks
+  const int64_t g = (int64_t)(blockIdx.x - 1) * PLAN_THREADS + threadIdx.x;
+  if (L <= PLAN_LDS_L) {
+    for (int t = threadIdx.x; t < L; t += PLAN_THREADS) first_s[t] = (int32_t)table[t].first_block;
+    __syncthreads();
+    if (g < total_blocks) ws.block_tensor[g] = batch_find([&](int t) { return (int64_t)first_s[t]; }, L, g);
+  } else if (g < total_blocks) {
+    ws.block_tensor[g] = batch_find([&](int t) { return table[t].first_block; }, L, g);
+  }
 }
 
 // Bytes of the arena a tensor of N groups takes at a width, as the plan counts them
@@ -3406,9 +3423,8 @@ __device__ __forceinline__ int64_t batch_span(int width, int64_t N) {
 
 // What the plan's workgroup 0 does: thread t sizes tensors t, t + 256, ...; the running packed-arena offset is carried across rounds of
 // 256 with an inclusive scan of each wave and the waves' totals.  One round, with the loads of all tensors under way at once, where a
-// wave alone took two (65 to 128 tensors).  entry(t) gives a tensor's size and type, place(t, width, offset) takes what the plan
-// finds for it.
-#define PLAN_THREADS 256
+// wave alone took two (65 to 128 tensors).  entry(t) loads all that is needed of a tensor, place(t, entry, offset) takes that and what
+// the plan finds for it.
 template <typename ENTRY, typename PLACE>
 __device__ __forceinline__ void batch_plan_sizes(const int32_t* __restrict__ bits, int L, int64_t capacity, const BatchWorkspace& ws,
                                                  int64_t* __restrict__ verdict, const ENTRY& entry, const PLACE& place) {
@@ -3424,21 +3440,17 @@ __device__ __forceinline__ void batch_plan_sizes(const int32_t* __restrict__ bit
     const int t = t0 + threadIdx.x;
     int64_t bytes = 0;
     int width = 0;
+    gact_batch_entry e = {};
     if (t < L) {
       const int given = bits[t];
-      const gact_batch_entry e = entry(t);
+      e = entry(t);
       const bool valid = given == 1 || given == 2 || given == 4 || given == 8;
       width = valid ? given : 8;
       if (!valid || e.dtype < 0 || e.dtype > 2) bad_s = 1;
       atomicAdd(&count_s[width_index(width)], 1);
       bytes = batch_span(width, (e.numel + GROUP - 1) / GROUP);
     }
-    int64_t incl = bytes;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int64_t up = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += up;
-    }
+    const int64_t incl = (int64_t)wave_running_sum((uint64_t)bytes);
     if (lane == 63) total_s[wave] = incl;
     __syncthreads();
     int64_t before = 0, all = 0;
@@ -3447,7 +3459,7 @@ __device__ __forceinline__ void batch_plan_sizes(const int32_t* __restrict__ bit
       before += w < wave ? total_s[w] : 0;
       all += total_s[w];
     }
-    if (t < L) place(t, base + before + incl - bytes);
+    if (t < L) place(t, e, base + before + incl - bytes);
     base += all;
     __syncthreads();
   }
@@ -3472,12 +3484,11 @@ __global__ void __launch_bounds__(PLAN_THREADS)
 batch_plan_kernel(gact_batch_entry* table, const int32_t* __restrict__ bits, int L, int64_t total_blocks,
                   int64_t capacity, BatchWorkspace ws, int64_t* __restrict__ verdict) {
   if (blockIdx.x > 0) {
-    const int64_t g = (int64_t)(blockIdx.x - 1) * blockDim.x + threadIdx.x;
-    if (g < total_blocks) ws.block_tensor[g] = batch_find(table, L, g);
+    batch_plan_blocks(table, L, total_blocks, ws);
     return;
   }
   batch_plan_sizes(bits, L, capacity, ws, verdict, [&](int t) { return table[t]; },
-                   [&](int t, int64_t offset) { table[t].packed_offset = offset; });
+                   [&](int t, const gact_batch_entry&, int64_t offset) { table[t].packed_offset = offset; });
 }
 
 // The plan of a table that the launch itself brings: what changes from call to call - a tensor's address and its seed - arrives in the
@@ -3494,17 +3505,19 @@ batch_plan_args_kernel(BatchArgs args, const gact_batch_entry* __restrict__ geom
                        const int32_t* __restrict__ bits, int32_t* __restrict__ kept, int L, int64_t total_blocks, int64_t capacity,
                        BatchWorkspace ws, int64_t* __restrict__ verdict) {
   if (blockIdx.x > 0) {
-    const int64_t g = (int64_t)(blockIdx.x - 1) * blockDim.x + threadIdx.x;
-    if (g < total_blocks) ws.block_tensor[g] = batch_find(geometry, L, g);
+    batch_plan_blocks(geometry, L, total_blocks, ws);
     return;
   }
   if (kept)
     for (int t = threadIdx.x; t < L; t += PLAN_THREADS) kept[t] = bits[t];
-  batch_plan_sizes(bits, L, capacity, ws, verdict, [&](int t) { return geometry[t]; },
-                   [&](int t, int64_t offset) {
+  batch_plan_sizes(bits, L, capacity, ws, verdict,
+                   [&](int t) {
                      gact_batch_entry e = geometry[t];
                      e.x = args.x[t];
                      e.seed = args.seed[t];
+                     return e;
+                   },
+                   [&](int t, gact_batch_entry e, int64_t offset) {
                      e.packed_offset = offset;
                      table[t] = e;
                    });
