@@ -1783,8 +1783,8 @@ quantize_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_
   // by dynamic LDS at five or four waves gets half of that back)
   constexpr bool PACKS = SMALL || !(std::is_same<T, f16>::value && BITS == 2 && NOISE != GACT_NOISE_REF);
   // bfloat16 widens here: ordered minima leave registers for more waves than HBM bears (67 M elements 1 bit 26.7 -> 27.5 us, 2 bit 25.7 -> 26.9,
-  // 8 M 5.58 -> 5.67), where batches (three waves on a SIMD instead of two: 686 M 562 -> 548 us a round trip, 83 M 97.5 -> 95.5) and tensors that
-  // are not contiguous (heads [64,12,512,64] 4 bit 14.1 -> 13.8) gain
+  // 8 M 5.58 -> 5.67), where batches (three waves on a SIMD instead of two: 686 M 562 -> 548 us a round trip, 83 M 97.5 -> 95.5) and runs of
+  // pieces (heads [64,12,512,64] 4 bit 14.1 -> 13.9) gain
   constexpr bool ORDERED = !std::is_same<T, bf16>::value;
   quantize_supergroup<T, BITS, NOISE, GIVEN, SGR, STAGE, LAZY, PACKS, ORDERED>(ContiguousSource<T>{x, numel}, N, sg0, threadIdx.x & 15, packed, scale_out, mn_io, mx_io,
                                                   (uint32_t)seed, (uint32_t)(seed >> 32), noise);
@@ -2064,8 +2064,9 @@ quantize_transposed_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t nu
   const uint64_t seed = seed_arg.value();
   const TileSource<T> src{tile, E0 / GROUP};
   for (int sg = (int)(threadIdx.x >> 4); sg * WPT * GROUP < L; sg += TRANSPOSED_THREADS / 16)
-    quantize_supergroup<T, BITS, NOISE, false>(src, N, E0 / (WPT * GROUP) + sg, threadIdx.x & 15, packed, scale_out, mn_out, mx_out,
-                                               (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
+    // bfloat16 widens its minima: [16,96,64,64] 2 bit 11.7 us, ordered 12.0, [64,512,28,28] 21.4 and 21.7
+    quantize_supergroup<T, BITS, NOISE, false, 1, 0, false, true, !std::is_same<T, bf16>::value>(
+        src, N, E0 / (WPT * GROUP) + sg, threadIdx.x & 15, packed, scale_out, mn_out, mx_out, (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
 }
 
 // The same layout where channels are long (K pixels hold a super-group and more): a workgroup owns a strip of channels, 64 bytes
@@ -2230,6 +2231,12 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
     n_first[c] = (((int64_t)b * g.M + m0 + m) * K + first) / GROUP;
   }
   uint32_t bytes[OWN][4];   // the lane's 16 bytes of each channel's super-group, in the order of their addresses
+  // Scale and minimum stay in the row until its 16 lanes hold those of STATS steps (or the channel ends): a step's own are pieces of a
+  // few bytes, one for every channel, and each costs the memory system what a whole line does.  Lane G * k + r keeps group r of
+  // the step k of its turn.  Stored step by step / by turns, us: half [64,256,56,56] 1 bit 42.6 / 41.0, 2 bit 37.5 / 36.7, 4 and 8 bit
+  // equal, float 2 bit 67.5 / 66.1, 4 bit 64.0 / 62.9, [32,64,112,112] 1 bit 38.9 / 37.9; tensors of 2 M elements equal to 2 % slower.
+  constexpr uint32_t STATS = 16 / (OWN * GS);
+  Stat kept_scale = (Stat)0.0f, kept_lo = (Stat)0.0f;
 
   const uint32_t most = (K + UNIT - 1) / STEP + 1;   // no channel has anything left after so many steps
   const uint32_t end = j_end + UNIT / STEP < most ? j_end + UNIT / STEP : most;
@@ -2265,29 +2272,35 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
 #pragma unroll
       for (int k = 0; k < CH; k++) Elem<T>::load_chunk(reinterpret_cast<const T*>(p) + chunk_col<T>(k, i), st[r], k);
     }
-    Elem<T>::template groups_minmax<G>(st, lo, hi);
+    Elem<T>::template groups_minmax<G, !std::is_same<T, bf16>::value>(st, lo, hi);   // bfloat16: nothing in it (36.1 / 36.4)
     {
       // one division per lane: lane r of the row takes group r % G
       const int mine = i & (G - 1);
       Stat lo_m = lo[0], hi_m = hi[0];
-      int64_t n = n_first[0] + j[0] * GS;
-      bool mine_due = due[0];
 #pragma unroll
       for (int r = 1; r < G; r++) {
         lo_m = mine == r ? lo[r] : lo_m;
         hi_m = mine == r ? hi[r] : hi_m;
       }
-      if (OWN > 1 && mine >= GS) {
-        n = n_first[OWN - 1] + j[OWN - 1] * GS;
-        mine_due = due[OWN - 1];
-      }
-      n += mine % GS;
+      const bool second = OWN > 1 && mine >= GS;   // the group is one of the row's second channel
+      const uint32_t j_m = second ? j[OWN - 1] : j[0], last_m = second ? last[OWN - 1] : last[0];
+      const bool due_m = second ? due[OWN - 1] : due[0];
+      const int64_t n_m = (second ? n_first[OWN - 1] : n_first[0]) + mine % GS;
       const Stat s_m = Elem<T>::make_scale(lo_m, hi_m, QMAX);
-      if (i < G && mine_due && n < N) {
-        scale_out[n] = s_m;
-        mn_out[n] = Elem<T>::elem_of(lo_m);
-        if (mx_out) mx_out[n] = Elem<T>::elem_of(hi_m);
+      const uint32_t turn = (uint32_t)i / G;
+      if ((j_m & (STATS - 1)) == turn) {
+        kept_scale = s_m;
+        kept_lo = lo_m;
       }
+      if (due_m && ((j_m & (STATS - 1)) == STATS - 1 || j_m + 1 == last_m)) {
+        const uint32_t at = (j_m & ~(STATS - 1)) + turn;
+        const int64_t n = n_m + (int64_t)at * GS;
+        if (at <= j_m && at >= j_first && n < N) {
+          scale_out[n] = kept_scale;
+          mn_out[n] = Elem<T>::elem_of(kept_lo);
+        }
+      }
+      if (mx_out && i < G && due_m && n_m + (int64_t)j_m * GS < N) mx_out[n_m + (int64_t)j_m * GS] = Elem<T>::elem_of(hi_m);
       sc[0] = G == 1 ? s_m : row_bcast<0>(s_m);
       if (G > 1) sc[1 % G] = row_bcast<1>(s_m);
       if (G > 2) {
