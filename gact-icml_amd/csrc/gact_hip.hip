@@ -1783,8 +1783,8 @@ quantize_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_
   // by dynamic LDS at five or four waves gets half of that back)
   constexpr bool PACKS = SMALL || !(std::is_same<T, f16>::value && BITS == 2 && NOISE != GACT_NOISE_REF);
   // bfloat16 widens here: ordered minima leave registers for more waves than HBM bears (67 M elements 1 bit 26.7 -> 27.5 us, 2 bit 25.7 -> 26.9,
-  // 8 M 5.58 -> 5.67), where batches (three waves on a SIMD instead of two: 686 M 562 -> 548 us a round trip, 83 M 97.5 -> 95.5) and runs of
-  // pieces (heads [64,12,512,64] 4 bit 14.1 -> 13.9) gain
+  // 8 M 5.58 -> 5.67), where batches (three waves on a SIMD instead of two: 686 M 562 -> 548 us a round trip, 83 M 97.5 -> 95.5) and tensors
+  // that are not contiguous (heads [64,12,512,64] 4 bit 14.1 -> 13.9) gain
   constexpr bool ORDERED = !std::is_same<T, bf16>::value;
   quantize_supergroup<T, BITS, NOISE, GIVEN, SGR, STAGE, LAZY, PACKS, ORDERED>(ContiguousSource<T>{x, numel}, N, sg0, threadIdx.x & 15, packed, scale_out, mn_io, mx_io,
                                                   (uint32_t)seed, (uint32_t)(seed >> 32), noise);
@@ -2061,12 +2061,19 @@ quantize_transposed_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t nu
   for (uint32_t at = (uint32_t)L + threadIdx.x; at < (uint32_t)g.tile; at += TRANSPOSED_THREADS)   // the padding of the last group
     *reinterpret_cast<T*>(tile + tile_byte<T>(at)) = (T)0.0f;
   __syncthreads();
-  const uint64_t seed = seed_arg.value();
   const TileSource<T> src{tile, E0 / GROUP};
-  for (int sg = (int)(threadIdx.x >> 4); sg * WPT * GROUP < L; sg += TRANSPOSED_THREADS / 16)
-    // bfloat16 widens its minima: [16,96,64,64] 2 bit 11.7 us, ordered 12.0, [64,512,28,28] 21.4 and 21.7
-    quantize_supergroup<T, BITS, NOISE, false, 1, 0, false, true, !std::is_same<T, bf16>::value>(
-        src, N, E0 / (WPT * GROUP) + sg, threadIdx.x & 15, packed, scale_out, mn_out, mx_out, (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
+  if constexpr (BITS == 1) {
+    // A wave per super-group: a tile of 64 KB holds 8 (float) or 16 of them, fewer than the workgroup has rows.  A row per super-group / this,
+    // us: float [64,512,28,28] 50.2 / 33.7, [110,512,32,32] 98.5 / 58.5, [128,512,14,14] 28.2 / 18.8, [16,64,14,14] 6.7 / 4.7; half equal, and
+    // with tiles of 48 KB [256,512,14,14] 22.9 / 19.0.  2 bit: float equal to 5 % slower, half 10 % slower: rows.
+    for (int sg = (int)(threadIdx.x >> 6); sg * WPT * GROUP < L; sg += WAVES)
+      quantize_wave8<T, BITS, NOISE>(seed_arg, src, E0 / (WPT * GROUP) + sg, N, packed, scale_out, mn_out, mx_out, (const float*)nullptr);
+  } else {
+    const uint64_t seed = seed_arg.value();
+    for (int sg = (int)(threadIdx.x >> 4); sg * WPT * GROUP < L; sg += TRANSPOSED_THREADS / 16)
+      quantize_supergroup<T, BITS, NOISE, false>(
+          src, N, E0 / (WPT * GROUP) + sg, threadIdx.x & 15, packed, scale_out, mn_out, mx_out, (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
+  }
 }
 
 // The same layout where channels are long (K pixels hold a super-group and more): a workgroup owns a strip of channels, 64 bytes
