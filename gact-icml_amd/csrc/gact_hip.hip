@@ -2071,6 +2071,7 @@ quantize_transposed_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t nu
   } else {
     const uint64_t seed = seed_arg.value();
     for (int sg = (int)(threadIdx.x >> 4); sg * WPT * GROUP < L; sg += TRANSPOSED_THREADS / 16)
+      // bfloat16 with ordered minima, whose registers let three workgroups onto a CU: [256,512,14,14] 2 bit 24.3 -> 20.3 us, 4 bit 20.2 -> 19.4
       quantize_supergroup<T, BITS, NOISE, false>(
           src, N, E0 / (WPT * GROUP) + sg, threadIdx.x & 15, packed, scale_out, mn_out, mx_out, (uint32_t)seed, (uint32_t)(seed >> 32), nullptr);
   }
@@ -3972,12 +3973,20 @@ inline StripCut strip_cut(int bits, int64_t strips, int64_t K) {
     return c;
   }
 }
-// Elements of a workgroup's tile: 64 KB, two workgroups to a CU, where that leaves a tile 16 channels and more (half
-// [64,512,28,28] 4 bit 23 us against 28 with one of 144 KB), else one of up to 144 KB (half [64,256,56,56] 1 bit 54 against 64;
-// [2,256,56,56] 9 against 13); as many tiles as the workgroups that the GPU holds, or a multiple of that.
-inline int transposed_tile(size_t elem_size, int64_t numel, int64_t K) {
-  int64_t slots = 512, most = 65536 / (int64_t)elem_size;
-  if ((most < numel / slots ? most : numel / slots) < 16 * K) {
+// Elements of a workgroup's tile: 48 KB, three workgroups to a CU that load and quantize by turns, where that leaves a tile 28 channels
+// and more; 64 KB, two workgroups, where that leaves it 16 (half [64,512,28,28] 4 bit 23 us against 28 with one of 144 KB), else one of
+// up to 144 KB (half [64,256,56,56] 1 bit 54 against 64; [2,256,56,56] 9 against 13); as many tiles as the workgroups that the GPU
+// holds, or a multiple of that.  64 / 48 KB, us: half 4 bit [512,512,7,7] 15.0 / 13.6, [256,512,14,14] 22.4 / 19.0, [64,512,20,20]
+// 13.2 / 12.2, [64,512,28,28] (31 channels) 21.5 / 20.4, [64,256,32,32] (24) 14.5 / 16.6; float 4 bit [2000,256,7,7] 37.1 / 32.0,
+// [128,512,14,14] 18.8 / 17.1, [64,512,20,20] (30) 20.1 / 17.0, [64,512,28,28] (15) 33.9 / 37.9.  32 KB: 2 % ahead to 19 % behind 48.
+// Float at 2 bit has registers for two workgroups only (106): [2000,256,7,7] 38.0 / 39.2.
+inline int transposed_tile(size_t elem_size, int bits, int64_t numel, int64_t K) {
+  int64_t slots = 768, most = 49152 / (int64_t)elem_size;
+  if ((elem_size == 4 && bits == 2) || (most < numel / slots ? most : numel / slots) < 28 * K) {
+    slots = 512;
+    most = 65536 / (int64_t)elem_size;
+  }
+  if (slots == 512 && (most < numel / slots ? most : numel / slots) < 16 * K) {
     slots = 256;
     most = 147456 / (int64_t)elem_size;
   }
@@ -4072,7 +4081,7 @@ int dispatch_quantize_strided(int n, const int64_t (&size)[8], const int64_t (&s
     }
   } else if (stride[n - 2] == 1 && stride[n - 1] != 1 && n <= 3 && (n == 2 || stride[0] != 1) && size[n - 2] % W == 0 &&
              size[n - 1] < (1 << 24) && numel / size[n - 1] < 0x7fffffffLL) {
-    const int tile = transposed_tile(sizeof(T), numel, size[n - 1]);
+    const int tile = transposed_tile(sizeof(T), bits, numel, size[n - 1]);
     const bool tiles = tiles_pay(sizeof(T), bits, numel, size[n - 2], size[n - 1], tile);
     // channels of one piece leave three quarters of a strip's lanes without work: half [1091,8,3844] 4 bit strips 77, copy 68 us,
     // [1551,8,2704] 2 bit 90, 63, where tiles (as odd numbers of pixels take) need half of the copy's time
