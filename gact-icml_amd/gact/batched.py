@@ -25,7 +25,7 @@ class BatchedPacked:
     calc_precision left at 32 is not) and whether the arena was large enough is only known on the
     device: when either fails the kernels write nothing.  ``ok()`` reads that verdict back (it
     synchronises); ``per_tensor`` calls it and raises.  ``BatchedQuantizer.dequantize`` raises by the copy of the
-    verdict that left for the host right behind the plan, so that it does not wait for the quantize kernels."""
+    verdict that the plan leaves on the host, so that it does not wait for the quantize kernels."""
 
     _arena_bytes = None     # of `packed` when the plan was made
     # the plan's verdict: of a native call what it waits by, else (event behind the copy, the workspace's first two words in

@@ -95,7 +95,7 @@ def native():
     """The operators' host side: functions on tensors that answer an ordinary call with one call of the library, and any other
     - what has to be refused included - with None and without a launch.  Called through Python a round trip of 8192 floats took 18.6 us,
     three extension calls on 16 MB 34.8; through these 11.9 and 18.6; a batch of 69 half tensors
-    (allocation of widths, quantize, dequantize) 54 where its copies and launches called from Python took 116."""
+    (allocation of widths, quantize, dequantize) 39 where its copies and launches called from Python took 116."""
     global _NATIVE
     if _NATIVE is None:
         lib()       # the library it is linked to, of the right version
