@@ -48,10 +48,10 @@ def test_the_verdict_waits_for_earlier_work(batch):
 def test_verdicts_dropped_before_the_plan_has_run(batch):
     """Their words are not handed out again before: pinned memory taken meanwhile keeps its values."""
     made, xs, bits = batch
-    torch.cuda._sleep(LONG)
-    for _ in range(50):
+    torch.cuda._sleep(5 * LONG)
+    for _ in range(30):
         made.quantize(xs, bits, [1, 2, 3])
-    words = [torch.full((2,), -7, dtype=torch.int64).pin_memory() for _ in range(100)]
+    words = [torch.full((2,), -7, dtype=torch.int64).pin_memory() for _ in range(50)]
     assert not torch.cuda.current_stream().query()
     torch.cuda.synchronize()
     assert all(w.tolist() == [-7, -7] for w in words)
