@@ -23,10 +23,12 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cstdint>
 #include <cstring>
 #include <thread>
+#include <vector>
 
 #include "gact_hip.h"
 
@@ -373,7 +375,7 @@ bool capturing(c10::Device device) {
 
 // What the plan says, two words in pinned memory (bytes the table needs, whether all is well) that its kernel writes through to the
 // host: they are there as soon as both have changed from kUnwritten.  An event behind the plan said the same and kept the stream 6 us
-// from the next kernel, as did the one that the allocator of pinned memory recorded when the words were dropped.  calc_precision, quantize
+// from the next kernel, as does the one that the allocator of pinned memory records where it is told of the stream.  calc_precision, quantize
 // and dequantize, us, events / words: 40 bfloat16 tensors of 9 M elements together 42.6 / 35.2, 44 float 10 M 44.3 / 36.6, 69 half 16 M
 // 44.5 / 39.3, 139 float 17 M 56.4 / 50.5, 20 bfloat16 83 M 92.6 / 86.3, 45 half 117 M 117.5 / 111.3, 119 float 168 M 260 / 253,
 // 120 half 1.83 G 1329 / 1325.
@@ -382,17 +384,23 @@ constexpr const char* kVerdict = "gact verdict";
 struct Verdict {
   at::Tensor words;
   c10::hip::HIPStream stream;
-  int64_t word(int i) const { return __atomic_load_n((const int64_t*)words.const_data_ptr() + i, __ATOMIC_ACQUIRE); }
-  bool written() const { return word(0) != kUnwritten && word(1) != kUnwritten; }
 };
-// Words that a plan has still to write are not handed out again before it has
+int64_t word_of(const at::Tensor& words, int i) { return __atomic_load_n((const int64_t*)words.const_data_ptr() + i, __ATOMIC_ACQUIRE); }
+bool written(const at::Tensor& words) { return word_of(words, 0) != kUnwritten && word_of(words, 1) != kUnwritten; }
+// Words that a plan has still to write are not handed out again before it has: those of a verdict that is dropped earlier are held here
+// until a later verdict comes or goes and finds them written.  As many as there are such plans under way; guarded by the GIL; never
+// destroyed, as a plan may outlast the process's own objects.
+void hold_unwritten(const at::Tensor* dropped) {
+  static std::vector<at::Tensor>* const held = new std::vector<at::Tensor>;
+  held->erase(std::remove_if(held->begin(), held->end(), written), held->end());
+  if (dropped && !written(*dropped)) held->push_back(*dropped);
+}
 void drop_verdict(PyObject* capsule) {
   Verdict* const v = (Verdict*)PyCapsule_GetPointer(capsule, kVerdict);
   try {
-    if (!v->written())
-      (void)at::getHostAllocator(at::kCUDA)->record_event(v->words.mutable_data_ptr(), v->words.storage().data_ptr().get_context(), v->stream.unwrap());
-  } catch (...) {   // nowhere to tell: the words stay allocated
-    (void)new at::Tensor(v->words);
+    hold_unwritten(&v->words);
+  } catch (...) {   // no memory to hold them in: they stay allocated
+    (void)v->words.unsafeReleaseTensorImpl();
   }
   delete v;
 }
@@ -413,6 +421,7 @@ PyObject* batch_quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (capturing(device)) Py_RETURN_NONE;
   const at::Tensor packed = make({arena}, at::kByte, device), scale = make({groups * 4}, at::kByte, device), mn = make({groups * 4}, at::kByte, device);
   const at::Tensor table = make({b.geometry->numel()}, at::kByte, device), kept = make(b.bits->sizes(), at::kInt, device), ws = make({ws_bytes}, at::kByte, device);
+  hold_unwritten(nullptr);
   const at::Tensor words = at::empty({2}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
   const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(device.index());
   used_on(*b.geometry, stream);
@@ -426,13 +435,16 @@ PyObject* batch_quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return nullptr;
   }
   int rc;
+  bool planned;
   Py_BEGIN_ALLOW_THREADS
   rc = gact_batch_plan_args((const gact_batch_entry*)in(*b.geometry), b.x.data(), b.seeds.data(), (gact_batch_entry*)out(table),
                             (const int32_t*)in(*b.bits), (int32_t*)out(kept), b.count, blocks, arena, out(ws), word, stream.stream());
-  if (rc == GACT_OK)
+  planned = rc == GACT_OK;
+  if (planned)
     rc = gact_quantize_batched((const gact_batch_entry*)out(table), (const int32_t*)out(kept), b.count, blocks, (int)mode, (int)dtypes, out(ws),
                                out(packed), out(scale), out(mn), stream.stream());
   Py_END_ALLOW_THREADS
+  if (!planned) word[0] = word[1] = 0;   // nobody will write them
   PyObject* const tensors = rc == GACT_OK ? tuple_of({packed, scale, mn, table, kept, ws}) : nullptr;
   if (rc != GACT_OK || !tensors) {
     Py_DECREF(capsule);
@@ -456,7 +468,7 @@ PyObject* verdict_wait(PyObject*, PyObject* const* args, Py_ssize_t n) {
   }
   hipError_t rc = hipSuccess;
   Py_BEGIN_ALLOW_THREADS
-  for (int spins = 0; !v->written(); spins++) {
+  for (int spins = 0; !written(v->words); spins++) {
     if (spins < 20000) {   // about a millisecond; a plan is a few microseconds behind what the stream has to do before it
       __builtin_ia32_pause();
       continue;
@@ -474,11 +486,11 @@ PyObject* verdict_wait(PyObject*, PyObject* const* args, Py_ssize_t n) {
     break;
   }
   Py_END_ALLOW_THREADS
-  if (!v->written()) {
+  if (!written(v->words)) {
     PyErr_SetString(PyExc_RuntimeError, rc != hipSuccess ? hipGetErrorString(rc) : "gact: the plan of a batch did not run");
     return nullptr;
   }
-  return Py_BuildValue("(LL)", (long long)v->word(0), (long long)v->word(1));
+  return Py_BuildValue("(LL)", (long long)word_of(v->words, 0), (long long)word_of(v->words, 1));
   END_HANDLE_TH_ERRORS
 }
 

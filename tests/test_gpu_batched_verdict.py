@@ -59,6 +59,23 @@ def test_verdicts_dropped_before_the_plan_has_run(batch):
     assert q._planned() == q.ok()
 
 
+def test_words_of_dropped_verdicts_are_used_again(batch):
+    """Pinned memory does not grow with the batches that nobody waits for."""
+    made, xs, bits = batch
+
+    def drop():
+        torch.cuda._sleep(LONG)
+        for _ in range(30):
+            made.quantize(xs, bits, [1, 2, 3])
+        torch.cuda.synchronize()
+        made.quantize(xs, bits, [1, 2, 3])              # finds the others' words written
+        torch.cuda.synchronize()
+        return torch.cuda.host_memory_stats()["num_host_alloc"]
+
+    first = drop()
+    assert [drop() for _ in range(3)] == [first] * 3
+
+
 def test_what_is_no_verdict_is_refused():
     for args in ((), (None,), (1, 2)):
         with pytest.raises((TypeError, ValueError)):

@@ -1,0 +1,56 @@
+"""A batch's verdict on the host - the words that a plan writes, who holds them until it has - without a GPU: the operators' source
+built with one function more, which makes a verdict of words that the test fills in as the plan's kernel would."""
+import importlib.util
+import subprocess
+import sys
+
+import pytest
+import torch
+
+from conftest import ROOT
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    spec = importlib.util.spec_from_file_location("gact_build", ROOT + "/gact-icml_amd/build.py")
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    out = str(tmp_path_factory.mktemp("host") / "verdict_host.so")
+    cmd = ["-O0" if c == "-O2" else out if c == build.TORCH_OUT else ROOT + "/tests/verdict_host.cpp" if c == build.TORCH_SRC else c
+           for c in build.torch_command()]
+    subprocess.run(cmd + ["-Wl,-rpath," + build.OUT_DIR], check=True)
+    spec = importlib.util.spec_from_file_location("verdict_host", out)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
+def words(need=-1, good=-1):
+    return torch.tensor([need, good], dtype=torch.int64)
+
+
+def test_a_verdict_that_is_there(host):
+    w = words(1024, 1)
+    assert host.verdict_wait(host.verdict(w)) == (1024, 1)
+    assert w._use_count() == 1
+
+
+def test_words_of_a_dropped_verdict_are_held_until_they_are_written(host):
+    """And no longer: they went to nobody again where the memory's allocator refused to watch the stream for them."""
+    held = [words() for _ in range(20)]
+    for w in held:
+        host.verdict(w)
+    host.verdict(words(1, 1))
+    assert all(w._use_count() == 2 for w in held)
+    for w in held[:10]:
+        w[0] = 512
+    host.verdict(words(1, 1))
+    assert all(w._use_count() == 2 for w in held)       # the second word is still to come
+    for w in held[:10]:
+        w[1] = 0
+    host.verdict(words(1, 1))
+    assert [w._use_count() for w in held] == [1] * 10 + [2] * 10
+    for w in held[10:]:
+        w.fill_(0)
+    host.verdict(words(1, 1))
+    assert all(w._use_count() == 1 for w in held)
