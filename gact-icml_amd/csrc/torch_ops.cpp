@@ -22,6 +22,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <algorithm>
 #include <chrono>
@@ -107,16 +108,20 @@ void* stream_on(c10::Device device) { return c10::hip::getCurrentHIPStream(devic
 const void* in(const at::Tensor& t) { return t.const_data_ptr(); }
 void* out(const at::Tensor& t) { return t.mutable_data_ptr(); }
 
+// The GIL is released as long as this lives, and is back before an exception that leaves its scope becomes one of Python's
+struct WithoutGil {
+  PyThreadState* const state = PyEval_SaveThread();
+  WithoutGil() = default;
+  WithoutGil(const WithoutGil&) = delete;
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
 // The library's call with the GIL released and the data's device current
 template <typename F>
 int on(c10::Device device, const F& call) {
   const c10::DeviceGuard guard(device);
   void* const stream = stream_on(device);
-  int rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = call(stream);
-  Py_END_ALLOW_THREADS
-  return rc;
+  const WithoutGil released;
+  return call(stream);
 }
 
 PyObject* tuple_of(std::initializer_list<at::Tensor> tensors) {
@@ -428,33 +433,22 @@ PyObject* batch_quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   int64_t* const word = (int64_t*)out(words);
   __atomic_store_n(word, kUnwritten, __ATOMIC_RELAXED);
   __atomic_store_n(word + 1, kUnwritten, __ATOMIC_RELEASE);
-  Verdict* const verdict = new Verdict{words, stream};
-  PyObject* const capsule = PyCapsule_New(verdict, kVerdict, drop_verdict);
-  if (!capsule) {
-    delete verdict;
-    return nullptr;
-  }
+  const THPObjectPtr capsule(PyCapsule_New(new Verdict{words, stream}, kVerdict, drop_verdict));
+  if (!capsule) return nullptr;
   int rc;
-  bool planned;
-  Py_BEGIN_ALLOW_THREADS
-  rc = gact_batch_plan_args((const gact_batch_entry*)in(*b.geometry), b.x.data(), b.seeds.data(), (gact_batch_entry*)out(table),
-                            (const int32_t*)in(*b.bits), (int32_t*)out(kept), b.count, blocks, arena, out(ws), word, stream.stream());
-  planned = rc == GACT_OK;
-  if (planned)
-    rc = gact_quantize_batched((const gact_batch_entry*)out(table), (const int32_t*)out(kept), b.count, blocks, (int)mode, (int)dtypes, out(ws),
-                               out(packed), out(scale), out(mn), stream.stream());
-  Py_END_ALLOW_THREADS
-  if (!planned) word[0] = word[1] = 0;   // nobody will write them
-  PyObject* const tensors = rc == GACT_OK ? tuple_of({packed, scale, mn, table, kept, ws}) : nullptr;
-  if (rc != GACT_OK || !tensors) {
-    Py_DECREF(capsule);
-    if (rc == GACT_OK) return nullptr;
-    Py_RETURN_NONE;
+  {
+    const WithoutGil released;
+    rc = gact_batch_plan_args((const gact_batch_entry*)in(*b.geometry), b.x.data(), b.seeds.data(), (gact_batch_entry*)out(table),
+                              (const int32_t*)in(*b.bits), (int32_t*)out(kept), b.count, blocks, arena, out(ws), word, stream.stream());
+    if (rc == GACT_OK)
+      rc = gact_quantize_batched((const gact_batch_entry*)out(table), (const int32_t*)out(kept), b.count, blocks, (int)mode, (int)dtypes, out(ws),
+                                 out(packed), out(scale), out(mn), stream.stream());
+    else
+      word[0] = word[1] = 0;   // nobody will write them
   }
-  PyObject* const result = PyTuple_Pack(2, tensors, capsule);
-  Py_DECREF(tensors);
-  Py_DECREF(capsule);
-  return result;
+  if (rc != GACT_OK) Py_RETURN_NONE;
+  const THPObjectPtr tensors(tuple_of({packed, scale, mn, table, kept, ws}));
+  return tensors ? PyTuple_Pack(2, tensors.get(), capsule.get()) : nullptr;
   END_HANDLE_TH_ERRORS
 }
 
@@ -467,25 +461,26 @@ PyObject* verdict_wait(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return nullptr;
   }
   hipError_t rc = hipSuccess;
-  Py_BEGIN_ALLOW_THREADS
-  for (int spins = 0; !written(v->words); spins++) {
-    if (spins < 20000) {   // about a millisecond; a plan is a few microseconds behind what the stream has to do before it
-      __builtin_ia32_pause();
-      continue;
+  {
+    const WithoutGil released;
+    for (int spins = 0; !written(v->words); spins++) {
+      if (spins < 20000) {   // about a millisecond; a plan is a few microseconds behind what the stream has to do before it
+        __builtin_ia32_pause();
+        continue;
+      }
+      // longer work before it: look every 20 us, and end with the stream, whatever became of it
+      std::this_thread::sleep_for(std::chrono::microseconds(20));
+      const c10::DeviceGuard guard(v->stream.device());
+      rc = hipStreamQuery(v->stream.stream());
+      if (rc == hipErrorNotReady) {
+        (void)hipGetLastError();
+        rc = hipSuccess;
+        continue;
+      }
+      if (rc == hipSuccess) rc = hipStreamSynchronize(v->stream.stream());
+      break;
     }
-    // longer work before it: look every 20 us, and end with the stream, whatever became of it
-    std::this_thread::sleep_for(std::chrono::microseconds(20));
-    const c10::DeviceGuard guard(v->stream.device());
-    rc = hipStreamQuery(v->stream.stream());
-    if (rc == hipErrorNotReady) {
-      (void)hipGetLastError();
-      rc = hipSuccess;
-      continue;
-    }
-    if (rc == hipSuccess) rc = hipStreamSynchronize(v->stream.stream());
-    break;
   }
-  Py_END_ALLOW_THREADS
   if (!written(v->words)) {
     PyErr_SetString(PyExc_RuntimeError, rc != hipSuccess ? hipGetErrorString(rc) : "gact: the plan of a batch did not run");
     return nullptr;

@@ -54,3 +54,19 @@ def test_words_of_a_dropped_verdict_are_held_until_they_are_written(host):
         w.fill_(0)
     host.verdict(words(1, 1))
     assert all(w._use_count() == 1 for w in held)
+
+
+def test_an_error_while_the_gil_is_released_is_raised(host):
+    """No such GPU, or none that has such a plan: the wait ends with an exception, not with the interpreter."""
+    code = ("import importlib.util, torch\n"
+            "spec = importlib.util.spec_from_file_location('verdict_host', %r)\n"
+            "host = importlib.util.module_from_spec(spec)\n"
+            "spec.loader.exec_module(host)\n"
+            "v = host.verdict(torch.full((2,), -1, dtype=torch.int64))\n"
+            "for _ in range(2):\n"
+            "    try:\n"
+            "        host.verdict_wait(v)\n"
+            "    except RuntimeError as e:\n"
+            "        print('raised', e)\n" % host.__file__)
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert done.returncode == 0 and done.stdout.count("raised") == 2, (done.returncode, done.stdout, done.stderr[-2000:])
