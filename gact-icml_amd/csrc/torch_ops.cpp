@@ -25,7 +25,6 @@
 #include <torch/csrc/utils/object_ptr.h>
 
 #include <algorithm>
-#include <chrono>
 #include <cstdint>
 #include <cstring>
 #include <thread>
@@ -388,7 +387,12 @@ constexpr int64_t kUnwritten = -1;
 constexpr const char* kVerdict = "gact verdict";
 struct Verdict {
   at::Tensor words;
-  c10::hip::HIPStream stream;
+  c10::Device device;
+  hipStream_t stream;         // one of torch's, which live as long as the process
+  hipEvent_t event = nullptr; // behind the plan, where the stream is not torch's own and may be gone before the wait
+  ~Verdict() {
+    if (event) (void)hipEventDestroy(event);
+  }
 };
 int64_t word_of(const at::Tensor& words, int i) { return __atomic_load_n((const int64_t*)words.const_data_ptr() + i, __ATOMIC_ACQUIRE); }
 bool written(const at::Tensor& words) { return word_of(words, 0) != kUnwritten && word_of(words, 1) != kUnwritten; }
@@ -433,23 +437,54 @@ PyObject* batch_quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   int64_t* const word = (int64_t*)out(words);
   __atomic_store_n(word, kUnwritten, __ATOMIC_RELAXED);
   __atomic_store_n(word + 1, kUnwritten, __ATOMIC_RELEASE);
-  const THPObjectPtr capsule(PyCapsule_New(new Verdict{words, stream}, kVerdict, drop_verdict));
-  if (!capsule) return nullptr;
-  int rc;
+  Verdict* const verdict = new Verdict{words, device, stream.stream()};
+  const THPObjectPtr capsule(PyCapsule_New(verdict, kVerdict, drop_verdict));
+  if (!capsule) {
+    delete verdict;
+    return nullptr;
+  }
+  // torch's name for a stream that it was given is the stream's own handle
+  const bool foreign = stream.stream() != nullptr && (int64_t)(intptr_t)stream.stream() == (int64_t)stream.id();
+  int rc = GACT_ELAUNCH;
   {
     const WithoutGil released;
-    rc = gact_batch_plan_args((const gact_batch_entry*)in(*b.geometry), b.x.data(), b.seeds.data(), (gact_batch_entry*)out(table),
-                              (const int32_t*)in(*b.bits), (int32_t*)out(kept), b.count, blocks, arena, out(ws), word, stream.stream());
-    if (rc == GACT_OK)
+    if (!foreign || hipEventCreateWithFlags(&verdict->event, hipEventDisableTiming) == hipSuccess)
+      rc = gact_batch_plan_args((const gact_batch_entry*)in(*b.geometry), b.x.data(), b.seeds.data(), (gact_batch_entry*)out(table),
+                                (const int32_t*)in(*b.bits), (int32_t*)out(kept), b.count, blocks, arena, out(ws), word, stream.stream());
+    if (rc != GACT_OK)
+      word[0] = word[1] = 0;   // nobody will write them
+    else if (foreign && hipEventRecord(verdict->event, stream.stream()) != hipSuccess)
+      rc = GACT_ELAUNCH;
+    else
       rc = gact_quantize_batched((const gact_batch_entry*)out(table), (const int32_t*)out(kept), b.count, blocks, (int)mode, (int)dtypes, out(ws),
                                  out(packed), out(scale), out(mn), stream.stream());
-    else
-      word[0] = word[1] = 0;   // nobody will write them
   }
   if (rc != GACT_OK) Py_RETURN_NONE;
   const THPObjectPtr tensors(tuple_of({packed, scale, mn, table, kept, ws}));
   return tensors ? PyTuple_Pack(2, tensors.get(), capsule.get()) : nullptr;
   END_HANDLE_TH_ERRORS
+}
+
+// Until the words are written, or cannot be any more.  A plan is a few microseconds behind what the stream has to do before it, so the
+// thread keeps looking, as one that waits for an event does; after about a millisecond it lets others run in between (sleeps of
+// 20 us came back 40 us late).  From then on it looks at the stream, too, every 50 ms or so, to end with it whatever became of it.
+hipError_t wait_written(const Verdict& v) {
+  if (v.event) return hipEventSynchronize(v.event);
+  for (int64_t looks = 0; !written(v.words); looks++) {
+    if (looks < 20000) {
+      __builtin_ia32_pause();
+      continue;
+    }
+    std::this_thread::yield();
+    if ((looks - 20000) % (1 << 16) != 0) continue;
+    const c10::DeviceGuard guard(v.device);
+    // "not ready" is an error of its own to the runtime: it must not take the place of one that another call left for its caller
+    const bool unread = hipPeekAtLastError() != hipSuccess;
+    const hipError_t rc = unread ? hipStreamSynchronize(v.stream) : hipStreamQuery(v.stream);
+    if (rc != hipErrorNotReady) return rc;
+    if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();
+  }
+  return hipSuccess;
 }
 
 // verdict_wait(verdict of batch_quantize) -> (bytes the table needs, 1 where all is well), once the plan has run
@@ -460,26 +495,10 @@ PyObject* verdict_wait(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "verdict_wait takes one verdict");
     return nullptr;
   }
-  hipError_t rc = hipSuccess;
+  hipError_t rc;
   {
     const WithoutGil released;
-    for (int spins = 0; !written(v->words); spins++) {
-      if (spins < 20000) {   // about a millisecond; a plan is a few microseconds behind what the stream has to do before it
-        __builtin_ia32_pause();
-        continue;
-      }
-      // longer work before it: look every 20 us, and end with the stream, whatever became of it
-      std::this_thread::sleep_for(std::chrono::microseconds(20));
-      const c10::DeviceGuard guard(v->stream.device());
-      rc = hipStreamQuery(v->stream.stream());
-      if (rc == hipErrorNotReady) {
-        (void)hipGetLastError();
-        rc = hipSuccess;
-        continue;
-      }
-      if (rc == hipSuccess) rc = hipStreamSynchronize(v->stream.stream());
-      break;
-    }
+    rc = wait_written(*v);
   }
   if (!written(v->words)) {
     PyErr_SetString(PyExc_RuntimeError, rc != hipSuccess ? hipGetErrorString(rc) : "gact: the plan of a batch did not run");

@@ -1,5 +1,7 @@
 """The verdict of a batch's plan, which the plan's kernel writes to the host: it is there while the stream still has later work, waits for
 earlier work, and may be dropped before the plan has run."""
+import ctypes
+
 import pytest
 import torch
 
@@ -43,6 +45,38 @@ def test_the_verdict_waits_for_earlier_work(batch):
             q = made.quantize(xs, bits, [1, 2, 3])
             assert not stream.query()
             assert q._planned() == q.ok()
+
+
+def test_an_error_that_nobody_has_read_outlasts_the_wait(batch):
+    made, xs, bits = batch
+    with open("/proc/self/maps") as maps:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    torch.cuda._sleep(LONG)
+    q = made.quantize(xs, bits, [1, 2, 3])
+    left = hip.hipSetDevice(torch.cuda.device_count() + 7)
+    assert left != 0
+    planned = q._planned()
+    assert hip.hipGetLastError() == left and hip.hipGetLastError() == 0
+    assert planned == q.ok() and planned[0]
+
+
+def test_a_stream_that_torch_was_given(batch):
+    """It may be gone before the wait: an event behind the plan says when it has run."""
+    made, xs, bits = batch
+    with open("/proc/self/maps") as maps:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    handle = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(handle)) == 0
+    with torch.cuda.stream(torch.cuda.ExternalStream(handle.value)):
+        for cycles in (0, LONG):
+            torch.cuda._sleep(cycles)
+            q = made.quantize(xs, bits, [1, 2, 3])
+            torch.cuda._sleep(LONG)
+            planned = q._planned()
+            assert not torch.cuda.current_stream().query()
+            assert planned == q.ok() and planned[0]
+            made.dequantize(q)
+        made.quantize(xs, bits, [1, 2, 3])
 
 
 def test_verdicts_dropped_before_the_plan_has_run(batch):

@@ -7,8 +7,7 @@ namespace {
 PyObject* verdict(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 1 || !THPVariable_Check(args[0])) Py_RETURN_NONE;
-  const c10::Stream stream(c10::Stream::UNSAFE, c10::Device(c10::DeviceType::HIP, 0), 0);
-  Verdict* const v = new Verdict{THPVariable_Unpack(args[0]), c10::hip::HIPStream(c10::hip::HIPStream::UNCHECKED, stream)};
+  Verdict* const v = new Verdict{THPVariable_Unpack(args[0]), c10::Device(c10::kCUDA, 0), nullptr};
   return PyCapsule_New(v, kVerdict, drop_verdict);
   END_HANDLE_TH_ERRORS
 }
