@@ -2280,7 +2280,11 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
 #pragma unroll
       for (int k = 0; k < CH; k++) Elem<T>::load_chunk(reinterpret_cast<const T*>(p) + chunk_col<T>(k, i), st[r], k);
     }
-    Elem<T>::template groups_minmax<G, !std::is_same<T, bf16>::value>(st, lo, hi);   // bfloat16: nothing in it (36.1 / 36.4)
+    // bfloat16 widens its elements for two groups at 4 bit only.  With one group a step the statistics that wait for their turn leave no
+    // registers for that: 128 and up to 37 spilled, against 126 and none with ordered minima.  Widened / ordered, us: one group [40,256,56,56]
+    // 4 bit 36.8 / 30.4, 2 bit 43.4 / 32.4, 1 bit 59.0 / 39.6, [22,256,56,56] 4 bit 27.9 / 21.7, [64,256,56,56] 8 bit 41.2 / 40.5; two groups
+    // [64,256,56,56] 1 bit 41.7 / 41.4, 2 bit 36.9 / 36.8, 4 bit 36.0 / 36.0, [16,256,56,56] 4 bit 14.5 / 14.7.
+    Elem<T>::template groups_minmax<G, !std::is_same<T, bf16>::value || GS == 1 || BITS != 4>(st, lo, hi);
     {
       // one division per lane: lane r of the row takes group r % G
       const int mine = i & (G - 1);
