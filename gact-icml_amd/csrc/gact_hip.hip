@@ -3977,25 +3977,29 @@ inline StripCut strip_cut(int bits, int64_t strips, int64_t K) {
     return c;
   }
 }
-// Elements of a workgroup's tile: 48 KB, three workgroups to a CU that load and quantize by turns, where that leaves a tile 28 channels
-// and more; 64 KB, two workgroups, where that leaves it 16 (half [64,512,28,28] 4 bit 23 us against 28 with one of 144 KB), else one of
-// up to 144 KB (half [64,256,56,56] 1 bit 54 against 64; [2,256,56,56] 9 against 13); as many tiles as the workgroups that the GPU
-// holds, or a multiple of that.  64 / 48 KB, us: half 4 bit [512,512,7,7] 15.0 / 13.6, [256,512,14,14] 22.4 / 19.0, [64,512,20,20]
-// 13.2 / 12.2, [64,512,28,28] (31 channels) 21.5 / 20.4, [64,256,32,32] (24) 14.5 / 16.6; float 4 bit [2000,256,7,7] 37.1 / 32.0,
-// [128,512,14,14] 18.8 / 17.1, [64,512,20,20] (30) 20.1 / 17.0, [64,512,28,28] (15) 33.9 / 37.9.  32 KB: 2 % ahead to 19 % behind 48.
+// Elements of a workgroup's tile: as many tiles as the workgroups that the GPU holds, or a multiple of that, in whole super-groups.  Up to
+// 48 KB, three workgroups to a CU that load and quantize by turns, where that leaves a tile 21 channels in the end, and either 28 KB or
+// the CU that gets most no more than the other way; up to 64 KB, two workgroups, where those would leave 16 channels before the rounds are
+// cut (half [64,512,28,28] 4 bit 23 us against 28 with one of 144 KB), else one of up to 144 KB (half [64,256,56,56] 1 bit 54 against 64;
+// [2,256,56,56] 9 against 13).  64 / 48 KB, us, with what the latter leaves: half 4 bit [512,512,7,7] 15.0 / 13.6 (36 KB, 376 channels),
+// [256,512,14,14] 22.4 / 19.0 (36 KB, 94), [64,512,20,20] 13.2 / 12.2 (36 KB, 46), [64,512,28,28] 21.5 / 20.4 (36 KB, 23); float 4 bit
+// [2000,256,7,7] 37.1 / 32.0 (48 KB, 251), [128,512,14,14] 18.8 / 17.1 (40 KB, 52), [64,512,20,20] 20.1 / 17.0 (40 KB, 26).  Fewer
+// channels: half [64,256,32,32] 4 bit 14.5 / 16.6 (44 KB, 22), [87,256,876] 2 bit 17.6 / 19.6, 4 bit 18.0 / 19.1 (28 KB, 16).  Smaller
+// tiles: half 4 bit [311,256,49] 6.9 / 7.7 (12 KB, 635 tiles: 36 KB for some CUs, where 477 of 16 KB are 32), [2164,256,9] 8.1 / 9.1 (16 KB,
+// 609: 48, 487 of 20 KB: 40), but [273,128,179] 9.5 / 8.1 (16 KB, 764: 48, 509 of 24 KB: 48).  Over 3900 layouts of 9 to 1225 pixels
+// and 1.3 to 64 M elements at the four widths this rule is 1.0 % behind the better way on average, one of 28 channels before the rounds are
+// cut 2.2, the 64 KB everywhere 4.7; the worst is float [974,256,49] 4 bit 19.5 / 23.2 (32 KB).
 // Float at 2 bit has registers for two workgroups only (106): [2000,256,7,7] 38.0 / 39.2.
 inline int transposed_tile(size_t elem_size, int bits, int64_t numel, int64_t K) {
-  int64_t slots = 768, most = 49152 / (int64_t)elem_size;
-  if ((elem_size == 4 && bits == 2) || (most < numel / slots ? most : numel / slots) < 28 * K) {
-    slots = 512;
-    most = 65536 / (int64_t)elem_size;
-  }
-  if (slots == 512 && (most < numel / slots ? most : numel / slots) < 16 * K) {
-    slots = 256;
-    most = 147456 / (int64_t)elem_size;
-  }
-  const int64_t rounds = (numel + slots * most - 1) / (slots * most);
-  return (int)(((numel + slots * rounds - 1) / (slots * rounds) + 2047) / 2048 * 2048);
+  const auto cut = [&](int64_t slots, int64_t most) {
+    const int64_t rounds = (numel + slots * most - 1) / (slots * most);
+    return ((numel + slots * rounds - 1) / (slots * rounds) + 2047) / 2048 * 2048;
+  };
+  const auto busiest = [&](int64_t tile) { return ((numel + tile - 1) / tile + 255) / 256 * tile; };   // CU, elements
+  const int64_t size = (int64_t)elem_size, most = 65536 / size, three = cut(768, 49152 / size);
+  const int64_t two = (most < numel / 512 ? most : numel / 512) < 16 * K ? cut(256, 147456 / size) : cut(512, most);
+  const bool by_threes = !(elem_size == 4 && bits == 2) && three >= 21 * K && (three * size >= 28672 || busiest(three) <= busiest(two));
+  return (int)(by_threes ? three : two);
 }
 // Where the tile kernel gains over the contiguous copy before quantize_kernel; elsewhere the caller makes that copy.  us, in place
 // / copy and quantize:

@@ -1,20 +1,21 @@
-"""Tiles of tensors whose last but one dimension is contiguous, on either side of the sizes at which a tile holds 48 KB, 64 KB and more, at
+"""Tiles of tensors whose last but one dimension is contiguous, on either side of the sizes at which a CU holds two or three of them, at
 1 bit (a wave per super-group) and the other widths, with ends inside a group, a super-group and a tile: against the same tensor made
 contiguous first, bit for bit."""
 import pytest
 import torch
 
 from gact import ops
-from gact.cpp_extension import _abi
 
 pytestmark = pytest.mark.gpu
 
 
-# batch, channels, pixels: 28 channels a tile of 48 KB (half 24576 elements, float 12288) and 768 tiles, one more pixel or one fewer
-# element, odd numbers of pixels, tensors of less than a tile
-@pytest.mark.parametrize("shape", [(1, 8, 49), (3, 72, 50), (90, 256, 49), (11, 128, 196), (75, 256, 196), (33, 512, 784), (45, 256, 877),
-                                   (45, 256, 878), (70, 256, 438), (70, 256, 439), (37, 512, 1024), (9, 264, 2025)],
-                         ids=lambda s: "%dx%dx%d" % s)
+# batch, channels, pixels.  Tiles of 48 KB and 21 channels with one pixel fewer, or more, than they hold (half 1170, float 585), of 28 KB and
+# small ones with tensors on either side of what takes them, one round and several, less than a tile
+SHAPES = [(1, 8, 49), (3, 72, 50), (11, 128, 196), (47, 512, 784), (25, 640, 1169), (25, 640, 1171), (25, 640, 585), (25, 640, 586),
+          (155, 512, 49), (188, 512, 49), (430, 512, 49), (130, 512, 405)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "%dx%dx%d" % s)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["f32", "f16", "bf16"])
 def test_tiles_equal_the_contiguous_tensor(shape, dtype):
     b, c, k = shape
