@@ -4,6 +4,7 @@ import itertools
 import pytest
 
 import strided_rules
+import test_gpu_strip_stats
 import test_gpu_tiles
 
 SIZES = (2, 4)
@@ -50,3 +51,15 @@ def test_the_shapes_of_the_tile_test_take_both_kinds_of_tiles():
         assert any(not three and size_ != "less" for three, size_, _ in seen)
         if not (size == 4 and bits == 2):
             assert (True, "48 KB", False) in seen and any(three and many for three, _, many in seen), seen
+
+
+def test_the_shapes_of_the_strip_test_are_strips():
+    seen = set()
+    for shape, size, bits in test_gpu_strip_stats.CASES:
+        cut = strided_rules.strip_cut(size, bits, shape)
+        assert cut, (shape, size, bits)
+        seen.add((size, bits, cut[0]))
+        if cut[1] > 1:
+            seen.add((size, bits, "segments"))
+    for size, bits in itertools.product(SIZES, BITS):
+        assert {(size, bits, 1), (size, bits, "segments")} <= seen and ((size, bits, 2) in seen or bits == 8), (size, bits)
