@@ -82,13 +82,19 @@ def test_a_stream_that_torch_was_given(batch):
 def test_verdicts_dropped_before_the_plan_has_run(batch):
     """Their words are not handed out again before: pinned memory taken meanwhile keeps its values."""
     made, xs, bits = batch
-    torch.cuda._sleep(5 * LONG)
-    for _ in range(30):
-        made.quantize(xs, bits, [1, 2, 3])
-    words = [torch.full((2,), -7, dtype=torch.int64).pin_memory() for _ in range(50)]
-    assert not torch.cuda.current_stream().query()
-    torch.cuda.synchronize()
-    assert all(w.tolist() == [-7, -7] for w in words)
+    cycles = LONG
+    for _ in range(8):          # until the stream had more to do before the plans than the host took for what follows
+        torch.cuda._sleep(cycles)
+        for _ in range(30):
+            made.quantize(xs, bits, [1, 2, 3])
+        words = [torch.full((2,), -7, dtype=torch.int64).pin_memory() for _ in range(50)]
+        under_way = not torch.cuda.current_stream().query()
+        torch.cuda.synchronize()
+        assert all(w.tolist() == [-7, -7] for w in words)
+        if under_way:
+            break
+        cycles *= 2
+    assert under_way
     q = made.quantize(xs, bits, [1, 2, 3])
     assert q._planned() == q.ok()
 
