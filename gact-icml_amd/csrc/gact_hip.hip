@@ -3098,18 +3098,16 @@ mask_unpack_kernel(const int32_t* __restrict__ mask, int64_t n, uint8_t* __restr
 // argmax restates it.  Keys are doubles narrowed to float exactly as the heap's pair<float, int64> does.
 // ------------------------------------------------------------------------------------------------
 __host__ __device__ inline int prec_next_bits(int b) { return b == 32 ? 8 : b == 8 ? 4 : b == 4 ? 2 : b == 2 ? 1 : 0; }
-__host__ __device__ inline float prec_key(float C, int b, int64_t w) {
-  const int nb = prec_next_bits(b);
-  const int coeff_2 = ((1 << nb) - 1) * ((1 << nb) - 1);
+// Widths by level: 1, 2, 4, 8, 32.  The key of the step down from a level, which saves so many bits.
+__host__ __device__ inline int prec_level(int bits) { return bits == 32 ? 4 : bits == 8 ? 3 : bits == 4 ? 2 : bits == 2 ? 1 : 0; }
+__host__ __device__ inline int prec_width(int level) { return level == 4 ? 32 : 1 << level; }
+__host__ __device__ inline float prec_level_key(float C, int level, int64_t saving) {
   double obj;
-  if (b == 32) {
-    obj = -(double)C / coeff_2;
-  } else {
-    const int coeff_1 = ((1 << b) - 1) * ((1 << b) - 1);
-    obj = C * (1.0 / coeff_1 - 1.0 / coeff_2);
-  }
-  return (float)(obj / (double)(w * (int64_t)(b - nb)));
+  if (level == 4) obj = -(double)C / 65025;
+  else obj = C * (level == 3 ? 1.0 / 65025 - 1.0 / 225 : level == 2 ? 1.0 / 225 - 1.0 / 9 : 1.0 / 9 - 1.0 / 1);
+  return (float)(obj / (double)saving);
 }
+__host__ __device__ inline float prec_key(float C, int b, int64_t w) { return prec_level_key(C, prec_level(b), w * (int64_t)(b - prec_next_bits(b))); }
 __host__ __device__ inline bool prec_valid_bits(int b) { return b == 1 || b == 2 || b == 4 || b == 8 || b == 32; }
 
 #define PREC_MAX_L 4096      /* tensors the device kernel handles (LDS tables, 12 bits of a candidate's key) */
@@ -3196,16 +3194,6 @@ __device__ __forceinline__ uint32_t wave_extreme(uint32_t v) {
 }
 __device__ __forceinline__ uint64_t read_lane(uint64_t v, int lane) {
   return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
-}
-
-// Widths by level: 1, 2, 4, 8, 32.  The step down from a level and its key, prec_key with the widths' constants worked out beforehand.
-__device__ __forceinline__ int prec_level(int bits) { return bits == 32 ? 4 : bits == 8 ? 3 : bits == 4 ? 2 : bits == 2 ? 1 : 0; }
-__device__ __forceinline__ int prec_width(int level) { return level == 4 ? 32 : 1 << level; }
-__device__ __forceinline__ float prec_level_key(float C, int level, int64_t saving) {
-  double obj;
-  if (level == 4) obj = -(double)C / 65025;
-  else obj = C * (level == 3 ? 1.0 / 65025 - 1.0 / 225 : level == 2 ? 1.0 / 225 - 1.0 / 9 : 1.0 / 9 - 1.0 / 1);
-  return (float)(obj / (double)saving);
 }
 
 // The greedy pops candidates (tensor i, step s) in descending (key, i) order.  A tensor's steps have
