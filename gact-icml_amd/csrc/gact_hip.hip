@@ -1783,8 +1783,8 @@ quantize_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel, int64_
   // by dynamic LDS at five or four waves gets half of that back)
   constexpr bool PACKS = SMALL || !(std::is_same<T, f16>::value && BITS == 2 && NOISE != GACT_NOISE_REF);
   // bfloat16 widens here: ordered minima leave registers for more waves than HBM bears (67 M elements 1 bit 26.7 -> 27.5 us, 2 bit 25.7 -> 26.9,
-  // 8 M 5.58 -> 5.67), where batches (three waves on a SIMD instead of two: 686 M 562 -> 548 us a round trip, 83 M 97.5 -> 95.5) and tensors
-  // that are not contiguous (heads [64,12,512,64] 4 bit 14.1 -> 13.9) gain
+  // 8 M 5.58 -> 5.67), where batches (three waves on a SIMD instead of two: 686 M 562 -> 548 us a round trip, 83 M 97.5 -> 95.5), runs of
+  // pieces (heads [64,12,512,64] 4 bit 14.1 -> 13.9) and tiles gain; strips are apart (see there)
   constexpr bool ORDERED = !std::is_same<T, bf16>::value;
   quantize_supergroup<T, BITS, NOISE, GIVEN, SGR, STAGE, LAZY, PACKS, ORDERED>(ContiguousSource<T>{x, numel}, N, sg0, threadIdx.x & 15, packed, scale_out, mn_io, mx_io,
                                                   (uint32_t)seed, (uint32_t)(seed >> 32), noise);
@@ -2242,7 +2242,8 @@ quantize_strips_kernel(SeedArg seed_arg, const T* __restrict__ x, int64_t numel,
   // Scale and minimum stay in the row until its 16 lanes hold those of STATS steps (or the channel ends): a step's own are pieces of a
   // few bytes, one for every channel, and each costs the memory system what a whole line does.  Lane G * k + r keeps group r of
   // the step k of its turn.  Stored step by step / by turns, us: half [64,256,56,56] 1 bit 42.6 / 41.0, 2 bit 37.5 / 36.7, 4 and 8 bit
-  // equal, float 2 bit 67.5 / 66.1, 4 bit 64.0 / 62.9, [32,64,112,112] 1 bit 38.9 / 37.9; tensors of 2 M elements equal to 2 % slower.
+  // equal, float 2 bit 67.5 / 66.1, 4 bit 64.0 / 62.9, [32,64,112,112] 1 bit 38.9 / 37.9; tensors of 2 M elements and fewer equal, but
+  // float 1-2 % slower (0.05-0.1 us of 4 to 7).
   constexpr uint32_t STATS = 16 / (OWN * GS);
   Stat kept_scale = (Stat)0.0f, kept_lo = (Stat)0.0f;
 
@@ -3412,7 +3413,8 @@ __device__ __forceinline__ int batch_find(const FIRST& first_block, int L, int64
 }
 // The plan's workgroups behind the first note the tensor of 256 blocks each.  The tensors' first blocks come into LDS at once (up to
 // PLAN_LDS_L of them): a search in memory is a chain of loads, one for every bit of L, and was what the plan's launch took longest for
-// (graph replay, a launch: 3 tensors 4.0 -> 2.6 us, 45 4.0 -> 2.55, 120 4.1 -> 2.7, 190 4.3 -> 2.9, whatever the number of blocks).
+// (graph replay, a launch: 3 tensors 4.0 -> 2.6 us, 45 4.0 -> 2.55, 120 4.1 -> 2.7, 190 4.3 -> 2.9, 400 4.1 -> 3.2, 800 5.3 -> 4.6, 2048 9.2 -> 7.9,
+// from one block a tensor to 512).
 #define PLAN_THREADS 256
 #define PLAN_LDS_L 2048
 __device__ __forceinline__ void batch_plan_blocks(const gact_batch_entry* __restrict__ table, int L, int64_t total_blocks, const BatchWorkspace& ws) {

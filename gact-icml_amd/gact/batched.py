@@ -24,8 +24,8 @@ class BatchedPacked:
     The widths come from device memory, so whether they were all valid (1, 2, 4 or 8 - a tensor that
     calc_precision left at 32 is not) and whether the arena was large enough is only known on the
     device: when either fails the kernels write nothing.  ``ok()`` reads that verdict back (it
-    synchronises); ``per_tensor`` calls it and raises.  ``BatchedQuantizer.dequantize`` raises by the copy of the
-    verdict that the plan leaves on the host, so that it does not wait for the quantize kernels."""
+    synchronises); ``per_tensor`` calls it and raises.  ``BatchedQuantizer.dequantize`` raises by the verdict that the
+    plan leaves on the host, so that it does not wait for the quantize kernels."""
 
     _arena_bytes = None     # of `packed` when the plan was made
     # the plan's verdict: of a native call what it waits by, else (event behind the copy, the workspace's first two words in
@@ -52,7 +52,8 @@ class BatchedPacked:
         return bool(vals[1]), vals[0]
 
     def _planned(self):
-        """What ok() returns, as of the plan of the quantize call; waits for that plan and its copy only."""
+        """What ok() returns, as of the plan of the quantize call; waits for that plan only (and, where the call was not native, for
+        the copy of its verdict)."""
         if self._verdict is None:
             return self.ok()
         if isinstance(self._verdict, tuple):
